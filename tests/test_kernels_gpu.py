@@ -1107,6 +1107,35 @@ def test_sampling_matches_plain_chain():
     assert mismatches <= 2
 
 
+@pytest.mark.parametrize("kind", ["ties", "flat", "negative", "peaked", "masked", "steep"])
+def test_sampling_from_the_list_of_largest_and_by_descent(kind):
+    """Rows that the list of the largest elements serves and rows it leaves to the descent (a flat row's first cut holds
+    more than the list), at sizes on either side of what stays in registers: the plain chain's token for the same u.
+    Ties are drawn in order of their ids; the plain chain adds float64 probabilities, so a u within 2e-6 of a boundary
+    may fall on its other side."""
+    g = torch.Generator().manual_seed(31)
+    for vocab in (1, 3, 1000, 4097, 32768, 32772, 40001):
+        n = 6
+        z = torch.randn(n, vocab, generator=g)
+        logits = {"ties": (z * 4).round() / 2, "flat": z * 1e-3 + 1.0, "negative": z - 30.0, "peaked": z,
+                  "masked": torch.where(z > 0.5, z, torch.full_like(z, -1e30)), "steep": z * 40.0}[kind]
+        if kind == "peaked":
+            logits[:, vocab // 2] += 25.0
+        if kind == "masked":
+            logits[:, vocab - 1] = 0.25
+        for t, k, p in ((0.7, 50, 0.95), (1.0, 0, 0.9), (1.0, 1, 1.0), (0.9, 0, 1.0), (1.0, 3000, 0.5)):
+            k = min(k, vocab)
+            seeds = torch.arange(n, dtype=torch.int64) * 104729 + vocab + k
+            ctrs = torch.arange(n, dtype=torch.int32) + 11
+            got = _sample(logits, temperature=torch.full((n,), t), top_k=torch.full((n,), k, dtype=torch.int32),
+                          top_p=torch.full((n,), p), seeds=seeds, counters=ctrs)
+            for i in range(n if vocab <= 4097 else 2):
+                u = plain.uniform_for(int(seeds[i]), int(ctrs[i]))
+                if got[i] != plain.sample_token(logits[i], t, k, p, u):
+                    near = {plain.sample_token(logits[i], t, k, p, min(max(u + d, 0.0), 0.999999)) for d in (-2e-6, 2e-6)}
+                    assert got[i] in near, (kind, vocab, t, k, p, i, got[i])
+
+
 def test_sampling_top_p_reference_vectors():
     # (ref) tests/logit_processors/test_sort_processors.cpp:120-200: with logits i/40 and logit[0] = 0.5,
     # p = 0.2 keeps ids {0, 19, 18, 17}; with logit[0] = 2 it keeps {0, 19}

@@ -1164,6 +1164,44 @@ def test_sampling_distribution():
     assert (counts - probs).abs().max() < 0.015
 
 
+# ------------------------------------------------------------ experts of few rows
+@pytest.mark.parametrize("T,top,E,K,N", [(1, 1, 1, 8, 4), (1, 4, 16, 2048, 1408), (3, 2, 5, 520, 46), (16, 4, 16, 512, 30),
+                                         (7, 9, 64, 1032, 10), (64, 1, 3, 704, 24), (15, 4, 4, 1536, 18), (2, 3, 8, 2056, 12),
+                                         (17, 4, 16, 264, 20)])
+def test_experts_of_few_rows(T, top, E, K, N):
+    """Rows up to and beyond those that share an expert's weights in one workgroup (64), inner sizes on either side of its
+    vectors of 512 and beyond its registers, every activation, a strided input, all rows on one expert: both products
+    against float64.  bfloat16 results are rounded once (2^-8 of their size; the gate's exponential adds little); a
+    float32 sum of K products in any order stays within K 2^-24 of the sum of their sizes."""
+    g = torch.Generator(device=DEV).manual_seed(T * 1000 + K)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g).to(torch.bfloat16)
+    wide = rnd(T, K + 8)
+    a, w, wd, z = wide[:, :K], rnd(E, N, K) * 0.05, rnd(E, N, K) * 0.05, rnd(T * top, K)
+    wts = torch.rand(T, top, device=DEV, generator=g)
+    base = torch.randn(T, N, device=DEV, generator=g)
+    for one in (False, True):
+        ids = torch.stack([torch.randperm(E, device=DEV, generator=g)[torch.arange(top, device=DEV) % E] for _ in range(T)])
+        if one:
+            ids = torch.full_like(ids, E - 1)
+        ids = ids.to(torch.int32).contiguous()
+        rows = [(t, j, int(ids[t, j])) for t in range(T) for j in range(top)]
+        sums = torch.stack([w[e].double() @ a[t].double() for t, j, e in rows])
+        for act in (None, "relu2", "swiglu"):
+            gated = act == "swiglu"
+            out = torch.empty(T * top, N // 2 if gated else N, device=DEV, dtype=torch.bfloat16)
+            ops().table_moe_up(a, w, None, ids, out, act)
+            want = sums if act is None else sums.clamp(min=0) ** 2 if act == "relu2" else \
+                sums[:, 0::2] * torch.sigmoid(sums[:, 0::2]) * sums[:, 1::2]
+            assert ((out.double() - want).abs() <= want.abs() * 2 ** -7 + 1e-4 * want.abs().max()).all(), act
+        part = torch.stack([wd[e].double() @ z[t * top + j].double() for t, j, e in rows]).view(T, top, N)
+        size = torch.stack([wd[e].double().abs() @ z[t * top + j].double().abs() for t, j, e in rows]).view(T, top, N)
+        out = base.clone()
+        ops().table_moe_down(z, wd, None, ids, out, 0.5, out, None, wts)
+        want = base.double() + 0.5 * (wts.double()[:, :, None] * part).sum(dim=1)
+        bound = (K + top + 2) * 2.0 ** -24 * ((wts.double()[:, :, None] * size).sum(dim=1) + base.abs())
+        assert ((out.double() - want).abs() <= bound).all()
+
+
 # ------------------------------------------------------------ seeded numbers
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_seeded_numbers_are_the_same_bits_on_host_and_device(dtype):

@@ -613,3 +613,39 @@ def test_gate_and_activation_rows():
         x = torch.randn(7, 50, generator=g).cuda()
         z = ops.activate_rows(x[:, 3:43], torch.empty(7, 40, dtype=dtype, device="cuda"), "relu2")
         assert (z.double() - torch.relu(x[:, 3:43].double()) ** 2).abs().max() < (1e-6 if dtype == torch.float32 else 5e-2)
+
+
+@pytest.mark.parametrize("C,R,H", [(512, 64, 16), (512, 56, 16), (496, 64, 20), (512, 64, 3), (16, 0, 16), (256, 8, 16)])
+def test_latent_decode_splits_and_sizes(C, R, H):
+    """One token a request against contexts that end inside a key tile, from one split to more than there are key tiles,
+    with a window, sinks and a gate, at the largest sizes (whose kernel knows them) and around them: against float64 over
+    the same cached bfloat16 rows.  The probabilities and the result are rounded to bfloat16 once each (2^-8 of the
+    values summed, and of the result)."""
+    from tiny_llm_amd.kernels import ops
+    g = torch.Generator(device="cuda:0").manual_seed(C + R + H)
+    rnd = lambda *s: torch.randn(*s, device="cuda:0", generator=g)
+    bs, ctxs = 16, [1, 15, 33, 517, 700]
+    T, per = len(ctxs), -(-max(ctxs) // bs)
+    lat, rope = rnd(T * per + 1, bs, C).bfloat16(), rnd(T * per + 1, bs, max(R, 1)).bfloat16()
+    table = (torch.randperm(T * per, device="cuda:0", generator=g).to(torch.int32) + 1).view(T, per).contiguous()
+    pos = torch.tensor([c - 1 for c in ctxs], dtype=torch.int32, device="cuda:0")
+    qa, sinks, gate = rnd(T, H, C + R) * 0.3, rnd(H), rnd(T, H).bfloat16()
+    scale = (C + R) ** -0.5
+    for window in (0, 40, 512):
+        want = torch.empty(T, H, C, dtype=torch.float64, device="cuda:0")
+        size = torch.empty_like(want)
+        for t, n in enumerate(ctxs):
+            rows = table[t].long()
+            c = lat[rows].reshape(-1, C)[:n].double()
+            k = torch.cat([c, rope[rows].reshape(-1, max(R, 1))[:n, :R].double()], 1)
+            s = qa[t].double() @ k.T * scale
+            if window:
+                s[:, :max(0, n - window)] = float("-inf")
+            p = torch.softmax(torch.cat([s, sinks[:, None].double()], 1), -1)[:, :-1] * torch.sigmoid(gate[t].double())[:, None]
+            want[t], size[t] = p @ c, p @ c.abs()
+        for splits in (1, 2, 9, 64):
+            out = torch.empty(T, H, C, dtype=torch.bfloat16, device="cuda:0")
+            part = torch.full((splits * T * H * (C + 2),), float("nan"), device="cuda:0")
+            ops.latent_flash(qa, lat, rope[:, :, :R].contiguous() if R else None, table, None, pos, out, scale, gate, splits, part,
+                             window=window, sinks=sinks)
+            assert ((out.double() - want).abs() <= 2.0 ** -7 * size + 1e-6).all(), (window, splits)

@@ -182,10 +182,13 @@ class LatentAttention(Mixer):
         qa = ops.scratch("latent_qa", (T, H, KR + R), torch.float32, dev)
         q3, qa2 = q.unflatten(1, (H, D + R)), qa.view(T, H * (KR + R))
         few = T <= ops.HEAD_PRODUCT_ROWS and max(D, KR) <= ops.HEAD_PRODUCT_INNER
-        many = self.dtype == torch.bfloat16 and not few and q.stride(0) % 8 == 0     # one launch on the matrix cores
-        if few:
+        gemm = self.dtype == torch.bfloat16 and q.stride(0) % 8 == 0     # one launch on the matrix cores
+        many = gemm and not few
+        # few rows with a short inner size too: 6 rows of 16 heads, 128 -> 512, take 8.7 us by rows and 2.8 on the matrix
+        # cores; 512 -> 128, four times the round trips, 6.5 (`_project_heads` has 5.2 for it)
+        if few and not (gemm and D <= 256 and D % 8 == 0 and R % 8 == 0):
             ops.head_products(q3[:, :, :D], self.w_uk_few, qa[:, :, :KR])
-        elif many:
+        elif gemm:
             ops.head_gemm(q3[:, :, :D], self.w_uk_t, qa[:, :, :KR])
         else:
             for n in range(H):

@@ -54,6 +54,32 @@ def test_rmsnorm(dtype, hidden):
         assert rel(out, ref) < tol(dtype, 2e-6, 5e-3)
 
 
+@pytest.mark.parametrize("hidden", [4, 2044, 2048, 2052, 2050, 8192, 8193, 8196])
+def test_norms_by_vectors_and_by_elements(hidden):
+    """The norm kernels around the widths at which they change their form, rows that begin off a vector's boundary among
+    them: against float64.  Statistics and results are float32 (a few 2^-24 of the normed size, sums of `hidden` terms)."""
+    g = torch.Generator(device=DEV).manual_seed(hidden)
+    f32 = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    n, eps = 3, 1e-5
+    for off in (0, 1):
+        at = lambda t: torch.cat([t.new_zeros(off), t.reshape(-1)])[off:].view(t.shape)
+        y, x, w, b, sc = at(f32(n, hidden)), at(f32(n, hidden)), at(1 + f32(hidden) * 0.1), at(f32(hidden) * 0.1), at(f32(hidden))
+        d = 0.5 * x.double() + y.double()
+        dev = d - d.mean(1, keepdim=True)
+        want = dev / torch.sqrt(dev.square().mean(1, keepdim=True) + eps) * w.double() + b.double()
+        got = x.clone()
+        ops().layer_norm_sum(y, w, b, got, 0.5, eps)
+        assert (got.double() - want).abs().max() < 2e-6 * want.abs().max() + 1e-6
+        unit = y.double() / torch.sqrt(y.double().square().mean(1, keepdim=True) + eps) * w.double()
+        got = x.clone()
+        ops().norm_scale_add(y, w, eps, got, sc)
+        want = x.double() + unit * sc.double()
+        assert (got.double() - want).abs().max() < 2e-6 * want.abs().max() + 1e-6
+        got = torch.empty(n, hidden, device=DEV)
+        ops().rmsnorm(y, w, eps, got)
+        assert (got.double() - unit).abs().max() < 2e-6 * unit.abs().max() + 1e-6
+
+
 def test_rmsnorm_gathers_rows():
     g = torch.Generator().manual_seed(2)
     x = torch.randn(10, 96, generator=g)

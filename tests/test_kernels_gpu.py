@@ -1190,6 +1190,24 @@ def test_sampling_distribution():
     assert (counts - probs).abs().max() < 0.015
 
 
+@pytest.mark.parametrize("M,K,cols", [(1, 8, (1, 3)), (6, 2048, (2048, 64, 17, 8, 2048)), (16, 520, (40, 15, 16, 33, 1, 250)), (9, 4096, (300,))])
+def test_linear_set(M, K, cols):
+    """Products of one launch: widths around a workgroup's 16 columns, rows of inputs and outputs that lie wider apart,
+    one product and the most there may be; every result within a float32 sum's bound of float64, nothing beyond written."""
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    sets, whole = [], []
+    for n in cols:
+        out = torch.full((M, n + 5), 7.0, device=DEV)
+        whole.append(out)
+        sets.append((rnd(M, K + 16).bfloat16()[:, :K], rnd(n, K).bfloat16(), out[:, :n]))
+    ops().linear_set(sets)
+    for (a, w, out), full in zip(sets, whole):
+        want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+        assert ((out.double() - want).abs() <= K * 2.0 ** -24 * size).all()
+        assert (full[:, out.shape[1]:] == 7.0).all()
+
+
 # ------------------------------------------------------------ experts of few rows
 @pytest.mark.parametrize("T,top,E,K,N", [(1, 1, 1, 8, 4), (1, 4, 16, 2048, 1408), (3, 2, 5, 520, 46), (16, 4, 16, 512, 30),
                                          (7, 9, 64, 1032, 10), (64, 1, 3, 704, 24), (15, 4, 4, 1536, 18), (2, 3, 8, 2056, 12),

@@ -143,9 +143,18 @@ constexpr int kCh = 16;           // tokens per staged chunk
 constexpr int kCols = 8;          // value columns per wave
 constexpr int kRecWaves = 4, kRecThreads = kRecWaves * TL_WAVE, kRecCols = kRecWaves * kCols;
 constexpr int kSlices = TL_WAVE / kCols;
-// the sum over the lanes c, c + 8, ..., c + 56; every lane gets it
-__device__ __forceinline__ float sum_over_slices(float v) { return sum_over_rows(v + dpp_f32<TL_DPP_ROR8>(v)); }
-template <int DS>
+// x and y summed over the lanes c, c + 8, ..., c + 56, every lane gets both: after the step over 8 lanes the two travel
+// together, x in the even and y in the odd rows of 16 lanes.
+__device__ __forceinline__ void sum_over_slices(float& x, float& y) {
+  x += dpp_f32<TL_DPP_ROR8>(x);
+  y += dpp_f32<TL_DPP_ROR8>(y);
+  const tl_u32x2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  float a, b;
+  pair32(__uint_as_float(r[0]) + __uint_as_float(r[1]), a, b);
+  pair16(a + b, x, y);
+}
+// VEC: the head's channels are a multiple of four, and their rows begin on 16 bytes.
+template <int DS, bool VEC>
 __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vc,
     const float* __restrict__ beta, const float* __restrict__ decay, float* __restrict__ state, int64_t state_stride,
@@ -154,7 +163,8 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
   constexpr int DP = kSlices * DS;                // key channels, padded
   constexpr int PER = (kCh * DP + kRecThreads - 1) / kRecThreads;    // floats of one staged array a thread moves per chunk
   constexpr int PERV = kCh * kRecCols / kRecThreads;
-  __shared__ float ks[kCh][DP], qs[kCh][DP], gs[kCh][DP], vs[kCh][kRecCols], bs[kCh];
+  __shared__ __attribute__((aligned(16))) float ks[kCh][DP], qs[kCh][DP], gs[kCh][DP];
+  __shared__ float vs[kCh][kRecCols], bs[kCh], kqs[kCh];
   const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE;
   const int s = lane / kCols, c = wave * kCols + lane % kCols;
   const int col = blockIdx.z * kRecCols + c;
@@ -166,17 +176,24 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
 #pragma unroll
   for (int i = 0; i < DS; ++i) S[i] = (live && s * DS + i < dim) ? S_mem[(int64_t)(s * DS + i) * vdim] : 0.f;
 
-  float rk[PER], rq[PER], rg[PER], rv[PERV], rb = 0.f;
+  constexpr int V = VEC ? 4 : 1, PIECES = (PER + V - 1) / V;
+  typedef float piece __attribute__((ext_vector_type(V)));
+  piece rk[PIECES], rq[PIECES], rg[PIECES];
+  float rv[PERV], rb = 0.f;
   // element e of a staged array: token e / DP of the chunk, channel e % DP (channels beyond dim: k = q = 0, g = 1)
   auto fetch = [&](int tc) {
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int e = j * kRecThreads + tid, tt = e / DP, i = e % DP;
+    for (int j = 0; j < PIECES; ++j) {
+      const int e = (j * kRecThreads + tid) * V, tt = e / DP, i = e % DP;
       const bool ok = e < kCh * DP && tc + tt < t1 && i < dim;
       const int64_t at = ((int64_t)(tc + tt) * heads + h) * dim + i;
-      rk[j] = ok ? kn[at] : 0.f;
-      rq[j] = ok ? qn[at] : 0.f;
-      rg[j] = ok ? decay[at] : 1.f;
+      rk[j] = rq[j] = 0.f;
+      rg[j] = 1.f;
+      if (ok) {
+        rk[j] = *(const piece*)(kn + at);
+        rq[j] = *(const piece*)(qn + at);
+        rg[j] = *(const piece*)(decay + at);
+      }
     }
 #pragma unroll
     for (int j = 0; j < PERV; ++j) {
@@ -190,12 +207,12 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
   for (int tc = t0; tc < t1; tc += kCh) {
     __syncthreads();                              // the chunk before has been read
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int e = j * kRecThreads + tid;
+    for (int j = 0; j < PIECES; ++j) {
+      const int e = (j * kRecThreads + tid) * V;
       if (e < kCh * DP) {
-        (&ks[0][0])[e] = rk[j];
-        (&qs[0][0])[e] = rq[j];
-        (&gs[0][0])[e] = rg[j];
+        *(piece*)(&ks[0][0] + e) = rk[j];
+        *(piece*)(&qs[0][0] + e) = rq[j];
+        *(piece*)(&gs[0][0] + e) = rg[j];
       }
     }
 #pragma unroll
@@ -203,12 +220,24 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
     if (tid < kCh) bs[tid] = rb;
     __syncthreads();
     if (tc + kCh < t1) fetch(tc + kCh);           // on its way while this chunk is worked on
+    {                                             // k . q of the chunk's tokens, sixteen threads a token
+      static_assert(kRecThreads == 16 * kCh, "sixteen threads a token");
+      const int tt = tid / 16;
+      float kq = 0.f;
+#pragma unroll
+      for (int i = 0; i < DP / 16; ++i) kq = fmaf(ks[tt][tid % 16 + i * 16], qs[tt][tid % 16 + i * 16], kq);
+      kq = group_sum<16>(kq);
+      if (tid % 16 == 0) kqs[tt] = kq;
+    }
+    __syncthreads();
     const int n = min(kCh, t1 - tc);
-    // With S' = diag(g) S:  o = (S' + k u^T)^T q = S'^T q + u (k . q).  Both sums over S' and k . q are
+    // With S' = diag(g) S:  o = (S' + k u^T)^T q = S'^T q + u (k . q).  Both sums over S' are
     // taken in ONE pass (in four independent parts) and meet in one round of exchanges between the
     // slices; the update of S hangs off it.  A token's operands are read from LDS while the token before
-    // it is worked on (two register sets, the loop goes two tokens at a time).
-    auto load = [&](int tt, float* k, float* q, float* g, float& v, float& bt) {
+    // it is worked on (two register sets, the loop goes two tokens at a time).  What a token costs is what its
+    // waves issue (two a SIMD): with k . q in every wave and the sums exchanged one by one 801 tokens (five shorter prompts beside them) took 364 us,
+    // now 319; 16 slices of half the rows, 4 columns a wave: 294, but 18 -> 26 us for eight prompts of 13 tokens.
+    auto load = [&](int tt, float* k, float* q, float* g, float& v, float& bt, float& kq) {
 #pragma unroll
       for (int i = 0; i < DS; ++i) {
         k[i] = ks[tt][s * DS + i];
@@ -217,31 +246,30 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
       }
       v = vs[tt][c];
       bt = bs[tt];
+      kq = kqs[tt];
     };
-    auto step = [&](int tt, const float* k, const float* q, const float* g, float v, float bt) {
-      float sk[4] = {0.f, 0.f, 0.f, 0.f}, sq[4] = {0.f, 0.f, 0.f, 0.f}, kq[4] = {0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int tt, const float* k, const float* q, const float* g, float v, float bt, float kq) {
+      float sk[4] = {0.f, 0.f, 0.f, 0.f}, sq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < DS; ++i) {
         S[i] *= g[i];
         sk[i & 3] = fmaf(S[i], k[i], sk[i & 3]);
         sq[i & 3] = fmaf(S[i], q[i], sq[i & 3]);
-        kq[i & 3] = fmaf(k[i], q[i], kq[i & 3]);
       }
-      const float sk_all = sum_over_slices((sk[0] + sk[1]) + (sk[2] + sk[3]));
-      const float sq_all = sum_over_slices((sq[0] + sq[1]) + (sq[2] + sq[3]));
-      const float kq_all = sum_over_slices((kq[0] + kq[1]) + (kq[2] + kq[3]));
+      float sk_all = (sk[0] + sk[1]) + (sk[2] + sk[3]), sq_all = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+      sum_over_slices(sk_all, sq_all);
       const float u = bt * (v - sk_all);
 #pragma unroll
       for (int i = 0; i < DS; ++i) S[i] = fmaf(k[i], u, S[i]);
-      if (s == 0 && live) out[((int64_t)(tc + tt) * heads + h) * vdim + col] = fmaf(u, kq_all, sq_all);
+      if (s == 0 && live) out[((int64_t)(tc + tt) * heads + h) * vdim + col] = fmaf(u, kq, sq_all);
     };
-    float ka[DS], qa2[DS], ga[DS], kb[DS], qb[DS], gb[DS], va, ba, vb, bb;
-    load(0, ka, qa2, ga, va, ba);
+    float ka[DS], qa2[DS], ga[DS], kb[DS], qb[DS], gb[DS], va, ba, vb, bb, da, db;
+    load(0, ka, qa2, ga, va, ba, da);
     for (int tt = 0; tt < n; tt += 2) {
-      load(min(tt + 1, kCh - 1), kb, qb, gb, vb, bb);
-      step(tt, ka, qa2, ga, va, ba);
-      load(min(tt + 2, kCh - 1), ka, qa2, ga, va, ba);
-      if (tt + 1 < n) step(tt + 1, kb, qb, gb, vb, bb);
+      load(min(tt + 1, kCh - 1), kb, qb, gb, vb, bb, db);
+      step(tt, ka, qa2, ga, va, ba, da);
+      load(min(tt + 2, kCh - 1), ka, qa2, ga, va, ba, da);
+      if (tt + 1 < n) step(tt + 1, kb, qb, gb, vb, bb, db);
     }
   }
 #pragma unroll
@@ -495,9 +523,10 @@ int tl_delta_recurrence(const float* qn, const float* kn, const float* vc, const
   if (heads <= 0 || heads > 65535 || dim <= 0 || dim > kMaxDim || vdim <= 0 || (vdim + kRecCols - 1) / kRecCols > 65535)
     return TL_ERR_ARG;
   dim3 g(n_requests, heads, (vdim + kRecCols - 1) / kRecCols), b(kRecThreads);
+  const bool vec = dim % 4 == 0 && !(((uintptr_t)qn | (uintptr_t)kn | (uintptr_t)decay) & 15);
 #define TL_REC(DS)                                                                                                   \
-  hipLaunchKernelGGL(delta_recurrence_kernel<DS>, g, b, 0, stream, qn, kn, vc, beta, decay, state, state_stride,     \
-                     cu_seqlens, state_slots, out, heads, dim, vdim)
+  hipLaunchKernelGGL((vec ? delta_recurrence_kernel<DS, true> : delta_recurrence_kernel<DS, false>), g, b, 0, stream, \
+                     qn, kn, vc, beta, decay, state, state_stride, cu_seqlens, state_slots, out, heads, dim, vdim)
   if (dim <= 16) TL_REC(2);
   else if (dim <= 32) TL_REC(4);
   else if (dim <= 64) TL_REC(8);

@@ -449,7 +449,8 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const float* 
 // Tiles of BM x BN outputs, k in steps of 64, WM x WN wave64, each owning (BM/WM) x (BN/WN)
 // outputs as 32x32x16 MFMA tiles.  Operand tiles go global -> registers -> LDS; LDS is
 // double-buffered so an iteration needs one barrier, and the global loads of the next k step are
-// in flight while the current one is multiplied.
+// in flight while the current one is multiplied.  Or they go straight into LDS, three or four buffers in turn
+// (launch_gemm_bf16 says where), and the loads of the next two or three k steps are in flight.
 //
 // Tile shapes: 256 x 256 (eight waves of 128 x 64), 256 x 128, 128 x 128 and 64 x 128.  The larger
 // the tile, the fewer operand bytes and LDS reads per flop and the higher the rate on a full chip;
@@ -462,6 +463,20 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const float* 
 constexpr int B_BK = 64;
 constexpr int B_LD = B_BK + 8;  // LDS row stride in elements: 144 bytes, keeps 16-byte alignment
 constexpr int B_XCDS = 8;
+
+// 16 bytes a lane from a buffer straight into LDS, side by side from `dst` on (the same for the whole wave).  Written
+// as one instruction block: given the builtin, the compiler waits for every load on its way ahead of each LDS read,
+// whichever buffer it reads.  Whoever reads the data waits for it first (tl_wait_loads, then a barrier).
+typedef int tl_rsrc_words __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void tl_load_to_lds(tl_rsrc_words buf, void* dst, int voffset, int soffset) {
+  const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(__attribute__((address_space(3))) void*)dst);
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(at), "v"(voffset), "s"(buf), "s"(soffset)
+               : "memory", "m0");
+}
+template <int LEFT>       // until at most LEFT of the wave's loads are still on their way
+__device__ __forceinline__ void tl_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
 
 // What the epilogue of the tiled kernel does to a row besides the product: a factor per row
 // (`row_scale`), or a norm handed from product to product as the few-row kernel does it (see
@@ -497,13 +512,20 @@ struct GemmShape {
   static constexpr int TM = BM / WM, TN = BN / WN;        // a wave's outputs
   static constexpr int MI = TM / 32, NJ = TN / 32;        // as 32 x 32 MFMA tiles
   static constexpr int AC = BM * (B_BK / 8) / THREADS, WC = BN * (B_BK / 8) / THREADS;
-  static constexpr size_t SMEM = (size_t)2 * (BM + BN) * B_LD * sizeof(bf16_t);      // the operand tiles
-  static constexpr size_t SMEM_ALL = SMEM + BM * sizeof(float);                      // and a factor per row behind them
+  // operand tiles in LDS: two, or, straight from memory, as many as make three in flight beside the one in use
+  static constexpr int BUFS = BM + BN > 384 ? 2 : BM + BN > 256 ? 3 : 4;
+  static constexpr size_t smem(bool direct) {
+    return direct ? (size_t)BUFS * (BM + BN) * B_BK * sizeof(bf16_t) : (size_t)2 * (BM + BN) * B_LD * sizeof(bf16_t);
+  }
+  static constexpr size_t smem_all(bool direct) { return smem(direct) + BM * sizeof(float); }     // and a factor per row
   static_assert(TM % 32 == 0 && TN % 32 == 0 && AC >= 1 && WC >= 1, "tile does not divide");
 };
 
 // K must be a multiple of 8 (16-byte chunks of bf16 never straddle the end).
-template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, bool FULL>
+// How operand tiles get into LDS: through registers, zeros beyond the end of a row (kTail); through registers, the inner
+// size a multiple of the k step (kWhole); likewise, but straight from memory (kDirect).
+constexpr int kTail = 0, kWhole = 1, kDirect = 2;
+template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, int MODE>
 __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16_t* __restrict__ a,
                                                                       const bf16_t* __restrict__ w,
                                                                       TO* __restrict__ out,
@@ -512,9 +534,12 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
                                                                       int64_t lda, int64_t ldo, int k_per_split) {
   using S = GemmShape<BM, BN, WM, WN>;
   constexpr int MI = S::MI, NJ = S::NJ, THREADS = S::THREADS;
+  constexpr bool DIRECT = MODE == kDirect;
+  constexpr int LD = DIRECT ? B_BK : B_LD;              // row stride of a staged tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  bf16_t* As = (bf16_t*)smem_raw;                       // [2][BM][B_LD]
-  bf16_t* Ws = As + 2 * BM * B_LD;                      // [2][BN][B_LD]
+  constexpr int BUFS = DIRECT ? S::BUFS : 2;
+  bf16_t* As = (bf16_t*)smem_raw;                       // [BUFS][BM][LD]
+  bf16_t* Ws = As + BUFS * BM * LD;                     // [BUFS][BN][LD]
   const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = tid / TL_WAVE;
   const int wm = wave / WN, wn = wave % WN;
   // k_per_split > 0 (a multiple of the k step): the inner size is split over workgroups, each
@@ -547,7 +572,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   // A norm handed over: the factors of this tile's rows are worked out once, here, where the loads
   // hide behind the main loop (16 threads share a row's parts out), and wait in LDS for the
   // epilogue; the barriers of the main loop lie in between.
-  float* row_factor = (float*)(smem_raw + S::SMEM);      // [BM]
+  float* row_factor = (float*)(smem_raw + S::smem(DIRECT));      // [BM]
   if (nm.in_sumsq) {      // uniform
     for (int r = tid / 16; r < BM; r += THREADS / 16) {
       const int64_t at = (int64_t)min(m0 + r, M - 1) * nm.in_parts;
@@ -565,14 +590,25 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   // without a branch.  (A piece beyond K within a row is zeroed when it is written to LDS.)
   constexpr int PIECES = S::AC + S::WC;
   bf16x8 stage[PIECES];
-  const int prow = tid / 8, pk = (tid % 8) * 8;            // this thread's row within a pass, k offset
+  const int prow = tid / 8;                                // this thread's row within a pass
+  // and its k offset.  DIRECT: the wave's 64 pieces land in LDS side by side, 8 rows of 8, so a row cannot be padded;
+  // piece c of row r holds the k of piece c ^ (r / 2 % 8) instead, and 16 rows at one k then touch every bank once.
+  const int pk = DIRECT ? ((tid % 8) ^ (prow / 2 % 8)) * 8 : (tid % 8) * 8;
   constexpr int PASS = THREADS / 8;                        // rows per pass
   auto tile_buffer = [](const bf16_t* first_row, int rows, int64_t ld, int K_) {
     const int64_t bytes = rows > 0 ? ((int64_t)(rows - 1) * ld + K_) * 2 : 0;
     return __builtin_amdgcn_make_buffer_rsrc((void*)first_row, 0, (int)(bytes < 0x7fffffff ? bytes : 0x7fffffff), 0x00020000);
   };
+  auto buffer_words = [](const bf16_t* first_row, int rows, int64_t ld, int K_) {      // the same as four words
+    const int64_t bytes = rows > 0 ? ((int64_t)(rows - 1) * ld + K_) * 2 : 0;
+    const uint64_t at = (uint64_t)first_row;
+    return tl_rsrc_words{(int)(uint32_t)at, (int)(uint32_t)(at >> 32) & 0xffff, (int)(bytes < 0x7fffffff ? bytes : 0x7fffffff),
+                         0x00020000};
+  };
   const __amdgpu_buffer_rsrc_t buf_a = tile_buffer(a + (int64_t)m0 * lda, min(M - m0, BM), lda, K);
   const __amdgpu_buffer_rsrc_t buf_w = tile_buffer(w + (int64_t)n0 * K, min(N - n0, BN), K, K);
+  const tl_rsrc_words words_a = buffer_words(a + (int64_t)m0 * lda, min(M - m0, BM), lda, K);
+  const tl_rsrc_words words_w = buffer_words(w + (int64_t)n0 * K, min(N - n0, BN), K, K);
   int piece_off[PIECES];                                   // bytes from the tile's first row
 #pragma unroll
   for (int p = 0; p < PIECES; ++p) {
@@ -586,25 +622,34 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
         tl_i32x4, __builtin_amdgcn_raw_buffer_load_b128(p < S::AC ? buf_a : buf_w, piece_off[p], k0 * 2, 0));
     stage[p] = __builtin_bit_cast(bf16x8, v);
   };
-  // FULL: K is a multiple of the k step (and M, N of the tile), so nothing is zeroed
   auto lds_write1 = [&](int buf, int k0, int p) {
     const bool is_a = p < S::AC;
     const int r = (is_a ? p : p - S::AC) * PASS + prow;
-    const bool ok = FULL || k0 + pk < K;
+    const bool ok = MODE != kTail || k0 + pk < K;
     bf16x8 z = {};
-    bf16_t* dst = is_a ? As + (buf * BM + r) * B_LD + pk : Ws + (buf * BN + r) * B_LD + pk;
+    bf16_t* dst = is_a ? As + (buf * BM + r) * LD + pk : Ws + (buf * BN + r) * LD + pk;
     *(bf16x8*)dst = ok ? stage[p] : z;
+  };
+  // DIRECT: piece p of the k step at k0, straight into a buffer.
+  auto direct1 = [&](int buf, int k0, int p) {
+    const bool is_a = p < S::AC;
+    const int r = (is_a ? p : p - S::AC) * PASS + wave * 8;
+    bf16_t* dst = is_a ? As + (buf * BM + r) * LD : Ws + (buf * BN + r) * LD;
+    tl_load_to_lds(is_a ? words_a : words_w, dst, piece_off[p], k0 * 2);
   };
   // MFMA operands of one k16 step: NJ weight pieces, then MI activation pieces, in the order of use
   struct Frag {
     bf16x8 w[NJ], a[MI];
   };
   constexpr int FRAG = NJ + MI;
-  const bf16_t* ra = As + (wm * S::TM + lane % 32) * B_LD + (lane / 32) * 8;
-  const bf16_t* rw = Ws + (wn * S::TN + lane % 32) * B_LD + (lane / 32) * 8;
+  const bf16_t* ra = As + (wm * S::TM + lane % 32) * LD;
+  const bf16_t* rw = Ws + (wn * S::TN + lane % 32) * LD;
+  int kcol[4];                                             // this lane's place in a row for every k16 step
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) kcol[ks] = DIRECT ? ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8 : ks * 16 + (lane / 32) * 8;
   auto lds_read1 = [&](Frag& f, int buf, int ks, int p) {
-    if (p < NJ) f.w[p] = *(const bf16x8*)(rw + (buf * BN + p * 32) * B_LD + ks * 16);
-    else f.a[p - NJ] = *(const bf16x8*)(ra + (buf * BM + (p - NJ) * 32) * B_LD + ks * 16);
+    if (p < NJ) f.w[p] = *(const bf16x8*)(rw + (buf * BN + p * 32) * LD + kcol[ks]);
+    else f.a[p - NJ] = *(const bf16x8*)(ra + (buf * BM + (p - NJ) * 32) * LD + kcol[ks]);
   };
   // The MFMAs of one k16 step, with memory operations issued between them: slot(n) comes after the
   // n-th MFMA.  The result tile is transposed (rows = n, columns = m) so that a lane holds four
@@ -636,15 +681,29 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   // kt + 2 are issued right after; the last k16 step of a tile is multiplied after the barrier,
   // while the first fragments of the next tile are on their way.
   const int nk = (kend - kbase + B_BK - 1) / B_BK;
+  if constexpr (DIRECT) {
 #pragma unroll
-  for (int p = 0; p < PIECES; ++p) gload1(kbase, p);
+    for (int p = 0; p < PIECES; ++p) direct1(0, kbase, p);
 #pragma unroll
-  for (int p = 0; p < PIECES; ++p) lds_write1(0, kbase, p);
-  if (nk > 1) {
+    for (int b = 1; b < BUFS; ++b)
+      if (b < nk) {
 #pragma unroll
-    for (int p = 0; p < PIECES; ++p) gload1(kbase + B_BK, p);
+        for (int p = 0; p < PIECES; ++p) direct1(b, kbase + b * B_BK, p);
+      }
+    if (nk >= BUFS) tl_wait_loads<(BUFS - 1) * PIECES>();
+    else tl_wait_loads<0>();
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) gload1(kbase, p);
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) lds_write1(0, kbase, p);
+    if (nk > 1) {
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p) gload1(kbase + B_BK, p);
+    }
+    __syncthreads();
   }
-  __syncthreads();
   Frag f0, f1;
 #pragma unroll
   for (int p = 0; p < FRAG; ++p) lds_read1(f0, 0, 0, p);
@@ -652,32 +711,32 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   constexpr int HALF = SLOTS / 2;
   auto step = [&](auto has_next, auto has_next2, int kt) {
     constexpr bool NX = decltype(has_next)::value, NX2 = decltype(has_next2)::value;
-    const int cur = kt & 1, nxt = cur ^ 1, k1 = kbase + (kt + 1) * B_BK, k2 = kbase + (kt + 2) * B_BK;
+    const int cur = DIRECT ? kt % BUFS : kt & 1, nxt = DIRECT ? (kt + 1) % BUFS : cur ^ 1;
+    const int k1 = kbase + (kt + 1) * B_BK, k2 = kbase + (kt + (DIRECT ? BUFS : 2)) * B_BK;
     group(f0, [&](int n) { spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f1, cur, 1, p); }); });
     group(f1, [&](int n) {
       spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f0, cur, 2, p); });
-      if constexpr (NX)
+      if constexpr (NX && !DIRECT)
         if (n >= SLOTS - HALF) spread(n - (SLOTS - HALF), PIECES / 2, HALF, [&](int p) { lds_write1(nxt, k1, p); });
     });
     group(f0, [&](int n) {
       spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f1, cur, 3, p); });
-      if constexpr (NX)
+      if constexpr (NX && !DIRECT)
         if (n < HALF) spread(n, PIECES - PIECES / 2, HALF, [&](int p) { lds_write1(nxt, k1, PIECES / 2 + p); });
-      if constexpr (NX2)
+      if constexpr (NX2 && !DIRECT)
         if (n >= SLOTS - HALF) spread(n - (SLOTS - HALF), PIECES, HALF, [&](int p) { gload1(k2, p); });
     });
+    if constexpr (DIRECT && NX) tl_wait_loads<NX2 ? (BUFS - 2) * PIECES : 0>();      // the next tile has arrived
     __syncthreads();
     group(f1, [&](int n) {
       if constexpr (NX) spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f0, nxt, 0, p); });
+      if constexpr (DIRECT && NX2) spread(n, PIECES, SLOTS, [&](int p) { direct1(cur, k2, p); });     // cur has been read
     });
   };
   {
     int kt = 0;
-    for (; kt + 2 < nk; ++kt) step(std::true_type{}, std::true_type{}, kt);
-    if (kt + 1 < nk) {
-      step(std::true_type{}, std::false_type{}, kt);
-      ++kt;
-    }
+    for (; kt + BUFS < nk; ++kt) step(std::true_type{}, std::true_type{}, kt);
+    for (; kt + 1 < nk; ++kt) step(std::true_type{}, std::false_type{}, kt);
     step(std::false_type{}, std::false_type{}, kt);
   }
 
@@ -688,11 +747,22 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   // row: 16 lanes then cover 256 contiguous bytes of one row, and so do the residual reads.
   static_assert(S::TN == 64, "the epilogue stages 64 columns per wave");
   constexpr int E_LD = 68;                 // floats per staged row: 16-byte aligned, conflict-free
-  static_assert((size_t)WM * WN * 32 * E_LD * sizeof(float) <= S::SMEM, "staging areas fit the tile buffers");
+  static_assert((size_t)WM * WN * 32 * E_LD * sizeof(float) <= S::smem(DIRECT), "staging areas fit the tile buffers");
   float* cstage = (float*)smem_raw + wave * (32 * E_LD);
   const bool vec_ok = (N % 4 == 0) && (ldo % 4 == 0);
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
+    // the residual of these 32 rows, requested together: out may be the residual, so the compiler asks for a piece only
+    // when the one before is stored (3,288 rows, 2,048 x 2,048: 43.9 -> 42.0 us, 5,632 inner: 96.0 -> 90.2)
+    f32x4 res[8];
+    if (!SWIGLU && residual && vec_ok) {
+#pragma unroll
+      for (int c8 = 0; c8 < 8; ++c8) {
+        const int c = c8 * TL_WAVE + lane;
+        const int m = m0 + wm * S::TM + i * 32 + c / 16, n = n0 + wn * S::TN + (c % 16) * 4;
+        res[c8] = m < M && n < N ? *(const f32x4*)(residual + (int64_t)m * ldo + n) : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -734,8 +804,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
       const int64_t o = (int64_t)m * ldo + n;
       if (vec_ok) {  // n + 3 < N because n and N are both multiples of 4
         if (residual) {
-          const f32x4 rv = *(const f32x4*)(residual + o);
-          v[0] += rv[0]; v[1] += rv[1]; v[2] += rv[2]; v[3] += rv[3];
+          v[0] += res[c8][0]; v[1] += res[c8][1]; v[2] += res[c8][2]; v[3] += res[c8][3];
         }
         if constexpr (sizeof(TO) == 4) {
           f32x4 sv = {v[0], v[1], v[2], v[3]};
@@ -780,15 +849,15 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   }
 }
 
-template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, bool FULL>
-static int launch_gemm_bf16_full(const bf16_t* a, const bf16_t* w, TO* out, const float* residual,
+template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, int MODE>
+static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, const float* residual,
                                  const TileNorm& row_scale, int M, int N, int K, int64_t lda, int64_t ldo,
                                  int k_per_split, hipStream_t stream) {
   using S = GemmShape<BM, BN, WM, WN>;
   static bool configured = false;
   if (!configured) {
-    if (hipFuncSetAttribute((const void*)gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, FULL>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::SMEM_ALL) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, MODE>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::smem_all(MODE == kDirect)) != hipSuccess)
       return TL_ERR_LAUNCH;
     configured = true;
   }
@@ -800,8 +869,8 @@ static int launch_gemm_bf16_full(const bf16_t* a, const bf16_t* w, TO* out, cons
   const int64_t total = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
   const int64_t grid = (total + B_XCDS - 1) / B_XCDS * B_XCDS;
   if (grid > 0x7fffffff) return TL_ERR_ARG;
-  hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, FULL>), dim3((unsigned)grid), dim3(S::THREADS),
-                     S::SMEM_ALL, stream, a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split);
+  hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, MODE>), dim3((unsigned)grid), dim3(S::THREADS),
+                     S::smem_all(MODE == kDirect), stream, a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split);
   static_assert(sizeof(TileNorm) <= 96, "passed by value");
   return TL_OK;
 }
@@ -809,11 +878,24 @@ static int launch_gemm_bf16_full(const bf16_t* a, const bf16_t* w, TO* out, cons
 template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU>
 static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const float* residual, const TileNorm& row_scale,
                             int M, int N, int K, int64_t lda, int64_t ldo, int k_per_split, hipStream_t stream) {
-  if (M % BM == 0 && N % BN == 0 && K % B_BK == 0)
-    return launch_gemm_bf16_full<BM, BN, WM, WN, TO, SWIGLU, true>(a, w, out, residual, row_scale, M, N, K, lda, ldo,
-                                                                   k_per_split, stream);
-  return launch_gemm_bf16_full<BM, BN, WM, WN, TO, SWIGLU, false>(a, w, out, residual, row_scale, M, N, K, lda, ldo,
-                                                                  k_per_split, stream);
+#define TL_GEMM(MODE)                                                                                                  \
+  launch_gemm_bf16_mode<BM, BN, WM, WN, TO, SWIGLU, MODE>(a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split, \
+                                                          stream)
+  if (K % B_BK) return TL_GEMM(kTail);
+  if constexpr (BM + BN == 384 || BM + BN == 256) {
+    const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
+    const int64_t wgs = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
+    // Straight into LDS where a unit has one workgroup at a time anyway, so that the tiles on their way cost none: the
+    // 128 x 128 tile with at most 256 of them (512 to 2,048 rows of 2,048 to 5,632 inner: 4 to 11 % faster, without
+    // this 60.2 and with it 53.8 us at 1,944 rows of 5,632; beyond, two workgroups a unit are worth more), and the
+    // 256 x 128 tile for float32 results (o and down of prompts: 1 to 5 %; bfloat16 results, whose products run beside
+    // the largest tile's on fewer workgroups, lose 1 to 2 %).  The 256 x 256 tile has room for two buffers only, one on
+    // its way: 8,192^3 takes 1,138 us so and 927 through registers.  Four waves of twice the outputs, which read a
+    // third less from LDS, are 2 to 10 % slower with either tile.
+    if (BM + BN == 384 ? sizeof(TO) == 4 : wgs <= 256) return TL_GEMM(kDirect);
+  }
+  return TL_GEMM(kWhole);
+#undef TL_GEMM
 }
 
 // Which tile: the one with the smallest estimated time.  A compute unit works through

@@ -326,6 +326,29 @@ def test_linear_two_part_launch(M, K, N):
     assert rel(two, one.double()) < 1e-6
 
 
+@pytest.mark.parametrize("tile", [1, 2, 3])
+@pytest.mark.parametrize("M,N", [(1, 128), (129, 132), (300, 260), (257, 130), (2049, 2052)])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 328])
+def test_linear_operand_tiles(tile, M, N, K):
+    """Operand tiles that go straight into LDS or through registers: inner sizes of fewer k steps than there are buffers,
+    as many and more, and one that ends within a step; rows and columns that end within a tile; few and many tiles; an
+    operand within wider rows, and the residual that is overwritten."""
+    g = torch.Generator().manual_seed(M + K + N)
+    wide = torch.randn(M, K + 72, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
+    res = torch.randn(M, N, generator=g)
+    a = wide[:, :K]
+    ref = a.double() @ w.double().T
+    # float32 sums of K exact products in any order, the last addition included: (K + 1) roundings of the absolute sum
+    bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + res.double().abs())
+    x = res.clone().to(DEV)
+    ops().linear(wide.to(DEV)[:, :K], w.to(DEV), x, x, tile=tile)
+    assert ((x.cpu().double() - (ref + res.double())).abs() <= bound).all()
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops().linear(wide.to(DEV)[:, :K], w.to(DEV), y, tile=tile)
+    assert ((y.cpu().double() - ref).abs() <= bound + 2.0 ** -8 * (ref.abs() + bound)).all()
+
+
 @pytest.mark.parametrize("M", [17, 50, 64, 65, 200, 512])
 @pytest.mark.parametrize("K,N", [(5632, 2048), (2048, 4100), (1096, 518), (2048, 2046), (256, 2560), (4096, 6144)])
 def test_linear_split_k(M, K, N):

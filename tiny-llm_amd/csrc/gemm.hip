@@ -592,7 +592,8 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   bf16x8 stage[PIECES];
   const int prow = tid / 8;                                // this thread's row within a pass
   // and its k offset.  DIRECT: the wave's 64 pieces land in LDS side by side, 8 rows of 8, so a row cannot be padded;
-  // piece c of row r holds the k of piece c ^ (r / 2 % 8) instead, and 16 rows at one k then touch every bank once.
+  // piece c of row r holds the k of piece c ^ (r / 2 % 8) instead, and 16 rows at one k then touch every bank once
+  // (conflicts are 0.7 % of the cycles LDS works, 1,944 rows, 2,048 x 5,632, and as many with padded rows: the epilogue's).
   const int pk = DIRECT ? ((tid % 8) ^ (prow / 2 % 8)) * 8 : (tid % 8) * 8;
   constexpr int PASS = THREADS / 8;                        // rows per pass
   auto tile_buffer = [](const bf16_t* first_row, int rows, int64_t ld, int K_) {
@@ -753,7 +754,8 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     // the residual of these 32 rows, requested together: out may be the residual, so the compiler asks for a piece only
-    // when the one before is stored (3,288 rows, 2,048 x 2,048: 43.9 -> 42.0 us, 5,632 inner: 96.0 -> 90.2)
+    // when the one before is stored (with the zeroing of kTail left out of ragged rows, 3,288 rows through registers,
+    // 2,048 x 2,048: 43.9 -> 42.0 us, 5,632 inner: 96.0 -> 90.2)
     f32x4 res[8];
     if (!SWIGLU && residual && vec_ok) {
 #pragma unroll
@@ -886,12 +888,12 @@ static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const flo
     const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
     const int64_t wgs = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
     // Straight into LDS where a unit has one workgroup at a time anyway, so that the tiles on their way cost none: the
-    // 128 x 128 tile with at most 256 of them (512 to 2,048 rows of 2,048 to 5,632 inner: 4 to 11 % faster, without
-    // this 60.2 and with it 53.8 us at 1,944 rows of 5,632; beyond, two workgroups a unit are worth more), and the
-    // 256 x 128 tile for float32 results (o and down of prompts: 1 to 5 %; bfloat16 results, whose products run beside
-    // the largest tile's on fewer workgroups, lose 1 to 2 %).  The 256 x 256 tile has room for two buffers only, one on
-    // its way: 8,192^3 takes 1,138 us so and 927 through registers.  Four waves of twice the outputs, which read a
-    // third less from LDS, are 2 to 10 % slower with either tile.
+    // 128 x 128 tile with at most 256 of them (1,944 rows, 2,048 x 5,632: 58.6 us through registers, 55.2 so; 1,536 rows:
+    // 53.4 and 49.4; beyond, two workgroups a unit are worth more), and the 256 x 128 tile for float32 results (2,048
+    // rows, 4,096 x 4,096: 74.3 and 73.5; 3,000 rows, 4,096 x 14,336: 323.9 and 316.1).  With bfloat16 results that tile
+    // loses (2,048 rows, 6,144 x 4,096: 98.3 and 100.1).  The 256 x 256 tile has room for two buffers only, one on
+    // its way: 8,192^3 takes 1,138 us so and 927 through registers.  Four waves of twice the outputs, which read less
+    // from LDS, lose with float32 results (1,944 rows, 2,048 x 5,632: 59.0; 3,288 rows: 88.2 -> 100.6).
     if (BM + BN == 384 ? sizeof(TO) == 4 : wgs <= 256) return TL_GEMM(kDirect);
   }
   return TL_GEMM(kWhole);

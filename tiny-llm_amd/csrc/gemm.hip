@@ -643,14 +643,12 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     bf16x8 w[NJ], a[MI];
   };
   constexpr int FRAG = NJ + MI;
-  const bf16_t* ra = As + (wm * S::TM + lane % 32) * LD;
-  const bf16_t* rw = Ws + (wn * S::TN + lane % 32) * LD;
-  int kcol[4];                                             // this lane's place in a row for every k16 step
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) kcol[ks] = DIRECT ? ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8 : ks * 16 + (lane / 32) * 8;
+  const bf16_t* ra = As + (wm * S::TM + lane % 32) * LD + (DIRECT ? 0 : (lane / 32) * 8);
+  const bf16_t* rw = Ws + (wn * S::TN + lane % 32) * LD + (DIRECT ? 0 : (lane / 32) * 8);
   auto lds_read1 = [&](Frag& f, int buf, int ks, int p) {
-    if (p < NJ) f.w[p] = *(const bf16x8*)(rw + (buf * BN + p * 32) * LD + kcol[ks]);
-    else f.a[p - NJ] = *(const bf16x8*)(ra + (buf * BM + (p - NJ) * 32) * LD + kcol[ks]);
+    const int at = DIRECT ? ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8 : ks * 16;     // this lane's place in a row
+    if (p < NJ) f.w[p] = *(const bf16x8*)(rw + (buf * BN + p * 32) * LD + at);
+    else f.a[p - NJ] = *(const bf16x8*)(ra + (buf * BM + (p - NJ) * 32) * LD + at);
   };
   // The MFMAs of one k16 step, with memory operations issued between them: slot(n) comes after the
   // n-th MFMA.  The result tile is transposed (rows = n, columns = m) so that a lane holds four

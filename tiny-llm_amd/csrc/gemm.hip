@@ -464,16 +464,18 @@ constexpr int B_BK = 64;
 constexpr int B_LD = B_BK + 8;  // LDS row stride in elements: 144 bytes, keeps 16-byte alignment
 constexpr int B_XCDS = 8;
 
-// 16 bytes a lane from a buffer straight into LDS, side by side from `dst` on (the same for the whole wave).  Written
-// as one instruction block: given the builtin, the compiler waits for every load on its way ahead of each LDS read,
-// whichever buffer it reads.  Whoever reads the data waits for it first (tl_wait_loads, then a barrier).
+// 16 bytes a lane from a buffer straight into LDS, side by side from `dst` on (the same for the whole wave; the
+// instruction takes its place from M0).  Written as an instruction block: given the builtin, the compiler waits for every
+// load on its way ahead of each LDS read, whichever buffer it reads.  M0 is an operand, so the compiler writes it and knows
+// that it is used; what it does not see is that the block holds a load, which needs a wait state behind that write: the
+// s_nop.  Whoever reads the data waits for it first (tl_wait_loads, then a barrier).
 typedef int tl_rsrc_words __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void tl_load_to_lds(tl_rsrc_words buf, void* dst, int voffset, int soffset) {
   const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(__attribute__((address_space(3))) void*)dst);
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :
-               : "s"(at), "v"(voffset), "s"(buf), "s"(soffset)
-               : "memory", "m0");
+               : "{m0}"(at), "v"(voffset), "s"(buf), "s"(soffset)
+               : "memory");
 }
 template <int LEFT>       // until at most LEFT of the wave's loads are still on their way
 __device__ __forceinline__ void tl_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }

@@ -330,9 +330,28 @@ def test_linear_two_part_launch(M, K, N):
 @pytest.mark.parametrize("M,N", [(1, 128), (129, 132), (300, 260), (257, 130), (2049, 2052)])
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 328])
 def test_linear_operand_tiles(tile, M, N, K):
-    """Operand tiles that go straight into LDS or through registers: inner sizes of fewer k steps than there are buffers,
-    as many and more, and one that ends within a step; rows and columns that end within a tile; few and many tiles; an
-    operand within wider rows, and the residual that is overwritten."""
+    """Operand tiles in LDS: inner sizes of few k steps and one that ends within a step; rows and columns that end within a
+    tile; few and many tiles; an operand within wider rows, and the residual that is overwritten."""
+    _operand_tiles(tile, M, N, K)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3])
+@pytest.mark.parametrize("M,N,K", [(129, 132, 960), (129, 132, 1024), (300, 260, 1088), (257, 130, 1152), (300, 260, 1216),
+                                   (1, 128, 1032), (2049, 2052, 1024), (2048, 2048, 1024), (2000, 2047, 1088),
+                                   (4096, 1024, 1024), (3970, 1024, 1088)])
+def test_linear_operand_tiles_straight_into_lds(tile, M, N, K):
+    """From 16 k steps on operand tiles may go straight into LDS: every number of steps against the three and four buffers,
+    and both sides of the limits (256 tiles of 128 x 128 in 16 columns or in 8)."""
+    _operand_tiles(tile, M, N, K)
+
+
+@pytest.mark.parametrize("M,N", [(4096, 4096), (4095, 4092), (2048, 1024)])
+def test_linear_residual_of_large_tiles(M, N):
+    """256 x 256 tiles: the residual piece by piece with 256 of them, requested ahead with fewer."""
+    _operand_tiles(0, M, N, 64)
+
+
+def _operand_tiles(tile, M, N, K):
     g = torch.Generator().manual_seed(M + K + N)
     wide = torch.randn(M, K + 72, generator=g).to(torch.bfloat16)
     w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)

@@ -527,6 +527,8 @@ struct GemmShape {
 // How operand tiles get into LDS: through registers, zeros beyond the end of a row (kTail); through registers, the inner
 // size a multiple of the k step (kWhole); likewise, but straight from memory (kDirect).
 constexpr int kTail = 0, kWhole = 1, kDirect = 2;
+// What is known of the residual where the epilogue is compiled (kNoResidual: none, or one of rows without whole vectors).
+constexpr int kNoResidual = 0, kResidual = 1, kAnyForm = 2;
 template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, int MODE>
 __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16_t* __restrict__ a,
                                                                       const bf16_t* __restrict__ w,
@@ -753,18 +755,6 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   const bool vec_ok = (N % 4 == 0) && (ldo % 4 == 0);
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
-    // the residual of these 32 rows, requested together: out may be the residual, so the compiler asks for a piece only
-    // when the one before is stored (with the zeroing of kTail left out of ragged rows, 3,288 rows through registers,
-    // 2,048 x 2,048: 43.9 -> 42.0 us, 5,632 inner: 96.0 -> 90.2)
-    f32x4 res[8];
-    if (!SWIGLU && residual && vec_ok) {
-#pragma unroll
-      for (int c8 = 0; c8 < 8; ++c8) {
-        const int c = c8 * TL_WAVE + lane;
-        const int m = m0 + wm * S::TM + i * 32 + c / 16, n = n0 + wn * S::TN + (c % 16) * 4;
-        res[c8] = m < M && n < N ? *(const f32x4*)(residual + (int64_t)m * ldo + n) : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -775,75 +765,102 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    auto leave = [&](auto form) {
+      constexpr int FORM = decltype(form)::value;
+      constexpr bool AHEAD = FORM != kNoResidual && sizeof(TO) == 4;
+      // whether this launch's are: see below
+      const bool ahead = AHEAD && (BM + BN < 512 || gridDim.x < 256) && residual && vec_ok;
+      f32x4 res[AHEAD ? 8 : 1];
+      if (FORM == kResidual || ahead) {
+        const int m = m0 + wm * S::TM + i * 32 + lane / 16, n = n0 + wn * S::TN + (lane % 16) * 4;
+        const float* from = residual + (int64_t)m * ldo + n;
 #pragma unroll
-    for (int c8 = 0; c8 < 8; ++c8) {
-      const int c = c8 * TL_WAVE + lane;
-      const int r = c / 16, col = (c % 16) * 4;
-      const int m = m0 + wm * S::TM + i * 32 + r, n = n0 + wn * S::TN + col;
-      if (m >= M || n >= N) continue;
-      // the row's factor (1 / rms of a norm left out of the operand): given, or that of a norm handed over
-      float rs = 1.f;
-      if (nm.in_sumsq) rs = row_factor[m - m0];
-      else if (nm.row_scale) rs = nm.row_scale[m];
-      const f32x4 s4 = *(const f32x4*)(cstage + r * E_LD + col);
-      float v[4] = {s4[0] * rs, s4[1] * rs, s4[2] * rs, s4[3] * rs};
-      if constexpr (SWIGLU) {   // (gate, up, gate, up) -> two outputs; N is even and n a multiple of 4
-        const int64_t oz = (int64_t)m * ldo + n / 2;
-        if (n + 2 < N) {
-          typedef TO to2 __attribute__((ext_vector_type(2)));
-          to2 sv = {from_f32<TO>(swiglu_pair_fast(v[0], v[1])), from_f32<TO>(swiglu_pair_fast(v[2], v[3]))};
-          if (ldo % 2 == 0) {
-            *(to2*)(out + oz) = sv;
-          } else {
-            out[oz] = sv[0];
-            out[oz + 1] = sv[1];
-          }
-        } else {
-          out[oz] = from_f32<TO>(swiglu_pair_fast(v[0], v[1]));
-        }
-        continue;
+        for (int c8 = 0; c8 < 8; ++c8)
+          if (m + c8 * 4 < M && n < N) res[c8] = *(const f32x4*)(from + c8 * 4 * ldo);      // others are not stored
       }
-      const int64_t o = (int64_t)m * ldo + n;
-      if (vec_ok) {  // n + 3 < N because n and N are both multiples of 4
-        if (residual) {
-          v[0] += res[c8][0]; v[1] += res[c8][1]; v[2] += res[c8][2]; v[3] += res[c8][3];
-        }
-        if constexpr (sizeof(TO) == 4) {
-          f32x4 sv = {v[0], v[1], v[2], v[3]};
-          *(f32x4*)((float*)out + o) = sv;
-          if constexpr (!SWIGLU) {
-            if (nm.emit_operand) {      // uniform; N is a multiple of 64: the 16 lanes of a row are all here or none is
-              float wn[4];
-              if (nm.emit_w_is_f32) {
-                const f32x4 w4 = *(const f32x4*)((const float*)nm.emit_w + n);
-                wn[0] = w4[0]; wn[1] = w4[1]; wn[2] = w4[2]; wn[3] = w4[3];
-              } else {
-                const bf16x4 w4 = *(const bf16x4*)((const bf16_t*)nm.emit_w + n);
-                wn[0] = (float)w4[0]; wn[1] = (float)w4[1]; wn[2] = (float)w4[2]; wn[3] = (float)w4[3];
-              }
-              bf16x4 ev = {(bf16_t)(wn[0] * v[0]), (bf16_t)(wn[1] * v[1]), (bf16_t)(wn[2] * v[2]), (bf16_t)(wn[3] * v[3])};
-              *(bf16x4*)(nm.emit_operand + (int64_t)m * nm.emit_ld + n) = ev;
-              const float sq = group_sum<16>((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]));
-              if (lane % 16 == 0) nm.emit_sumsq[(int64_t)m * nm.emit_parts + n / 64] = sq;
+#pragma unroll
+      for (int c8 = 0; c8 < 8; ++c8) {
+        const int c = c8 * TL_WAVE + lane;
+        const int r = c / 16, col = (c % 16) * 4;
+        const int m = m0 + wm * S::TM + i * 32 + r, n = n0 + wn * S::TN + col;
+        if (m >= M || n >= N) continue;
+        // the row's factor (1 / rms of a norm left out of the operand): given, or that of a norm handed over
+        float rs = 1.f;
+        if (nm.in_sumsq) rs = row_factor[m - m0];
+        else if (nm.row_scale) rs = nm.row_scale[m];
+        const f32x4 s4 = *(const f32x4*)(cstage + r * E_LD + col);
+        float v[4] = {s4[0] * rs, s4[1] * rs, s4[2] * rs, s4[3] * rs};
+        if constexpr (SWIGLU) {   // (gate, up, gate, up) -> two outputs; N is even and n a multiple of 4
+          const int64_t oz = (int64_t)m * ldo + n / 2;
+          if (n + 2 < N) {
+            typedef TO to2 __attribute__((ext_vector_type(2)));
+            to2 sv = {from_f32<TO>(swiglu_pair_fast(v[0], v[1])), from_f32<TO>(swiglu_pair_fast(v[2], v[3]))};
+            if (ldo % 2 == 0) {
+              *(to2*)(out + oz) = sv;
+            } else {
+              out[oz] = sv[0];
+              out[oz + 1] = sv[1];
             }
+          } else {
+            out[oz] = from_f32<TO>(swiglu_pair_fast(v[0], v[1]));
+          }
+          continue;
+        }
+        const int64_t o = (int64_t)m * ldo + n;
+        if (vec_ok) {  // n + 3 < N because n and N are both multiples of 4
+          if (FORM == kResidual || (FORM == kAnyForm && residual)) {
+            f32x4 rv;
+            if (FORM == kResidual || ahead) rv = res[AHEAD ? c8 : 0];
+            else rv = *(const f32x4*)(residual + o);
+            v[0] += rv[0]; v[1] += rv[1]; v[2] += rv[2]; v[3] += rv[3];
+          }
+          if constexpr (sizeof(TO) == 4) {
+            f32x4 sv = {v[0], v[1], v[2], v[3]};
+            *(f32x4*)((float*)out + o) = sv;
+            if constexpr (!SWIGLU) {
+              if (nm.emit_operand) {      // uniform; N is a multiple of 64: the 16 lanes of a row are all here or none is
+                float wn[4];
+                if (nm.emit_w_is_f32) {
+                  const f32x4 w4 = *(const f32x4*)((const float*)nm.emit_w + n);
+                  wn[0] = w4[0]; wn[1] = w4[1]; wn[2] = w4[2]; wn[3] = w4[3];
+                } else {
+                  const bf16x4 w4 = *(const bf16x4*)((const bf16_t*)nm.emit_w + n);
+                  wn[0] = (float)w4[0]; wn[1] = (float)w4[1]; wn[2] = (float)w4[2]; wn[3] = (float)w4[3];
+                }
+                bf16x4 ev = {(bf16_t)(wn[0] * v[0]), (bf16_t)(wn[1] * v[1]), (bf16_t)(wn[2] * v[2]), (bf16_t)(wn[3] * v[3])};
+                *(bf16x4*)(nm.emit_operand + (int64_t)m * nm.emit_ld + n) = ev;
+                const float sq = group_sum<16>((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]));
+                if (lane % 16 == 0) nm.emit_sumsq[(int64_t)m * nm.emit_parts + n / 64] = sq;
+              }
+            }
+          } else {
+            if (nm.act != kActNone) {     // uniform
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[e] = act_value(v[e], nm.act);
+            }
+            bf16x4 sv = {(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+            *(bf16x4*)((bf16_t*)out + o) = sv;
           }
         } else {
-          if (nm.act != kActNone) {     // uniform
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = act_value(v[e], nm.act);
+          for (int e = 0; e < 4 && n + e < N; ++e) {
+            float x = v[e];
+            if (residual) x += residual[o + e];
+            if constexpr (sizeof(TO) == 2) x = act_value(x, nm.act);
+            out[o + e] = from_f32<TO>(x);
           }
-          bf16x4 sv = {(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
-          *(bf16x4*)((bf16_t*)out + o) = sv;
-        }
-      } else {
-        for (int e = 0; e < 4 && n + e < N; ++e) {
-          float x = v[e];
-          if (residual) x += residual[o + e];
-          if constexpr (sizeof(TO) == 2) x = act_value(x, nm.act);
-          out[o + e] = from_f32<TO>(x);
         }
       }
-    }
+    };
+    // A float32 result's residual is requested for all 32 rows together: out may be the residual, so the compiler asks for
+    // a piece only when the one before is stored (4,096 rows, 640 x 512: 13.6 -> 12.0 us; 3,000 rows, 1,280 x 256: 12.2 ->
+    // 10.6).  Where 256 x 256 tiles occupy every unit their requests come in one burst: 4,096 rows, 4,096 x 512, took 39.3
+    // us piece by piece and 40.7 so, and stay piece by piece.  The smallest tile, whose products are mostly launch, has the
+    // two forms apart: 65 to 4,096 rows, 520 x 264, take 2 % more without a residual where one piece of code serves both,
+    // bfloat16 results 3 % (they come without one, and load it piece by piece).  The larger tiles would lose waves by it:
+    // 108 registers where 84 let four a SIMD run.
+    if constexpr (BM > 64 || sizeof(TO) != 4) leave(std::integral_constant<int, SWIGLU ? kNoResidual : kAnyForm>{});
+    else if (!SWIGLU && residual && vec_ok) leave(std::integral_constant<int, kResidual>{});
+    else leave(std::integral_constant<int, kNoResidual>{});
     // the area is written again for the next 32 rows
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -888,13 +905,17 @@ static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const flo
     const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
     const int64_t wgs = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
     // Straight into LDS where a unit has one workgroup at a time anyway, so that the tiles on their way cost none: the
-    // 128 x 128 tile with at most 256 of them (1,944 rows, 2,048 x 5,632: 58.6 us through registers, 55.2 so; 1,536 rows:
-    // 53.4 and 49.4; beyond, two workgroups a unit are worth more), and the 256 x 128 tile for float32 results (2,048
-    // rows, 4,096 x 4,096: 74.3 and 73.5; 3,000 rows, 4,096 x 14,336: 323.9 and 316.1).  With bfloat16 results that tile
-    // loses (2,048 rows, 6,144 x 4,096: 98.3 and 100.1).  The 256 x 256 tile has room for two buffers only, one on
-    // its way: 8,192^3 takes 1,138 us so and 927 through registers.  Four waves of twice the outputs, which read less
-    // from LDS, lose with float32 results (1,944 rows, 2,048 x 5,632: 59.0; 3,288 rows: 88.2 -> 100.6).
-    if (BM + BN == 384 ? sizeof(TO) == 4 : wgs <= 256) return TL_GEMM(kDirect);
+    // 128 x 128 tile with fewer than 256 of them, or with 256 in at least 16 columns of tiles (through registers and so:
+    // 3,000 rows, 1,280 x 4,096 46.5 and 42.6 us; 2,048 rows, 2,048 x 4,096 44.7 and 43.6; but 4,096 rows, 1,024 x 2,048, 8
+    // columns, 25.6 and 26.4; beyond 256, two workgroups a unit are worth more), and the 256 x 128 tile for float32 results
+    // (2,048 rows, 4,096 x 4,096: 74.3 and 73.5; 3,000 rows, 4,096 x 14,336: 323.9 and 316.1).  From 16 k steps on: with
+    // fewer the buffers are hardly filled when the last is asked for (4,096 rows, 1,000 x 512: 12.0 and 12.4).  With
+    // bfloat16 results the 256 x 128 tile loses (2,048 rows, 6,144 x 4,096: 98.3 and 100.1).  The 256 x 256 tile has room
+    // for two buffers only, one on its way: 8,192^3 takes 1,138 us so and 927 through registers.  Four waves of twice the
+    // outputs, which read less from LDS, lose with float32 results (1,944 rows, 2,048 x 5,632: 59.0; 3,288 rows: 88.2 ->
+    // 100.6).
+    const bool few = wgs < 256 || (wgs == 256 && (N + BN - 1) / BN >= 16);
+    if (K >= 16 * B_BK && (BM + BN == 384 ? sizeof(TO) == 4 : few)) return TL_GEMM(kDirect);
   }
   return TL_GEMM(kWhole);
 #undef TL_GEMM

@@ -1253,9 +1253,11 @@ def test_linear_set(M, K, cols):
 # ------------------------------------------------------------ experts of few rows
 @pytest.mark.parametrize("T,top,E,K,N", [(1, 1, 1, 8, 4), (1, 4, 16, 2048, 1408), (3, 2, 5, 520, 46), (16, 4, 16, 512, 30),
                                          (7, 9, 64, 1032, 10), (64, 1, 3, 704, 24), (15, 4, 4, 1536, 18), (2, 3, 8, 2056, 12),
-                                         (17, 4, 16, 264, 20)])
+                                         (17, 4, 16, 264, 20),
+                                         (16, 4, 4, 520, 2018), (7, 9, 9, 1032, 1026), (64, 1, 3, 1544, 1026), (15, 4, 4, 2040, 1030),
+                                         (5, 2, 8, 264, 4100), (6, 5, 40, 1536, 1044), (2, 2, 3, 1032, 16), (3, 2, 3, 1024, 1024)])
 def test_experts_of_few_rows(T, top, E, K, N):
-    """Rows up to and beyond those that share an expert's weights in one workgroup (64), inner sizes on either side of its
+    """Experts on either side of a million weights, from which on they are read once; rows up to and beyond those that share an expert's weights in one workgroup (64), inner sizes on either side of its
     vectors of 512 and beyond its registers, every activation, a strided input, all rows on one expert: both products
     against float64.  bfloat16 results are rounded once (2^-8 of their size; the gate's exponential adds little); a
     float32 sum of K products in any order stays within K 2^-24 of the sum of their sizes."""

@@ -2,7 +2,7 @@
 of a decode step's requests."""
 import pytest
 
-from tiny_llm_amd.kernels import ops
+from tiny_llm_amd.kernels import library, ops
 
 
 @pytest.fixture
@@ -59,3 +59,16 @@ def test_prompt_portions_split_their_keys_where_it_was_measured_to_pay():
         for ctx in (rows, 4096, 32768, 131072):
             if ctx >= rows:
                 assert 1 <= ops.prefill_key_splits(rows, ctx, tile_waves=4, **heads) <= 8
+
+
+def test_small_experts_products_go_by_rows():
+    """Which experts' weights are read once for all their rows: large ones, and any in the second product of one or two
+    tokens (small ones took up to four times as long that way)."""
+    by_expert = library.load(verbose=False).tl_table_moe_by_expert
+    up = lambda N, K, act=0: by_expert(0, 6, 4, N, K, act)
+    down = lambda n_tokens, top, N, K: by_expert(1, n_tokens, top, N, K, 0)
+    gate = 2
+    assert up(2 * 704, 2048, gate) and up(704, 2048) and up(1408, 2048) and up(2048, 512, gate)
+    assert not up(128, 512) and not up(2048, 1024) and not up(2 * 256, 1024, gate) and not up(256, 2048)
+    assert down(6, 4, 2048, 704) and down(32, 2, 1024, 1024) and not down(8, 8, 1024, 256) and not down(64, 1, 512, 1536)
+    assert down(1, 8, 256, 64) and down(2, 2, 64, 32) and not down(2, 1, 512, 128) and not down(3, 2, 256, 128)

@@ -222,7 +222,7 @@ __device__ __forceinline__ void load_lanes(const bf16_t* __restrict__ row, int K
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ bf16x2 pair_of(bf16x8 v, int j) { return bf16x2{v[2 * j], v[2 * j + 1]}; }
 
-// The four products of one row (or of two at once, x1 not null: the weights are widened once for both).
+// The four products of one row, or of two that share the weights in the registers (TWO; else x1 is not read).
 template <int NIT, bool TWO>
 __device__ __forceinline__ void dot_held4(const bf16_t* __restrict__ x0, const bf16_t* __restrict__ x1, const bf16x8 (*y)[NIT],
                                           int K, int lane, float* out0, float* out1) {
@@ -247,6 +247,11 @@ __device__ __forceinline__ void dot_held4(const bf16_t* __restrict__ x0, const b
     if constexpr (TWO) out1[c] = wave_sum(acc1[c]);
   }
 }
+// The expert of row `at` (= t * top + j).  Without token ids the table has these rows in this order.
+__device__ __forceinline__ int expert_of_row(const int32_t* tokens, const int32_t* table, int at, int top, int vocab, int experts) {
+  if (tokens) return expert_of(tokens, table, at / top, at % top, top, vocab, experts);
+  return min(max(table[at], 0), experts - 1);
+}
 // v[lane] of the first four lanes without an indexed array
 __device__ __forceinline__ float of_lane(const float* v, int lane) {
   return lane == 0 ? v[0] : lane == 1 ? v[1] : lane == 2 ? v[2] : v[3];
@@ -262,7 +267,7 @@ __global__ __launch_bounds__(kThreads) void table_moe_up_shared_kernel(
     int act) {
   const int wave = threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE;
   const int at = min(lane, rows - 1);
-  const int mine = expert_of(tokens, table, at / top, at % top, top, vocab, experts);
+  const int mine = expert_of_row(tokens, table, at, top, vocab, experts);
   const bool by_row = (int)gridDim.x == rows;
   const int e = by_row ? __builtin_amdgcn_readlane(mine, blockIdx.x) : (int)blockIdx.x;
   const unsigned long long all = __ballot(lane < rows && mine == e);
@@ -319,7 +324,7 @@ __global__ __launch_bounds__(kDownCols / 4 * kDownSlots * TL_WAVE) void table_mo
   const int wave = threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE;
   const int group = wave % (kDownCols / 4), slot = wave / (kDownCols / 4), n = blockIdx.x * kDownCols + group * 4;
   const int at = min(lane, rows - 1);
-  const int mine = expert_of(tokens, table, at / top, at % top, top, vocab, experts);
+  const int mine = expert_of_row(tokens, table, at, top, vocab, experts);
   unsigned long long open = rows >= TL_WAVE ? ~0ull : (1ull << rows) - 1;
   for (int nth = 0; open; ++nth) {
     const int e = __builtin_amdgcn_readlane(mine, __builtin_ctzll(open));
@@ -352,6 +357,21 @@ __global__ __launch_bounds__(kDownCols / 4 * kDownSlots * TL_WAVE) void table_mo
     for (int j = 0; j < top; ++j) acc = fmaf(row_w ? row_w[(int64_t)t * top + j] : 1.f, part[t * top + j][c], acc);
     out[(int64_t)t * N + col] = fmaf(coef, acc, b);
   }
+}
+
+// Whether an expert's weights (N rows of K) are worth a walk over its rows, one or two at a time, by the waves that hold
+// them: that walk is a chain, and rows on workgroups of their own find the weights of a small expert in the caches.
+// From a million weights on the walk wins (4 rows and more, first product: 0.55 to 1.06 of the time by rows, gated or with
+// rows of more than 1,024; second product with 1,024 columns or more: 0.37 to 0.97).  Below it loses: first product of 16
+// experts of 128 x 512, 16 and 64 rows, 7.7 -> 10.4 and 8.6 -> 15.6 us for three layers; of 16 plain experts of 2,048 x
+// 1,024, 16 rows, 35 -> 44; second product of 128 experts of 1,024 x 256, 64 rows, 32 -> 53.  One or two tokens' second
+// product it wins at every size, because the other kernel takes a token's experts one after another: 4 of 256 x 128 11.5 ->
+// 9.1, 128 of 256 x 64 30 -> 16.
+static bool shared_up_pays(int N, int K, int act) {
+  return (int64_t)N * K >= 1 << 20 && (act == kActSiluGate || K > 1024);
+}
+static bool shared_down_pays(int n_tokens, int top, int N, int K) {
+  return (N >= 1024 && (int64_t)N * K >= 1 << 20) || (n_tokens <= 2 && top >= 2);
 }
 
 // Whether the kernels above take these rows: whole vectors, and few enough of them for a lane's registers.
@@ -795,6 +815,12 @@ int tl_moe_combine(const float* y, const float* base, const float* base_scale, c
   return tl_launch_status();
 }
 
+// Which kernel takes the products of few rows: 1 if an expert's weights are read once for its rows.  For the first
+// (down 0) or the second product (down 1); act as below.
+int tl_table_moe_by_expert(int down, int n_tokens, int top, int N, int K, int act) {
+  return down ? shared_down_pays(n_tokens, top, N, K) : shared_up_pays(N, K, act);
+}
+
 // a: [n_tokens, K] (row stride a_stride); w: [experts, N, K]; table: int32 [vocab, top], looked up by tokens[t], or
 // (tokens null) by t itself; out: [n_tokens * top, N], with the activation `act` (0 none, 1 squared relu) applied.
 int tl_table_moe_up(const void* a, int64_t a_stride, const void* w, const int32_t* tokens, const int32_t* table, void* out,
@@ -807,7 +833,7 @@ int tl_table_moe_up(const void* a, int64_t a_stride, const void* w, const int32_
   const int kCols = (int64_t)n_tokens * top <= kFewRows ? kColsFew : kColsWide;
   const int n_out = act == kActSiluGate ? N / 2 : N;      // output columns
   dim3 g(n_tokens * top, (n_out + kCols - 1) / kCols), b(kThreads);
-  const int nit = shared_vectors((int64_t)n_tokens * top, K, dtype, a_stride, a, w);
+  const int nit = shared_up_pays(N, K, act) ? shared_vectors((int64_t)n_tokens * top, K, dtype, a_stride, a, w) : 0;
   if (nit) {
     const int cols = (act == kActSiluGate ? 2 : 4) * kWaves;
     g = dim3(n_tokens * top < experts ? n_tokens * top : experts, (n_out + cols - 1) / cols);
@@ -844,7 +870,7 @@ int tl_table_moe_down(const void* z, const void* w, const int32_t* tokens, const
     return TL_ERR_ARG;
   const int kCols = (int64_t)n_tokens * top <= kFewRows ? kColsFew : kColsWide;
   dim3 g(n_tokens, (N + kCols - 1) / kCols), b(kThreads);
-  const int nit = shared_vectors((int64_t)n_tokens * top, K, dtype, 0, z, w);
+  const int nit = shared_down_pays(n_tokens, top, N, K) ? shared_vectors((int64_t)n_tokens * top, K, dtype, 0, z, w) : 0;
   if (nit) {
     g = dim3((N + kDownCols - 1) / kDownCols);
     b = dim3(kDownCols / 4 * kDownSlots * TL_WAVE);

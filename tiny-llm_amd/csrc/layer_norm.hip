@@ -18,15 +18,15 @@ constexpr int kWaves = kThreads / TL_WAVE;
 // v[j] = alpha * x[row, j] + y[row, j] (y optional); x[row] <- LN(v) * w + b (when `inplace`), out[row] likewise
 // in TO (optional).  `rows` (optional) gathers: output row i reads stream row rows[i].  One workgroup a row.  A decode
 // step's rows leave the chip empty, so the kernel is its round trips: everything the row needs is requested before the
-// first sum, in vectors of four where the row allows it (VEC 4: KEEP vectors a thread; VEC 1: KEEP elements).  Six rows
-// of 2,048: 7.9 us with element loads and weights behind the sums, 4.7 so (a launch and one round trip are 4.1).
-template <typename TO, int KEEP, int VEC>
+// first sum, KEEP vectors of four a thread.  Six rows of 2,048: 7.9 us with element loads and weights behind the sums, 4.7 so
+// (a launch and one round trip are 4.1).
+template <typename TO, int KEEP>
 __global__ __launch_bounds__(kThreads) void layer_norm_kernel(const float* __restrict__ y, const float* __restrict__ w,
                                                               const float* __restrict__ b, float* __restrict__ x,
                                                               const int32_t* __restrict__ rows, TO* __restrict__ out,
                                                               int hidden, float alpha, float eps, int inplace) {
-  typedef float vec __attribute__((ext_vector_type(VEC)));
-  typedef TO out_vec __attribute__((ext_vector_type(VEC)));
+  typedef float vec __attribute__((ext_vector_type(4)));
+  typedef TO out_vec __attribute__((ext_vector_type(4)));
   __shared__ float red[kWaves];
   const int64_t src_row = rows ? rows[blockIdx.x] : blockIdx.x;
   float* xr = x + src_row * hidden;
@@ -36,37 +36,37 @@ __global__ __launch_bounds__(kThreads) void layer_norm_kernel(const float* __res
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
-    const int j = (threadIdx.x + i * kThreads) * VEC;
+    const int j = (threadIdx.x + i * kThreads) * 4;
     const vec zero = {};
     const bool in = j < hidden;
     const vec xv = in ? *(const vec*)(xr + j) : zero, yv = in && yr ? *(const vec*)(yr + j) : zero;
     wv[i] = in ? *(const vec*)(w + j) : zero;
     bv[i] = in ? *(const vec*)(b + j) : zero;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) v[i][e] = yr ? fmaf(alpha, xv[e], yv[e]) : alpha * xv[e];
+    for (int e = 0; e < 4; ++e) v[i][e] = yr ? fmaf(alpha, xv[e], yv[e]) : alpha * xv[e];
   }
 #pragma unroll
   for (int i = 0; i < KEEP; ++i)
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) s += v[i][e];
+    for (int e = 0; e < 4; ++e) s += v[i][e];
   const float mean = block_sum<kWaves>(s, red) * inv_n;
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < KEEP; ++i)
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float d = (threadIdx.x + i * kThreads) * VEC < hidden ? v[i][e] - mean : 0.f;
+    for (int e = 0; e < 4; ++e) {
+      const float d = (threadIdx.x + i * kThreads) * 4 < hidden ? v[i][e] - mean : 0.f;
       q += d * d;
     }
   const float r = 1.f / sqrtf(block_sum<kWaves>(q, red) * inv_n + eps);
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
-    const int j = (threadIdx.x + i * kThreads) * VEC;
+    const int j = (threadIdx.x + i * kThreads) * 4;
     if (j >= hidden) continue;
     vec o;
     out_vec c;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
+    for (int e = 0; e < 4; ++e) {
       o[e] = (v[i][e] - mean) * r * wv[i][e] + bv[i][e];
       c[e] = from_f32<TO>(o[e]);
     }
@@ -75,18 +75,50 @@ __global__ __launch_bounds__(kThreads) void layer_norm_kernel(const float* __res
   }
 }
 
-// The same for rows longer than the registers hold: formed again in every pass.
-template <typename TO>
-__global__ __launch_bounds__(kThreads) void layer_norm_long_kernel(const float* __restrict__ y, const float* __restrict__ w,
-                                                                   const float* __restrict__ b, float* __restrict__ x,
-                                                                   const int32_t* __restrict__ rows, TO* __restrict__ out,
-                                                                   int hidden, float alpha, float eps, int inplace) {
+// The same for rows of no whole vectors, element by element, and for rows longer than the registers hold, which are formed
+// again in every pass.  The weights are read behind the sums here: held beside the elements they cost more waves than a
+// round trip (2,048 rows of 2,050: 13.1 and 20.6 us).
+template <typename TO, int KEEP>
+__global__ __launch_bounds__(kThreads) void layer_norm_elements_kernel(const float* __restrict__ y, const float* __restrict__ w,
+                                                                       const float* __restrict__ b, float* __restrict__ x,
+                                                                       const int32_t* __restrict__ rows, TO* __restrict__ out,
+                                                                       int hidden, float alpha, float eps, int inplace) {
   __shared__ float red[kWaves];
   const int64_t src_row = rows ? rows[blockIdx.x] : blockIdx.x;
   float* xr = x + src_row * hidden;
   const float* yr = y ? y + src_row * hidden : nullptr;
   TO* dst = out ? out + (int64_t)blockIdx.x * hidden : nullptr;
   const float inv_n = 1.f / (float)hidden;
+  if (hidden <= KEEP * kThreads) {
+    float v[KEEP];
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+      const int j = threadIdx.x + i * kThreads;
+      v[i] = 0.f;
+      if (j < hidden) v[i] = yr ? fmaf(alpha, xr[j], yr[j]) : alpha * xr[j];
+      s += v[i];
+    }
+    const float mean = block_sum<kWaves>(s, red) * inv_n;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+      const int j = threadIdx.x + i * kThreads;
+      const float d = j < hidden ? v[i] - mean : 0.f;
+      q += d * d;
+    }
+    const float r = 1.f / sqrtf(block_sum<kWaves>(q, red) * inv_n + eps);
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+      const int j = threadIdx.x + i * kThreads;
+      if (j < hidden) {
+        const float o = (v[i] - mean) * r * w[j] + b[j];
+        if (inplace) xr[j] = o;
+        if (dst) dst[j] = from_f32<TO>(o);
+      }
+    }
+    return;
+  }
   float s = 0.f;
   for (int j = threadIdx.x; j < hidden; j += kThreads) s += yr ? fmaf(alpha, xr[j], yr[j]) : alpha * xr[j];
   const float mean = block_sum<kWaves>(s, red) * inv_n;
@@ -252,16 +284,13 @@ template <typename TO>
 int launch(const float* y, const float* w, const float* b, float* x, const int32_t* rows, TO* out, int n, int hidden,
            float alpha, float eps, int inplace, hipStream_t stream) {
   dim3 g(n), blk(kThreads);
-#define TL_LN(KEEP, VEC)                                                                                                  \
-  hipLaunchKernelGGL((layer_norm_kernel<TO, KEEP, VEC>), g, blk, 0, stream, y, w, b, x, rows, out, hidden, alpha, eps,     \
-                     inplace)
+#define TL_LN(KERNEL, KEEP)                                                                                        \
+  hipLaunchKernelGGL((KERNEL<TO, KEEP>), g, blk, 0, stream, y, w, b, x, rows, out, hidden, alpha, eps, inplace)
   const bool vec = hidden % 4 == 0 && !(((uintptr_t)y | (uintptr_t)w | (uintptr_t)b | (uintptr_t)x | (uintptr_t)out) & 15);
-  if (vec && hidden <= 8 * kThreads) TL_LN(2, 4);
-  else if (vec && hidden <= 32 * kThreads) TL_LN(8, 4);
-  else if (hidden <= 8 * kThreads) TL_LN(8, 1);
-  else if (hidden <= 32 * kThreads) TL_LN(32, 1);
-  else
-    hipLaunchKernelGGL(layer_norm_long_kernel<TO>, g, blk, 0, stream, y, w, b, x, rows, out, hidden, alpha, eps, inplace);
+  if (vec && hidden <= 8 * kThreads) TL_LN(layer_norm_kernel, 2);
+  else if (vec && hidden <= 32 * kThreads) TL_LN(layer_norm_kernel, 8);
+  else if (hidden <= 8 * kThreads) TL_LN(layer_norm_elements_kernel, 8);
+  else TL_LN(layer_norm_elements_kernel, 32);
 #undef TL_LN
   return tl_launch_status();
 }

@@ -13,16 +13,15 @@ constexpr int kWaves = kThreads / TL_WAVE;
 // x[t] += scale * w * y[t] / sqrt(mean(y[t]^2) + eps); copy[t] = x[t] in TC (optional).
 // One workgroup per row.  `w` is the norm's effective weight, `scale` (optional) a factor per channel.
 // A row stays in registers between the two passes, and what the second pass needs (x, w, scale) is requested before the
-// sum of squares is known: KEEP vectors of four a thread, or KEEP elements where the row has no whole vectors (six rows
-// of 2,048: 6.1 us by elements, 4.7 by vectors).  Rows beyond 8,192 elements are read twice.
-template <typename TC, int KEEP, int VEC>
+// sum of squares is known: KEEP vectors of four a thread (six rows of 2,048: 6.1 us by elements, 4.7 by vectors).
+template <typename TC, int KEEP>
 __global__ __launch_bounds__(kThreads) void norm_scale_add_kernel(const float* __restrict__ y,
                                                                   const float* __restrict__ w,
                                                                   const float* __restrict__ scale,
                                                                   float* __restrict__ x, TC* __restrict__ copy,
                                                                   int hidden, float eps) {
-  typedef float vec __attribute__((ext_vector_type(VEC)));
-  typedef TC copy_vec __attribute__((ext_vector_type(VEC)));
+  typedef float vec __attribute__((ext_vector_type(4)));
+  typedef TC copy_vec __attribute__((ext_vector_type(4)));
   __shared__ float red[kWaves];
   const float* src = y + (int64_t)blockIdx.x * hidden;
   float* dst = x + (int64_t)blockIdx.x * hidden;
@@ -30,7 +29,7 @@ __global__ __launch_bounds__(kThreads) void norm_scale_add_kernel(const float* _
   vec yv[KEEP], xv[KEEP], wv[KEEP], sv[KEEP];
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
-    const int j = (threadIdx.x + i * kThreads) * VEC;
+    const int j = (threadIdx.x + i * kThreads) * 4;
     const vec zero = {};
     const bool in = j < hidden;
     yv[i] = in ? *(const vec*)(src + j) : zero;
@@ -41,17 +40,17 @@ __global__ __launch_bounds__(kThreads) void norm_scale_add_kernel(const float* _
 #pragma unroll
   for (int i = 0; i < KEEP; ++i)
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) ss += yv[i][e] * yv[i][e];
+    for (int e = 0; e < 4; ++e) ss += yv[i][e] * yv[i][e];
   ss = block_sum<kWaves>(ss, red);
   const float r = 1.f / sqrtf(ss / (float)hidden + eps);
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
-    const int j = (threadIdx.x + i * kThreads) * VEC;
+    const int j = (threadIdx.x + i * kThreads) * 4;
     if (j >= hidden) continue;
     vec s;
     copy_vec c;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
+    for (int e = 0; e < 4; ++e) {
       s[e] = xv[i][e] + yv[i][e] * r * (scale ? wv[i][e] * sv[i][e] : wv[i][e]);
       c[e] = from_f32<TC>(s[e]);
     }
@@ -60,17 +59,41 @@ __global__ __launch_bounds__(kThreads) void norm_scale_add_kernel(const float* _
   }
 }
 
-// The same for rows longer than the registers hold: read twice.
-template <typename TC>
-__global__ __launch_bounds__(kThreads) void norm_scale_add_long_kernel(const float* __restrict__ y,
-                                                                       const float* __restrict__ w,
-                                                                       const float* __restrict__ scale,
-                                                                       float* __restrict__ x, TC* __restrict__ copy,
-                                                                       int hidden, float eps) {
+// The same for rows of no whole vectors, element by element; rows beyond 8,192 elements are read twice.
+template <typename TC, int KEEP>
+__global__ __launch_bounds__(kThreads) void norm_scale_add_elements_kernel(const float* __restrict__ y,
+                                                                           const float* __restrict__ w,
+                                                                           const float* __restrict__ scale,
+                                                                           float* __restrict__ x, TC* __restrict__ copy,
+                                                                           int hidden, float eps) {
   __shared__ float red[kWaves];
   const float* src = y + (int64_t)blockIdx.x * hidden;
   float* dst = x + (int64_t)blockIdx.x * hidden;
   float ss = 0.f;
+  if (hidden <= KEEP * kThreads) {
+    float yv[KEEP], xv[KEEP], wv[KEEP];
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+      const int j = threadIdx.x + i * kThreads;
+      const bool in = j < hidden;
+      yv[i] = in ? src[j] : 0.f;
+      xv[i] = in ? dst[j] : 0.f;
+      wv[i] = in ? (scale ? w[j] * scale[j] : w[j]) : 0.f;
+      ss += yv[i] * yv[i];
+    }
+    ss = block_sum<kWaves>(ss, red);
+    const float r = 1.f / sqrtf(ss / (float)hidden + eps);
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+      const int j = threadIdx.x + i * kThreads;
+      if (j < hidden) {
+        const float s = xv[i] + yv[i] * r * wv[i];
+        dst[j] = s;
+        if (copy) copy[(int64_t)blockIdx.x * hidden + j] = from_f32<TC>(s);
+      }
+    }
+    return;
+  }
   for (int j = threadIdx.x; j < hidden; j += kThreads) {
     const float v = src[j];
     ss += v * v;
@@ -90,14 +113,12 @@ template <typename TC>
 int launch_norm_scale_add(const float* y, const float* w, const float* scale, float* x, TC* copy, int n_rows, int hidden,
                           float eps, hipStream_t stream) {
   dim3 g(n_rows), b(kThreads);
-#define TL_NSA(KEEP, VEC) \
-  hipLaunchKernelGGL((norm_scale_add_kernel<TC, KEEP, VEC>), g, b, 0, stream, y, w, scale, x, copy, hidden, eps)
+#define TL_NSA(KERNEL, KEEP) hipLaunchKernelGGL((KERNEL<TC, KEEP>), g, b, 0, stream, y, w, scale, x, copy, hidden, eps)
   const bool vec = hidden % 4 == 0 && !(((uintptr_t)y | (uintptr_t)w | (uintptr_t)scale | (uintptr_t)x | (uintptr_t)copy) & 15);
-  if (vec && hidden <= 8 * kThreads) TL_NSA(2, 4);
-  else if (vec && hidden <= 32 * kThreads) TL_NSA(8, 4);
-  else if (hidden <= 8 * kThreads) TL_NSA(8, 1);
-  else if (hidden <= 32 * kThreads) TL_NSA(32, 1);
-  else hipLaunchKernelGGL(norm_scale_add_long_kernel<TC>, g, b, 0, stream, y, w, scale, x, copy, hidden, eps);
+  if (vec && hidden <= 8 * kThreads) TL_NSA(norm_scale_add_kernel, 2);
+  else if (vec && hidden <= 32 * kThreads) TL_NSA(norm_scale_add_kernel, 8);
+  else if (hidden <= 8 * kThreads) TL_NSA(norm_scale_add_elements_kernel, 8);
+  else TL_NSA(norm_scale_add_elements_kernel, 32);
 #undef TL_NSA
   return tl_launch_status();
 }

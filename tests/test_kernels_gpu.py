@@ -1204,6 +1204,31 @@ def test_sampling_from_the_list_of_largest_and_by_descent(kind):
                     assert got[i] in near, (kind, vocab, t, k, p, i, got[i])
 
 
+@pytest.mark.parametrize("kind", ["ties", "normal", "peaked"])
+def test_sampling_at_the_limits_of_ranks_and_lists(kind):
+    """Rows and lists of up to 256 elements (ranks), of up to 1,024 (descents over one element a thread) and beyond: the plain
+    chain's token for the same u, as above."""
+    g = torch.Generator().manual_seed(37)
+    for vocab in (255, 256, 257, 1023, 1024, 1025, 6000):
+        n = 3
+        logits = torch.randn(n, vocab, generator=g) * 3
+        if kind == "ties":
+            logits = (logits * 2).round() / 2 + 0.0       # + 0.0: -0 is a key of its own below 0
+        if kind == "peaked":
+            logits[:, 3] += 12.0
+        for t, k, p in ((1.0, 0, 1.0), (1.0, 0, 0.97), (0.8, 256, 1.0), (1.5, 257, 0.9), (1.0, 1000, 0.99), (3.0, 1024, 1.0), (3.0, 1025, 0.9)):
+            k = min(k, vocab)
+            seeds = torch.arange(n, dtype=torch.int64) * 15485863 + vocab + k
+            ctrs = torch.arange(n, dtype=torch.int32) + 5
+            got = _sample(logits, temperature=torch.full((n,), t), top_k=torch.full((n,), k, dtype=torch.int32),
+                          top_p=torch.full((n,), p), seeds=seeds, counters=ctrs)
+            for i in range(n):
+                u = plain.uniform_for(int(seeds[i]), int(ctrs[i]))
+                if got[i] != plain.sample_token(logits[i], t, k, p, u):
+                    near = {plain.sample_token(logits[i], t, k, p, min(max(u + d, 0.0), 0.999999)) for d in (-2e-6, 2e-6)}
+                    assert got[i] in near, (kind, vocab, t, k, p, i, got[i])
+
+
 def test_sampling_top_p_reference_vectors():
     # (ref) tests/logit_processors/test_sort_processors.cpp:120-200: with logits i/40 and logit[0] = 0.5,
     # p = 0.2 keeps ids {0, 19, 18, 17}; with logit[0] = 2 it keeps {0, 19}

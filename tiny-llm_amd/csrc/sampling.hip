@@ -16,11 +16,13 @@
 // added with integer atomics, so the result does not depend on the order in which
 // threads arrive and a (seed, position) pair always gives the same token.
 //
-// Nearly every row needs none of the four passes: what the three cuts look at lies within a few hundred of the
-// largest logits, whatever lies below.  One histogram over the distance from the row's maximum (`candidates`) finds
-// a bin behind which nothing matters, the elements ahead of it are gathered into LDS, and every cut is read off their
-// ranks.  The counts and masses are the same integers, so the token is the descent's token; a row whose first cut
-// reaches beyond kMaxListed elements, or that is flat and has no top-k, takes the descent.
+// Nearly every row needs none of the four passes over all of its elements: what the three cuts look at lies within a few
+// hundred of the largest logits, whatever lies below.  One histogram over the distance from the row's maximum
+// (`candidates`) finds a bin behind which nothing matters, and the elements ahead of it are gathered into LDS, at most one
+// a thread.  Every cut is read off the ranks of a short list; a longer one (and a whole row of no more elements than
+// threads) takes the descent over the threads' own elements.  The counts and masses are the same integers, so the token
+// is the descent's token; a row whose first cut reaches beyond kMaxListed elements, or that is flat and has no top-k,
+// takes the descent over all elements.
 //
 // One workgroup per row.  u comes from a counter-based generator keyed by the
 // row's seed and the row's position counter.
@@ -53,8 +55,10 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
 // values share a handful of exponents, so bins of the key's leading byte (the descent's first pass) are hit by
 // thousands of elements each and their LDS atomics queue up: that is what the descent's passes wait for.
 constexpr int kDistShift = 15, kDistBins = 2048;
-// Most elements the ranks are formed of (one a thread; each looks at all of them).
-constexpr int kMaxListed = S_THREADS;
+// Most elements of a list (one a thread), and most of which the ranks are formed, for which each looks at all of them.  8
+// rows of 32,000: the 200 best and three cuts take 34 us by ranks; the 1,000 best and one cut 132 us by ranks, 32 by
+// descents over the list and 110 by descents over the row.
+constexpr int kMaxListed = S_THREADS, kMaxRanked = 256;
 // Rows of up to this many logits are read once and stay in registers.
 constexpr int kHeldVecs = 8, kHeldVocab = kHeldVecs * 4 * S_THREADS;
 
@@ -102,8 +106,10 @@ __device__ __forceinline__ unsigned long long mass_of(const Row& r, float x) {
 // Finds the key K* at which the running measure, taken over keys in descending
 // order, first reaches `target` (>= 1).  by_mass selects the measure.  On return
 // (in sh): above_mass / above_cnt = mass and count of keys > K*; bin_mass / bin_cnt
-// = mass and count of keys == K*.  Returns K*.
-__device__ uint32_t descend(const Row& r, Shared& sh, bool by_mass, unsigned long long target) {
+// = mass and count of keys == K*.  Returns K*.  `each` calls its argument with the key of every element of the calling
+// thread and a function that gives its mass.
+template <typename E>
+__device__ uint32_t descend(const E& each, Shared& sh, bool by_mass, unsigned long long target) {
   uint32_t prefix = 0;
   unsigned long long above_mass = 0;
   unsigned int above_cnt = 0;
@@ -113,16 +119,14 @@ __device__ uint32_t descend(const Row& r, Shared& sh, bool by_mass, unsigned lon
       sh.hcnt[b] = 0;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < r.vocab; i += S_THREADS) {
-      const float x = scaled(r, i);
-      const uint32_t key = order_key(x);
+    each([&](uint32_t key, auto mass) {
       const bool match = (shift == 24) || ((key >> (shift + 8)) == (prefix >> (shift + 8)));
       if (match) {
         const int bin = (key >> shift) & 255;
-        atomicAdd(&sh.hmass[bin], mass_of(r, x));
+        atomicAdd(&sh.hmass[bin], mass());
         atomicAdd(&sh.hcnt[bin], 1u);
       }
-    }
+    });
     __syncthreads();
     if (threadIdx.x < TL_WAVE) {
       // lane L owns bins 255-4L .. 252-4L, i.e. the scan runs from the largest keys down
@@ -239,9 +243,10 @@ __device__ __forceinline__ unsigned long long sum64(Shared& sh, unsigned long lo
 
 // Gathers (key, id, mass) of a set of the row's largest elements that reaches `target` of the measure (counts, or mass)
 // and holds every element of the smallest key in it.  Returns their number, or 0: beyond the bins or beyond the list.
+// `kmin`: no smaller key is in the set.
 template <bool HELD>
 __device__ int candidates(const Row& r, Shared& sh, const f32x4* held, uint32_t kmax, bool by_mass,
-                          unsigned long long target) {
+                          unsigned long long target, uint32_t* kmin) {
   for (int b = threadIdx.x; b < kDistBins; b += S_THREADS) {
     sh.dmass[b] = 0;
     sh.dcnt[b] = 0;
@@ -291,6 +296,8 @@ __device__ int candidates(const Row& r, Shared& sh, const f32x4* held, uint32_t 
   __syncthreads();
   const unsigned int last = sh.bin;
   const int n = last < kDistBins ? (int)sh.bin_cnt : 0;
+  const uint32_t reach = ((last + 1) << kDistShift) - 1;      // how far below the maximum they go
+  *kmin = n > 0 && reach < kmax ? kmax - reach : 0u;
   __syncthreads();                          // the list takes the histograms' place
   if (n <= 0 || n > kMaxListed) return 0;
   for_row<HELD>(r, held, [&](float x, int i) {
@@ -306,48 +313,73 @@ __device__ int candidates(const Row& r, Shared& sh, const f32x4* held, uint32_t 
   return n;
 }
 
-// The whole chain on the gathered elements, whose first cut lies at z (all of the row's mass where there is no top-k);
-// false: this row takes the passes over all of its elements.
-template <bool HELD>
-__device__ bool sample_listed(const Row& r, Shared& sh, const f32x4* held, uint32_t kmax, int k, float p, double u,
-                              unsigned long long z, int32_t* out) {
-  const bool top_k = k > 0 && k < r.vocab;
-  unsigned long long target;
-  if (top_k) {
-    target = (unsigned long long)k;
-  } else {
-    target = p < 1.f ? min(max((unsigned long long)((double)fmaxf(p, 0.f) * (double)z), 1ull), z)
-                     : min((unsigned long long)(u * (double)z) + 1ull, z);
+// At most one element a thread.
+struct Own {
+  bool mine;
+  uint32_t key;
+  int id;
+  unsigned long long mass;
+};
+
+// The whole chain (top-k, top-p, the draw) by descents over the elements of `each`.  Returns the drawn key, with in `nth`
+// which of the `ties` elements that share it.
+template <typename E>
+__device__ uint32_t cut_and_draw(const E& each, Shared& sh, bool cut_k, int k, float p, double u, unsigned long long z,
+                                 unsigned int* nth, unsigned int* ties) {
+  uint32_t key = 0;
+  for (int cut = cut_k ? 0 : 1; cut < 3; ++cut) {
+    if (cut == 1 && !(p < 1.f)) continue;
+    unsigned long long target = (unsigned long long)k;
+    if (cut == 1) {             // the shortest prefix whose mass reaches p * z
+      target = (unsigned long long)((double)fmaxf(p, 0.f) * (double)z);
+      target = min(max(target, 1ull), z);
+    } else if (cut == 2) {      // the first token at which the running mass exceeds u * z
+      target = min((unsigned long long)(u * (double)z) + 1ull, z);
+    }
+    key = descend(each, sh, cut > 0, target);
+    *ties = sh.bin_cnt;
+    if (cut == 0) {             // mass of the k largest
+      z = sh.above_mass + (unsigned long long)((unsigned int)k - sh.above_cnt) * (sh.bin_mass / sh.bin_cnt);
+    } else {
+      const unsigned long long w = max(sh.bin_mass / sh.bin_cnt, 1ull);
+      const unsigned long long n = min(max((target - sh.above_mass + w - 1) / w, 1ull), (unsigned long long)sh.bin_cnt);
+      z = sh.above_mass + n * w;
+      *nth = (unsigned int)n;
+    }
+    __syncthreads();
   }
-  const int n = candidates<HELD>(r, sh, held, kmax, !top_k, target);
-  if (n == 0) return false;
-  // every element's place: how many and how much lies above it, how many share its key, how many of those come first
-  const bool mine = (int)threadIdx.x < n;
-  const uint32_t key = mine ? sh.lkey[threadIdx.x] : 0u;
-  const int id = mine ? sh.lid[threadIdx.x] : 0;
-  const unsigned long long mass = mine ? sh.lmass[threadIdx.x] : 0ull;
+  return key;
+}
+
+// The same for a short list of which each thread below n has an element (key, id and mass of all of them are in LDS): every
+// element's place is formed at once, how many and how much lies above it, how many share its key, how many of those
+// come first.
+__device__ void draw_by_rank(const Own& own, Shared& sh, int n, bool cut_k, int k, float p, double u, unsigned long long z,
+                             int32_t* out) {
   unsigned int above = 0, ties = 0, earlier = 0;
   unsigned long long above_mass = 0;
-  if (mine)
+  if (own.mine) {
+#pragma unroll 4
     for (int j = 0; j < n; ++j) {
       const uint32_t kj = sh.lkey[j];
-      if (kj > key) {
-        above += 1;
-        above_mass += sh.lmass[j];
-      } else if (kj == key) {
-        ties += 1;
-        earlier += sh.lid[j] < id;
-      }
+      const unsigned long long mj = sh.lmass[j];
+      const int ij = sh.lid[j];
+      above += kj > own.key;
+      above_mass += kj > own.key ? mj : 0ull;
+      ties += kj == own.key;
+      earlier += kj == own.key && ij < own.id;
     }
-  const bool first = mine && earlier == 0;            // one element speaks for its key
-  const unsigned long long w = max(mass, 1ull), through = above_mass + mass * ties;
-  if (top_k) {
+  }
+  const bool first = own.mine && earlier == 0;            // one element speaks for its key
+  const unsigned long long w = max(own.mass, 1ull), through = above_mass + own.mass * ties;
+  if (cut_k) {
     if (first && above < (unsigned int)k && above + ties >= (unsigned int)k)
-      sh.above_mass = above_mass + (unsigned long long)((unsigned int)k - above) * mass;
+      sh.above_mass = above_mass + (unsigned long long)((unsigned int)k - above) * own.mass;
     __syncthreads();
     z = sh.above_mass;
     __syncthreads();
   }
+  unsigned long long target;
   if (p < 1.f) {
     target = (unsigned long long)((double)fmaxf(p, 0.f) * (double)z);
     target = min(max(target, 1ull), z);
@@ -360,11 +392,81 @@ __device__ bool sample_listed(const Row& r, Shared& sh, const f32x4* held, uint3
     __syncthreads();
   }
   target = min((unsigned long long)(u * (double)z) + 1ull, z);
-  if (mine && above_mass < target && through >= target) {
+  if (own.mine && above_mass < target && through >= target) {
     const unsigned long long nth = min(max((target - above_mass + w - 1) / w, 1ull), (unsigned long long)ties);
-    if (earlier + 1 == nth) *out = id;
+    if (earlier + 1 == nth) *out = own.id;
   }
+}
+
+// The chain over the threads' own elements, n of them.  ORDERED: the ids ascend with the threads.
+template <bool ORDERED>
+__device__ void draw_own(const Own& own, Shared& sh, int n, bool cut_k, int k, float p, double u, unsigned long long z,
+                         int32_t* out) {
+  if (n <= kMaxRanked) return draw_by_rank(own, sh, n, cut_k, k, p, u, z, out);
+  __syncthreads();                          // the descent's histograms take the list's place
+  unsigned int nth = 0, ties = 0;
+  const uint32_t key = cut_and_draw([&](auto f) { if (own.mine) f(own.key, [&] { return own.mass; }); }, sh, cut_k, k, p, u,
+                                    z, &nth, &ties);
+  const bool drawn = own.mine && own.key == key;
+  if (ties == 1) {
+    if (drawn) *out = own.id;
+    return;
+  }
+  if constexpr (ORDERED) {
+    const int lane = threadIdx.x % TL_WAVE, wave = threadIdx.x / TL_WAVE;
+    const unsigned long long all = __ballot(drawn);
+    if (lane == 0) sh.red32[wave] = __popcll(all);
+    __syncthreads();
+    unsigned int before = __popcll(all & ((1ull << lane) - 1));
+    for (int wv = 0; wv < wave; ++wv) before += sh.red32[wv];
+    if (drawn && before + 1 == nth) *out = own.id;
+  } else {          // the nth in ascending order of the ids: the nth largest of their complements
+    const uint32_t id = ~descend([&](auto f) { if (drawn) f(~(uint32_t)own.id, [] { return 0ull; }); }, sh, false, nth);
+    if (threadIdx.x == 0) *out = (int32_t)id;
+  }
+}
+
+// By way of a list of the row's largest elements; z is the row's mass where there is no top-k.  False: this row takes the
+// descent over all of its elements from `kmin` on.
+template <bool HELD>
+__device__ bool draw_listed(const Row& r, Shared& sh, const f32x4* held, uint32_t kmax, bool cut_k, int k, float p, double u,
+                            unsigned long long z, uint32_t* kmin, int32_t* out) {
+  unsigned long long target;
+  if (cut_k) {
+    target = (unsigned long long)k;
+  } else {
+    target = p < 1.f ? min(max((unsigned long long)((double)fmaxf(p, 0.f) * (double)z), 1ull), z)
+                     : min((unsigned long long)(u * (double)z) + 1ull, z);
+  }
+  const int n = candidates<HELD>(r, sh, held, kmax, !cut_k, target, kmin);
+  if (n == 0) return false;
+  Own own = {(int)threadIdx.x < n, 0u, 0, 0ull};
+  if (own.mine) {
+    own.key = sh.lkey[threadIdx.x];
+    own.id = sh.lid[threadIdx.x];
+    own.mass = sh.lmass[threadIdx.x];
+  }
+  draw_own<false>(own, sh, n, cut_k, k, p, u, z, out);
   return true;
+}
+
+// Over all of the row's elements, read again in every pass (registers for 32 of them a thread would spill).  None below
+// `kmin` matters to any cut, and without them the passes' atomics meet less often, which pays for the search that did not
+// end in a list.
+__device__ void draw_from_all(const Row& r, Shared& sh, uint32_t kmin, bool cut_k, int k, float p, double u,
+                              unsigned long long z, int32_t* out) {
+  unsigned int nth = 0, ties = 0;
+  const uint32_t key = cut_and_draw(
+      [&](auto f) {
+        for (int i = threadIdx.x; i < r.vocab; i += S_THREADS) {
+          const float x = scaled(r, i);
+          const uint32_t key = order_key(x);
+          if (key >= kmin) f(key, [&] { return mass_of(r, x); });
+        }
+      },
+      sh, cut_k, k, p, u, z, &nth, &ties);
+  const int tok = nth_with_key(r, sh, key, nth);
+  if (threadIdx.x == 0) *out = tok;
 }
 
 __global__ __launch_bounds__(S_THREADS) void sample_kernel(
@@ -453,48 +555,38 @@ __global__ __launch_bounds__(S_THREADS) void sample_kernel(
     __syncthreads();
   }
 
+  int32_t* token = out + row;
+  const bool finite = fabsf(r.xmax) < INFINITY;       // else there are no masses to rank
+  if (finite && vocab <= S_THREADS) {       // an element a thread: no list to look for
+    Own own = {(int)threadIdx.x < vocab, 0u, (int)threadIdx.x, 0ull};
+    if (own.mine) {
+      const float x = scaled(r, threadIdx.x);
+      own.key = order_key(x);
+      own.mass = mass_of(r, x);
+      if (vocab <= kMaxRanked) {
+        sh.lkey[threadIdx.x] = own.key;
+        sh.lid[threadIdx.x] = own.id;
+        sh.lmass[threadIdx.x] = own.mass;
+      }
+    }
+    __syncthreads();
+    return draw_own<true>(own, sh, vocab, cut_k, k, p, u, z, token);
+  }
+
   // Rows of 32,000 logits with the default options (temperature 0.7, the 50 best, mass 0.95): 154 us for one row and 163
-  // us for 64 by the descent, 20 and 22 us from the list; 128,256 logits 569 and 63 us.  Without a top-k the list is
+  // us for 64 by the descent, 20 us from the list; 128,256 logits 569 and 63 us.  Without a top-k the list is
   // tried where the first cut cannot lie far down, the likeliest token holding a 64th of the mass or more (70 -> 23 us);
   // behind a flat row's first pass (normal logits: a thousandth) the list would only be found too short (70 -> 85 us).
-  // A maximum that is no finite number has no masses to rank.
-  if (fabsf(r.xmax) < INFINITY && (cut_k ? k <= kMaxListed : z < 64ull << 40)) {
-    const bool done = held_row ? sample_listed<true>(r, sh, held, kmax, k, p, u, z, out + row)
-                               : sample_listed<false>(r, sh, held, kmax, k, p, u, z, out + row);
+  // Where it is found too short all the same, what the search learned makes up for it (normal logits of spread 3, mass 0.9,
+  // 64 rows: 128 us by descents alone, 110 so); a row whose largest logit is so near zero that the first cut lies beyond
+  // the bins takes 3 to 5 % more.
+  uint32_t kmin = 0;
+  if (finite && (cut_k ? k <= kMaxListed : z < 64ull << 40)) {
+    const bool done = held_row ? draw_listed<true>(r, sh, held, kmax, cut_k, k, p, u, z, &kmin, token)
+                               : draw_listed<false>(r, sh, held, kmax, cut_k, k, p, u, z, &kmin, token);
     if (done) return;
   }
-
-  // top-k: mass of the k largest
-  if (cut_k) {
-    descend(r, sh, false, (unsigned long long)k);
-    const unsigned int ties = (unsigned int)k - sh.above_cnt;
-    const unsigned long long w = sh.bin_mass / sh.bin_cnt;
-    z = sh.above_mass + (unsigned long long)ties * w;
-    __syncthreads();
-  }
-
-  // top-p: shortest prefix whose mass reaches p * z
-  if (p < 1.f) {
-    unsigned long long target = (unsigned long long)((double)fmaxf(p, 0.f) * (double)z);
-    target = min(max(target, 1ull), z);
-    descend(r, sh, true, target);
-    const unsigned long long w = max(sh.bin_mass / sh.bin_cnt, 1ull);
-    unsigned long long ties = (target - sh.above_mass + w - 1) / w;
-    ties = min(max(ties, 1ull), (unsigned long long)sh.bin_cnt);
-    z = sh.above_mass + ties * w;
-    __syncthreads();
-  }
-
-  // multinomial: first token at which the running mass exceeds u * z
-  unsigned long long target = (unsigned long long)(u * (double)z) + 1ull;
-  target = min(target, z);
-  const uint32_t key = descend(r, sh, true, target);
-  const unsigned long long w = max(sh.bin_mass / sh.bin_cnt, 1ull);
-  unsigned long long nth = (target - sh.above_mass + w - 1) / w;
-  nth = min(max(nth, 1ull), (unsigned long long)sh.bin_cnt);
-  __syncthreads();
-  const int tok = nth_with_key(r, sh, key, (unsigned int)nth);
-  if (threadIdx.x == 0) out[row] = tok;
+  draw_from_all(r, sh, kmin, cut_k, k, p, u, z, token);
 }
 
 }  // namespace

@@ -767,7 +767,12 @@ __global__ __launch_bounds__(kThreads) void head_products_kernel(const TI* __res
 // 2 x 2 tiles of v_mfma_f32_16x16x32_bf16; both operands go straight from memory into registers (a
 // lane's eight consecutive k of one row).  The product is computed transposed (columns as the
 // instruction's rows), so a lane ends with four consecutive output columns of one row.
-template <typename TO>
+// STEPS: k steps of 32 whose operands are requested together, each with a sum of its own.  With few rows the kernel is its
+// round trips to memory and takes four: 6 rows of 16 heads, 512 -> 128, 7.0 us one by one and 6.1 so.  Four sums also keep its
+// error where the kernel of few rows has it (5.7e-8 of the result against 64 bits; in one sum 8.5e-8).  Many rows find
+// their operands in the caches and lose waves by it: 64 rows of 16 heads, 128 -> 512, 6.1 us by one step and 6.3 by four.
+constexpr int kHeadFewRows = 32;
+template <typename TO, int STEPS>
 __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* __restrict__ in, int64_t in_stride,
                                                                   int in_head_width, const bf16_t* __restrict__ w,
                                                                   TO* __restrict__ out, int64_t out_stride,
@@ -783,17 +788,18 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
     wp[a] = w + ((int64_t)h * cols + min(col0 + a * 16 + c, cols - 1)) * inner;
     xp[a] = in + (int64_t)min(row0 + a * 16 + c, n_rows - 1) * in_stride + (int64_t)h * in_head_width;
   }
-  f32x4 acc[2][2];
+  f32x4 sum[STEPS][2][2];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int p = 0; p < STEPS; ++p)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) sum[p][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  // four steps' operands are requested together: with few rows the kernel is its round trips to memory
-  for (int k0 = 0; k0 < inner; k0 += 128) {
-    bf16x8 wa[4][2], xb[4][2];
+  for (int k0 = 0; k0 < inner; k0 += STEPS * 32) {
+    bf16x8 wa[STEPS][2], xb[STEPS][2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < STEPS; ++u) {
       const int d0 = k0 + u * 32 + g * 8;
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
@@ -802,12 +808,23 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
       }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < STEPS; ++u)
+      if (u == 0 || k0 + u * 32 < inner) {       // uniform
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][a], xb[u][b], acc[a][b], 0, 0, 0);
+          for (int b = 0; b < 2; ++b)
+            sum[u][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][a], xb[u][b], sum[u][a][b], 0, 0, 0);
+      }
   }
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if constexpr (STEPS == 4) acc[a][b] = (sum[0][a][b] + sum[1][a][b]) + (sum[2][a][b] + sum[3][a][b]);
+      else acc[a][b] = sum[0][a][b];
+    }
   // acc[a][b][i] = out[row0 + b*16 + c][col0 + a*16 + g*4 + i]
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
@@ -995,12 +1012,13 @@ int tl_head_gemm(const void* in, int64_t in_stride, int in_head_width, const voi
       in_stride % 8 || in_head_width % 8 || (n_rows + 63) / 64 > 65535 || (cols + 63) / 64 > 65535)
     return TL_ERR_ARG;
   dim3 g(heads, (cols + 63) / 64, (n_rows + 63) / 64), b(kThreads);
+  const bool few = n_rows <= kHeadFewRows;
   if (out_dtype == 0)
-    hipLaunchKernelGGL(head_gemm_bf16_kernel<float>, g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width,
+    hipLaunchKernelGGL((few ? head_gemm_bf16_kernel<float, 4> : head_gemm_bf16_kernel<float, 1>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width,
                        (const bf16_t*)w, (float*)out, out_stride, out_head_width, n_rows, inner, cols,
                        (const bf16_t*)gate, gate_stride);
   else if (out_dtype == 1)
-    hipLaunchKernelGGL(head_gemm_bf16_kernel<bf16_t>, g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width,
+    hipLaunchKernelGGL((few ? head_gemm_bf16_kernel<bf16_t, 4> : head_gemm_bf16_kernel<bf16_t, 1>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width,
                        (const bf16_t*)w, (bf16_t*)out, out_stride, out_head_width, n_rows, inner, cols,
                        (const bf16_t*)gate, gate_stride);
   else

@@ -201,3 +201,16 @@ def test_every_expert_variant_weighs_by_score():
     w = {k: v.double() for k, v in random_weights(ODD, 1).items()}
     logits = plain.forward(ODD, w, random_tokens(20, ODD["vocab"], 0))
     assert logits.shape == (20, ODD["vocab"]) and torch.isfinite(logits).all()
+
+
+@pytest.mark.parametrize("dtype,head_dim,by_rows", [(torch.bfloat16, 128, False), (torch.bfloat16, 256, False),
+                                                    (torch.bfloat16, 264, True), (torch.float32, 128, True)])
+def test_a_layer_keeps_the_key_products_weights_once(dtype, head_dim, by_rows):
+    """W_uk is laid out for the products by rows only where steps of few rows take them; the matrix cores read it as the
+    many rows do."""
+    from tiny_llm_amd.parts.latent_attention import LatentAttention
+    layer = LatentAttention("a", dtype, "cpu", hidden_size=64, num_heads=2, head_dim=head_dim, rot_dim=0, value_dim=16,
+                            q_rank=0, kv_rank=32, scale=1.0, eps=1e-5, gated=False)
+    layer.bind({w.name: torch.zeros(w.shape, dtype=dtype) for w in layer.weights()})
+    assert (layer.w_uk_few is not None) == by_rows
+    assert tuple(layer.w_uk_t.shape) == (2, 32, head_dim)

@@ -92,6 +92,9 @@ class LatentAttention(Mixer):
         self.kv_off = _pad8(self.q_rank or self.q_width)
         self.g_off = self.kv_off + (0 if self.shares_cache else _pad8(self.kv_rank + self.rot_dim))
         self.down_width = self.g_off + _pad8(self.gate_width)
+        # Few rows' products with W_uk by rows or on the matrix cores: 6 rows of 16 heads, 128 -> 512, take 8.7 us by rows and
+        # 3.8 on the matrix cores; 512 -> 128, four times the round trips, 6.1 (`_project_heads` has 5.2 for it).
+        self.keys_by_rows = dtype != torch.bfloat16 or self.head_dim > 256
         self.w_down = self.w_uq = self.w_uk_t = self.w_uv = self.w_o = self.w_uk_few = self.w_uv_few = None
         self.w_dq_norm = self.w_dkv_norm = self.sinks = None
 
@@ -137,7 +140,7 @@ class LatentAttention(Mixer):
         self.w_uk_t = uk.transpose(1, 2).contiguous()
         self.w_uv = tensors[n["uv"]].contiguous()
         # the same two as [heads, inner, cols], for the one-launch products of steps with few rows
-        self.w_uk_few = ops.head_product_weights(uk)
+        self.w_uk_few = ops.head_product_weights(uk) if self.keys_by_rows else None
         self.w_uv_few = ops.head_product_weights(self.w_uv.view(H, self.value_dim, self.kv_rank).transpose(1, 2))
         # for steps of few rows the value products are rows against the weights of each row's own head: row t * H + n
         # takes head n (the table the per-row kernel of the experts looks its weights up in)
@@ -184,9 +187,7 @@ class LatentAttention(Mixer):
         few = T <= ops.HEAD_PRODUCT_ROWS and max(D, KR) <= ops.HEAD_PRODUCT_INNER
         gemm = self.dtype == torch.bfloat16 and q.stride(0) % 8 == 0     # one launch on the matrix cores
         many = gemm and not few
-        # few rows with a short inner size too: 6 rows of 16 heads, 128 -> 512, take 8.7 us by rows and 2.8 on the matrix
-        # cores; 512 -> 128, four times the round trips, 6.5 (`_project_heads` has 5.2 for it)
-        if few and not (gemm and D <= 256 and D % 8 == 0 and R % 8 == 0):
+        if few and self.keys_by_rows:
             ops.head_products(q3[:, :, :D], self.w_uk_few, qa[:, :, :KR])
         elif gemm:
             ops.head_gemm(q3[:, :, :D], self.w_uk_t, qa[:, :, :KR])

@@ -670,9 +670,14 @@ def test_gated_experts_by_every_route(dtype, tokens):
 
 
 @pytest.mark.parametrize("H,G,D,V,taps", [(4, 2, 16, 8, 4), (3, 3, 24, 40, 2), (2, 1, 64, 64, 3), (1, 1, 128, 128, 4),
-                                          (3, 1, 5, 9, 3)])
+                                          (3, 1, 5, 9, 3),
+                                          (1, 1, 256, 256, 4), (2, 1, 256, 132, 4), (2, 2, 192, 160, 3), (1, 1, 200, 256, 2),
+                                          (2, 1, 32, 48, 4), (1, 1, 17, 8, 2), (2, 2, 33, 128, 3), (1, 1, 132, 4, 1),
+                                          (344, 344, 40, 24, 3), (352, 176, 128, 32, 4), (342, 342, 12, 132, 2)])
 def test_delta_state_over_slots_and_tiny_portions(H, G, D, V, taps):
-    """The delta rule's kernels alone with one decay per head, full-rank pre-activations and the SiLU gate: three
+    """The delta rule's kernels alone with one decay per head, full-rank pre-activations and the SiLU gate, with every split
+    of a decode step's heads over threads (4, 8 and 16 slices, one and two channels a thread, heads of the most channels
+    and columns, few and more than 1,024 pairs of request and head): three
     requests of unequal length in slots out of order, fed in portions of 1 to 7 tokens (single tokens take the one-kernel
     decode step), against the plain scan over each whole sequence."""
     from tiny_llm_amd.parts.delta_rule import ChannelDelta

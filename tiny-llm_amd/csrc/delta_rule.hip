@@ -337,9 +337,9 @@ __device__ __forceinline__ void store_saved(float* __restrict__ saved, const flo
 // State phase of the kernel: thread (sl, cq) keeps rows [sl * DS, (sl + 1) * DS) of the FOUR value columns
 // 4 cq .. 4 cq + 3 of S in registers (16-byte loads and stores: a lane that moves four bytes at a time gets a
 // fraction of what a compute unit can fetch), the slices' partial sums meet in LDS in a fixed order.  There are few
-// (request, head) pairs, so a workgroup is as wide as it may be: 16 slices (8 beyond 128 columns) where four kept two
-// waves busy for 32 rows each, and a thread per channel of q, k and v: 16.9 -> 9.9 us for 6 requests of 16
-// heads of 128 x 128.
+// (request, head) pairs as a rule, so a workgroup is as wide as it may be: 16 slices where four kept two waves busy for 32
+// rows each, and a thread per channel of q, k and v: 16.9 -> 9.9 us for 6 requests of 16 heads of 128 x 128
+// (tl_delta_decode says where it is narrower).
 template <typename T, typename TZ, int DS>
 __global__ __launch_bounds__(kDecodeThreads) void delta_decode_kernel(
     const T* __restrict__ p, int64_t p_stride, int conv_off, int b_off, const float* __restrict__ a, int64_t a_stride,
@@ -548,10 +548,19 @@ int tl_delta_decode(const void* p, int64_t p_stride, int conv_off, int b_off, co
       vdim > kDecodeCols || vdim % 4 || state_stride % 4 || taps < 1 || taps > 4 ||
       (update_saved && heads != kv_heads) || gate_kind < 0 || gate_kind > 1 || !a || !gate)
     return TL_ERR_ARG;
-  // a thread per column quad and slice, and at most two of the head's channels a thread
-  const int quads = vdim / 4, slices = quads <= 32 ? 16 : 8;
+  // A thread per column quad and slice.  16 slices of the key channels (8 beyond 128 columns); fewer where a slice would
+  // have less than four of them (4 heads of 32 x 32: 6.8 us by 16, 6.5 by 8; of 8 x 8: 6.8 by 16, 6.1 by 4).  With 1,024
+  // (request, head) pairs, four a unit, waves beyond the state's own are in the way: 8 slices, and two of the head's
+  // channels a thread (64 requests of 16 heads of 128 x 64: 23.9 us by 16 slices and a channel a thread, 17.8 so; 128 x
+  // 128: 28.8 and 24.8; 32 heads of 64 x 128, 32 and 64 requests: 0.76 and 0.84 of the time).
+  const int quads = vdim / 4;
+  const bool many = (int64_t)n_requests * heads >= 1024;
+  int slices = dim <= 16 ? 4 : dim <= 32 || many ? 8 : 16;
+  if (quads > 32 && slices > 8) slices = 8;
+  const int items = 2 * dim + vdim;         // the head's channels: at most two a thread, and a thread a key channel
   int threads = quads * slices;
-  if (threads < 2 * dim + vdim) threads = 2 * dim + vdim;
+  const int least = many ? (dim > (items + 1) / 2 ? dim : (items + 1) / 2) : items;
+  if (threads < least) threads = least;
   threads = threads > kDecodeThreads ? kDecodeThreads : (threads + TL_WAVE - 1) / TL_WAVE * TL_WAVE;
   const int ds = (dim + slices - 1) / slices;
   dim3 g(n_requests, heads), b(threads);

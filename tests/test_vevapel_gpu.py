@@ -669,6 +669,40 @@ def test_gated_experts_by_every_route(dtype, tokens):
     assert err < (1e-5 if dtype == "float32" else 3e-2)
 
 
+@pytest.mark.parametrize("dim,vdim", [(8, 8), (30, 32), (32, 40), (36, 33), (50, 64), (64, 32), (66, 31), (128, 64), (130, 32), (256, 40)])
+def test_delta_recurrence_of_every_length_of_chunk(dim, vdim):
+    """`delta_recurrence` alone, whole vectors and not, for every number of key channels a lane keeps: portions of one
+    token, around the 16 that are staged together, and none at all (its state stays), from states that hold something.
+    Bound: an output is a sum of `dim` products in at least 32 parts (less than 20 roundings) over a state of up to 33
+    updates of two roundings, 90 * 2^-24 = 5e-6 of the largest term; four times that."""
+    from tiny_llm_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(dim)
+    H, lens, slots = 3, [1, 16, 0, 2, 33, 15, 17, 4], [6, 0, 9, 3, 8, 1, 7, 2]
+    T = sum(lens)
+    unit = lambda *n: torch.nn.functional.normalize(torch.randn(*n, generator=g), dim=-1)
+    q, k, v = unit(T, H, dim), unit(T, H, dim), torch.randn(T, H, vdim, generator=g)
+    beta, decay = torch.rand(T, H, generator=g), 0.5 + 0.5 * torch.rand(T, H, dim, generator=g)
+    state = torch.randn(10, H * dim * vdim + 4, generator=g)
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32)
+    want, S_all = torch.zeros(T, H, vdim, dtype=torch.float64), state.double().clone()
+    for r, (n, slot) in enumerate(zip(lens, slots)):
+        S = S_all[slot, :H * dim * vdim].view(H, dim, vdim)
+        for t in range(int(cu[r]), int(cu[r]) + n):
+            S *= decay[t].double()[:, :, None]
+            u = beta[t].double()[:, None] * (v[t].double() - torch.einsum("hdv,hd->hv", S, k[t].double()))
+            S += k[t].double()[:, :, None] * u[:, None, :]
+            want[t] = torch.einsum("hdv,hd->hv", S, q[t].double())
+    st, out = state.cuda(), torch.empty(T * H * vdim, device="cuda")
+    flat = lambda x: x.reshape(-1).cuda()
+    ops.delta_recurrence(flat(q), flat(k), flat(v), flat(beta), flat(decay), st, cu.cuda(),
+                         torch.tensor(slots, dtype=torch.int32, device="cuda"), out, H, dim, vdim)
+    assert (out.double().cpu().view(T, H, vdim) - want).abs().max() <= 2e-5 * want.abs().max()
+    assert (st.double().cpu() - S_all).abs().max() <= 2e-5 * S_all.abs().max()
+    untouched = [s for s in range(10) if s not in slots or lens[slots.index(s)] == 0]
+    assert torch.equal(st.cpu()[untouched], state[untouched]) and torch.equal(st.cpu()[:, -4:], state[:, -4:])
+
+
 @pytest.mark.parametrize("H,G,D,V,taps", [(4, 2, 16, 8, 4), (3, 3, 24, 40, 2), (2, 1, 64, 64, 3), (1, 1, 128, 128, 4),
                                           (3, 1, 5, 9, 3),
                                           (1, 1, 256, 256, 4), (2, 1, 256, 132, 4), (2, 2, 192, 160, 3), (1, 1, 200, 256, 2),

@@ -172,10 +172,6 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
   if (t1 <= t0) return;                           // a padding request owns no state
   const bool live = col < vdim;
   float* S_mem = state + (int64_t)state_slots[r] * state_stride + (int64_t)h * dim * vdim + col;
-  float S[DS];
-#pragma unroll
-  for (int i = 0; i < DS; ++i) S[i] = (live && s * DS + i < dim) ? S_mem[(int64_t)(s * DS + i) * vdim] : 0.f;
-
   constexpr int V = VEC ? 4 : 1, PIECES = (PER + V - 1) / V;
   typedef float piece __attribute__((ext_vector_type(V)));
   piece rk[PIECES], rq[PIECES], rg[PIECES];
@@ -203,7 +199,19 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
     }
     rb = (tid < kCh && tc + tid < t1) ? beta[(int64_t)(tc + tid) * heads + h] : 0.f;
   };
+  // The state is requested behind the first chunk, which is staged (and its k . q formed) while the state is on its way: a
+  // portion of a few tokens is little else.  32 requests of 32 heads and two tokens, 64 x 128, behind the state 18.9 us, so
+  // 16.5.  With 32 rows a lane the two are more loads than a wave can tell apart (63), so that it would wait for all.
+  float S[DS];
+  if constexpr (DS == 32) {
+#pragma unroll
+    for (int i = 0; i < DS; ++i) S[i] = (live && s * DS + i < dim) ? S_mem[(int64_t)(s * DS + i) * vdim] : 0.f;
+  }
   fetch(t0);
+  if constexpr (DS < 32) {
+#pragma unroll
+    for (int i = 0; i < DS; ++i) S[i] = (live && s * DS + i < dim) ? S_mem[(int64_t)(s * DS + i) * vdim] : 0.f;
+  }
   for (int tc = t0; tc < t1; tc += kCh) {
     __syncthreads();                              // the chunk before has been read
 #pragma unroll
@@ -220,17 +228,19 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
     if (tid < kCh) bs[tid] = rb;
     __syncthreads();
     if (tc + kCh < t1) fetch(tc + kCh);           // on its way while this chunk is worked on
+    const int n = min(kCh, t1 - tc);
     {                                             // k . q of the chunk's tokens, sixteen threads a token
       static_assert(kRecThreads == 16 * kCh, "sixteen threads a token");
       const int tt = tid / 16;
-      float kq = 0.f;
+      if (tt < n) {
+        float kq = 0.f;
 #pragma unroll
-      for (int i = 0; i < DP / 16; ++i) kq = fmaf(ks[tt][tid % 16 + i * 16], qs[tt][tid % 16 + i * 16], kq);
-      kq = group_sum<16>(kq);
-      if (tid % 16 == 0) kqs[tt] = kq;
+        for (int i = 0; i < DP / 16; ++i) kq = fmaf(ks[tt][tid % 16 + i * 16], qs[tt][tid % 16 + i * 16], kq);
+        kq = group_sum<16>(kq);
+        if (tid % 16 == 0) kqs[tt] = kq;
+      }
     }
     __syncthreads();
-    const int n = min(kCh, t1 - tc);
     // With S' = diag(g) S:  o = (S' + k u^T)^T q = S'^T q + u (k . q).  Both sums over S' are
     // taken in ONE pass (in four independent parts) and meet in one round of exchanges between the
     // slices; the update of S hangs off it.  A token's operands are read from LDS while the token before
@@ -524,14 +534,19 @@ int tl_delta_recurrence(const float* qn, const float* kn, const float* vc, const
     return TL_ERR_ARG;
   dim3 g(n_requests, heads, (vdim + kRecCols - 1) / kRecCols), b(kRecThreads);
   const bool vec = dim % 4 == 0 && !(((uintptr_t)qn | (uintptr_t)kn | (uintptr_t)decay) & 15);
-#define TL_REC(DS)                                                                                                   \
-  hipLaunchKernelGGL((vec ? delta_recurrence_kernel<DS, true> : delta_recurrence_kernel<DS, false>), g, b, 0, stream, \
-                     qn, kn, vc, beta, decay, state, state_stride, cu_seqlens, state_slots, out, heads, dim, vdim)
-  if (dim <= 16) TL_REC(2);
-  else if (dim <= 32) TL_REC(4);
-  else if (dim <= 64) TL_REC(8);
-  else if (dim <= 128) TL_REC(16);
-  else TL_REC(32);
+#define TL_REC(DS, VEC)                                                                                           \
+  hipLaunchKernelGGL((delta_recurrence_kernel<DS, VEC>), g, b, 0, stream, qn, kn, vc, beta, decay, state, state_stride, \
+                     cu_seqlens, state_slots, out, heads, dim, vdim)
+  // Up to 32 channels a thread stages two elements at most; vectors leave half the threads without a piece and cost 13
+  // registers, two waves a SIMD
+  if (dim <= 16) TL_REC(2, false);
+  else if (dim <= 32) TL_REC(4, false);
+  else if (dim <= 64 && vec) TL_REC(8, true);
+  else if (dim <= 64) TL_REC(8, false);
+  else if (dim <= 128 && vec) TL_REC(16, true);
+  else if (dim <= 128) TL_REC(16, false);
+  else if (vec) TL_REC(32, true);
+  else TL_REC(32, false);
 #undef TL_REC
   return tl_launch_status();
 }

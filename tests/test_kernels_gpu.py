@@ -54,7 +54,7 @@ def test_rmsnorm(dtype, hidden):
         assert rel(out, ref) < tol(dtype, 2e-6, 5e-3)
 
 
-@pytest.mark.parametrize("hidden", [4, 2044, 2048, 2052, 2050, 8192, 8193, 8196])
+@pytest.mark.parametrize("hidden", [4, 252, 256, 260, 2044, 2048, 2052, 2050, 8192, 8193, 8196])
 def test_norms_by_vectors_and_by_elements(hidden):
     """The norm kernels around the widths at which they change their form, rows that begin off a vector's boundary among
     them: against float64.  Statistics and results are float32 (a few 2^-24 of the normed size, sums of `hidden` terms)."""

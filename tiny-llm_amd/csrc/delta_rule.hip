@@ -229,24 +229,24 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
     __syncthreads();
     if (tc + kCh < t1) fetch(tc + kCh);           // on its way while this chunk is worked on
     const int n = min(kCh, t1 - tc);
-    {                                             // k . q of the chunk's tokens, sixteen threads a token
+    // k . q of the chunk's tokens, sixteen threads a token (all sixteen: skipping those that are not there cost 801 tokens 3 %)
+    {
       static_assert(kRecThreads == 16 * kCh, "sixteen threads a token");
       const int tt = tid / 16;
-      if (tt < n) {
-        float kq = 0.f;
+      float kq = 0.f;
 #pragma unroll
-        for (int i = 0; i < DP / 16; ++i) kq = fmaf(ks[tt][tid % 16 + i * 16], qs[tt][tid % 16 + i * 16], kq);
-        kq = group_sum<16>(kq);
-        if (tid % 16 == 0) kqs[tt] = kq;
-      }
+      for (int i = 0; i < DP / 16; ++i) kq = fmaf(ks[tt][tid % 16 + i * 16], qs[tt][tid % 16 + i * 16], kq);
+      kq = group_sum<16>(kq);
+      if (tid % 16 == 0) kqs[tt] = kq;
     }
     __syncthreads();
     // With S' = diag(g) S:  o = (S' + k u^T)^T q = S'^T q + u (k . q).  Both sums over S' are
     // taken in ONE pass (in four independent parts) and meet in one round of exchanges between the
     // slices; the update of S hangs off it.  A token's operands are read from LDS while the token before
     // it is worked on (two register sets, the loop goes two tokens at a time).  What a token costs is what its
-    // waves issue (two a SIMD): with k . q in every wave and the sums exchanged one by one 801 tokens (five shorter prompts beside them) took 364 us,
-    // now 319; 16 slices of half the rows, 4 columns a wave: 294, but 18 -> 26 us for eight prompts of 13 tokens.
+    // waves issue (two a SIMD): with k . q in every wave and the sums exchanged one by one 801 tokens (five shorter prompts
+    // beside them) took 314 us, now 275.  16 slices of half the rows, 4 columns a wave, took 8 % less for them in an
+    // earlier form, but 1.45 times as long for eight prompts of 13 tokens.
     auto load = [&](int tt, float* k, float* q, float* g, float& v, float& bt, float& kq) {
 #pragma unroll
       for (int i = 0; i < DS; ++i) {

@@ -515,14 +515,16 @@ def test_latent_window_and_sink_find_one_key(kernel, window, heads):
 
 @pytest.mark.parametrize("kernel", ["general float32", "matrix cores", "matrix cores, many rows"])
 @pytest.mark.parametrize("window,heads", [(9, 6), (40, 3), (0, 16)])
-def test_latent_attention_of_a_prompt(kernel, window, heads):
+@pytest.mark.parametrize("C,R", [(48, 16), (512, 64), (512, 56), (496, 64)])
+def test_latent_attention_of_a_prompt(kernel, window, heads, C, R):
     """One request's portion of 150 tokens behind 37 cached ones: tiles hold several tokens of the request, and
-    every row sees its own window."""
+    every row sees its own window.  A small size, the largest (whose kernels know it) and two beside it; the scale keeps
+    the scores' spread."""
     from tiny_llm_amd.kernels import ops
     from tiny_llm_amd.engine.step import tile_lists
     dtype = torch.float32 if "float32" in kernel else torch.bfloat16
     g = torch.Generator().manual_seed(window + heads)
-    n0, T, C, R, block = 37, 150, 48, 16, 8
+    n0, T, block = 37, 150, 8
     n = n0 + T
     lat, kr = torch.randn(n, C, generator=g), torch.randn(n, R, generator=g)
     table = torch.randperm(40, generator=g)[: -(-n // block)].tolist()
@@ -534,7 +536,7 @@ def test_latent_attention_of_a_prompt(kernel, window, heads):
     out = torch.empty(T, heads, C, dtype=dtype, device="cuda")
     tpt = 16 // min(heads, 16)
     dev = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
-    scale = 0.3
+    scale = 0.3 * (64 / (C + R)) ** 0.5
     if kernel.startswith("general"):
         ops.latent_attention(q.cuda(), l_pages, r_pages, bt, torch.zeros(T, dtype=torch.int32, device="cuda"), pos_dev, out,
                              scale, None, window, sinks.cuda())

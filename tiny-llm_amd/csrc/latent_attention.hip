@@ -179,8 +179,9 @@ __global__ __launch_bounds__(TL_WAVE) void latent_attention_kernel(
 // product as a sum of two bfloat16 terms (staged once per tile), so nothing of their float32 value is
 // lost against float32 scores over bfloat16 keys; scores, softmax and sums are float32.
 // A decode step's waves have a key tile or two each, so the kernel is a chain of latencies: requests made before
-// anything is waited for, scores in four sums, one merge through LDS instead of a round a wave: 28.9 -> 20 us with the
-// merge kernel for 6 tokens of 16 heads in a window of 512 (14 with the sizes known when compiled).
+// anything is waited for, scores in four sums, one merge through LDS instead of a round a wave: 6 tokens of 16 heads in a
+// window of 512, the merge kernel included, 30.3 -> 22.3 us for latents of 512 with 32 rotated dims, 22.8 -> 17.6 for 256
+// with 64, 15.9 -> 12.5 for 16 with 8; 512 with 64: 30.4 -> 12.7, see WHOLE.
 constexpr int LF_WAVES = 4;
 constexpr int LF_MAXKS = 18;        // (512 + 64) / 32 steps of the score product
 constexpr int LF_MAXDT = 32;        // 512 / 16 tiles of the output
@@ -206,8 +207,8 @@ __device__ __forceinline__ void lf_wave_sync() {      // a wave's LDS operations
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// WHOLE: latents of 512 and 64 rotated dims, the largest sizes, known when compiled (no test in front of every step:
-// 17.7 -> 11.9 us for 6 tokens of 16 heads in a window of 512, the merge included).
+// WHOLE: latents of 512 and 64 rotated dims, the largest sizes, known when compiled, so that no test stands in front of
+// every step (12.7 us where 496 with 64 take 22.2).
 template <bool WHOLE>
 __global__ __launch_bounds__(LF_WAVES * TL_WAVE) void latent_flash_bf16_kernel(
     const float* __restrict__ qa, const bf16_t* __restrict__ latent, const bf16_t* __restrict__ rope,
@@ -417,8 +418,10 @@ __global__ __launch_bounds__(LF_WAVES * TL_WAVE) void latent_flash_bf16_kernel(
 // LDS.  A wave keeps its own (max, sum, output): nothing is merged.
 // What bounds it is what a SIMD's one wave issues per 32 keys: 72 matrix instructions for the scores in four sums, 32
 // for the values (both halves of the keys in one operand, in the order in which the scores leave the registers), and
-// the output's rescaling only where a maximum rose.  2,048 tokens of 16 heads: 721 -> 514 us, in a window of 512 tokens
-// 287 -> 222 us (half the keys an instruction and every output rescaled, before).
+// the output's rescaling only where a maximum rose.  2,048 tokens of 16 heads: 707 -> 496 us, in a window of 512 tokens
+// 271 -> 209 us (half the keys an instruction and every output rescaled, before).  The form for other sizes takes every
+// register there is and keeps 12 values in scratch: 2,048 tokens, latents of 496 with 64 rotated dims 698 -> 621 us, of
+// 256 with 64 551 -> 474, of 64 with 32 414 -> 343; ten sizes in six shapes of step took 0.80 to 0.99 of the time before.
 constexpr int LP_KEYS = 32;         // keys a staged tile holds (two 16-key tiles of the products)
 constexpr int LP_NPF = 9;           // 16-byte pieces of a staged tile a thread fetches: 32 * 72 / 256
 // WHOLE: as in latent_flash_bf16_kernel.

@@ -1063,6 +1063,51 @@ def _fused_against_separate(nq, nkv, hd, bs, n_splits, window, seed):
     assert torch.equal(out3, out2) and torch.equal(kc3, kc2) and torch.equal(vc3, vc2)
 
 
+@pytest.mark.parametrize("nq,nkv,hd,bs,opts", [
+    (4, 4, 32, 16, {}), (15, 1, 64, 32, {}), (16, 1, 128, 16, {}), (8, 2, 128, 64, {"window": 65}), (6, 2, 64, 16, {"window": -100}),
+    (8, 2, 128, 16, {"window": 130, "keep": 5}), (4, 1, 64, 128, {"window": 64, "keep": 70, "softcap": 20.0}),
+    (4, 2, 32, 16, {"softcap": 15.0, "out_scale": 0.5}), (8, 2, 128, 16, {"sink": True, "finish": True, "window": 100}),
+    (8, 1, 64, 16, {"finish": True, "value_dim": 38, "f32": True}), (4, 1, 128, 16, {"value_dim": 100, "finish": True})])
+@pytest.mark.parametrize("n_splits", [1, 3])
+def test_decode_steps_without_tile_lists_give_the_bits_of_those_with(nq, nkv, hd, bs, opts, n_splits):
+    """Row i is request i's one new token: said by tile lists or known without (then pages of 16 keys and more and heads of
+    32, 64 and 128 have a kernel of their own).  The same products in the same order: the same bits, over every mask and
+    finish, contexts around the 64-key tiles and more splits than tiles, with NaN wherever no key of the request lies."""
+    opts = dict(opts)
+    f32, finish = opts.pop("f32", False), opts.pop("finish", False)
+    g = torch.Generator().manual_seed(nq * 131 + hd + bs)
+    lens = [1, 15, 16, 17, 63, 64, 65, 128, 191, 300, 513, 1]
+    R = len(lens)
+    mb = max(-(-l // bs) for l in lens) + 1
+    nblocks = sum(-(-l // bs) for l in lens) + 2
+    perm = (torch.randperm(nblocks - 1, generator=g) + 1).tolist()
+    bt = torch.full((R, mb), -1, dtype=torch.int32)
+    kc = torch.full((nblocks, nkv, bs, hd), float("nan"), dtype=torch.bfloat16)
+    vc = kc.clone()
+    for r, L in enumerate(lens):
+        for b in range(-(-L // bs)):
+            bt[r, b] = perm.pop()
+            rows = min(bs, L - b * bs)
+            kc[bt[r, b], :, :rows] = torch.randn(nkv, rows, hd, generator=g).to(torch.bfloat16)
+            vc[bt[r, b], :, :rows] = torch.randn(nkv, rows, hd, generator=g).to(torch.bfloat16)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    q = torch.randn(R, nq * hd + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :nq * hd]
+    if finish:
+        opts["gate"] = torch.randn(R, nq, generator=g).to(DEV)
+        if opts.get("sink"):
+            opts["sinks"] = torch.randn(nq, generator=g).to(DEV)
+    cols = nq * (opts.get("value_dim") or hd)
+    kc, vc, bt, pos = kc.to(DEV), vc.to(DEV), bt.to(DEV), i32([l - 1 for l in lens])
+    got = []
+    for tiles in ((i32(list(range(R))), i32(list(range(R))), i32([1] * R)), None):
+        out = torch.zeros(R, cols + 1, dtype=torch.float32 if f32 else torch.bfloat16, device=DEV)[:, :cols]
+        scratch = torch.full((n_splits * R * nq * (hd + 2),), float("nan"), device=DEV)
+        ops().flash_attention(q, kc, vc, bt, tiles, pos, out, nq, nkv, hd, hd ** -0.5, n_splits=n_splits, scratch=scratch, **opts)
+        got.append(out)
+    assert torch.isfinite(got[0].float()).all() and got[0].float().abs().max() > 0.1
+    assert torch.equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("hd", [48, 80, 112])
 def test_fused_rotation_head_sizes_that_end_inside_a_k_step(hd):
     """Head sizes that are no multiple of 32: the last k step of the score product has slots beyond

@@ -234,9 +234,11 @@ struct FusedRope {
 
 // Rotate-half of 8 dims starting at d0 (a multiple of 8): own chunk x, partner chunk y = the dims
 // d0 +- HD/2, with the 8 angles of the chunk in registers (c8, s8 = cos and sin of the pairs
-// j0 .. j0 + 7).  The expressions are rope_store_kernel's; how the compiler fuses their
-// multiplications and additions is its own choice in each kernel, so once in some ten thousand
-// elements the two kernels differ in the last bit of a rotated value.
+// j0 .. j0 + 7).  The products are fused here as written, so that the kernels of this file rotate alike to the bit.  The
+// expressions are rope_store_kernel's, where the compiler fuses as it likes: once in some ten thousand elements that kernel
+// differs in the last bit of a rotated value.
+__device__ __forceinline__ float rotated_first(float c, float s, float a, float b) { return fmaf(c, a, -(s * b)); }
+__device__ __forceinline__ float rotated_second(float c, float s, float a, float b) { return fmaf(s, a, c * b); }
 template <int HD>
 __device__ __forceinline__ bf16x8 rotate_chunk_regs(const bf16x8 x, const bf16x8 y, int d0, const float* c8,
                                                     const float* s8) {
@@ -246,7 +248,7 @@ __device__ __forceinline__ bf16x8 rotate_chunk_regs(const bf16x8 x, const bf16x8
   for (int e = 0; e < 8; ++e) {
     const float a = first ? (float)x[e] : (float)y[e];     // the pair's first-half value
     const float b = first ? (float)y[e] : (float)x[e];     // and its second-half value
-    r[e] = (bf16_t)(first ? c8[e] * a - s8[e] * b : s8[e] * a + c8[e] * b);
+    r[e] = (bf16_t)(first ? rotated_first(c8[e], s8[e], a, b) : rotated_second(c8[e], s8[e], a, b));
   }
   return r;
 }
@@ -638,6 +640,357 @@ __global__ __launch_bounds__(WAVES * TL_WAVE) void flash_attn_bf16_kernel(
         float* ml = part_ml + (((int64_t)split * n_tokens + t) * nq + h) * 2;
         ml[0] = M;       // in units of log2 e
         ml[1] = L;
+      }
+    }
+  }
+}
+
+// flash_decode_bf16_kernel: flash_attn_bf16_kernel for the steps it runs most, a decode step whose row i is the one new token of
+// request i (no tile lists), with pages of a power of two of at least 16 keys and heads of 32, 64 or 128.  The same tiles go
+// to the same waves and are worked on in the same order, so the results are the same to the bit.
+//
+// What bounds it is how many instructions a wave issues one after the other: there is one wave a SIMD, and with a context of
+// 15 keys in the caches flash_attn_bf16_kernel takes 5.65 us from its first instruction to its last, 0.9 of them waiting for
+// memory.  Here everything a row shares (position, key range, pages of 16 keys, addresses) is one scalar for the wave, the
+// waves need no division for their share of the tiles, the mask is applied to the tiles that need it, the rotated query and the
+// new key go through the same instructions (the key as a row of its own behind the G query rows), and the merge writes four
+// outputs a thread of the G rows there are: 3.9 us for those 15 keys, 6.4 where 576 keys a request took 10.2, none of 234
+// forms (1 to 64 requests of 9 to 32,768 keys) slower, the long ones 5 to 15 % faster.  Odd page sizes, other head sizes and
+// fused groups of 16 heads, which leave no row for the key, stay with flash_attn_bf16_kernel.
+template <int HDT, int WAVES, int KIND>
+__global__ __launch_bounds__(WAVES * TL_WAVE) void flash_decode_bf16_kernel(
+    const bf16_t* __restrict__ q, const int32_t* __restrict__ positions, const int32_t* __restrict__ block_tables,
+    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, int q_stride, int max_blocks, int bs_shift, int nkv,
+    int G, int n_splits, const FusedRope fused, float scale, KeyMask mask, const Finish fin, bf16_t* __restrict__ out,
+    int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, int n_tokens, int vec_out) {
+  constexpr int HD = HDT * 16;
+  static_assert(HD % 32 == 0 && TL_WAVE % (HD / 8) == 0, "a wave's load covers whole rows");
+  constexpr bool CAP = KIND == kMaskCapped, KEEPS = KIND == kMaskKeeps || CAP, FIN = KIND != kMaskPlain;
+  const int keep = KEEPS ? mask.keep : 0;
+  constexpr int KS = HD / 32;              // k-steps of the score product
+  constexpr int VS = HD + FA_VPAD;         // row stride of a wave's V tile in LDS
+  constexpr int WAVE_ELEMS = FA_KT * VS;
+  constexpr int VCH = HD / 8, VROWS = TL_WAVE / VCH;      // pieces of a value row, rows a load of the wave covers
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  bf16_t* smem = (bf16_t*)smem_raw;
+  const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TL_WAVE);
+  const int r16 = lane % 16, g = lane / 16;
+  const int tok = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
+  const int mine = split * WAVES + wave, stride = WAVES * n_splits;
+  const bool do_rope = fused.cos_t != nullptr;
+  bf16_t* Vl = smem + wave * WAVE_ELEMS;
+  // the first round trip: everything whose address the launch gives
+  const int32_t* bt = block_tables + (int64_t)tok * max_blocks;
+  int pg[4];
+#pragma unroll
+  for (int kt = 0; kt < 4; ++kt) pg[kt] = bt[min((mine * FA_KT + kt * 16) >> bs_shift, max_blocks - 1)];
+  const int pos = positions[tok];
+  // row r16 of the matrix tile: query head r16 of the group; behind them, in fused mode, the new token's key
+  const bf16_t* token_row = q + (int64_t)tok * q_stride;
+  const bf16_t* row = token_row + (r16 < G || !do_rope ? (kvh * G + min(r16, G - 1)) * HD : fused.k_off + kvh * HD);
+  bf16x8 x[KS], y, new_v;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) x[ks] = *(const bf16x8*)(row + ks * 32 + g * 8);
+  if (do_rope) {
+    if constexpr (KS == 1) y = *(const bf16x8*)(row + (g * 8 + HD / 2) % HD);
+    new_v = *(const bf16x8*)(token_row + fused.v_off + kvh * HD + (lane % VCH) * 8);
+  }
+  float row_sink = 0.f, row_gate = 0.f;
+  if constexpr (FIN) {
+    const int head = kvh * G + min(r16, G - 1);
+    if (fin.sinks) row_sink = fin.sinks[head];
+    if (fin.gate) row_gate = fin.gate[(int64_t)tok * fin.gate_stride + head];
+  }
+  // the key range and this wave's tiles: numbers mine, mine + stride, ... (see flash_attn_bf16_kernel)
+  const int kv_begin = first_visible_key(pos, mask.window), kv_end = pos + 1;
+  const int first_tile = kv_begin / FA_KT, new_tile = pos >> 6;
+  const int n_kept = KEEPS ? kept_key_tiles(keep, first_tile) : 0, skip = keep > 0 ? first_tile - n_kept : 0;
+  const int n_end = (kv_end + FA_KT - 1) / FA_KT - skip;
+  int n = mine;
+  bool looked_up = true;       // pg holds the pages of number n
+  if (keep > 0 || first_tile > 0) {
+    if (keep <= 0) n += first_tile / stride * stride;
+    if (keep <= 0 && n < first_tile) n += stride;
+    looked_up = n == mine && n < (keep > 0 ? n_kept : n_end);
+  }
+  auto tile_of = [&](int i) { return KEEPS && i >= n_kept ? i + skip : i; };
+  float m_run = kNegBig, l_run = 0.f;
+  f32x4 o[HDT];
+#pragma unroll
+  for (int dt = 0; dt < HDT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float c_log2 = CAP ? 1.f : scale * 1.44269504088896341f;
+  const float cap_in = CAP ? scale * 2.88539008177792681f / mask.cap : 0.f, cap_out = mask.cap * 1.44269504088896341f;
+
+  // A tile is fetched in groups of 16 keys, which lie in one page.  A group without a visible key reads from page 0; the rows
+  // of a group beyond the key range may hold anything: the mask replaces their scores, their values become zeros on the way
+  // to LDS (0 * NaN is NaN).
+  bf16x8 k_op[4][KS], v_stage[VCH];
+  int64_t at[4];               // elements from the start of a cache to each group
+  auto fetch = [&](int base) {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      const int j = base + kt * 16;
+      const bool any = (j + 15 >= kv_begin || (KEEPS && j < keep)) && j < kv_end;
+      const int page = any ? max(pg[kt], 0) : 0;
+      at[kt] = (int64_t)(((page * nkv + kvh) << bs_shift) + (j & ((1 << bs_shift) - 1))) * HD;
+    }
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) k_op[kt][ks] = *(const bf16x8*)(k_cache + at[kt] + (r16 * HD + g * 8 + ks * 32));
+#pragma unroll
+    for (int c = 0; c < VCH; ++c) v_stage[c] = *(const bf16x8*)(v_cache + at[c / KS] + (lane * 8 + (c % KS) * (TL_WAVE * 8)));
+  };
+  auto seen = [&](int j, int more) {      // key j + more: one comparison where no kept keys are
+    const bool in = (unsigned)(j - kv_begin + more) < (unsigned)(kv_end - kv_begin);
+    return KEEPS ? in || (j + more < keep && j + more < kv_end) : in;
+  };
+  int next_pages = 0;
+  auto look_up = [&](int i) { next_pages = bt[min((tile_of(i) * FA_KT + lane) >> bs_shift, max_blocks - 1)]; };
+  auto take_pages = [&]() {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) pg[kt] = __builtin_amdgcn_readlane(next_pages, kt * 16);
+  };
+  if (n < n_end) {
+    if (!looked_up) {
+      look_up(n);
+      take_pages();
+    }
+    fetch(tile_of(n) * FA_KT);
+    if (n + stride < n_end) look_up(n + stride);
+  }
+  // query rows (B operand), rotated in fused mode, and with them the new key: the angles of dims d and d + HD/2 are one
+  bf16x8 qf[KS];
+  if (do_rope) {
+    constexpr int SETS = KS > 1 ? KS / 2 : 1;
+    float c8[SETS][8], s8[SETS][8];
+    const float* cs = fused.cos_t + (int64_t)max(pos, 0) * (HD / 2);
+    const float* sn = fused.sin_t + (int64_t)max(pos, 0) * (HD / 2);
+#pragma unroll
+    for (int a = 0; a < SETS; ++a) {
+      const int j0 = (a * 32 + g * 8) % (HD / 2);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const f32x4 c4 = *(const f32x4*)(cs + j0 + h * 4), s4 = *(const f32x4*)(sn + j0 + h * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          c8[a][h * 4 + e] = c4[e];
+          s8[a][h * 4 + e] = s4[e];
+        }
+      }
+    }
+    if constexpr (KS == 1) {
+      qf[0] = rotate_chunk_regs<HD>(x[0], y, g * 8, c8[0], s8[0]);
+    } else {
+#pragma unroll
+      for (int a = 0; a < SETS; ++a)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float u = (float)x[a][e], v = (float)x[a + SETS][e];
+          qf[a][e] = (bf16_t)rotated_first(c8[a][e], s8[a][e], u, v);
+          qf[a + SETS][e] = (bf16_t)rotated_second(c8[a][e], s8[a][e], u, v);
+        }
+    }
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = x[ks];
+  }
+
+  for (; n < n_end; n += stride) {
+    const int base = tile_of(n) * FA_KT;
+    if (do_rope && base == new_tile * FA_KT) {
+      // the new token's key, of row 15, takes the place of what its cache row held, its value that of what was fetched; both
+      // go to the cache
+      const int at_row = pos % FA_KT;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const u32x4 mine4 = __builtin_bit_cast(u32x4, qf[ks]);
+        u32x4 key;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) key[w] = (uint32_t)dpp_i32<TL_DPP_ROW_LANE15>((int)mine4[w]);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+          if (kt == at_row / 16) {
+            if (r16 == at_row % 16) {
+              k_op[kt][ks] = __builtin_bit_cast(bf16x8, key);
+              *(bf16x8*)(fused.k_cache_w + at[kt] + (r16 * HD + g * 8 + ks * 32)) = k_op[kt][ks];
+            }
+          }
+      }
+#pragma unroll
+      for (int c = 0; c < VCH; ++c)
+        if (c == at_row / VROWS) {
+          if (lane / VCH == at_row % VROWS) {
+            v_stage[c] = new_v;
+            *(bf16x8*)(fused.v_cache_w + at[c / KS] + (lane * 8 + (c % KS) * (TL_WAVE * 8))) = new_v;
+          }
+        }
+    }
+    const bool all_seen = base + FA_KT <= kv_end && (base >= kv_begin || (KEEPS && base + FA_KT <= keep));
+    if (!all_seen) {
+#pragma unroll
+      for (int c = 0; c < VCH; ++c) {
+        const bf16x8 z = {};
+        if (!seen(base + lane / VCH, c * VROWS)) v_stage[c] = z;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < VCH; ++c) *(bf16x8*)(Vl + (c * VROWS + lane / VCH) * VS + (lane % VCH) * 8) = v_stage[c];
+    // scores, transposed: sc[kt][r] = S^T[key kt*16 + g*4 + r][row r16]
+    f32x4 sc[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      sc[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k_op[kt][ks], qf[ks], sc[kt], 0, 0, 0);
+    }
+    if (n + stride < n_end) {
+      take_pages();
+      fetch(tile_of(n + stride) * FA_KT);
+      if (n + 2 * stride < n_end) look_up(n + 2 * stride);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if constexpr (CAP) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[kt][r] = capped_score(sc[kt][r], cap_in, cap_out);
+    }
+    if (!all_seen) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (!seen(base + g * 4, kt * 16 + r)) sc[kt][r] = -INFINITY;
+    }
+    float m_tile = kNegBig;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m_tile = fmaxf(m_tile, sc[kt][r]);
+    m_tile = max_over_rows(m_tile);
+    const float m_new = fmaxf(m_run, m_tile * c_log2);   // the scale is positive: the maximum commutes
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    float psum = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(sc[kt][r], c_log2, -m_new));
+        sc[kt][r] = p;
+        psum += p;
+      }
+    psum = sum_over_rows(psum);
+    l_run = l_run * alpha + psum;
+    m_run = m_new;
+#pragma unroll
+    for (int dt = 0; dt < HDT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      // probabilities as two bfloat16 terms, p = hi + lo: the product then carries 16 bits of p
+      u32x4 hi, lo;
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        uint32_t h0, l0, h1, l1;
+        split_pair(sc[2 * st][2 * r], sc[2 * st][2 * r + 1], h0, l0);
+        split_pair(sc[2 * st + 1][2 * r], sc[2 * st + 1][2 * r + 1], h1, l1);
+        hi[r] = h0;
+        lo[r] = l0;
+        hi[2 + r] = h1;
+        lo[2 + r] = l1;
+      }
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, hi), pl = __builtin_bit_cast(bf16x8, lo);
+      const bf16_t* vsrc = Vl + ((2 * st) * 16 + g * 4 + r16 / 4) * VS + 4 * (r16 % 4);
+      bf16x8 vf[HDT];
+#pragma unroll
+      for (int dt = 0; dt < HDT; ++dt) {
+        const bf16x4 lo4 = lds_read_transposed(vsrc + dt * 16);
+        const bf16x4 hi4 = lds_read_transposed(vsrc + 16 * VS + dt * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          vf[dt][r] = lo4[r];
+          vf[dt][4 + r] = hi4[r];
+        }
+      }
+#pragma unroll
+      for (int dt = 0; dt < HDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb, o[dt], 0, 0, 0);
+#pragma unroll
+      for (int dt = 0; dt < HDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pl, o[dt], 0, 0, 0);
+    }
+    // this wave's reads of its area are done before the next tile is written over it
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+
+  // merge the waves: each leaves (m, l, O) of the group's rows in its own LDS area, whose tile only it has read
+  constexpr int MROW = HD + 4;
+  float* Mw = (float*)(smem + wave * WAVE_ELEMS);
+  if (r16 < G) {
+#pragma unroll
+    for (int dt = 0; dt < HDT; ++dt) *(f32x4*)(Mw + r16 * MROW + dt * 16 + g * 4) = o[dt];
+    if (g == 0) {
+      f32x4 ml = {m_run, l_run, 0.f, 1.f};
+      if constexpr (FIN) {
+        ml[2] = row_sink;
+        ml[3] = fin.gate ? mask.out_scale / (1.f + expf(-row_gate)) : mask.out_scale;
+      }
+      *(f32x4*)(Mw + r16 * MROW + HD) = ml;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < G * (HD / 4); e += WAVES * TL_WAVE) {      // four output elements a thread
+    const int r = e / (HD / 4), d = e % (HD / 4) * 4, h = kvh * G + r;
+    f32x4 ml[WAVES], part[WAVES];
+    float M = kNegBig;
+#pragma unroll
+    for (int wv = 0; wv < WAVES; ++wv) {
+      const float* area = (const float*)(smem + wv * WAVE_ELEMS) + r * MROW;
+      ml[wv] = *(const f32x4*)(area + HD);
+      part[wv] = *(const f32x4*)(area + d);
+    }
+#pragma unroll
+    for (int wv = 0; wv < WAVES; ++wv) M = fmaxf(M, ml[wv][0]);
+    float L = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int wv = 0; wv < WAVES; ++wv) {
+      const float wgt = __builtin_amdgcn_exp2f(ml[wv][0] - M);      // a wave without keys has l = 0 and O = 0
+      L += wgt * ml[wv][1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] += wgt * part[wv][i];
+    }
+    if (n_splits == 1) {
+      const float Ls = with_sink(L, M, fin.flags, FIN ? ml[0][2] : 0.f), f = FIN ? ml[0][3] : 1.f;
+      f32x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = Ls > 0.f ? acc[i] * f / Ls : 0.f;
+      const int width = FIN ? fin.vdim : HD;
+      const int64_t to = (int64_t)tok * out_stride + (int64_t)h * width + d;
+      if (vec_out) {      // uniform: pieces of four are whole and aligned
+        if (FIN && d >= width) continue;
+        if (fin.flags & kFlagOutF32) {
+          *(f32x4*)((float*)out + to) = v;
+        } else {
+          const bf16x4 b = {(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+          *(bf16x4*)(out + to) = b;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (!FIN || d + i < width) store_result(out, to + i, v[i], fin.flags);
+      }
+    } else {
+      const int64_t to = ((int64_t)split * n_tokens + tok) * nkv * G + h;
+      *(f32x4*)(part_o + to * HD + d) = acc;
+      if (d == 0) {
+        part_ml[to * 2] = M;       // in units of log2 e
+        part_ml[to * 2 + 1] = L;
       }
     }
   }
@@ -1532,8 +1885,30 @@ static int launch_flash_w(const bf16_t* q, int64_t q_stride, const bf16_t* k_cac
                           hipStream_t stream) {
   constexpr int HD = HDT * 16;
   constexpr size_t stage = (size_t)WAVES * FA_KT * (HD + FA_VPAD) * sizeof(bf16_t);
-  static_assert((size_t)FA_KT * (HD + FA_VPAD) * sizeof(bf16_t) >= 16 * (HD + 2) * sizeof(float),
+  static_assert((size_t)FA_KT * (HD + FA_VPAD) * sizeof(bf16_t) >= 16 * (HD + 4) * sizeof(float),
                 "a wave's merge area must fit its staging area");
+  if constexpr (HDT == 2 || HDT == 4 || HDT == 8) {
+    int bs_shift = -1;      // log2 of the page size where it is a power of two
+    for (int sh = 0; sh < 31; ++sh)
+      if ((1 << sh) == block_size) bs_shift = sh;
+    // Row 15 of the matrix tile is the new key's, so a fused group has at most 15 query heads.
+    if (!tile_req && bs_shift >= 4 && (!fused.cos_t || nq / nkv < 16) && q_stride <= 0x7fffffff &&
+        (n_splits == 1 || (uintptr_t)part_o % 16 == 0)) {
+      const int piece = fin.flags & kFlagOutF32 ? 16 : 8;      // bytes of four outputs
+      const bool vec_out = (uintptr_t)out % piece == 0 && out_stride % 4 == 0 && fin.vdim % 4 == 0;
+      static bool configured = false;
+      if (!configured) {
+        if (hipFuncSetAttribute((const void*)flash_decode_bf16_kernel<HDT, WAVES, KIND>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)stage) != hipSuccess)
+          return TL_ERR_LAUNCH;
+        configured = true;
+      }
+      hipLaunchKernelGGL((flash_decode_bf16_kernel<HDT, WAVES, KIND>), dim3(n_tiles, nkv, n_splits), dim3(WAVES * TL_WAVE),
+                         stage, stream, q, positions, block_tables, k_cache, v_cache, (int)q_stride, max_blocks, bs_shift, nkv,
+                         nq / nkv, n_splits, fused, scale, mask, fin, out, out_stride, part_o, part_ml, n_tokens, (int)vec_out);
+      return TL_OK;
+    }
+  }
   static bool configured = false;
   if (!configured) {
     if (hipFuncSetAttribute((const void*)flash_attn_bf16_kernel<HDT, WAVES, KIND>,

@@ -30,6 +30,7 @@ template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return
 typedef unsigned int tl_u32x2 __attribute__((ext_vector_type(2)));
 constexpr int TL_DPP_XOR1 = 0xB1, TL_DPP_XOR2 = 0x4E;              // quad_perm [1,0,3,2], [2,3,0,1]
 constexpr int TL_DPP_MIRROR = 0x140, TL_DPP_HALF_MIRROR = 0x141;   // lane 15 - i of the row, 7 - i of the half row
+constexpr int TL_DPP_ROW_LANE15 = 0x15F;                             // lane 15 of the row, to all of it
 constexpr int TL_DPP_ROR1 = 0x121, TL_DPP_ROR2 = 0x122, TL_DPP_ROR4 = 0x124, TL_DPP_ROR8 = 0x128;   // rotate the row
 template <int CTRL>
 __device__ __forceinline__ int dpp_i32(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false); }

@@ -351,6 +351,14 @@ def test_linear_residual_of_large_tiles(M, N):
     _operand_tiles(0, M, N, 64)
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 260, 64), (257, 516, 128), (1281, 258, 192), (2049, 260, 256), (2305, 514, 320),
+                                   (3329, 70, 448)])
+def test_linear_large_tile_in_quarters(M, N, K):
+    """The 256 x 256 tile replaces its operands by quarters, in pairs of k steps: one step, two, odd and even numbers, and
+    rows in bands of tiles (five and six in one band, nine in two, fourteen in three of which the last is not full)."""
+    _operand_tiles(1, M, N, K)
+
+
 def _operand_tiles(tile, M, N, K):
     g = torch.Generator().manual_seed(M + K + N)
     wide = torch.randn(M, K + 72, generator=g).to(torch.bfloat16)

@@ -450,7 +450,8 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const float* 
 // outputs as 32x32x16 MFMA tiles.  Operand tiles go global -> registers -> LDS; LDS is
 // double-buffered so an iteration needs one barrier, and the global loads of the next k step are
 // in flight while the current one is multiplied.  Or they go straight into LDS, three or four buffers in turn
-// (launch_gemm_bf16 says where), and the loads of the next two or three k steps are in flight.
+// (launch_gemm_bf16 says where), and the loads of the next two or three k steps are in flight; the 256 x 256 tile's two
+// buffers are replaced quarter by quarter (kPhased).
 //
 // Tile shapes: 256 x 256 (eight waves of 128 x 64), 256 x 128, 128 x 128 and 64 x 128.  The larger
 // the tile, the fewer operand bytes and LDS reads per flop and the higher the rate on a full chip;
@@ -470,8 +471,10 @@ constexpr int B_XCDS = 8;
 // that it is used; what it does not see is that the block holds a load, which needs a wait state behind that write: the
 // s_nop.  Whoever reads the data waits for it first (tl_wait_loads, then a barrier).
 typedef int tl_rsrc_words __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void tl_load_to_lds(tl_rsrc_words buf, void* dst, int voffset, int soffset) {
-  const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(__attribute__((address_space(3))) void*)dst);
+__device__ __forceinline__ unsigned int tl_lds_address(void* p) {
+  return __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(__attribute__((address_space(3))) void*)p);
+}
+__device__ __forceinline__ void tl_load_to_lds(tl_rsrc_words buf, unsigned int at, int voffset, int soffset) {
   asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :
                : "{m0}"(at), "v"(voffset), "s"(buf), "s"(soffset)
@@ -526,7 +529,8 @@ struct GemmShape {
 // K must be a multiple of 8 (16-byte chunks of bf16 never straddle the end).
 // How operand tiles get into LDS: through registers, zeros beyond the end of a row (kTail); through registers, the inner
 // size a multiple of the k step (kWhole); likewise, but straight from memory (kDirect).
-constexpr int kTail = 0, kWhole = 1, kDirect = 2;
+// Straight from memory in quarters, each replaced as soon as it has been read (kPhased: the 256 x 256 tile).
+constexpr int kTail = 0, kWhole = 1, kDirect = 2, kPhased = 3;
 // What is known of the residual where the epilogue is compiled (kNoResidual: none, or one of rows without whole vectors).
 constexpr int kNoResidual = 0, kResidual = 1, kAnyForm = 2;
 template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, int MODE>
@@ -538,7 +542,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
                                                                       int64_t lda, int64_t ldo, int k_per_split) {
   using S = GemmShape<BM, BN, WM, WN>;
   constexpr int MI = S::MI, NJ = S::NJ, THREADS = S::THREADS;
-  constexpr bool DIRECT = MODE == kDirect;
+  constexpr bool PHASED = MODE == kPhased, DIRECT = MODE == kDirect || PHASED;
   constexpr int LD = DIRECT ? B_BK : B_LD;              // row stride of a staged tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   constexpr int BUFS = DIRECT ? S::BUFS : 2;
@@ -555,12 +559,16 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   const int t_all = (blockIdx.x % B_XCDS) * per_xcd + blockIdx.x / B_XCDS;
   if (t_all >= total) return;                           // the grid is padded to a multiple of 8
   const int split = t_all / tiles, t = t_all % tiles;
-  const int m0 = (t % tiles_m) * BM, n0 = (t / tiles_m) * BN;
+  // The tiles that an XCD works on at a time make a block about as high as it is wide, which asks the fewest rows of both
+  // operands of its L2 (8192^3 in columns of 32 tiles 927 us, in bands of four 781): bands of 4 to 7 tiles of rows.
+  const int tiles_n = (N + BN - 1) / BN, bands = max(tiles_m / 4, 1), band_m = (tiles_m + bands - 1) / bands;
+  const int band = t / (band_m * tiles_n), in_band = t - band * band_m * tiles_n, high = min(band_m, tiles_m - band * band_m);
+  const int m0 = (band * band_m + in_band % high) * BM, n0 = in_band / high * BN;
   const int kbase = split * k_per_split;
   const int kend = k_per_split > 0 ? min(K, kbase + k_per_split) : K;
   if (k_per_split > 0) out += (int64_t)split * M * ldo;
   if (nm.tile_group) {      // uniform: this tile's rows belong to one group, with weights of its own
-    const int group = nm.tile_group[m0 / nm.group_rows];
+    const int group = __builtin_amdgcn_readfirstlane(nm.tile_group[m0 / nm.group_rows]);
     if (group < 0) return;
     w += (int64_t)group * nm.group_stride;
   }
@@ -640,7 +648,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     const bool is_a = p < S::AC;
     const int r = (is_a ? p : p - S::AC) * PASS + wave * 8;
     bf16_t* dst = is_a ? As + (buf * BM + r) * LD : Ws + (buf * BN + r) * LD;
-    tl_load_to_lds(is_a ? words_a : words_w, dst, piece_off[p], k0 * 2);
+    tl_load_to_lds(is_a ? words_a : words_w, tl_lds_address(dst), piece_off[p], k0 * 2);
   };
   // MFMA operands of one k16 step: NJ weight pieces, then MI activation pieces, in the order of use
   struct Frag {
@@ -684,6 +692,110 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   // kt + 2 are issued right after; the last k16 step of a tile is multiplied after the barrier,
   // while the first fragments of the next tile are on their way.
   const int nk = (kend - kbase + B_BK - 1) / B_BK;
+  if constexpr (PHASED) {
+    static_assert(BM == 256 && BN == 256 && WM == 2 && WN == 4 && BUFS == 2, "quarters of the 256 x 256 tile");
+    // With both operands through registers and one barrier a k step the matrix pipes were busy for 69 % of the time (8192^3;
+    // the loads of two whole buffers straight into LDS are too late, 1,138 us where registers take 889); so, 783 us.  2,048
+    // rows, 28,672 x 4,096: 428 -> 389 us (1.24 PFLOP/s); 4,096 x 14,336 260 -> 217, where half the units work and run at
+    // 2.2 GHz; on a full chip the part clocks at 1.7 to 1.75 GHz, and that bounds it.
+    // A k step is four items of 128 rows, in the order in which they are read: a weight half, the first half of the
+    // activations, the other weight half, the rest of the activations.  A half holds the rows that every wave needs for half
+    // of its outputs: of the activations 64 of each 128, of the weights 32 of each 64.  Which weight half comes first
+    // alternates from step to step, so that a phase of eight matrix instructions always has one new half to read.  Phase f
+    // reads item f + 1 into registers, asks for item f + 7 and waits for item f + 2: five items, a step and a quarter of
+    // work, stay on their way.  The waves of a SIMD take turns: while one multiplies, the other reads; between two barriers
+    // each half of the workgroup does one of the two, the second half a turn behind.  Item f + 7 takes the place of item
+    // f - 1: it was read in phase f - 2, and by the end of that phase's products, which both halves have behind them a
+    // barrier before the first asks for item f + 7, its reads have been waited for.
+    const unsigned int lds_wave = tl_lds_address(As + __builtin_amdgcn_readfirstlane(wave) * 8 * LD);
+    int off[2][2][2];                                      // of a thread's two pieces of an item: [weights][half][piece]
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        off[0][h][q] = (int)(((int64_t)(q * 128 + h * 64 + prow) * lda + pk) * 2);
+        off[1][h][q] = (int)(((int64_t)(q * 128 + prow / 32 * 64 + h * 32 + prow % 32) * K + pk) * 2);
+      }
+    // Half h of the operand's k step kt.  A step behind the last is asked for from a buffer of no bytes: it reads as zeros.
+    auto fill = [&](int buf, bool weights, int h, int kt) {
+      const unsigned int dst = lds_wave + ((weights ? BUFS * BM : 0) + (buf * 2 + h) * 128) * LD * 2;
+      tl_rsrc_words from = weights ? words_w : words_a;
+      from[2] = kt < nk ? from[2] : 0;
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        tl_load_to_lds(from, dst + q * 64 * LD * 2, off[weights][h][q], (kbase + min(kt, nk - 1) * B_BK) * 2);
+    };
+    bf16x8 fa[4][2], fw[2][4];                             // fragments of a half of the activations, of both weight halves
+    const bf16_t* pa = As + (wm * 64 + lane % 32) * LD;
+    const bf16_t* pw = Ws + (wn * 32 + lane % 32) * LD;
+    auto read_a = [&](int buf, int h) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          fa[ks][i] = *(const bf16x8*)(pa + ((buf * 2 + h) * 128 + i * 32) * LD + ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8);
+    };
+    auto read_w = [&](int buf, int h) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        fw[h][ks] = *(const bf16x8*)(pw + (buf * 2 + h) * 128 * LD + ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8);
+    };
+    auto meet = [&]() {
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // Phase P of the k step kt, whose weight half F comes first.
+    auto phase = [&](auto p_, auto first, int kt) {
+      constexpr int P = decltype(p_)::value, F = decltype(first)::value;
+      if constexpr (P == 0) read_a(F, 0);
+      if constexpr (P == 1) read_w(F, F ^ 1);
+      if constexpr (P == 2) read_a(F, 1);
+      if constexpr (P == 3) read_w(F ^ 1, F ^ 1);
+      if constexpr (P == 0) fill(F ^ 1, false, 1, kt + 1);
+      else fill(F, P % 2 == 1, P == 1 ? F : P == 3 ? F ^ 1 : 0, kt + 2);
+      tl_wait_loads<10>();
+      meet();
+      constexpr int A = P / 2, B = P == 0 || P == 3 ? F : F ^ 1;
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          acc[A * 2 + i][B] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[B][ks], fa[ks][i], acc[A * 2 + i][B], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+      if constexpr (P == 3) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // what it read is used a phase later
+      meet();
+    };
+    auto step = [&](auto first, int kt) {
+      phase(std::integral_constant<int, 0>{}, first, kt);
+      phase(std::integral_constant<int, 1>{}, first, kt);
+      phase(std::integral_constant<int, 2>{}, first, kt);
+      phase(std::integral_constant<int, 3>{}, first, kt);
+    };
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {                          // items 0 to 6
+      fill(b, true, b, b);
+      fill(b, false, 0, b);
+      fill(b, true, b ^ 1, b);
+      if (b == 0) fill(b, false, 1, b);
+    }
+    tl_wait_loads<10>();
+    meet();
+    read_w(0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    meet();
+    if (wm == 1) meet();                                   // this half of the waves stays one turn behind
+    for (int kt = 0; kt < nk; kt += 2) {                   // an odd number of steps ends with one of zeros
+      step(std::integral_constant<int, 0>{}, kt);
+      step(std::integral_constant<int, 1>{}, kt + 1);
+    }
+    tl_wait_loads<0>();
+    if (wm == 0) meet();
+    meet();
+  } else {
   if constexpr (DIRECT) {
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) direct1(0, kbase, p);
@@ -742,6 +854,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     for (; kt + 1 < nk; ++kt) step(std::true_type{}, std::false_type{}, kt);
     step(std::false_type{}, std::false_type{}, kt);
   }
+  }
 
   // Epilogue.  A lane's accumulators hold four consecutive n of 32 different rows, so stored from
   // there a row would go out in 16-byte pieces.  Each wave therefore passes its result, 32 rows x
@@ -753,6 +866,34 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   static_assert((size_t)WM * WN * 32 * E_LD * sizeof(float) <= S::smem(DIRECT), "staging areas fit the tile buffers");
   float* cstage = (float*)smem_raw + wave * (32 * E_LD);
   const bool vec_ok = (N % 4 == 0) && (ldo % 4 == 0);
+  // Where a unit holds one workgroup and registers cost no wave, what 32 rows need from LDS is read together, and the residual
+  // of the next 32 rows is requested before these are stored: one 256 x 256 tile of 64 k takes its epilogue from 6.6 to 4.5 us,
+  // with a residual from 9.2 to 6.0 (on a full chip from 31 to 15); 3,288 rows, 2,048 x 2,048 with a residual, 256 x 128
+  // tiles: 41.3 -> 35.7 us.
+  constexpr bool TOGETHER = DIRECT || BM + BN > 256, NEXT = TOGETHER && sizeof(TO) == 4 && !SWIGLU;
+  f32x4 res_next[NEXT ? 8 : 1];
+  auto request_residual = [&](int i) {
+    const int m = m0 + wm * S::TM + i * 32 + lane / 16, n = n0 + wn * S::TN + (lane % 16) * 4;
+    const float* from = residual + (int64_t)m * ldo + n;
+#pragma unroll
+    for (int c8 = 0; c8 < 8; ++c8)
+      if (m + c8 * 4 < M && n < N) res_next[NEXT ? c8 : 0] = *(const f32x4*)(from + c8 * 4 * ldo);      // others are not stored
+  };
+  auto load_emit_w = [&](float* wn, int n) {
+    if (nm.emit_w_is_f32) {
+      const f32x4 w4 = *(const f32x4*)((const float*)nm.emit_w + n);
+      wn[0] = w4[0]; wn[1] = w4[1]; wn[2] = w4[2]; wn[3] = w4[3];
+    } else {
+      const bf16x4 w4 = *(const bf16x4*)((const bf16_t*)nm.emit_w + n);
+      wn[0] = (float)w4[0]; wn[1] = (float)w4[1]; wn[2] = (float)w4[2]; wn[3] = (float)w4[3];
+    }
+  };
+  float emit_w[4] = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (NEXT) {
+    const int n = n0 + wn * S::TN + (lane % 16) * 4;
+    if (residual && vec_ok) request_residual(0);
+    if (nm.emit_operand && n < N) load_emit_w(emit_w, n);
+  }
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
 #pragma unroll
@@ -767,9 +908,9 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     auto leave = [&](auto form) {
       constexpr int FORM = decltype(form)::value;
-      constexpr bool AHEAD = FORM != kNoResidual && sizeof(TO) == 4;
+      constexpr bool AHEAD = FORM != kNoResidual && sizeof(TO) == 4 && !NEXT;
       // whether this launch's are: see below
-      const bool ahead = AHEAD && (BM + BN < 512 || gridDim.x < 256) && residual && vec_ok;
+      const bool ahead = AHEAD && residual && vec_ok;
       f32x4 res[AHEAD ? 8 : 1];
       if (FORM == kResidual || ahead) {
         const int m = m0 + wm * S::TM + i * 32 + lane / 16, n = n0 + wn * S::TN + (lane % 16) * 4;
@@ -777,6 +918,32 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
 #pragma unroll
         for (int c8 = 0; c8 < 8; ++c8)
           if (m + c8 * 4 < M && n < N) res[c8] = *(const f32x4*)(from + c8 * 4 * ldo);      // others are not stored
+      }
+      f32x4 all[TOGETHER ? 8 : 1];
+      float all_rs[TOGETHER ? 8 : 1];
+      f32x4 res_now[NEXT ? 8 : 1];
+      if constexpr (TOGETHER) {
+        const int r0 = wm * S::TM + i * 32 + lane / 16;
+#pragma unroll
+        for (int c8 = 0; c8 < 8; ++c8) all[c8] = *(const f32x4*)(cstage + (c8 * 4 + lane / 16) * E_LD + (lane % 16) * 4);
+        if (nm.in_sumsq) {
+#pragma unroll
+          for (int c8 = 0; c8 < 8; ++c8) all_rs[c8] = row_factor[r0 + c8 * 4];
+        } else if (nm.row_scale) {
+#pragma unroll
+          for (int c8 = 0; c8 < 8; ++c8) all_rs[c8] = nm.row_scale[min(m0 + r0 + c8 * 4, M - 1)];
+        } else {
+#pragma unroll
+          for (int c8 = 0; c8 < 8; ++c8) all_rs[c8] = 1.f;
+        }
+        // used here, so that no read is put off into the branch of its row
+        asm volatile("" : "+v"(all[0]), "+v"(all[1]), "+v"(all[2]), "+v"(all[3]), "+v"(all[4]), "+v"(all[5]), "+v"(all[6]), "+v"(all[7]));
+        asm volatile("" : "+v"(all_rs[0]), "+v"(all_rs[1]), "+v"(all_rs[2]), "+v"(all_rs[3]), "+v"(all_rs[4]), "+v"(all_rs[5]), "+v"(all_rs[6]), "+v"(all_rs[7]));
+        if constexpr (NEXT) {
+#pragma unroll
+          for (int c8 = 0; c8 < 8; ++c8) res_now[c8] = res_next[c8];
+          if (i + 1 < MI && residual && vec_ok) request_residual(i + 1);
+        }
       }
 #pragma unroll
       for (int c8 = 0; c8 < 8; ++c8) {
@@ -786,9 +953,15 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
         if (m >= M || n >= N) continue;
         // the row's factor (1 / rms of a norm left out of the operand): given, or that of a norm handed over
         float rs = 1.f;
-        if (nm.in_sumsq) rs = row_factor[m - m0];
-        else if (nm.row_scale) rs = nm.row_scale[m];
-        const f32x4 s4 = *(const f32x4*)(cstage + r * E_LD + col);
+        f32x4 s4;
+        if constexpr (TOGETHER) {
+          rs = all_rs[c8];
+          s4 = all[c8];
+        } else {
+          if (nm.in_sumsq) rs = row_factor[m - m0];
+          else if (nm.row_scale) rs = nm.row_scale[m];
+          s4 = *(const f32x4*)(cstage + r * E_LD + col);
+        }
         float v[4] = {s4[0] * rs, s4[1] * rs, s4[2] * rs, s4[3] * rs};
         if constexpr (SWIGLU) {   // (gate, up, gate, up) -> two outputs; N is even and n a multiple of 4
           const int64_t oz = (int64_t)m * ldo + n / 2;
@@ -810,7 +983,8 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
         if (vec_ok) {  // n + 3 < N because n and N are both multiples of 4
           if (FORM == kResidual || (FORM == kAnyForm && residual)) {
             f32x4 rv;
-            if (FORM == kResidual || ahead) rv = res[AHEAD ? c8 : 0];
+            if constexpr (NEXT) rv = res_now[c8];
+            else if (FORM == kResidual || ahead) rv = res[AHEAD ? c8 : 0];
             else rv = *(const f32x4*)(residual + o);
             v[0] += rv[0]; v[1] += rv[1]; v[2] += rv[2]; v[3] += rv[3];
           }
@@ -820,12 +994,11 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
             if constexpr (!SWIGLU) {
               if (nm.emit_operand) {      // uniform; N is a multiple of 64: the 16 lanes of a row are all here or none is
                 float wn[4];
-                if (nm.emit_w_is_f32) {
-                  const f32x4 w4 = *(const f32x4*)((const float*)nm.emit_w + n);
-                  wn[0] = w4[0]; wn[1] = w4[1]; wn[2] = w4[2]; wn[3] = w4[3];
+                if constexpr (TOGETHER) {
+#pragma unroll
+                  for (int e = 0; e < 4; ++e) wn[e] = emit_w[e];
                 } else {
-                  const bf16x4 w4 = *(const bf16x4*)((const bf16_t*)nm.emit_w + n);
-                  wn[0] = (float)w4[0]; wn[1] = (float)w4[1]; wn[2] = (float)w4[2]; wn[3] = (float)w4[3];
+                  load_emit_w(wn, n);
                 }
                 bf16x4 ev = {(bf16_t)(wn[0] * v[0]), (bf16_t)(wn[1] * v[1]), (bf16_t)(wn[2] * v[2]), (bf16_t)(wn[3] * v[3])};
                 *(bf16x4*)(nm.emit_operand + (int64_t)m * nm.emit_ld + n) = ev;
@@ -853,8 +1026,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     };
     // A float32 result's residual is requested for all 32 rows together: out may be the residual, so the compiler asks for
     // a piece only when the one before is stored (4,096 rows, 640 x 512: 13.6 -> 12.0 us; 3,000 rows, 1,280 x 256: 12.2 ->
-    // 10.6).  Where 256 x 256 tiles occupy every unit their requests come in one burst: 4,096 rows, 4,096 x 512, took 39.3
-    // us piece by piece and 40.7 so, and stay piece by piece.  The smallest tile, whose products are mostly launch, has the
+    // 10.6).  The smallest tile, whose products are mostly launch, has the
     // two forms apart: 65 to 4,096 rows, 520 x 264, take 2 % more without a residual where one piece of code serves both,
     // bfloat16 results 3 % (they come without one, and load it piece by piece).  The larger tiles would lose waves by it:
     // 108 registers where 84 let four a SIMD run.
@@ -876,7 +1048,7 @@ static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, cons
   static bool configured = false;
   if (!configured) {
     if (hipFuncSetAttribute((const void*)gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, MODE>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::smem_all(MODE == kDirect)) != hipSuccess)
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::smem_all(MODE >= kDirect)) != hipSuccess)
       return TL_ERR_LAUNCH;
     configured = true;
   }
@@ -889,7 +1061,7 @@ static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, cons
   const int64_t grid = (total + B_XCDS - 1) / B_XCDS * B_XCDS;
   if (grid > 0x7fffffff) return TL_ERR_ARG;
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, MODE>), dim3((unsigned)grid), dim3(S::THREADS),
-                     S::smem_all(MODE == kDirect), stream, a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split);
+                     S::smem_all(MODE >= kDirect), stream, a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split);
   static_assert(sizeof(TileNorm) <= 96, "passed by value");
   return TL_OK;
 }
@@ -901,6 +1073,9 @@ static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const flo
   launch_gemm_bf16_mode<BM, BN, WM, WN, TO, SWIGLU, MODE>(a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split, \
                                                           stream)
   if (K % B_BK) return TL_GEMM(kTail);
+  if constexpr (BM + BN == 512) {
+    return K > 0 ? TL_GEMM(kPhased) : TL_GEMM(kTail);
+  } else {
   if constexpr (BM + BN == 384 || BM + BN == 256) {
     const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
     const int64_t wgs = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
@@ -910,14 +1085,14 @@ static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const flo
     // columns, 25.6 and 26.4; beyond 256, two workgroups a unit are worth more), and the 256 x 128 tile for float32 results
     // (2,048 rows, 4,096 x 4,096: 74.3 and 73.5; 3,000 rows, 4,096 x 14,336: 323.9 and 316.1).  From 16 k steps on: with
     // fewer the buffers are hardly filled when the last is asked for (4,096 rows, 1,000 x 512: 12.0 and 12.4).  With
-    // bfloat16 results the 256 x 128 tile loses (2,048 rows, 6,144 x 4,096: 98.3 and 100.1).  The 256 x 256 tile has room
-    // for two buffers only, one on its way: 8,192^3 takes 1,138 us so and 927 through registers.  Four waves of twice the
+    // bfloat16 results the 256 x 128 tile loses (2,048 rows, 6,144 x 4,096: 98.3 and 100.1).  Four waves of twice the
     // outputs, which read less from LDS, lose with float32 results (1,944 rows, 2,048 x 5,632: 59.0; 3,288 rows: 88.2 ->
     // 100.6).
     const bool few = wgs < 256 || (wgs == 256 && (N + BN - 1) / BN >= 16);
     if (K >= 16 * B_BK && (BM + BN == 384 ? sizeof(TO) == 4 : few)) return TL_GEMM(kDirect);
   }
   return TL_GEMM(kWhole);
+  }
 #undef TL_GEMM
 }
 
@@ -928,7 +1103,7 @@ struct TileChoice {
   int bm, bn;
   double rate;
 };
-static const TileChoice kTiles[4] = {{256, 256, 1060.}, {256, 128, 900.}, {128, 128, 760.}, {64, 128, 640.}};
+static const TileChoice kTiles[4] = {{256, 256, 1230.}, {256, 128, 920.}, {128, 128, 775.}, {64, 128, 650.}};
 
 static double tile_cost(int c, int M, int N) {
   const int64_t wgs = (int64_t)((M + kTiles[c].bm - 1) / kTiles[c].bm) * ((N + kTiles[c].bn - 1) / kTiles[c].bn);

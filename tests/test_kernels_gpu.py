@@ -376,6 +376,36 @@ def _operand_tiles(tile, M, N, K):
     assert ((y.cpu().double() - ref).abs() <= bound + 2.0 ** -8 * (ref.abs() + bound)).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 130, 32), (257, 2048, 96), (300, 258, 288), (640, 2050, 256), (640, 2562, 64), (900, 4100, 32),
+                                   (400, 11266, 96), (1000, 2562, 512), (1500, 2050, 160), (1800, 2060, 544), (270, 2, 2080),
+                                   (333, 36, 320), (474, 2050, 64), (319, 4100, 32), (722, 2562, 32), (1373, 11266, 32)])
+def test_linear_f32_tiles_cut_to_fit(M, N, K):
+    """The float32 product whose tile is chosen by its sizes (32 to 128 rows, 64 or 128 columns; ends inside a tile, columns
+    that are no whole vectors, fewer steps of 32 than its ring holds, inner sizes that end inside a block of 256): against
+    float64, and the same bits as the few-row kernel gives its first and last rows."""
+    g = torch.Generator().manual_seed(M + N + K)
+    wide = torch.randn(M, K + 8, generator=g)
+    w = torch.randn(N, K, generator=g) / math.sqrt(K)
+    res, scale = torch.randn(M, N, generator=g), torch.rand(M, generator=g) + 0.5
+    a = wide[:, :K]
+    ref = (a.double() @ w.double().T) * scale.double()[:, None]
+    # K products, their sums in any order, the factor and the last addition: at most K + 3 roundings of the absolute sum
+    bound = (K + 3) * 2.0 ** -24 * ((a.double().abs() @ w.double().abs().T) * scale.double()[:, None] + res.double().abs())
+    da, dw, dr, ds = wide.to(DEV)[:, :K], w.to(DEV), res.to(DEV), scale.to(DEV)
+    x = dr.clone()
+    ops().linear(da, dw, x, x, row_scale=ds)
+    assert ((x.cpu().double() - (ref + res.double())).abs() <= bound).all()
+    z = torch.full((M, N // 2), float("nan"), device=DEV)
+    ops().linear(da, dw, z, epilogue="swiglu")
+    for rows in (slice(0, 16), slice(M - 33, M)):
+        few = dr[rows].clone()
+        ops().linear(da[rows], dw, few, few, row_scale=ds[rows].contiguous())
+        assert torch.equal(few, x[rows])
+        few_z = torch.empty(few.shape[0], N // 2, device=DEV)
+        ops().linear(da[rows], dw, few_z, epilogue="swiglu")
+        assert torch.equal(few_z, z[rows])
+
+
 @pytest.mark.parametrize("M", [17, 50, 64, 65, 200, 512])
 @pytest.mark.parametrize("K,N", [(5632, 2048), (2048, 4100), (1096, 518), (2048, 2046), (256, 2560), (4096, 6144)])
 def test_linear_split_k(M, K, N):

@@ -4,10 +4,10 @@
 // residual add that the reference runs as a separate kernel
 // (tiny_llm/ops/cuda/arithmetic.cu:13) is folded into the epilogue.
 //
-//  * gemm_f32_kernel (tiles of 128 x 128 or 64 x 64), and gemm_f32_rows_kernel for at most 64 rows:
-//    true float32 on the matrix cores (v_mfma_f32_16x16x4_f32), no reduced-precision mode.  Both add
-//    in ONE order, so a row gives the same bits whether it is computed alone or in a batch, by
-//    either kernel.
+//  * gemm_f32_ring_kernel (tiles of 32 to 128 rows and 64 or 128 columns), gemm_f32_kernel (any rows and inner size), and
+//    gemm_f32_rows_kernel for few rows: true float32 on the matrix cores (v_mfma_f32_16x16x4_f32), no
+//    reduced-precision mode.  All add in ONE order, so a row gives the same bits whether it is computed
+//    alone or in a batch, by any of them.
 //  * gemm_bf16_kernel: bf16 inputs on the matrix cores (v_mfma_f32_32x32x16_bf16), float32
 //    accumulation, 256 x 256, 256 x 128, 128 x 128 or 64 x 128 tiles with k steps of 64 staged through
 //    double-buffered LDS; optionally over a share of the inner size (split k).
@@ -22,8 +22,8 @@ namespace {
 
 // ===================================================================== float32
 // True float32 on the matrix cores: v_mfma_f32_16x16x4_f32 takes float32 operands and keeps float32
-// sums (no reduced-precision mode).  Both kernels below add the terms of an output element in ONE
-// order, so that a row gives the same bits alone and in any batch, by either kernel:
+// sums (no reduced-precision mode).  The kernels below add the terms of an output element in ONE
+// order, so that a row gives the same bits alone and in any batch, by any of them:
 //   * k runs in blocks of 256, each block summed from zero, the block sums added in ascending order;
 //   * inside a block, groups of 16 k in ascending order; a group is four matrix instructions, the
 //     e-th of which takes k = 16 group + {0, 4, 8, 12} + e (a lane holds four consecutive k of its row,
@@ -52,6 +52,40 @@ __device__ __forceinline__ float swiglu_pair(float g, float u) { return g / (1.f
 // were a tenth of the gate/up product's time.
 __device__ __forceinline__ float swiglu_pair_fast(float g, float u) {
   return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g)) * u;
+}
+
+// 16 bytes a lane from a buffer straight into LDS, side by side from `dst` on (the same for the whole wave; the
+// instruction takes its place from M0).  Written as an instruction block: given the builtin, the compiler waits for every
+// load on its way ahead of each LDS read, whichever buffer it reads.  M0 is an operand, so the compiler writes it and knows
+// that it is used; what it does not see is that the block holds a load, which needs a wait state behind that write: the
+// s_nop.  Whoever reads the data waits for it first (tl_wait_loads, then a barrier).
+typedef int tl_rsrc_words __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ unsigned int tl_lds_address(void* p) {
+  return __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(__attribute__((address_space(3))) void*)p);
+}
+__device__ __forceinline__ void tl_load_to_lds(tl_rsrc_words buf, unsigned int at, int voffset, int soffset) {
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "{m0}"(at), "v"(voffset), "s"(buf), "s"(soffset)
+               : "memory");
+}
+template <int LEFT>       // until at most LEFT of the wave's loads are still on their way
+__device__ __forceinline__ void tl_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
+
+// Workgroups are handed to the eight XCDs in turn, each with an L2 of its own.  The index is remapped so that an XCD owns a
+// contiguous run of tiles, and the tiles that it works on at a time make a block about as high as it is wide, which asks the
+// fewest rows of both operands of its L2 (8192^3 with 256 x 256 tiles in columns of 32 927 us, in bands of four 781): bands
+// of 4 to 7 tiles of rows, column by column.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_tile(int block, int total) {
+  const int per_xcd = (total + kXcds - 1) / kXcds;
+  return (block % kXcds) * per_xcd + block / kXcds;
+}
+__device__ __forceinline__ void tile_place(int t, int tiles_m, int tiles_n, int* tm, int* tn) {
+  const int bands = max(tiles_m / 4, 1), band_m = (tiles_m + bands - 1) / bands;
+  const int band = t / (band_m * tiles_n), in_band = t - band * band_m * tiles_n, high = min(band_m, tiles_m - band * band_m);
+  *tm = band * band_m + in_band % high;
+  *tn = in_band / high;
 }
 
 // Four consecutive k of one row, zero beyond K; VEC: 16-byte aligned rows and K a multiple of 4.
@@ -245,6 +279,231 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f32_kernel(const float* __rest
       }
     }
   }
+}
+
+// gemm_f32_ring_kernel: the same for rows of 16-byte pieces and an inner size that is a multiple of 32.  Four waves side by
+// side, each with MT x NT matrix tiles (16 MT rows, 16 NT columns), so that a tile can be cut to make the chip's 256 units
+// equally busy: 640 rows x 2,048 are 256 tiles of 80 x 64.  What bounds it are the matrix pipes (32 clocks an instruction, one
+// wave a SIMD): operands go straight into LDS as a ring of R steps of 32 k, R - 2 of them on their way, the fragments of the
+// next 16 k are read while these are multiplied, and there is one barrier a step, in the middle of its products.
+// 640 rows, 2,048 x 2,048: 100 -> 54 us (100 TFLOP/s of 155 that a loop of these instructions reaches), 2,048 x 5,632
+// 261 -> 138, 11,264 x 2,048 332 -> 240 (123); 333 rows, 1,000 x 2,080: 74 -> 27.  Tiles of 64 x 64, one barrier every 16 k,
+// had a fragment's way from LDS and the barrier between any 16 instructions, and 320 of them kept 64 units twice as busy.
+template <int MT, int NT>
+struct F32Ring {
+  static constexpr int BM = 16 * MT, BN = 64 * NT, BK = 32;
+  static constexpr int GROUPS = (BM + BN) / 8;             // 8 rows of 128 bytes: what one load of a wave brings
+  static constexpr int PW = (GROUPS + 3) / 4;              // loads of a wave a step
+  static constexpr int BYTES = PW * 4 * 1024;              // of a step in LDS
+  static constexpr int R = 80 * 1024 / BYTES < 4 ? 4 : 80 * 1024 / BYTES > 6 ? 6 : 80 * 1024 / BYTES;
+};
+template <bool SWIGLU, int MT, int NT>
+__global__ __launch_bounds__(F_THREADS) void gemm_f32_ring_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                  float* __restrict__ out, const float* __restrict__ residual,
+                                                                  int M, int N, int K, int64_t lda, int64_t ldo,
+                                                                  const float* __restrict__ row_scale, int vec_out) {
+  using S = F32Ring<MT, NT>;
+  constexpr int BM = S::BM, BN = S::BN, R = S::R, PW = S::PW;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char f32_ring[];
+  const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TL_WAVE);
+  const int l16 = lane % 16, kk = lane / 16;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int t = xcd_tile(blockIdx.x, tiles_m * tiles_n);
+  if (t >= tiles_m * tiles_n) return;                      // the grid is padded to a multiple of 8
+  int tile_m, tile_n;
+  tile_place(t, tiles_m, tiles_n, &tile_m, &tile_n);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  // Each buffer begins at the tile's first row and ends with the matrix: rows beyond it read as zeros.
+  auto buffer_words = [](const float* first_row, int rows, int64_t ld, int K_) {
+    const int64_t bytes = ((int64_t)(rows - 1) * ld + K_) * 4;
+    const uint64_t at = (uint64_t)first_row;
+    return tl_rsrc_words{(int)(uint32_t)at, (int)(uint32_t)(at >> 32) & 0xffff, (int)bytes, 0x00020000};
+  };
+  const tl_rsrc_words words_a = buffer_words(a + (int64_t)m0 * lda, min(M - m0, BM), lda, K);
+  const tl_rsrc_words words_w = buffer_words(w + (int64_t)n0 * K, min(N - n0, BN), K, K);
+  // Wave v brings groups v, v + 4, ... of a step: the activations' 2 MT, then the weights' 8 NT, then, where they do not share
+  // out evenly, nothing into a place that nobody reads.  Row r holds the four k of piece c at place c ^ (r / 2 % 8).
+  int off[PW];
+#pragma unroll
+  for (int j = 0; j < PW; ++j) {
+    const int gi = wave + 4 * j, row = (gi < BM / 8 ? gi : gi - BM / 8) * 8 + lane / 8;
+    const int64_t ld = gi < BM / 8 ? lda : (int64_t)K;
+    off[j] = gi < S::GROUPS ? (int)((row * ld + ((lane % 8) ^ (row / 2 % 8)) * 4) * 4) : 0;
+  }
+  const unsigned int lds = tl_lds_address(f32_ring);
+  const int steps = K / S::BK;
+  auto fill = [&](int s) {                                 // steps behind the last read as zeros from a buffer of no bytes
+#pragma unroll
+    for (int j = 0; j < PW; ++j) {
+      const int gi = wave + 4 * j;
+      tl_rsrc_words from = gi < BM / 8 ? words_a : words_w;
+      from[2] = s < steps && gi < S::GROUPS ? from[2] : 0;
+      tl_load_to_lds(from, lds + (s % R) * S::BYTES + gi * 1024, off[j], min(s, steps - 1) * S::BK * 4);
+    }
+  };
+  f32x4 acc[NT][MT], tot[NT][MT], av[2][MT], wv[2][NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      tot[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  auto read = [&](int s, int half) {                       // the fragments of 16 k
+    const float* buf = (const float*)(f32_ring + (s % R) * S::BYTES) + ((half * 4 + kk) ^ (l16 / 2 % 8)) * 4 + l16 * 32;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) wv[half][nt] = *(const f32x4*)(buf + (BM + (wave * NT + nt) * 16) * 32);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) av[half][mt] = *(const f32x4*)(buf + mt * 16 * 32);
+  };
+  auto multiply = [&](int half) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[half][nt][e], av[half][mt][e], acc[nt][mt], 0, 0, 0);
+  };
+  auto meet = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int s = 0; s < R - 1; ++s) fill(s);
+  tl_wait_loads<(R - 2) * PW>();
+  meet();
+  read(0, 0);
+  for (int s = 0; s < steps; ++s) {
+    read(s, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    // step s + 1 has arrived; and step s - 1, whose fragments every wave has multiplied, can be written over
+    tl_wait_loads<(R - 3) * PW>();
+    meet();
+    fill(s + R - 1);
+    read(s + 1, 0);                                        // behind the last step: read, not used
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+    if ((s + 1) % (F_KBLOCK / S::BK) == 0 || s + 1 == steps) {      // a block of the order of addition ends
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          tot[nt][mt] += acc[nt][mt];
+          acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+  tl_wait_loads<0>();                                      // nothing may arrive in LDS that is no longer this workgroup's
+  // lane (l16, kk) of tile (nt, mt) holds row m = mt*16 + l16, columns n = nt*16 + 4 kk + r
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = m0 + mt * 16 + l16;
+    if (m >= M) continue;
+    const float f = row_scale ? row_scale[m] : 1.f;        // the factor of a norm in front (norm_prescale_f32_kernel)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = n0 + (wave * NT + nt) * 16 + kk * 4;
+      if (n >= N) continue;
+      f32x4 v = tot[nt][mt];
+      if (row_scale) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] *= f;
+      }
+      if constexpr (SWIGLU) {   // columns (2j, 2j+1) = (gate_j, up_j); N is even
+#pragma unroll
+        for (int r = 0; r < 4; r += 2)
+          if (n + r < N) out[(int64_t)m * ldo + (n + r) / 2] = swiglu_pair(v[r], v[r + 1]);
+      } else {
+        const int64_t at = (int64_t)m * ldo + n;
+        if (vec_out) {          // uniform: rows are whole, aligned pieces of four
+          if (residual) {
+            const f32x4 x = *(const f32x4*)(residual + at);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += x[r];
+          }
+          *(f32x4*)(out + at) = v;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < N) out[at + r] = residual ? v[r] + residual[at + r] : v[r];
+        }
+      }
+    }
+  }
+}
+
+template <bool SWIGLU, int MT, int NT>
+static int launch_f32_ring(const float* a, const float* w, float* out, const float* residual, int M, int N, int K, int64_t lda,
+                           int64_t ldo, const float* row_scale, int vec_out, hipStream_t stream) {
+  using S = F32Ring<MT, NT>;
+  static bool configured = false;
+  if (!configured) {
+    if (hipFuncSetAttribute((const void*)gemm_f32_ring_kernel<SWIGLU, MT, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            S::R * S::BYTES) != hipSuccess)
+      return TL_ERR_LAUNCH;
+    configured = true;
+  }
+  const int64_t total = (int64_t)((M + S::BM - 1) / S::BM) * ((N + S::BN - 1) / S::BN);
+  const int64_t grid = (total + kXcds - 1) / kXcds * kXcds;
+  if (grid > 0x7fffffff) return TL_ERR_ARG;
+  hipLaunchKernelGGL((gemm_f32_ring_kernel<SWIGLU, MT, NT>), dim3((unsigned)grid), dim3(F_THREADS), S::R * S::BYTES, stream, a, w,
+                     out, residual, M, N, K, lda, ldo, row_scale, vec_out);
+  return TL_OK;
+}
+
+// The tile whose rounds over 256 units are shortest, and the smaller of equals: a wave's matrix tiles and half of one for a
+// step's barrier (with two for it, as one round takes, large tiles came out ahead of small ones that share units: 640 x
+// 11,264 x 2,048 287 us instead of 240, 128 rows 77 instead of 61; 2,048 rows 874 instead of 892).  Returns an estimate of
+// the time: 0.107 us for each matrix tile and two more a step of
+// 32 k, 6 us for launch, first loads and epilogue (640 rows: 2,048 x 5,632 138 us estimated, 138 measured; 11,264 x 2,048
+// 252 and 240; 257 rows, 2,048 x 2,048: 40 and 37).
+static double f32_ring_us(int M, int N, int K, int* mt, int* nt) {
+  double best = 0., units = 0.;
+  for (int n = 1; n <= 2; ++n)
+    for (int m = 2; m <= 8; ++m) {
+      const int64_t wgs = (int64_t)((M + 16 * m - 1) / (16 * m)) * ((N + 64 * n - 1) / (64 * n));
+      const double rounds = (double)((wgs + 255) / 256), cost = rounds * (m * n + 0.5);
+      if (best == 0. || cost < best) {
+        best = cost;
+        units = rounds * (m * n + 2);
+        *mt = m;
+        *nt = n;
+      }
+    }
+  return 6.0 + units * 0.107 * (K / 32);
+}
+
+// Whether it takes this product: whole vectors, and rows of a tile addressed with 32-bit byte offsets from its first.
+static bool f32_ring_ok(bool vec, int K, int64_t lda) {
+  return vec && K % 32 == 0 && 128 * lda * 4 < 0x7fffffff && (int64_t)128 * K * 4 < 0x7fffffff;
+}
+
+template <bool SWIGLU>
+static int launch_f32_ring_any(const float* a, const float* w, float* out, const float* residual, int M, int N, int K,
+                               int64_t lda, int64_t ldo, const float* row_scale, hipStream_t stream) {
+  const int vec_out = N % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out | (uintptr_t)residual) % 16 == 0;
+  int mt = 2, nt = 1;
+  f32_ring_us(M, N, K, &mt, &nt);
+#define TL_RING(MT)                                                                                                         \
+  case MT:                                                                                                                  \
+    return nt == 1 ? launch_f32_ring<SWIGLU, MT, 1>(a, w, out, residual, M, N, K, lda, ldo, row_scale, vec_out, stream)      \
+                   : launch_f32_ring<SWIGLU, MT, 2>(a, w, out, residual, M, N, K, lda, ldo, row_scale, vec_out, stream)
+  switch (mt) {
+    TL_RING(2);
+    TL_RING(3);
+    TL_RING(4);
+    TL_RING(5);
+    TL_RING(6);
+    TL_RING(7);
+    TL_RING(8);
+  }
+#undef TL_RING
+  return TL_ERR_ARG;
 }
 
 // The same product for few rows (decode steps): the weights stream once, straight from memory
@@ -457,31 +716,8 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const float* 
 // the tile, the fewer operand bytes and LDS reads per flop and the higher the rate on a full chip;
 // small products take small tiles all the same, because 256 compute units want at least that many
 // workgroups (launch_gemm_bf16_any estimates the time of each shape and takes the best).
-//
-// Workgroups are handed to the eight XCDs in turn, each with an L2 of its own.  The tile index is
-// therefore remapped so that an XCD owns a contiguous run of tiles in column-major order: it then
-// reads only its own share of the weight matrix (plus the activations), instead of all of it.
 constexpr int B_BK = 64;
 constexpr int B_LD = B_BK + 8;  // LDS row stride in elements: 144 bytes, keeps 16-byte alignment
-constexpr int B_XCDS = 8;
-
-// 16 bytes a lane from a buffer straight into LDS, side by side from `dst` on (the same for the whole wave; the
-// instruction takes its place from M0).  Written as an instruction block: given the builtin, the compiler waits for every
-// load on its way ahead of each LDS read, whichever buffer it reads.  M0 is an operand, so the compiler writes it and knows
-// that it is used; what it does not see is that the block holds a load, which needs a wait state behind that write: the
-// s_nop.  Whoever reads the data waits for it first (tl_wait_loads, then a barrier).
-typedef int tl_rsrc_words __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ unsigned int tl_lds_address(void* p) {
-  return __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(__attribute__((address_space(3))) void*)p);
-}
-__device__ __forceinline__ void tl_load_to_lds(tl_rsrc_words buf, unsigned int at, int voffset, int soffset) {
-  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "{m0}"(at), "v"(voffset), "s"(buf), "s"(soffset)
-               : "memory");
-}
-template <int LEFT>       // until at most LEFT of the wave's loads are still on their way
-__device__ __forceinline__ void tl_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
 
 // What the epilogue of the tiled kernel does to a row besides the product: a factor per row
 // (`row_scale`), or a norm handed from product to product as the few-row kernel does it (see
@@ -555,15 +791,12 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   // them up.  That is how products with few output tiles still fill the chip.
   const int splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
   const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + BN - 1) / BN), total = tiles * splits;
-  const int per_xcd = (total + B_XCDS - 1) / B_XCDS;
-  const int t_all = (blockIdx.x % B_XCDS) * per_xcd + blockIdx.x / B_XCDS;
+  const int t_all = xcd_tile(blockIdx.x, total);
   if (t_all >= total) return;                           // the grid is padded to a multiple of 8
   const int split = t_all / tiles, t = t_all % tiles;
-  // The tiles that an XCD works on at a time make a block about as high as it is wide, which asks the fewest rows of both
-  // operands of its L2 (8192^3 in columns of 32 tiles 927 us, in bands of four 781): bands of 4 to 7 tiles of rows.
-  const int tiles_n = (N + BN - 1) / BN, bands = max(tiles_m / 4, 1), band_m = (tiles_m + bands - 1) / bands;
-  const int band = t / (band_m * tiles_n), in_band = t - band * band_m * tiles_n, high = min(band_m, tiles_m - band * band_m);
-  const int m0 = (band * band_m + in_band % high) * BM, n0 = in_band / high * BN;
+  int tile_m, tile_n;
+  tile_place(t, tiles_m, (N + BN - 1) / BN, &tile_m, &tile_n);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int kbase = split * k_per_split;
   const int kend = k_per_split > 0 ? min(K, kbase + k_per_split) : K;
   if (k_per_split > 0) out += (int64_t)split * M * ldo;
@@ -1058,7 +1291,7 @@ static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, cons
   if (row_scale.in_sumsq && k_per_split > 0) return TL_ERR_ARG;      // a split product has no epilogue of its own
   const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
   const int64_t total = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
-  const int64_t grid = (total + B_XCDS - 1) / B_XCDS * B_XCDS;
+  const int64_t grid = (total + kXcds - 1) / kXcds * kXcds;
   if (grid > 0x7fffffff) return TL_ERR_ARG;
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, MODE>), dim3((unsigned)grid), dim3(S::THREADS),
                      S::smem_all(MODE >= kDirect), stream, a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split);
@@ -2119,15 +2352,18 @@ int tl_linear_tile(const void* a, const void* w, void* out, const float* residua
     const int ct = f32_rows_col_tiles(M, N, K, cols, &cols_wg);
     const size_t rows_smem = (size_t)tiles_wg * nkb * 16 * cols * ct * sizeof(float);
     // Up to 64 rows the few-row kernel; up to 256 where it is estimated faster than the tiled kernel, whose few
-    // tiles each walk the whole inner size (measured at inner size 2048: 87 us a round of up to 352 tiles of
-    // 64 x 64, 204 us a round of 128 x 128; the few-row kernel 0.66 us per row tile and million weights:
-    // 2048 x 2048 at 128 rows 25 us against 89, 5632 x 2048 at 256 rows 124 against 232).  The bits are the same.
+    // tiles each walk the whole inner size (f32_ring_us; where rows are no whole vectors, measured at inner size 2048: 87 us a
+    // round of up to 352 tiles of 64 x 64, 204 us a round of 128 x 128; the few-row kernel 0.66 us per row tile and million
+    // weights: 100 rows of 2560 x 2048 35 us, estimated 32, against 33; 200 rows of 2048 x 5632 119 against 81).  The bits are
+    // the same.
     bool few_rows = M <= 16 * FR_MAX_MT;
     if (!few_rows && M <= 256) {
       const int64_t big_t = ceil_div64(N, 128) * ceil_div64(M, 128), small_t = ceil_div64(N, 64) * ceil_div64(M, 64);
       const bool small_tiles = (double)ceil_div64(small_t, 256) / (4 * 0.6) < (double)ceil_div64(big_t, 256);
-      const double tiled_us = (K / 2048.0) * (small_tiles ? 87.0 * (small_t > 352 ? small_t / 352.0 : 1.0)
-                                                          : 204.0 * (double)ceil_div64(big_t, 256));
+      int mt, nt;
+      const double tiled_us = f32_ring_ok(vec, K, lda) ? f32_ring_us(M, N, K, &mt, &nt)
+                              : (K / 2048.0) * (small_tiles ? 87.0 * (small_t > 352 ? small_t / 352.0 : 1.0)
+                                                            : 204.0 * (double)ceil_div64(big_t, 256));
       // (a long inner size leaves LDS for the block sums of one or two row tiles a workgroup only, and the
       // weights are then fetched once per row tile: 14336 x 4096 at 256 rows 876 us against 657)
       const double per_tile = tiles_wg >= 4 ? 0.66 : (tiles_wg >= 2 ? 0.8 : 0.98);
@@ -2176,6 +2412,13 @@ int tl_linear_tile(const void* a, const void* w, void* out, const float* residua
 #undef TL_F32_ROWS
 #undef TL_F32_ROWS_K
       return tl_launch_status();
+    }
+    if (f32_ring_ok(vec, K, lda)) {
+      const int rc = swiglu ? launch_f32_ring_any<true>((const float*)a, (const float*)w, (float*)out, nullptr, M, N, K, lda, ldo,
+                                                        row_scale, stream)
+                            : launch_f32_ring_any<false>((const float*)a, (const float*)w, (float*)out, residual, M, N, K, lda,
+                                                         ldo, row_scale, stream);
+      return rc == TL_OK ? tl_launch_status() : rc;
     }
     // 128 x 128 tiles, or 64 x 64 where those take fewer rounds of workgroups over the 256 compute
     // units even at 0.6 of the larger tile's rate (it fetches twice the operand bytes per flop)

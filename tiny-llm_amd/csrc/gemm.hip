@@ -74,7 +74,7 @@ __device__ __forceinline__ void tl_wait_loads() { asm volatile("s_waitcnt vmcnt(
 
 // Workgroups are handed to the eight XCDs in turn, each with an L2 of its own.  The index is remapped so that an XCD owns a
 // contiguous run of tiles, and the tiles that it works on at a time make a block about as high as it is wide, which asks the
-// fewest rows of both operands of its L2 (8192^3 with 256 x 256 tiles in columns of 32 927 us, in bands of four 781): bands
+// fewest rows of both operands of its L2 (8192^3 with 256 x 256 tiles in columns of 32 927 us, in bands of four 786): bands
 // of 4 to 7 tiles of rows, column by column.
 constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_tile(int block, int total) {
@@ -706,7 +706,7 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const float* 
 
 // ==================================================================== bfloat16
 // Tiles of BM x BN outputs, k in steps of 64, WM x WN wave64, each owning (BM/WM) x (BN/WN)
-// outputs as 32x32x16 MFMA tiles.  Operand tiles go global -> registers -> LDS; LDS is
+// outputs as 32x32x16 MFMA tiles (16x16x32 in the 256 x 256 tile).  Operand tiles go global -> registers -> LDS; LDS is
 // double-buffered so an iteration needs one barrier, and the global loads of the next k step are
 // in flight while the current one is multiplied.  Or they go straight into LDS, three or four buffers in turn
 // (launch_gemm_bf16 says where), and the loads of the next two or three k steps are in flight; the 256 x 256 tile's two
@@ -813,6 +813,11 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  f32x4 acc4[2 * MI][2 * NJ];                              // kPhased: 16 x 16 tiles
+#pragma unroll
+  for (int i = 0; i < 2 * MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * NJ; ++j) acc4[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // A norm handed over: the factors of this tile's rows are worked out once, here, where the loads
   // hide behind the main loop (16 threads share a row's parts out), and wait in LDS for the
@@ -928,13 +933,14 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   if constexpr (PHASED) {
     static_assert(BM == 256 && BN == 256 && WM == 2 && WN == 4 && BUFS == 2, "quarters of the 256 x 256 tile");
     // With both operands through registers and one barrier a k step the matrix pipes were busy for 69 % of the time (8192^3;
-    // the loads of two whole buffers straight into LDS are too late, 1,138 us where registers take 889); so, 783 us.  2,048
-    // rows, 28,672 x 4,096: 428 -> 389 us (1.24 PFLOP/s); 4,096 x 14,336 260 -> 217, where half the units work and run at
-    // 2.2 GHz; on a full chip the part clocks at 1.7 to 1.75 GHz, and that bounds it.
+    // the loads of two whole buffers straight into LDS are too late, 1,138 us where registers take 889); so, 723 us.  2,048
+    // rows, 28,672 x 4,096: 428 -> 360 us (1.34 PFLOP/s); 4,096 x 14,336 260 -> 217, where half the units work and run at
+    // 2.2 GHz; on a full chip the part clocks at 1.7 to 1.75 GHz, and power bounds it: instructions of 16 x 16 x 32 move
+    // half the sums of those of 32 x 32 x 16 for the same products (781 -> 723 and 381 -> 360 us; the bits are the same).
     // A k step is four items of 128 rows, in the order in which they are read: a weight half, the first half of the
     // activations, the other weight half, the rest of the activations.  A half holds the rows that every wave needs for half
     // of its outputs: of the activations 64 of each 128, of the weights 32 of each 64.  Which weight half comes first
-    // alternates from step to step, so that a phase of eight matrix instructions always has one new half to read.  Phase f
+    // alternates from step to step, so that a phase of sixteen matrix instructions always has one new half to read.  Phase f
     // reads item f + 1 into registers, asks for item f + 7 and waits for item f + 2: five items, a step and a quarter of
     // work, stay on their way.  The waves of a SIMD take turns: while one multiplies, the other reads; between two barriers
     // each half of the workgroup does one of the two, the second half a turn behind.  Item f + 7 takes the place of item
@@ -958,20 +964,23 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
       for (int q = 0; q < 2; ++q)
         tl_load_to_lds(from, dst + q * 64 * LD * 2, off[weights][h][q], (kbase + min(kt, nk - 1) * B_BK) * 2);
     };
-    bf16x8 fa[4][2], fw[2][4];                             // fragments of a half of the activations, of both weight halves
-    const bf16_t* pa = As + (wm * 64 + lane % 32) * LD;
-    const bf16_t* pw = Ws + (wn * 32 + lane % 32) * LD;
+    bf16x8 fa[2][4], fw[2][2][2];                          // fragments of a half of the activations, of both weight halves
+    const bf16_t* pa = As + (wm * 64 + lane % 16) * LD;
+    const bf16_t* pw = Ws + (wn * 32 + lane % 16) * LD;
+    const int key = lane % 16 / 2;
     auto read_a = [&](int buf, int h) {
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-          fa[ks][i] = *(const bf16x8*)(pa + ((buf * 2 + h) * 128 + i * 32) * LD + ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8);
+        for (int i = 0; i < 4; ++i)
+          fa[ks][i] = *(const bf16x8*)(pa + ((buf * 2 + h) * 128 + i * 16) * LD + ((ks * 4 + lane / 16) ^ key) * 8);
     };
     auto read_w = [&](int buf, int h) {
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-        fw[h][ks] = *(const bf16x8*)(pw + (buf * 2 + h) * 128 * LD + ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8);
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          fw[h][ks][j] = *(const bf16x8*)(pw + ((buf * 2 + h) * 128 + j * 16) * LD + ((ks * 4 + lane / 16) ^ key) * 8);
     };
     auto meet = [&]() {
       __builtin_amdgcn_sched_barrier(0);
@@ -994,10 +1003,13 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
       constexpr int A = P / 2, B = P == 0 || P == 3 ? F : F ^ 1;
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-          acc[A * 2 + i][B] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[B][ks], fa[ks][i], acc[A * 2 + i][B], 0, 0, 0);
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc4[A * 4 + i][B * 2 + j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[B][ks][j], fa[ks][i], acc4[A * 4 + i][B * 2 + j], 0, 0, 0);
       __builtin_amdgcn_s_setprio(0);
       if constexpr (P == 3) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // what it read is used a phase later
       meet();
@@ -1129,6 +1141,13 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   }
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
+    if constexpr (PHASED) {
+#pragma unroll
+      for (int ii = 0; ii < 2; ++ii)
+#pragma unroll
+        for (int j = 0; j < 2 * NJ; ++j)
+          *(f32x4*)(cstage + (ii * 16 + lane % 16) * E_LD + j * 16 + (lane / 16) * 4) = acc4[i * 2 + ii][j];
+    } else
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -1336,7 +1355,7 @@ struct TileChoice {
   int bm, bn;
   double rate;
 };
-static const TileChoice kTiles[4] = {{256, 256, 1230.}, {256, 128, 920.}, {128, 128, 775.}, {64, 128, 650.}};
+static const TileChoice kTiles[4] = {{256, 256, 1320.}, {256, 128, 920.}, {128, 128, 775.}, {64, 128, 650.}};
 
 static double tile_cost(int c, int M, int N) {
   const int64_t wgs = (int64_t)((M + kTiles[c].bm - 1) / kTiles[c].bm) * ((N + kTiles[c].bn - 1) / kTiles[c].bn);

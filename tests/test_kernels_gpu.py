@@ -359,6 +359,14 @@ def test_linear_large_tile_in_quarters(M, N, K):
     _operand_tiles(1, M, N, K)
 
 
+@pytest.mark.parametrize("tile,M,N,K", [(t, 300, 260, k) for t in (2, 3) for k in (192, 256, 320, 384, 448, 576)] +
+                         [(0, 1944, 704, 2048), (0, 512, 2048, 2048), (0, 150, 4096, 1024), (0, 66, 1024, 512), (0, 700, 2048, 4096)])
+def test_linear_few_steps_and_splits(tile, M, N, K):
+    """Operand tiles straight into LDS from four k steps on, around the number of buffers; and sizes on both sides of what is
+    split: unsplit since the tiles go that way, or split into fewer parts."""
+    _operand_tiles(tile, M, N, K)
+
+
 def _operand_tiles(tile, M, N, K):
     g = torch.Generator().manual_seed(M + K + N)
     wide = torch.randn(M, K + 72, generator=g).to(torch.bfloat16)

@@ -706,7 +706,7 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const float* 
 
 // ==================================================================== bfloat16
 // Tiles of BM x BN outputs, k in steps of 64, WM x WN wave64, each owning (BM/WM) x (BN/WN)
-// outputs as 32x32x16 MFMA tiles (16x16x32 in the 256 x 256 tile).  Operand tiles go global -> registers -> LDS; LDS is
+// outputs as 32x32x16 MFMA tiles, or as 16x16x32 (operands straight into LDS).  Operand tiles go global -> registers -> LDS; LDS is
 // double-buffered so an iteration needs one barrier, and the global loads of the next k step are
 // in flight while the current one is multiplied.  Or they go straight into LDS, three or four buffers in turn
 // (launch_gemm_bf16 says where), and the loads of the next two or three k steps are in flight; the 256 x 256 tile's two
@@ -751,7 +751,6 @@ template <int BM, int BN, int WM, int WN>
 struct GemmShape {
   static constexpr int THREADS = WM * WN * TL_WAVE;
   static constexpr int TM = BM / WM, TN = BN / WN;        // a wave's outputs
-  static constexpr int MI = TM / 32, NJ = TN / 32;        // as 32 x 32 MFMA tiles
   static constexpr int AC = BM * (B_BK / 8) / THREADS, WC = BN * (B_BK / 8) / THREADS;
   // operand tiles in LDS: two, or, straight from memory, as many as make three in flight beside the one in use
   static constexpr int BUFS = BM + BN > 384 ? 2 : BM + BN > 256 ? 3 : 4;
@@ -777,7 +776,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
                                                                       const TileNorm nm, int M, int N, int K,
                                                                       int64_t lda, int64_t ldo, int k_per_split) {
   using S = GemmShape<BM, BN, WM, WN>;
-  constexpr int MI = S::MI, NJ = S::NJ, THREADS = S::THREADS;
+  constexpr int THREADS = S::THREADS;
   constexpr bool PHASED = MODE == kPhased, DIRECT = MODE == kDirect || PHASED;
   constexpr int LD = DIRECT ? B_BK : B_LD;              // row stride of a staged tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -806,18 +805,23 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     w += (int64_t)group * nm.group_stride;
   }
 
-  f32x16 acc[MI][NJ];
+  // Straight from memory: 16 x 16 matrix tiles; through registers: 32 x 32.
+  constexpr int MI = S::TM / 16, NJ = S::TN / 16, MI32 = S::TM / 32, NJ32 = S::TN / 32;
+  f32x4 acc[DIRECT ? MI : 1][DIRECT ? NJ : 1];
+  f32x16 acc32[DIRECT ? 1 : MI32][DIRECT ? 1 : NJ32];
+  if constexpr (DIRECT) {
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  } else {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  f32x4 acc4[2 * MI][2 * NJ];                              // kPhased: 16 x 16 tiles
+    for (int i = 0; i < MI32; ++i)
 #pragma unroll
-  for (int i = 0; i < 2 * MI; ++i)
+      for (int j = 0; j < NJ32; ++j)
 #pragma unroll
-    for (int j = 0; j < 2 * NJ; ++j) acc4[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < 16; ++r) acc32[i][j][r] = 0.f;
+  }
 
   // A norm handed over: the factors of this tile's rows are worked out once, here, where the loads
   // hide behind the main loop (16 threads share a row's parts out), and wait in LDS for the
@@ -888,33 +892,6 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     bf16_t* dst = is_a ? As + (buf * BM + r) * LD : Ws + (buf * BN + r) * LD;
     tl_load_to_lds(is_a ? words_a : words_w, tl_lds_address(dst), piece_off[p], k0 * 2);
   };
-  // MFMA operands of one k16 step: NJ weight pieces, then MI activation pieces, in the order of use
-  struct Frag {
-    bf16x8 w[NJ], a[MI];
-  };
-  constexpr int FRAG = NJ + MI;
-  const bf16_t* ra = As + (wm * S::TM + lane % 32) * LD + (DIRECT ? 0 : (lane / 32) * 8);
-  const bf16_t* rw = Ws + (wn * S::TN + lane % 32) * LD + (DIRECT ? 0 : (lane / 32) * 8);
-  auto lds_read1 = [&](Frag& f, int buf, int ks, int p) {
-    const int at = DIRECT ? ((ks * 2 + lane / 32) ^ (lane % 32 / 2 % 8)) * 8 : ks * 16;     // this lane's place in a row
-    if (p < NJ) f.w[p] = *(const bf16x8*)(rw + (buf * BN + p * 32) * LD + at);
-    else f.a[p - NJ] = *(const bf16x8*)(ra + (buf * BM + (p - NJ) * 32) * LD + at);
-  };
-  // The MFMAs of one k16 step, with memory operations issued between them: slot(n) comes after the
-  // n-th MFMA.  The result tile is transposed (rows = n, columns = m) so that a lane holds four
-  // consecutive n of one output row and can store them as one vector.  The scheduling barriers
-  // keep the compiler from gathering the memory operations back into one place.
-  constexpr int SLOTS = MI * NJ;
-  auto group = [&](const Frag& f, auto&& slot) {
-#pragma unroll
-    for (int n = 0; n < SLOTS; ++n) {
-      acc[n / NJ][n % NJ] =
-          __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[n % NJ], f.a[n / NJ], acc[n / NJ][n % NJ], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      slot(n);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
   // pieces [n * per, (n + 1) * per) of `total`, for spreading `total` operations over slots
   auto spread = [](int n, int total, int slots, auto&& op) {
     const int per = (total + slots - 1) / slots;
@@ -923,12 +900,6 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
       if (p < total) op(p);
   };
 
-  // The loop is software-pipelined by hand, because all waves of a workgroup meet at the barrier
-  // of every k step and so cannot cover for each other: while the MFMAs of one k16 step run, the
-  // fragments of the next are read; the tile of step kt + 1 (loaded into registers during step
-  // kt - 1) is written to the other LDS buffer in the middle of step kt, and the loads of tile
-  // kt + 2 are issued right after; the last k16 step of a tile is multiplied after the barrier,
-  // while the first fragments of the next tile are on their way.
   const int nk = (kend - kbase + B_BK - 1) / B_BK;
   if constexpr (PHASED) {
     static_assert(BM == 256 && BN == 256 && WM == 2 && WN == 4 && BUFS == 2, "quarters of the 256 x 256 tile");
@@ -1008,8 +979,8 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j)
-            acc4[A * 4 + i][B * 2 + j] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[B][ks][j], fa[ks][i], acc4[A * 4 + i][B * 2 + j], 0, 0, 0);
+            acc[A * 4 + i][B * 2 + j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[B][ks][j], fa[ks][i], acc[A * 4 + i][B * 2 + j], 0, 0, 0);
       __builtin_amdgcn_s_setprio(0);
       if constexpr (P == 3) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // what it read is used a phase later
       meet();
@@ -1040,8 +1011,43 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     tl_wait_loads<0>();
     if (wm == 0) meet();
     meet();
-  } else {
-  if constexpr (DIRECT) {
+  } else if constexpr (DIRECT) {
+    // Two k32 steps a buffer, software-pipelined by hand, because all waves of a workgroup meet at the barrier of every k step:
+    // while the MFMAs of one run, the fragments of the next are read; the second is multiplied behind the barrier, ahead of
+    // which the wave has waited for its part of the next buffer, and asks for the pieces that replace this one.
+    // (1,944 rows, 2,048 x 5,632, 128 x 128 tiles: 52.9 us with 32 x 32 x 16 instructions, 48.8 so; 2,048 rows, 4,096 x 14,336,
+    // 256 x 128 tiles: 213 and 201.  Through registers the same takes 5 to 20 % more: LDS writes then stand right ahead of the
+    // barrier, or the loads behind them come late.)
+    // MFMA operands of one k32 step: NJ weight pieces, then MI activation pieces, in the order of use
+    struct Frag {
+      bf16x8 w[NJ], a[MI];
+    };
+    constexpr int FRAG = NJ + MI;
+    const bf16_t* ra = As + (wm * S::TM + lane % 16) * LD;
+    const bf16_t* rw = Ws + (wn * S::TN + lane % 16) * LD;
+    auto lds_read1 = [&](Frag& f, int buf, int ks, int p) {
+      const int at = ((ks * 4 + lane / 16) ^ (lane % 16 / 2)) * 8;         // this lane's place in a row
+      if (p < NJ) f.w[p] = *(const bf16x8*)(rw + (buf * BN + p * 16) * LD + at);
+      else f.a[p - NJ] = *(const bf16x8*)(ra + (buf * BM + (p - NJ) * 16) * LD + at);
+    };
+    // The MFMAs of one k32 step, with memory operations issued between them: slot(n) comes after the
+    // n-th pair.  The result tile is transposed (rows = n, columns = m) so that a lane holds four
+    // consecutive n of one output row and can store them as one vector.  The scheduling barriers
+    // keep the compiler from gathering the memory operations back into one place.
+    constexpr int SLOTS = MI * NJ / 2;
+    auto group = [&](const Frag& f, auto&& slot) {
+#pragma unroll
+      for (int n = 0; n < SLOTS; ++n) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int i = n * 2 / NJ, j = n * 2 % NJ + h;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[j], f.a[i], acc[i][j], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        slot(n);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) direct1(0, kbase, p);
 #pragma unroll
@@ -1053,7 +1059,61 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     if (nk >= BUFS) tl_wait_loads<(BUFS - 1) * PIECES>();
     else tl_wait_loads<0>();
     __syncthreads();
+    Frag f0, f1;
+#pragma unroll
+    for (int p = 0; p < FRAG; ++p) lds_read1(f0, 0, 0, p);
+    static_assert(SLOTS >= 2, "a wave owns at least two pairs of MFMA tiles");
+    auto step = [&](auto has_next, auto has_next2, int kt) {
+      constexpr bool NX = decltype(has_next)::value, NX2 = decltype(has_next2)::value;
+      const int cur = kt % BUFS, nxt = (kt + 1) % BUFS, k2 = kbase + (kt + BUFS) * B_BK;
+      group(f0, [&](int n) {
+        if (n < SLOTS / 2) spread(n, FRAG, SLOTS / 2, [&](int p) { lds_read1(f1, cur, 1, p); });
+      });
+      if constexpr (NX) tl_wait_loads<NX2 ? (BUFS - 2) * PIECES : 0>();      // the next tile has arrived
+      __syncthreads();
+      group(f1, [&](int n) {
+        if constexpr (NX) spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f0, nxt, 0, p); });
+        if constexpr (NX2) spread(n, PIECES, SLOTS, [&](int p) { direct1(cur, k2, p); });     // cur has been read
+      });
+    };
+    int kt = 0;
+    for (; kt + BUFS < nk; ++kt) step(std::true_type{}, std::true_type{}, kt);
+    for (; kt + 1 < nk; ++kt) step(std::true_type{}, std::false_type{}, kt);
+    step(std::false_type{}, std::false_type{}, kt);
   } else {
+    // MFMA operands of one k16 step: NJ32 weight pieces, then MI32 activation pieces, in the order of use
+    struct Frag {
+      bf16x8 w[NJ32], a[MI32];
+    };
+    constexpr int FRAG = NJ32 + MI32;
+    const bf16_t* ra = As + (wm * S::TM + lane % 32) * LD + (lane / 32) * 8;
+    const bf16_t* rw = Ws + (wn * S::TN + lane % 32) * LD + (lane / 32) * 8;
+    auto lds_read1 = [&](Frag& f, int buf, int ks, int p) {
+      const int at = ks * 16;
+      if (p < NJ32) f.w[p] = *(const bf16x8*)(rw + (buf * BN + p * 32) * LD + at);
+      else f.a[p - NJ32] = *(const bf16x8*)(ra + (buf * BM + (p - NJ32) * 32) * LD + at);
+    };
+    // The MFMAs of one k16 step, with memory operations issued between them: slot(n) comes after the
+    // n-th MFMA.  The result tile is transposed (rows = n, columns = m) so that a lane holds four
+    // consecutive n of one output row and can store them as one vector.  The scheduling barriers
+    // keep the compiler from gathering the memory operations back into one place.
+    constexpr int SLOTS = MI32 * NJ32;
+    auto group = [&](const Frag& f, auto&& slot) {
+#pragma unroll
+      for (int n = 0; n < SLOTS; ++n) {
+        acc32[n / NJ32][n % NJ32] =
+            __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[n % NJ32], f.a[n / NJ32], acc32[n / NJ32][n % NJ32], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        slot(n);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // The loop is software-pipelined by hand, because all waves of a workgroup meet at the barrier
+    // of every k step and so cannot cover for each other: while the MFMAs of one k16 step run, the
+    // fragments of the next are read; the tile of step kt + 1 (loaded into registers during step
+    // kt - 1) is written to the other LDS buffer in the middle of step kt, and the loads of tile
+    // kt + 2 are issued right after; the last k16 step of a tile is multiplied after the barrier,
+    // while the first fragments of the next tile are on their way.
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) gload1(kbase, p);
 #pragma unroll
@@ -1063,42 +1123,36 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
       for (int p = 0; p < PIECES; ++p) gload1(kbase + B_BK, p);
     }
     __syncthreads();
-  }
-  Frag f0, f1;
+    Frag f0, f1;
 #pragma unroll
-  for (int p = 0; p < FRAG; ++p) lds_read1(f0, 0, 0, p);
-  static_assert(SLOTS >= 2, "a wave owns at least two MFMA tiles");
-  constexpr int HALF = SLOTS / 2;
-  auto step = [&](auto has_next, auto has_next2, int kt) {
-    constexpr bool NX = decltype(has_next)::value, NX2 = decltype(has_next2)::value;
-    const int cur = DIRECT ? kt % BUFS : kt & 1, nxt = DIRECT ? (kt + 1) % BUFS : cur ^ 1;
-    const int k1 = kbase + (kt + 1) * B_BK, k2 = kbase + (kt + (DIRECT ? BUFS : 2)) * B_BK;
-    group(f0, [&](int n) { spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f1, cur, 1, p); }); });
-    group(f1, [&](int n) {
-      spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f0, cur, 2, p); });
-      if constexpr (NX && !DIRECT)
-        if (n >= SLOTS - HALF) spread(n - (SLOTS - HALF), PIECES / 2, HALF, [&](int p) { lds_write1(nxt, k1, p); });
-    });
-    group(f0, [&](int n) {
-      spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f1, cur, 3, p); });
-      if constexpr (NX && !DIRECT)
-        if (n < HALF) spread(n, PIECES - PIECES / 2, HALF, [&](int p) { lds_write1(nxt, k1, PIECES / 2 + p); });
-      if constexpr (NX2 && !DIRECT)
-        if (n >= SLOTS - HALF) spread(n - (SLOTS - HALF), PIECES, HALF, [&](int p) { gload1(k2, p); });
-    });
-    if constexpr (DIRECT && NX) tl_wait_loads<NX2 ? (BUFS - 2) * PIECES : 0>();      // the next tile has arrived
-    __syncthreads();
-    group(f1, [&](int n) {
-      if constexpr (NX) spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f0, nxt, 0, p); });
-      if constexpr (DIRECT && NX2) spread(n, PIECES, SLOTS, [&](int p) { direct1(cur, k2, p); });     // cur has been read
-    });
-  };
-  {
+    for (int p = 0; p < FRAG; ++p) lds_read1(f0, 0, 0, p);
+    static_assert(SLOTS >= 2, "a wave owns at least two MFMA tiles");
+    constexpr int HALF = SLOTS / 2;
+    auto step = [&](auto has_next, auto has_next2, int kt) {
+      constexpr bool NX = decltype(has_next)::value, NX2 = decltype(has_next2)::value;
+      const int cur = kt & 1, nxt = cur ^ 1, k1 = kbase + (kt + 1) * B_BK, k2 = kbase + (kt + 2) * B_BK;
+      group(f0, [&](int n) { spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f1, cur, 1, p); }); });
+      group(f1, [&](int n) {
+        spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f0, cur, 2, p); });
+        if constexpr (NX)
+          if (n >= SLOTS - HALF) spread(n - (SLOTS - HALF), PIECES / 2, HALF, [&](int p) { lds_write1(nxt, k1, p); });
+      });
+      group(f0, [&](int n) {
+        spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f1, cur, 3, p); });
+        if constexpr (NX)
+          if (n < HALF) spread(n, PIECES - PIECES / 2, HALF, [&](int p) { lds_write1(nxt, k1, PIECES / 2 + p); });
+        if constexpr (NX2)
+          if (n >= SLOTS - HALF) spread(n - (SLOTS - HALF), PIECES, HALF, [&](int p) { gload1(k2, p); });
+      });
+      __syncthreads();
+      group(f1, [&](int n) {
+        if constexpr (NX) spread(n, FRAG, SLOTS, [&](int p) { lds_read1(f0, nxt, 0, p); });
+      });
+    };
     int kt = 0;
-    for (; kt + BUFS < nk; ++kt) step(std::true_type{}, std::true_type{}, kt);
+    for (; kt + 2 < nk; ++kt) step(std::true_type{}, std::true_type{}, kt);
     for (; kt + 1 < nk; ++kt) step(std::true_type{}, std::false_type{}, kt);
     step(std::false_type{}, std::false_type{}, kt);
-  }
   }
 
   // Epilogue.  A lane's accumulators hold four consecutive n of 32 different rows, so stored from
@@ -1140,21 +1194,23 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     if (nm.emit_operand && n < N) load_emit_w(emit_w, n);
   }
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    if constexpr (PHASED) {
+  for (int i = 0; i < MI32; ++i) {
+    if constexpr (DIRECT) {
 #pragma unroll
       for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
-        for (int j = 0; j < 2 * NJ; ++j)
-          *(f32x4*)(cstage + (ii * 16 + lane % 16) * E_LD + j * 16 + (lane / 16) * 4) = acc4[i * 2 + ii][j];
-    } else
+        for (int j = 0; j < NJ; ++j)
+          *(f32x4*)(cstage + (ii * 16 + lane % 16) * E_LD + j * 16 + (lane / 16) * 4) = acc[i * 2 + ii][j];
+    } else {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+      for (int j = 0; j < NJ32; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        f32x4 v4 = {acc[i][j][q * 4 + 0], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
-        *(f32x4*)(cstage + (lane % 32) * E_LD + j * 32 + q * 8 + (lane / 32) * 4) = v4;
-      }
+        for (int q = 0; q < 4; ++q) {
+          const f32x16& c = acc32[i][j];
+          *(f32x4*)(cstage + (lane % 32) * E_LD + j * 32 + q * 8 + (lane / 32) * 4) =
+              f32x4{c[q * 4 + 0], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
+        }
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1194,7 +1250,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
         if constexpr (NEXT) {
 #pragma unroll
           for (int c8 = 0; c8 < 8; ++c8) res_now[c8] = res_next[c8];
-          if (i + 1 < MI && residual && vec_ok) request_residual(i + 1);
+          if (i + 1 < MI32 && residual && vec_ok) request_residual(i + 1);
         }
       }
 #pragma unroll
@@ -1329,19 +1385,13 @@ static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const flo
     return K > 0 ? TL_GEMM(kPhased) : TL_GEMM(kTail);
   } else {
   if constexpr (BM + BN == 384 || BM + BN == 256) {
-    const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
-    const int64_t wgs = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
-    // Straight into LDS where a unit has one workgroup at a time anyway, so that the tiles on their way cost none: the
-    // 128 x 128 tile with fewer than 256 of them, or with 256 in at least 16 columns of tiles (through registers and so:
-    // 3,000 rows, 1,280 x 4,096 46.5 and 42.6 us; 2,048 rows, 2,048 x 4,096 44.7 and 43.6; but 4,096 rows, 1,024 x 2,048, 8
-    // columns, 25.6 and 26.4; beyond 256, two workgroups a unit are worth more), and the 256 x 128 tile for float32 results
-    // (2,048 rows, 4,096 x 4,096: 74.3 and 73.5; 3,000 rows, 4,096 x 14,336: 323.9 and 316.1).  From 16 k steps on: with
-    // fewer the buffers are hardly filled when the last is asked for (4,096 rows, 1,000 x 512: 12.0 and 12.4).  With
-    // bfloat16 results the 256 x 128 tile loses (2,048 rows, 6,144 x 4,096: 98.3 and 100.1).  Four waves of twice the
-    // outputs, which read less from LDS, lose with float32 results (1,944 rows, 2,048 x 5,632: 59.0; 3,288 rows: 88.2 ->
-    // 100.6).
-    const bool few = wgs < 256 || (wgs == 256 && (N + BN - 1) / BN >= 16);
-    if (K >= 16 * B_BK && (BM + BN == 384 ? sizeof(TO) == 4 : few)) return TL_GEMM(kDirect);
+    // Straight into LDS: the tiles on their way cost no registers, and a unit's one workgroup multiplies for the two that the
+    // 128 x 128 tile had through registers (4,096^3 145 us through registers, 130 so; 2,048 rows, 2,048 x 512 10.0 and 9.0;
+    // with 256 x 128 tiles 2,048 rows, 4,096 x 4,096 65.0 and 59.0; 4,096 rows, 1,024 x 512 10.1 and 9.2; 2,048 x 4,096 x 512,
+    // where two workgroups a unit cover for each other's first loads, 15.3 and 16.0).  With fewer than four steps the buffers
+    // are not even filled.  Four waves of twice the outputs, which read less from LDS, lose with float32 results (1,944 rows,
+    // 2,048 x 5,632: 59.0; 3,288 rows: 88.2 -> 100.6).
+    if (K >= 4 * B_BK) return TL_GEMM(kDirect);
   }
   return TL_GEMM(kWhole);
   }
@@ -1355,7 +1405,7 @@ struct TileChoice {
   int bm, bn;
   double rate;
 };
-static const TileChoice kTiles[4] = {{256, 256, 1320.}, {256, 128, 920.}, {128, 128, 775.}, {64, 128, 650.}};
+static const TileChoice kTiles[4] = {{256, 256, 1400.}, {256, 128, 1130.}, {128, 128, 980.}, {64, 128, 650.}};
 
 static double tile_cost(int c, int M, int N) {
   const int64_t wgs = (int64_t)((M + kTiles[c].bm - 1) / kTiles[c].bm) * ((N + kTiles[c].bn - 1) / kTiles[c].bn);
@@ -1685,7 +1735,11 @@ static int splitk_plan(int M, int N, int K, int* tile, int* k_per_split) {
   const int64_t weights = (int64_t)N * K;
   const bool ring_rows = M <= O_BM || (M <= 128 && N <= 6144 && weights <= ((int64_t)26 << 20)) ||
                          (M <= 256 && weights <= ((int64_t)6 << 20));
-  if (M > 16 && ring_rows && K % O_SLAB_K == 0 && K >= 4 * O_SLAB_K) {
+  // Beyond 64 rows it and its second kernel have to beat the 128 x 128 tile unsplit, 0.365 us a k step (150 rows, inner size
+  // 1,024: 2,048 columns 10.1 us against 10.3, 4,096 12.5 against 10.7; inner size 512: never).  Only a split product can hand over
+  // a norm of a width that is no multiple of 64: those stay split.
+  const bool ring_pays = M <= O_BM || N % 64 || 7.0 + 1.05e-5 * M * N < 4.6 + 0.365 * (K / B_BK);
+  if (M > 16 && ring_rows && ring_pays && K % O_SLAB_K == 0 && K >= 4 * O_SLAB_K) {
     int slabs;
     const int one = oneshot_plan(M, N, K, &slabs);
     *tile = -1;
@@ -1698,13 +1752,36 @@ static int splitk_plan(int M, int N, int K, int* tile, int* k_per_split) {
   if (wgs >= 160) return 1;
   if (M <= 64 && (int64_t)N * K < (int64_t)8 << 20) return 1;      // small weights: the few-row kernel is faster
   const int nk = (K + B_BK - 1) / B_BK;
-  const int want = (int)((256 + wgs - 1) / wgs);
-  int per = (nk + want - 1) / want;
-  if (per < 4) per = 4;
-  const int splits = (nk + per - 1) / per;
-  if (splits < 2) return 1;
+  int splits = 1;
+  if (N % 64 || K % B_BK || M <= 64) {      // (M <= 64 is the ring kernel's but for the shortest and odd inner sizes)
+    const int want = (int)((256 + wgs - 1) / wgs);
+    const int per = max((nk + want - 1) / want, 4);
+    splits = (nk + per - 1) / per;
+    *k_per_split = per * B_BK;
+  } else {
+    // The number of splits with the smallest estimated time in us: rounds of workgroups over the 256 units (the tile's buffers
+    // leave room for one on each), 4 each and 0.36 to 0.42 a k step, and behind a split the second kernel, which reads the parts
+    // and about as much again (512 rows: 2,048 x 2,048 unsplit 17.1, in four 21.4; 2,048 x 4,096 29.2 and 20.9; 1,944 rows,
+    // 704 x 2,048 18.0 and, in three, 25.7).
+    double best = 0.;
+    for (int want = 1; want <= 64; ++want) {
+      const int per = (nk + want - 1) / want, got = (nk + per - 1) / per;
+      if (want > 1 && (per < 4 || got < want)) continue;
+      const int64_t all = wgs * got;
+      const double t = (double)((all + 255) / 256) * (4. + per * (all <= 128 ? 0.36 : 0.42)) +
+                       (got > 1 ? 2.5 + (got + 2.) * M * N * 4 / 4e6 : 0.);
+      if (best == 0. || t < best) {
+        best = t;
+        splits = got;
+        *k_per_split = per * B_BK;
+      }
+    }
+  }
+  if (splits < 2) {
+    *k_per_split = 0;
+    return 1;
+  }
   *tile = M <= 64 ? 4 : 3;
-  *k_per_split = per * B_BK;
   return splits;
 }
 

@@ -1437,3 +1437,27 @@ def test_handover_probe_runs_and_its_waits_are_bounded():
     except ops().KernelError as e:
         assert "ran out" in str(e)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("experts,top,groups,keep", [(1, 1, 1, 1), (5, 5, 1, 1), (16, 4, 4, 2), (48, 7, 6, 3), (63, 8, 1, 1), (64, 64, 1, 1),
+                                                     (64, 6, 8, 8), (64, 5, 32, 3), (66, 6, 6, 2)])
+def test_router_places_by_lanes(experts, top, groups, keep):
+    """Routers of up to 64 experts, one a lane, and past that: logits of a few values, so that most scores and runs of experts
+    tie and the lower index has to come first; rows with -inf (a score of zero); the weights against float64."""
+    g = torch.Generator().manual_seed(experts + top)
+    z = torch.randint(-2, 3, (37, experts), generator=g).float()
+    z[5:9, ::2] = -math.inf
+    z[:, -1] = 1.0
+    ids = torch.full((37, top), -1, dtype=torch.int32, device=DEV)
+    wts = torch.full((37, top), float("nan"), device=DEV)
+    ops().moe_route(z.to(DEV), ids, wts, groups, keep, 1.5)
+    p = z.double().softmax(1)
+    for t in range(37):
+        by_run = p[t].view(groups, -1).amax(1)
+        runs = sorted(range(groups), key=lambda r: (-by_run[r].item(), r))[:keep if groups > 1 else groups]
+        allowed = [e for e in range(experts) if e // (experts // groups) in runs]
+        want = sorted(allowed, key=lambda e: (-p[t, e].item(), e))[:top]
+        assert ids[t].tolist() == want
+        w = p[t, want] / (p[t, want].sum() + 1e-20) * 1.5
+        # exp, the sum over the experts, the division, the sum of the chosen, its division and the scale
+        assert ((wts[t].cpu().double() - w).abs() <= (experts + top + 8) * 2.0 ** -24 * w.abs() + 1e-30).all()

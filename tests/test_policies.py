@@ -72,3 +72,21 @@ def test_small_experts_products_go_by_rows():
     assert not up(128, 512) and not up(2048, 1024) and not up(2 * 256, 1024, gate) and not up(256, 2048)
     assert down(6, 4, 2048, 704) and down(32, 2, 1024, 1024) and not down(8, 8, 1024, 256) and not down(64, 1, 512, 1536)
     assert down(1, 8, 256, 64) and down(2, 2, 64, 32) and not down(2, 1, 512, 128) and not down(3, 2, 256, 128)
+
+
+def test_split_products_keep_their_number_of_parts():
+    """How many float32 parts a split product's sums are added in, and so what its results round to: sizes of the ring
+    kernel (two to sixteen parts), and of 128 x 128 tiles, shared out over 256 workgroups with at least four steps of 64 each."""
+    plan = library.load(verbose=False).tl_splitk_plan
+    ring = {(66, 1024, 512): 2, (80, 2048, 2048): 8, (128, 4096, 4096): 4, (150, 4096, 1024): 2, (200, 2048, 512): 2,
+            (256, 2560, 2048): 3, (128, 1408, 2048): 8}
+    for sizes, parts in ring.items():
+        assert plan(*sizes) == parts, sizes
+    for M in (257, 300, 400, 512, 640, 700, 1000, 1944, 2500):
+        for N in (256, 518, 704, 1280, 2048, 2560, 4096, 6144, 11264):
+            for K in (256, 512, 520, 1024, 1096, 2048, 4096, 5632, 14336):
+                tiles, steps, parts = -(-M // 128) * -(-N // 128), -(-K // 64), 1
+                if K >= 512 and tiles < 160:
+                    share = max(-(-steps // -(-256 // tiles)), 4)
+                    parts = -(-steps // share)
+                assert plan(M, N, K) == parts, (M, N, K)

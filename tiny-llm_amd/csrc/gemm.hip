@@ -1725,7 +1725,9 @@ __global__ __launch_bounds__(R_THREADS) void splitk_reduce_kernel(const ReduceAr
 // How a bfloat16 product of these sizes is best split: returns the number of splits (1: not at
 // all) and sets the tile (as tl_linear_tile's) and the inner size per split.  Splitting pays when
 // the output has too few tiles to fill 256 compute units and the rows are too many for the
-// few-row kernel to stream the weights at full rate.
+// few-row kernel to stream the weights at full rate.  The number of parts is the order in which a result's float32 sums are
+// added, and the sizes here are those of a step's rows: another number moves the logits of a batch (0.2 to 0.9 % of their norm
+// where an estimate from products replayed on cached weights chose fewer).
 static int splitk_plan(int M, int N, int K, int* tile, int* k_per_split) {
   *tile = 0;
   *k_per_split = 0;
@@ -1735,11 +1737,7 @@ static int splitk_plan(int M, int N, int K, int* tile, int* k_per_split) {
   const int64_t weights = (int64_t)N * K;
   const bool ring_rows = M <= O_BM || (M <= 128 && N <= 6144 && weights <= ((int64_t)26 << 20)) ||
                          (M <= 256 && weights <= ((int64_t)6 << 20));
-  // Beyond 64 rows it and its second kernel have to beat the 128 x 128 tile unsplit, 0.365 us a k step (150 rows, inner size
-  // 1,024: 2,048 columns 10.1 us against 10.3, 4,096 12.5 against 10.7; inner size 512: never).  Only a split product can hand over
-  // a norm of a width that is no multiple of 64: those stay split.
-  const bool ring_pays = M <= O_BM || N % 64 || 7.0 + 1.05e-5 * M * N < 4.6 + 0.365 * (K / B_BK);
-  if (M > 16 && ring_rows && ring_pays && K % O_SLAB_K == 0 && K >= 4 * O_SLAB_K) {
+  if (M > 16 && ring_rows && K % O_SLAB_K == 0 && K >= 4 * O_SLAB_K) {
     int slabs;
     const int one = oneshot_plan(M, N, K, &slabs);
     *tile = -1;
@@ -1752,36 +1750,13 @@ static int splitk_plan(int M, int N, int K, int* tile, int* k_per_split) {
   if (wgs >= 160) return 1;
   if (M <= 64 && (int64_t)N * K < (int64_t)8 << 20) return 1;      // small weights: the few-row kernel is faster
   const int nk = (K + B_BK - 1) / B_BK;
-  int splits = 1;
-  if (N % 64 || K % B_BK || M <= 64) {      // (M <= 64 is the ring kernel's but for the shortest and odd inner sizes)
-    const int want = (int)((256 + wgs - 1) / wgs);
-    const int per = max((nk + want - 1) / want, 4);
-    splits = (nk + per - 1) / per;
-    *k_per_split = per * B_BK;
-  } else {
-    // The number of splits with the smallest estimated time in us: rounds of workgroups over the 256 units (the tile's buffers
-    // leave room for one on each), 4 each and 0.36 to 0.42 a k step, and behind a split the second kernel, which reads the parts
-    // and about as much again (512 rows: 2,048 x 2,048 unsplit 17.1, in four 21.4; 2,048 x 4,096 29.2 and 20.9; 1,944 rows,
-    // 704 x 2,048 18.0 and, in three, 25.7).
-    double best = 0.;
-    for (int want = 1; want <= 64; ++want) {
-      const int per = (nk + want - 1) / want, got = (nk + per - 1) / per;
-      if (want > 1 && (per < 4 || got < want)) continue;
-      const int64_t all = wgs * got;
-      const double t = (double)((all + 255) / 256) * (4. + per * (all <= 128 ? 0.36 : 0.42)) +
-                       (got > 1 ? 2.5 + (got + 2.) * M * N * 4 / 4e6 : 0.);
-      if (best == 0. || t < best) {
-        best = t;
-        splits = got;
-        *k_per_split = per * B_BK;
-      }
-    }
-  }
-  if (splits < 2) {
-    *k_per_split = 0;
-    return 1;
-  }
+  const int want = (int)((256 + wgs - 1) / wgs);
+  int per = (nk + want - 1) / want;
+  if (per < 4) per = 4;
+  const int splits = (nk + per - 1) / per;
+  if (splits < 2) return 1;
   *tile = M <= 64 ? 4 : 3;
+  *k_per_split = per * B_BK;
   return splits;
 }
 

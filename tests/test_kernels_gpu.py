@@ -362,8 +362,8 @@ def test_linear_large_tile_in_quarters(M, N, K):
 @pytest.mark.parametrize("tile,M,N,K", [(t, 300, 260, k) for t in (2, 3) for k in (192, 256, 320, 384, 448, 576)] +
                          [(0, 1944, 704, 2048), (0, 512, 2048, 2048), (0, 150, 4096, 1024), (0, 66, 1024, 512), (0, 700, 2048, 4096)])
 def test_linear_few_steps_and_splits(tile, M, N, K):
-    """Operand tiles straight into LDS from four k steps on, around the number of buffers; and sizes on both sides of what is
-    split: unsplit since the tiles go that way, or split into fewer parts."""
+    """Operand tiles straight into LDS from four k steps on, around the number of buffers; and sizes whose inner size is split
+    into shares of a few steps, in the ring kernel and in tiles."""
     _operand_tiles(tile, M, N, K)
 
 

@@ -1374,26 +1374,37 @@ static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, cons
   return TL_OK;
 }
 
+// How the operands of a tile reach LDS.  Straight from memory where the inner size is whole steps: always in the 256 x 256
+// tile; in the 256 x 128 tile from four steps on (with fewer its buffers are not even filled; 2,047 rows, 4,096 x 4,096, weights
+// from memory: 68.1 us through registers, 61.8 so; 4,096 x 256 11.3 and 10.5); in the 128 x 128 tile likewise, if each
+// workgroup has a unit to itself.  Its four buffers leave a unit room for one workgroup, where through registers two share it,
+// and a second round for a few more workgroups than units costs a whole one (1,500 rows, 1,408 x 1,088 in two parts, 264
+// workgroups: 23.3 us through registers, 25.9 so; 300 rows, 2,048 x 2,048 in six 20.0 and 22.8).  532 products of up to 256
+// workgroups: 1.0 to 1.26x as fast so, median 1.09; 340 of more and 4 to 16 steps: 0.74 to 1.16x, median 0.91; beyond, where
+// the larger tiles serve nearly all, 0.83 to 1.19x, median 1.05.  Four waves of twice the outputs, which read less from LDS,
+// lose with float32 results (1,944 rows, 2,048 x 5,632: 59.0; 3,288 rows: 88.2 -> 100.6).
+static int tile_mode(int bm, int bn, int M, int N, int K, int k_per_split) {
+  if (K % B_BK) return kTail;
+  if (bm + bn == 512) return kPhased;
+  const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
+  const int64_t wgs = (int64_t)((N + bn - 1) / bn) * ((M + bm - 1) / bm) * splits;
+  return K >= 4 * B_BK && (bm + bn == 384 || (bm + bn == 256 && wgs <= 256)) ? kDirect : kWhole;
+}
+
 template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU>
 static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const float* residual, const TileNorm& row_scale,
                             int M, int N, int K, int64_t lda, int64_t ldo, int k_per_split, hipStream_t stream) {
 #define TL_GEMM(MODE)                                                                                                  \
   launch_gemm_bf16_mode<BM, BN, WM, WN, TO, SWIGLU, MODE>(a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split, \
                                                           stream)
-  if (K % B_BK) return TL_GEMM(kTail);
+  const int mode = tile_mode(BM, BN, M, N, K, k_per_split);
+  if (mode == kTail) return TL_GEMM(kTail);
   if constexpr (BM + BN == 512) {
-    return K > 0 ? TL_GEMM(kPhased) : TL_GEMM(kTail);
+    return TL_GEMM(kPhased);
   } else {
-  if constexpr (BM + BN == 384 || BM + BN == 256) {
-    // Straight into LDS: the tiles on their way cost no registers, and a unit's one workgroup multiplies for the two that the
-    // 128 x 128 tile had through registers (4,096^3 145 us through registers, 130 so; 2,048 rows, 2,048 x 512 10.0 and 9.0;
-    // with 256 x 128 tiles 2,048 rows, 4,096 x 4,096 65.0 and 59.0; 4,096 rows, 1,024 x 512 10.1 and 9.2; 2,048 x 4,096 x 512,
-    // where two workgroups a unit cover for each other's first loads, 15.3 and 16.0).  With fewer than four steps the buffers
-    // are not even filled.  Four waves of twice the outputs, which read less from LDS, lose with float32 results (1,944 rows,
-    // 2,048 x 5,632: 59.0; 3,288 rows: 88.2 -> 100.6).
-    if (K >= 4 * B_BK) return TL_GEMM(kDirect);
-  }
-  return TL_GEMM(kWhole);
+    if constexpr (BM + BN >= 256)
+      if (mode == kDirect) return TL_GEMM(kDirect);
+    return TL_GEMM(kWhole);
   }
 #undef TL_GEMM
 }
@@ -2674,6 +2685,12 @@ int tl_handoff_parts(int M, int N, int K) {
   const bool one_tile = M <= 16 || N < 256 * 32;
   const int cw = one_tile ? skinny_cols_wg(N) : S_COLS;
   return (N + cw - 1) / cw;
+}
+
+// How the operands of a tile (1 to 4, as tl_linear_tile's) reach LDS at these sizes (see tile_mode): 0 and 1 through
+// registers, 2 and 3 straight from memory.
+int tl_tile_mode(int tile, int M, int N, int K, int k_per_split) {
+  return tile >= 1 && tile <= 4 ? tile_mode(kTiles[tile - 1].bm, kTiles[tile - 1].bn, M, N, K, k_per_split) : -1;
 }
 
 // See splitk_plan.  A caller that gets more than one split allocates a float32 workspace of

@@ -1411,23 +1411,29 @@ static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const flo
 
 // Which tile: the one with the smallest estimated time.  A compute unit works through
 // ceil(workgroups / 256) tiles one after the other, each at the rate that its tile shape reaches
-// on a full chip (measured, TFLOP/s: the larger the tile, the fewer operand bytes per flop).
+// on a full chip (measured, TFLOP/s: the larger the tile, the fewer operand bytes per flop): `straight` from eight whole steps
+// on, where all but the 64 x 128 tile get their operands straight from memory, and `rate` for inner sizes that end within a
+// step, whose tiles go through registers, and for fewer steps, where first loads and the epilogue (10 us a 256 x 256 tile,
+// whose step takes 1) count for more than the loop (2,200 rows, 3,712 x 64: 9.8 us with the 64 x 128 tiles that `rate`
+// chooses, 12.5 with the 256 x 256 that `straight` would; 700 rows, 11,264 x 192 13.4 and 15.3; x 256 14.8 and 15.2; x 512
+// 20.8 and 19.1; x 2,048 53.1 and 43.6).
 struct TileChoice {
   int bm, bn;
-  double rate;
+  double rate, straight;
 };
-static const TileChoice kTiles[4] = {{256, 256, 1400.}, {256, 128, 1130.}, {128, 128, 980.}, {64, 128, 650.}};
+static const TileChoice kTiles[4] = {{256, 256, 1060., 1400.}, {256, 128, 900., 1130.}, {128, 128, 760., 980.}, {64, 128, 640., 650.}};
 
-static double tile_cost(int c, int M, int N) {
+static double tile_cost(int c, int M, int N, int K) {
   const int64_t wgs = (int64_t)((M + kTiles[c].bm - 1) / kTiles[c].bm) * ((N + kTiles[c].bn - 1) / kTiles[c].bn);
-  return (double)((wgs + 255) / 256) * kTiles[c].bm * kTiles[c].bn / kTiles[c].rate;
+  const double rate = K % B_BK == 0 && K >= 8 * B_BK ? kTiles[c].straight : kTiles[c].rate;
+  return (double)((wgs + 255) / 256) * kTiles[c].bm * kTiles[c].bn / rate;
 }
 
-static int best_tile(int M, int N, double* cost) {
+static int best_tile(int M, int N, int K, double* cost) {
   int best = 0;
   double best_cost = 0.;
   for (int c = 0; c < 4; ++c) {
-    const double t = tile_cost(c, M, N);
+    const double t = tile_cost(c, M, N, K);
     if (c == 0 || t < best_cost) {
       best = c;
       best_cost = t;
@@ -1469,15 +1475,15 @@ static int launch_gemm_bf16_any(const bf16_t* a, const bf16_t* w, TO* out, const
     return launch_gemm_bf16_tile<TO, SWIGLU>(tile - 1, a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split,
                                              stream);
   double whole_cost;
-  const int whole = best_tile(M, N, &whole_cost);
+  const int whole = best_tile(M, N, K, &whole_cost);
   if (k_per_split == 0) {
     const int tiles_m = (M + 255) / 256;
     const int cols_per_round = 256 / tiles_m * 256;          // columns that one round of 256 x 256 tiles covers
     const int n_first = cols_per_round > 0 ? N / cols_per_round * cols_per_round : 0;
     if (n_first > 0 && n_first < N) {
       double rest_cost;
-      const int rest = best_tile(M, N - n_first, &rest_cost);
-      if (tile_cost(0, M, n_first) + rest_cost < whole_cost) {
+      const int rest = best_tile(M, N - n_first, K, &rest_cost);
+      if (tile_cost(0, M, n_first, K) + rest_cost < whole_cost) {
         int rc = launch_gemm_bf16_tile<TO, SWIGLU>(0, a, w, out, residual, row_scale, M, n_first, K, lda, ldo, 0, stream);
         if (rc != TL_OK) return rc;
         const int64_t o_off = SWIGLU ? n_first / 2 : n_first;
@@ -2692,6 +2698,9 @@ int tl_handoff_parts(int M, int N, int K) {
 int tl_tile_mode(int tile, int M, int N, int K, int k_per_split) {
   return tile >= 1 && tile <= 4 ? tile_mode(kTiles[tile - 1].bm, kTiles[tile - 1].bn, M, N, K, k_per_split) : -1;
 }
+
+// The tile (1 to 4) that a product of these sizes takes unless it is split or launched in two parts.
+int tl_best_tile(int M, int N, int K) { return best_tile(M, N, K, nullptr) + 1; }
 
 // See splitk_plan.  A caller that gets more than one split allocates a float32 workspace of
 // splits * M * N elements and calls tl_linear_splitk with the same sizes.

@@ -1,5 +1,7 @@
 """Decisions the host takes about a launch, checked without a GPU: how many workgroups share the keys
 of a decode step's requests."""
+import ctypes
+
 import pytest
 
 from tiny_llm_amd.kernels import library, ops
@@ -118,3 +120,20 @@ def test_a_tile_is_chosen_by_the_rates_of_the_way_its_operands_go():
             assert best(M, N, K) == 1, (M, N, K)
     for K in (64, 72, 256, 512, 1000, 2048):
         assert best(2048, 28672, K) == 1 and best(2048, 4096, K) == 2 and best(2048, 2048, K) == 3 and best(512, 2048, K) == 4, K
+
+
+def _places(tiles_m, tiles_n, banded):
+    place = library.load(verbose=False).tl_tile_place
+    at, places = (ctypes.c_int * 2)(), []
+    for t in range(tiles_m * tiles_n):
+        place(t, tiles_m, tiles_n, banded, at)
+        places.append((at[0], at[1]))
+    assert sorted(places) == [(m, n) for m in range(tiles_m) for n in range(tiles_n)]      # every tile, once
+    return places
+
+
+@pytest.mark.parametrize("tiles_m", list(range(1, 45)) + [64, 101])
+def test_tiles_through_registers_and_few_rows_of_tiles_stand_in_columns(tiles_m):
+    columns = [(m, n) for n in range(5) for m in range(tiles_m)]
+    assert _places(tiles_m, 5, 0) == columns
+    assert (_places(tiles_m, 5, 1) == columns) == (tiles_m < 8)

@@ -73,15 +73,23 @@ template <int LEFT>       // until at most LEFT of the wave's loads are still on
 __device__ __forceinline__ void tl_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
 
 // Workgroups are handed to the eight XCDs in turn, each with an L2 of its own.  The index is remapped so that an XCD owns a
-// contiguous run of tiles, and the tiles that it works on at a time make a block about as high as it is wide, which asks the
-// fewest rows of both operands of its L2 (8192^3 with 256 x 256 tiles in columns of 32 927 us, in bands of four 786): bands
-// of 4 to 7 tiles of rows, column by column.
+// contiguous run of tiles, and, `banded`, the tiles that it works on at a time make a block about as high as it is wide, which
+// asks the fewest rows of both operands of its L2 (8192^3 with 256 x 256 tiles in columns of 32 927 us, in bands of four 786):
+// bands of 4 to 7 tiles of rows, column by column.  Fewer than eight rows of tiles are one band, found by one division: three
+// more took 0.1 to 0.25 us a launch.  128 x 128 and 64 x 128 tiles through registers stand in columns, whatever their number:
+// two to four share a unit and short steps wait for each other, not for the L2 (2,102 rows, 3,712 x 128 in 128 x 128 tiles
+// 8.94 us in bands, 8.63 so; 4,096 rows, 2,560 x 328 18.5 and 17.4; 2,047 rows, 4,096 x 192 with a residual 16.9 and 14.4).
 constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_tile(int block, int total) {
   const int per_xcd = (total + kXcds - 1) / kXcds;
   return (block % kXcds) * per_xcd + block / kXcds;
 }
-__device__ __forceinline__ void tile_place(int t, int tiles_m, int tiles_n, int* tm, int* tn) {
+__host__ __device__ __forceinline__ void tile_place(int t, int tiles_m, int tiles_n, bool banded, int* tm, int* tn) {
+  if (!banded || tiles_m < 8) {
+    *tm = t % tiles_m;
+    *tn = t / tiles_m;
+    return;
+  }
   const int bands = max(tiles_m / 4, 1), band_m = (tiles_m + bands - 1) / bands;
   const int band = t / (band_m * tiles_n), in_band = t - band * band_m * tiles_n, high = min(band_m, tiles_m - band * band_m);
   *tm = band * band_m + in_band % high;
@@ -311,7 +319,7 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f32_ring_kernel(const float* _
   const int t = xcd_tile(blockIdx.x, tiles_m * tiles_n);
   if (t >= tiles_m * tiles_n) return;                      // the grid is padded to a multiple of 8
   int tile_m, tile_n;
-  tile_place(t, tiles_m, tiles_n, &tile_m, &tile_n);
+  tile_place(t, tiles_m, tiles_n, true, &tile_m, &tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   // Each buffer begins at the tile's first row and ends with the matrix: rows beyond it read as zeros.
   auto buffer_words = [](const float* first_row, int rows, int64_t ld, int K_) {
@@ -794,7 +802,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   if (t_all >= total) return;                           // the grid is padded to a multiple of 8
   const int split = t_all / tiles, t = t_all % tiles;
   int tile_m, tile_n;
-  tile_place(t, tiles_m, (N + BN - 1) / BN, &tile_m, &tile_n);
+  tile_place(t, tiles_m, (N + BN - 1) / BN, DIRECT || BM == 256, &tile_m, &tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int kbase = split * k_per_split;
   const int kend = k_per_split > 0 ? min(K, kbase + k_per_split) : K;
@@ -2701,6 +2709,11 @@ int tl_tile_mode(int tile, int M, int N, int K, int k_per_split) {
 
 // The tile (1 to 4) that a product of these sizes takes unless it is split or launched in two parts.
 int tl_best_tile(int M, int N, int K) { return best_tile(M, N, K, nullptr) + 1; }
+
+// Where tile t of tiles_m x tiles_n stands (see tile_place): place[0] its row of tiles, place[1] its column.
+void tl_tile_place(int t, int tiles_m, int tiles_n, int banded, int* place) {
+  tile_place(t, tiles_m, tiles_n, banded != 0, place, place + 1);
+}
 
 // See splitk_plan.  A caller that gets more than one split allocates a float32 workspace of
 // splits * M * N elements and calls tl_linear_splitk with the same sizes.

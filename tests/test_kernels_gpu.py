@@ -340,14 +340,15 @@ def test_linear_operand_tiles(tile, M, N, K):
                                    (1, 128, 1032), (2049, 2052, 1024), (2048, 2048, 1024), (2000, 2047, 1088),
                                    (4096, 1024, 1024), (3970, 1024, 1088)])
 def test_linear_operand_tiles_straight_into_lds(tile, M, N, K):
-    """From 16 k steps on operand tiles may go straight into LDS: every number of steps against the three and four buffers,
-    and both sides of the limits (256 tiles of 128 x 128 in 16 columns or in 8)."""
+    """Operand tiles straight into LDS: every number of steps against the three and four buffers, and 128 x 128 tiles of 256
+    workgroups, the most that go this way, and of more, which go through registers."""
     _operand_tiles(tile, M, N, K)
 
 
 @pytest.mark.parametrize("M,N", [(4096, 4096), (4095, 4092), (2048, 1024)])
 def test_linear_residual_of_large_tiles(M, N):
-    """256 x 256 tiles: the residual piece by piece with 256 of them, requested ahead with fewer."""
+    """The residual of 256 x 256 tiles, requested 32 rows ahead, also where rows and columns end inside a tile; and that of the
+    smallest tile, requested for its own 32 rows."""
     _operand_tiles(0, M, N, 64)
 
 
@@ -1119,11 +1120,27 @@ def test_decode_steps_without_tile_lists_give_the_bits_of_those_with(nq, nkv, hd
     """Row i is request i's one new token: said by tile lists or known without (then pages of 16 keys and more and heads of
     32, 64 and 128 have a kernel of their own).  The same products in the same order: the same bits, over every mask and
     finish, contexts around the 64-key tiles and more splits than tiles, with NaN wherever no key of the request lies."""
+    _with_and_without_tile_lists(nq, nkv, hd, bs, opts, n_splits, False)
+
+
+@pytest.mark.parametrize("nq,nkv,hd,bs,opts", [
+    (4, 4, 32, 16, {}), (15, 1, 64, 32, {}), (16, 1, 128, 16, {}), (8, 2, 128, 64, {"window": 65}), (6, 2, 64, 16, {"window": -100}),
+    (8, 2, 128, 16, {"window": 130, "keep": 5}), (4, 1, 64, 128, {"window": 64, "keep": 70, "softcap": 20.0}),
+    (4, 2, 32, 16, {"softcap": 15.0, "out_scale": 0.5}), (8, 2, 128, 16, {"sink": True, "finish": True, "window": 100}),
+    (8, 1, 64, 16, {"finish": True, "value_dim": 38, "f32": True}), (4, 1, 128, 16, {"value_dim": 100, "finish": True})])
+@pytest.mark.parametrize("n_splits", [1, 3])
+def test_fused_decode_steps_without_tile_lists_give_the_bits_of_those_with(nq, nkv, hd, bs, opts, n_splits):
+    """The same with the rotation and the cache write inside, over every mask and finish: the same bits, of the cache's rows,
+    too, where the new token's row and every row behind it held NaN."""
+    _with_and_without_tile_lists(nq, nkv, hd, bs, opts, n_splits, True)
+
+
+def _with_and_without_tile_lists(nq, nkv, hd, bs, opts, n_splits, fused):
     opts = dict(opts)
     f32, finish = opts.pop("f32", False), opts.pop("finish", False)
     g = torch.Generator().manual_seed(nq * 131 + hd + bs)
     lens = [1, 15, 16, 17, 63, 64, 65, 128, 191, 300, 513, 1]
-    R = len(lens)
+    R, kept = len(lens), 1 if fused else 0       # fused: the new token's row of the cache is not written yet
     mb = max(-(-l // bs) for l in lens) + 1
     nblocks = sum(-(-l // bs) for l in lens) + 2
     perm = (torch.randperm(nblocks - 1, generator=g) + 1).tolist()
@@ -1133,11 +1150,14 @@ def test_decode_steps_without_tile_lists_give_the_bits_of_those_with(nq, nkv, hd
     for r, L in enumerate(lens):
         for b in range(-(-L // bs)):
             bt[r, b] = perm.pop()
-            rows = min(bs, L - b * bs)
+            rows = max(0, min(bs, L - kept - b * bs))
             kc[bt[r, b], :, :rows] = torch.randn(nkv, rows, hd, generator=g).to(torch.bfloat16)
             vc[bt[r, b], :, :rows] = torch.randn(nkv, rows, hd, generator=g).to(torch.bfloat16)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
-    q = torch.randn(R, nq * hd + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :nq * hd]
+    q = torch.randn(R, (nq + kept * 2 * nkv) * hd + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :nq * hd]
+    if fused:
+        from tiny_llm_amd.parts.rotary import RotaryEmbedding
+        opts["fused_rope"] = RotaryEmbedding("r", torch.bfloat16, DEV, head_dim=hd, theta=10000.0, max_position=600).rotary_tables()[:2]
     if finish:
         opts["gate"] = torch.randn(R, nq, generator=g).to(DEV)
         if opts.get("sink"):
@@ -1148,10 +1168,14 @@ def test_decode_steps_without_tile_lists_give_the_bits_of_those_with(nq, nkv, hd
     for tiles in ((i32(list(range(R))), i32(list(range(R))), i32([1] * R)), None):
         out = torch.zeros(R, cols + 1, dtype=torch.float32 if f32 else torch.bfloat16, device=DEV)[:, :cols]
         scratch = torch.full((n_splits * R * nq * (hd + 2),), float("nan"), device=DEV)
-        ops().flash_attention(q, kc, vc, bt, tiles, pos, out, nq, nkv, hd, hd ** -0.5, n_splits=n_splits, scratch=scratch, **opts)
-        got.append(out)
-    assert torch.isfinite(got[0].float()).all() and got[0].float().abs().max() > 0.1
-    assert torch.equal(got[0], got[1])
+        k, v = kc.clone(), vc.clone()
+        ops().flash_attention(q, k, v, bt, tiles, pos, out, nq, nkv, hd, hd ** -0.5, n_splits=n_splits, scratch=scratch, **opts)
+        got.append((out, k.view(torch.int16), v.view(torch.int16)))
+    out, k, v = got[0]
+    assert torch.isfinite(out.float()).all() and out.float().abs().max() > 0.1
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    keys = sum(lens) * nkv * hd                  # every key of a request, and no other row, holds numbers
+    assert torch.isfinite(k.view(torch.bfloat16).float()).sum() == keys == torch.isfinite(v.view(torch.bfloat16).float()).sum()
 
 
 @pytest.mark.parametrize("hd", [48, 80, 112])
@@ -1461,3 +1485,46 @@ def test_router_places_by_lanes(experts, top, groups, keep):
         w = p[t, want] / (p[t, want].sum() + 1e-20) * 1.5
         # exp, the sum over the experts, the division, the sum of the chosen, its division and the scale
         assert ((wts[t].cpu().double() - w).abs() <= (experts + top + 8) * 2.0 ** -24 * w.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("experts,top,groups,keep,opts", [
+    (16, 4, 4, 2, {}), (64, 8, 8, 4, {"correction": True}), (64, 64, 1, 1, {"bias": True, "correction": True}),
+    (60, 7, 12, 5, {"score": "sigmoid", "correction": True, "group_top2": True}), (5, 3, 1, 1, {"score": "sigmoid", "bias": True}),
+    (48, 6, 6, 3, {"correction": True, "group_top2": True, "normalize": False}), (64, 9, 1, 1, {"correction": True, "normalize": False}),
+    (32, 2, 32, 2, {"score": "sigmoid", "group_top2": True, "normalize": False})])
+def test_router_by_lanes_gives_the_bits_of_the_general_form(experts, top, groups, keep, opts):
+    """The same logits for up to 64 experts, one a lane, and with experts of logits -inf behind them, past 64, which the
+    general form takes: the same experts and the same bits of their weights.  Also rows that the form by lanes leaves to the
+    general one: +inf, NaN and nothing but -inf among the logits (where every score is NaN, any expert of the row may come),
+    and corrections of both infinities."""
+    opts = dict(opts)
+    g = torch.Generator().manual_seed(experts + top + groups)
+    per = experts // groups
+    wide = -(-80 // per) * per
+    bias, correction = opts.pop("bias", False), opts.pop("correction", False)
+    z = torch.full((203, wide), -math.inf)
+    z[:, :experts] = torch.randn(203, experts, generator=g) * 2
+    z[100:140, :experts] = torch.randint(-2, 3, (40, experts), generator=g).float()
+    z[200, 1], z[201, 2], z[202, :experts] = math.inf, math.nan, -math.inf
+    add = lambda on, scale, rest: torch.cat([torch.randn(experts, generator=g) * scale, torch.full((wide - experts,), rest)]) if on else None
+    bias, correction = add(bias, 1.0, 0.0), add(correction, 0.3, -math.inf)
+    corrections = [correction]
+    if correction is not None:
+        corrections.append(correction.clone())
+        corrections[1][3], corrections[1][4] = math.inf, -math.inf
+    for c in corrections:
+        got = []
+        for n in (experts, wide):
+            ids = torch.full((203, top), -1, dtype=torch.int32, device=DEV)
+            wts = torch.full((203, top), -7.0, device=DEV)
+            cut = lambda v: None if v is None else v[:n].contiguous().to(DEV)
+            ops().moe_route(z.to(DEV)[:, :n], ids, wts, groups if n == experts else wide // per if groups > 1 else 1, keep, 1.5, bias=cut(bias),
+                            correction=cut(c), **opts)
+            got.append((ids.cpu(), wts.cpu()))
+        (ids, wts), (want_ids, want_wts) = got
+        assert ((ids >= 0) & (ids < experts)).all()
+        good = torch.ones(203, dtype=torch.bool)
+        good[200:] = opts.get("score") == "sigmoid"      # softmax: one +inf or NaN makes every score of its row NaN
+        assert torch.equal(ids[good], want_ids[good])
+        assert torch.equal(wts[good].view(torch.int32), want_wts[good].view(torch.int32))
+        assert wts[~good].isnan().all()

@@ -8,9 +8,9 @@
 //    gemm_f32_rows_kernel for few rows: true float32 on the matrix cores (v_mfma_f32_16x16x4_f32), no
 //    reduced-precision mode.  All add in ONE order, so a row gives the same bits whether it is computed
 //    alone or in a batch, by any of them.
-//  * gemm_bf16_kernel: bf16 inputs on the matrix cores (v_mfma_f32_32x32x16_bf16), float32
-//    accumulation, 256 x 256, 256 x 128, 128 x 128 or 64 x 128 tiles with k steps of 64 staged through
-//    double-buffered LDS; optionally over a share of the inner size (split k).
+//  * gemm_bf16_kernel: bf16 inputs on the matrix cores, float32 accumulation, 256 x 256, 256 x 128, 128 x 128 or 64 x 128 tiles
+//    with k steps of 64: operands straight from memory into two to four buffers in LDS (v_mfma_f32_16x16x32_bf16), or through
+//    registers into two (v_mfma_f32_32x32x16_bf16; tile_mode says where); optionally over a share of the inner size (split k).
 //  * gemm_oneshot_bf16_kernel: the split product for few rows, operands streamed through a ring of
 //    LDS slabs filled straight from memory; splitk_reduce_kernel adds the parts and applies the epilogue.
 //  * gemm_skinny_bf16_kernel: at most 64 rows (decode steps), weights streamed once into registers.
@@ -75,7 +75,8 @@ __device__ __forceinline__ void tl_wait_loads() { asm volatile("s_waitcnt vmcnt(
 // Workgroups are handed to the eight XCDs in turn, each with an L2 of its own.  The index is remapped so that an XCD owns a
 // contiguous run of tiles, and, `banded`, the tiles that it works on at a time make a block about as high as it is wide, which
 // asks the fewest rows of both operands of its L2 (8192^3 with 256 x 256 tiles in columns of 32 927 us, in bands of four 786):
-// bands of 4 to 7 tiles of rows, column by column.  Fewer than eight rows of tiles are one band, found by one division: three
+// bands of 4 to 7 rows of tiles, column by column, of which the last may be lower (as even as can be was no faster: 256 x 256
+// tiles, 21 rows of them, 8,192 x 2,048 144.8 us and 145.8 even; 11 rows, 11,264 x 2,048 97.6 and 99.6).  Fewer than eight rows of tiles are one band, found by one division: three
 // more took 0.1 to 0.25 us a launch.  128 x 128 and 64 x 128 tiles through registers stand in columns, whatever their number:
 // two to four share a unit and short steps wait for each other, not for the L2 (2,102 rows, 3,712 x 128 in 128 x 128 tiles
 // 8.94 us in bands, 8.63 so; 4,096 rows, 2,560 x 328 18.5 and 17.4; 2,047 rows, 4,096 x 192 with a residual 16.9 and 14.4).
@@ -725,7 +726,7 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const F32Rows
 // outputs as 32x32x16 MFMA tiles, or as 16x16x32 (operands straight into LDS).  Operand tiles go global -> registers -> LDS; LDS is
 // double-buffered so an iteration needs one barrier, and the global loads of the next k step are
 // in flight while the current one is multiplied.  Or they go straight into LDS, three or four buffers in turn
-// (launch_gemm_bf16 says where), and the loads of the next two or three k steps are in flight; the 256 x 256 tile's two
+// (tile_mode says where), and the loads of the next two or three k steps are in flight; the 256 x 256 tile's two
 // buffers are replaced quarter by quarter (kPhased).
 //
 // Tile shapes: 256 x 256 (eight waves of 128 x 64), 256 x 128, 128 x 128 and 64 x 128.  The larger
@@ -1174,7 +1175,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     step(std::false_type{}, std::false_type{}, kt);
   }
 
-  // Epilogue.  A lane's accumulators hold four consecutive n of 32 different rows, so stored from
+  // Epilogue.  A lane's accumulators hold four consecutive n of 16 rows (straight from memory) or 32, so stored from
   // there a row would go out in 16-byte pieces.  Each wave therefore passes its result, 32 rows x
   // 64 columns at a time, through an LDS area of its own (the operand tiles are no longer read:
   // the last fragments were fetched before the loop's last barrier) and reads it back row by
@@ -1353,10 +1354,10 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     };
     // A float32 result's residual is requested for all 32 rows together: out may be the residual, so the compiler asks for
     // a piece only when the one before is stored (4,096 rows, 640 x 512: 13.6 -> 12.0 us; 3,000 rows, 1,280 x 256: 12.2 ->
-    // 10.6).  The smallest tile, whose products are mostly launch, has the
-    // two forms apart: 65 to 4,096 rows, 520 x 264, take 2 % more without a residual where one piece of code serves both,
-    // bfloat16 results 3 % (they come without one, and load it piece by piece).  The larger tiles would lose waves by it:
-    // 108 registers where 84 let four a SIMD run.
+    // 10.6).  What follows concerns the tiles of up to 128 x 128 through registers; the others asked for it 32 rows ago
+    // (NEXT).  The smallest tile, whose products are mostly launch, has the two forms apart: 65 to 4,096 rows, 520 x 264, take
+    // 2 % more without a residual where one piece of code serves both, bfloat16 results 3 % (they come without one, and load it
+    // piece by piece).  The 128 x 128 tile would lose waves by it: 108 registers where 84 let four a SIMD run.
     if constexpr (BM > 64 || sizeof(TO) != 4) leave(std::integral_constant<int, SWIGLU ? kNoResidual : kAnyForm>{});
     else if (!SWIGLU && residual && vec_ok) leave(std::integral_constant<int, kResidual>{});
     else leave(std::integral_constant<int, kNoResidual>{});
@@ -1528,7 +1529,7 @@ static int launch_gemm_bf16_any(const bf16_t* a, const bf16_t* w, TO* out, const
 // (global_load_lds_dwordx4: no registers in between), as a ring of six slabs of 64 k, so that five
 // slabs (120 KB) are on their way while one is multiplied; a share of up to six slabs is requested
 // at once and the kernel is one round trip to memory long.  The tiled kernel above keeps one k
-// step of 64 in flight and pays a round trip for each.
+// step of 64 in flight through registers, two or three straight into LDS, and pays a round trip for each so many.
 // A slab in LDS: [A: 8 groups of 8 rows | W: 16 groups of 8 rows][8 rows x 128 bytes]; one load
 // instruction of a wave fills one group (1 KB, lane i -> bytes 16 i); the 16-byte chunk c of row r
 // stands at position c ^ (r % 8), so that the fragment reads of 32 rows do not collide.

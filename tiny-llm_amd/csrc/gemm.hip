@@ -1763,8 +1763,8 @@ __global__ __launch_bounds__(R_THREADS) void splitk_reduce_kernel(const ReduceAr
 // all) and sets the tile (as tl_linear_tile's) and the inner size per split.  Splitting pays when
 // the output has too few tiles to fill 256 compute units and the rows are too many for the
 // few-row kernel to stream the weights at full rate.  The number of parts is the order in which a result's float32 sums are
-// added, and the sizes here are those of a step's rows: another number moves the logits of a batch (0.2 to 0.9 % of their norm
-// where an estimate from products replayed on cached weights chose fewer).
+// added, and the sizes here are those of a step's rows: another number moves the logits of a batch (by 0.2 to 1 % of their norm
+// where an estimate of the time chose fewer).
 static int splitk_plan(int M, int N, int K, int* tile, int* k_per_split) {
   *tile = 0;
   *k_per_split = 0;

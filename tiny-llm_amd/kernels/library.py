@@ -29,7 +29,8 @@ LIB_NAME = "libtinyllm_gfx950.so"
 ARCH = "gfx950"
 # -packed-fp32-ops is switched off: hipcc would otherwise form v_pk_*_f32 from scalar code.
 # A kernel's first 16 words of plain arguments arrive in registers: it begins without the round trip that fetches them (a
-# decode step of 183 launches: 0.1 us a launch, 1.7 % of a workload of mostly such steps; structs are fetched as before).
+# decode step of 183 launches: 0.1 us a launch, 1.7 % of a workload of mostly such steps; structs are fetched as before;
+# the float32 products of few rows, which lose by it, begin with one).
 HIPCC_FLAGS = ["-O3", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                "-Wno-unused-command-line-argument", "-Wno-unknown-attributes"]

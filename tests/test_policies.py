@@ -95,14 +95,14 @@ def test_split_products_keep_their_number_of_parts():
 
 
 def test_operands_go_straight_into_lds_where_it_is_the_faster_way():
-    """128 x 128 tiles: through registers again beyond 256 workgroups, also where splitting the inner size makes them so many;
-    every tile: through registers for inner sizes that end within a step."""
+    """128 x 128 tiles: through registers beyond 256 workgroups of fewer than 32 steps, also where splitting the inner size makes
+    them so many; every tile: through registers for inner sizes that end within a step."""
     mode = library.load(verbose=False).tl_tile_mode
     tail, whole, direct, quarters = 0, 1, 2, 3
-    for M, N, K, share in ((1500, 1408, 1088, 576), (300, 2048, 2048, 384), (66, 11264, 2048, 704), (2102, 3968, 2048, 0),
-                           (300, 2048, 128, 0), (128, 257 * 128, 4096, 0)):
+    for M, N, K, share in ((1500, 1408, 1088, 576), (300, 2048, 2048, 384), (66, 11264, 2048, 704), (2102, 3968, 1984, 0),
+                           (300, 2048, 128, 0), (128, 257 * 128, 4096, 2048)):
         assert mode(3, M, N, K, share) == whole, (M, N, K, share)
-    for M, N, K, share in ((1500, 1408, 1088, 0), (300, 2048, 2048, 512), (128, 256 * 128, 256, 0)):
+    for M, N, K, share in ((1500, 1408, 1088, 0), (300, 2048, 2048, 512), (128, 256 * 128, 256, 0), (2102, 3968, 2048, 0)):
         assert mode(3, M, N, K, share) == direct, (M, N, K, share)
     assert mode(2, 2102, 3968, 256, 0) == direct and mode(2, 2102, 3968, 192, 0) == whole
     assert mode(1, 100, 300, 64, 0) == quarters and mode(4, 100, 300, 4096, 0) == whole

@@ -1397,18 +1397,20 @@ static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, cons
 // How the operands of a tile reach LDS.  Straight from memory where the inner size is whole steps: always in the 256 x 256
 // tile; in the 256 x 128 tile from four steps on (with fewer its buffers are not even filled; 2,047 rows, 4,096 x 4,096, weights
 // from memory: 68.1 us through registers, 61.8 so; 4,096 x 256 11.3 and 10.5); in the 128 x 128 tile likewise, if each
-// workgroup has a unit to itself.  Its four buffers leave a unit room for one workgroup, where through registers two share it,
-// and a second round for a few more workgroups than units costs a whole one (1,500 rows, 1,408 x 1,088 in two parts, 264
-// workgroups: 23.3 us through registers, 25.9 so; 300 rows, 2,048 x 2,048 in six 20.0 and 22.8).  532 products of up to 256
-// workgroups: 1.0 to 1.26x as fast so, median 1.09; 340 of more and 4 to 16 steps: 0.74 to 1.16x, median 0.91; beyond, where
-// the larger tiles serve nearly all, 0.83 to 1.19x, median 1.05.  Four waves of twice the outputs, which read less from LDS,
+// workgroup has a unit to itself, or each has 32 steps and more.  Its four buffers leave a unit room for one workgroup, where
+// through registers two share it, cover for each other's first loads, and make a second round for a few more workgroups than
+// units cheap (1,500 rows, 1,408 x 1,088 in two parts, 264 workgroups: 23.3 us through registers, 25.9 so; 300 rows, 2,048 x
+// 2,048 in six 20.0 and 22.8).  532 products of up to 256 workgroups: 1.0 to 1.26x as fast so, median 1.09; 340 of more and 4
+// to 16 steps: 0.74 to 1.16x, median 0.91; where the choice below takes this tile for more and the inner size is whole, 4 to 11
+// steps 0.76 to 1.05x, 16 0.97 to 1.08, 32 and 64 1.03 to 1.13 (2,102 rows, 3,712 x 4,096 76.3 and 72.4 us).  Four waves of twice the outputs, which read less from LDS,
 // lose with float32 results (1,944 rows, 2,048 x 5,632: 59.0; 3,288 rows: 88.2 -> 100.6).
 static int tile_mode(int bm, int bn, int M, int N, int K, int k_per_split) {
   if (K % B_BK) return kTail;
   if (bm + bn == 512) return kPhased;
   const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
   const int64_t wgs = (int64_t)((N + bn - 1) / bn) * ((M + bm - 1) / bm) * splits;
-  return K >= 4 * B_BK && (bm + bn == 384 || (bm + bn == 256 && wgs <= 256)) ? kDirect : kWhole;
+  const bool alone = wgs <= 256 || (splits == 1 && K >= 32 * B_BK);
+  return K >= 4 * B_BK && (bm + bn == 384 || (bm + bn == 256 && alone)) ? kDirect : kWhole;
 }
 
 template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU>

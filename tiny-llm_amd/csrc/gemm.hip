@@ -1433,21 +1433,22 @@ static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const flo
 
 // Which tile: the one with the smallest estimated time.  A compute unit works through
 // ceil(workgroups / 256) tiles one after the other, each at the rate that its tile shape reaches
-// on a full chip (measured, TFLOP/s: the larger the tile, the fewer operand bytes per flop): `straight` from eight whole steps
-// on, where all but the 64 x 128 tile get their operands straight from memory, and `rate` for inner sizes that end within a
-// step, whose tiles go through registers, and for fewer steps, where first loads and the epilogue (10 us a 256 x 256 tile,
-// whose step takes 1) count for more than the loop (2,200 rows, 3,712 x 64: 9.8 us with the 64 x 128 tiles that `rate`
-// chooses, 12.5 with the 256 x 256 that `straight` would; 700 rows, 11,264 x 192 13.4 and 15.3; x 256 14.8 and 15.2; x 512
-// 20.8 and 19.1; x 2,048 53.1 and 43.6).
+// on a full chip (measured, TFLOP/s: the larger the tile, the fewer operand bytes per flop).  With fewer than eight steps first
+// loads and the epilogue (10 us a 256 x 256 tile, whose step takes 1) count for more than the loop, and large tiles are worth
+// less: `few` (2,200 rows, 3,712 x 64: 9.8 us with the 64 x 128 tiles that `few` chooses, 12.5 with the 256 x 256 that `rate`
+// would; 700 rows, 11,264 x 192 13.4 and 15.3; x 512 20.8 and 19.1; x 2,048 53.1 and 43.6).  40 products for which the two
+// choose another tile, in three forms, time of `few`'s choice over that of `rate`'s: inner size 64 to 200 0.96 to 1.0, 256 to
+// 456 1.0 to 1.03, 512 and 520 1.04 and 1.02, 1,000 to 1,096 1.06 to 1.08, 2,048 to 4,104 1.09 to 1.12; sizes that end within a
+// step, whose tiles all go through registers, as the others.
 struct TileChoice {
   int bm, bn;
-  double rate, straight;
+  double few, rate;
 };
 static const TileChoice kTiles[4] = {{256, 256, 1060., 1400.}, {256, 128, 900., 1130.}, {128, 128, 760., 980.}, {64, 128, 640., 650.}};
 
 static double tile_cost(int c, int M, int N, int K) {
   const int64_t wgs = (int64_t)((M + kTiles[c].bm - 1) / kTiles[c].bm) * ((N + kTiles[c].bn - 1) / kTiles[c].bn);
-  const double rate = K % B_BK == 0 && K >= 8 * B_BK ? kTiles[c].straight : kTiles[c].rate;
+  const double rate = K >= 8 * B_BK ? kTiles[c].rate : kTiles[c].few;
   return (double)((wgs + 255) / 256) * kTiles[c].bm * kTiles[c].bn / rate;
 }
 

@@ -11,6 +11,8 @@
 // convolutions' last inputs: channels x (taps - 1), oldest first].
 #include "common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kPrepThreads = 128;
@@ -287,6 +289,455 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
     if (live && s * DS + i < dim) S_mem[(int64_t)(s * DS + i) * vdim] = S[i];
 }
 
+// The recurrence in chunks of 16 tokens, on the matrix cores.  With G_t the product of a chunk's decays up to token t and
+// S_0 the state ahead of the chunk,
+//     u_t = beta_t (v_t - S_0^T (G_t k_t) - sum_(s<t) A_ts u_s),     A_ts = sum_i k_t[i] k_s[i] (g_(s+1) .. g_t)[i]
+//     o_t = S_0^T (G_t q_t) + sum_(s<=t) B_ts u_s,                   B_ts = sum_i q_t[i] k_s[i] (g_(s+1) .. g_t)[i]
+//     S   = diag(G_16) S_0 + sum_s (g_(s+1) .. g_16 k_s) u_s^T
+// A, B and the solution of the first line for u = U0 - W S_0 (W and U0 by forward substitution, row by row as the recurrence
+// goes) do not depend on the state: delta_chunk_kernel makes them for all chunks at once.  What is left for
+// delta_chunk_scan_kernel to do in order are three products of 16 x dim (x vdim columns) a chunk.  Products of decays are
+// taken of the decays themselves (none exceeds one), never as quotients, so decays near zero lose nothing.  Within its chunk
+// a number that is not finite reaches the request's tokens ahead of it too.
+// 1,944 tokens of six requests, the longest 801, 16 heads of 128 x 128: convolutions and decays 97 us and the recurrence 299,
+// now 46 and 79; one request of 2,047 tokens 102 and 704, now 45 and 101.  What bounds them: the first its convolutions' and
+// decays' functions; the second a chain of 0.75 us a chunk, of which the matrix instructions take a half.  Error against 64
+// bits (2-norm, 1,000 tokens, 128 x 128): one decay a channel 1.38e-7 and 1.44e-7 for two draws, token by token 1.46e-7 and
+// 1.55e-7; one a head 1.35e-7 and 1.38e-7, token by token 1.28e-7 and 1.39e-7; 64 x 64 1.53e-7 and 1.58e-7.
+constexpr int kCT = 16;                // tokens of a chunk
+constexpr int kChunkMaxDim = 128;      // channels and value columns a head may have here: a thread each
+constexpr int kChunkThreads = 256;
+constexpr int kChunkTaps = 4;
+
+// What a (chunk, head) leaves for the scan, in floats: W, Q, K [dp / 16][64][4], U0 [vp / 16][64][4], B [64][4], G [dp].  A lane's
+// four numbers are what it holds of a matrix operand in four instructions of 16 x 16 x 4: of W and Q token l % 16, channels
+// 4 (l / 16) + j of sixteen; of K channel l % 16 of sixteen, tokens 4 (l / 16) + j; of U0 column l % 16, of B row l % 16, likewise.
+// A request's chunks lie side by side from place t0 / 16 + r on, t0 its first row: rows of at most t0 / 16 + r chunks lie in front.
+__host__ __device__ __forceinline__ int chunk_place(int t0, int r) { return t0 / kCT + r; }
+__host__ __device__ __forceinline__ int64_t chunk_floats(int dp, int vp) { return 3 * kCT * dp + kCT * vp + kCT * kCT + dp; }
+
+// v[t] summed over a row of sixteen lanes, t = 0 .. 15: lane l of the row gets the sum of v[l].  Lanes exchange halves of
+// what they hold: 15 exchanges for sixteen sums.
+__device__ __forceinline__ float scatter_sums(float* v, int l) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float keep = l & 8 ? v[8 + i] : v[i], send = l & 8 ? v[i] : v[8 + i];
+    v[i] = keep + dpp_f32<TL_DPP_MIRROR>(send);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float keep = l & 4 ? v[4 + i] : v[i], send = l & 4 ? v[i] : v[4 + i];
+    v[i] = keep + dpp_f32<TL_DPP_HALF_MIRROR>(send);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float keep = l & 2 ? v[2 + i] : v[i], send = l & 2 ? v[i] : v[2 + i];
+    v[i] = keep + dpp_f32<TL_DPP_XOR2>(send);
+  }
+  const float keep = l & 1 ? v[1] : v[0], send = l & 1 ? v[0] : v[1];
+  return keep + dpp_f32<TL_DPP_XOR1>(send);
+}
+
+// One workgroup per (chunk, head).  Thread i < DP convolves q's channel i, i + DP k's; the others than the first DP also a value
+// column each.  The decays, the dearest functions here, are shared out so that both are equally busy.
+template <typename T, int DP>
+__global__ __launch_bounds__(kChunkThreads) void delta_chunk_kernel(
+    const T* __restrict__ p, int64_t p_stride, int conv_off, int b_off, const float* __restrict__ a, int64_t a_stride,
+    const float* __restrict__ conv_w, const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+    const float* __restrict__ state, int64_t state_stride, int64_t saved_off, const int32_t* __restrict__ cu_seqlens,
+    const int32_t* __restrict__ state_slots, const int32_t* __restrict__ tile_req, const int32_t* __restrict__ tile_tok0,
+    const int32_t* __restrict__ tile_ntok, float* __restrict__ items, int heads, int kv_heads, int dim, int vdim, int taps,
+    float q_scale, int a_per_head) {
+  constexpr int LD = DP + 4;
+  __shared__ __attribute__((aligned(16))) float qs[kCT][LD], ks[kCT][LD], gs[kCT][LD];
+  __shared__ __attribute__((aligned(16))) float As[kCT][kCT], Bs[kCT][kCT];      // A[s][t], B[t][s]
+  __shared__ __attribute__((aligned(16))) float beta[kCT];
+  const int tile = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int n = tile_ntok[tile];
+  if (n <= 0) return;                    // a padding tile
+  const int req = tile_req[tile], tok0 = tile_tok0[tile], t0 = cu_seqlens[req];
+  const int kh = h / (heads / kv_heads), vp = (vdim + 31) / 32 * 32;
+  const float* saved = state + (int64_t)state_slots[req] * state_stride + saved_off;
+  float* item = items + ((int64_t)(chunk_place(t0, req) + (tok0 - t0) / kCT) * heads + h) * chunk_floats(DP, vp);
+  // One channel's convolution and SiLU for the chunk's tokens, zero behind the last of them; inputs ahead of the request's
+  // first token of this step come from its state.
+  auto conv = [&](int ch, float* y) {
+    constexpr int BACK = kChunkTaps - 1;
+    const T* col = p + (int64_t)tok0 * p_stride + conv_off + ch;
+    T in[kCT + BACK];
+    float x[kCT + BACK], wt[kChunkTaps];
+#pragma unroll
+    for (int j = 0; j < kCT + BACK; ++j) in[j] = col[(int64_t)(j < BACK ? (tok0 > t0 ? j - BACK : 0) : min(j - BACK, n - 1)) * p_stride];
+#pragma unroll
+    for (int j = 0; j < kChunkTaps; ++j) wt[j] = j >= kChunkTaps - taps ? conv_w[(int64_t)ch * taps + j - (kChunkTaps - taps)] : 0.f;
+#pragma unroll
+    for (int j = 0; j < kCT + BACK; ++j) x[j] = to_f32(in[j]);
+    if (tok0 == t0) {
+      const float* sv = saved + (int64_t)ch * (taps - 1);
+#pragma unroll
+      for (int j = 0; j < BACK; ++j) x[j] = j >= kChunkTaps - taps ? sv[j - (kChunkTaps - taps)] : 0.f;
+    }
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) {
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < kChunkTaps; ++j) acc = fmaf(wt[j], x[t + j], acc);
+      y[t] = t < n ? silu(acc) : 0.f;
+    }
+  };
+  float y[kCT];
+  const bool channel = tid < DP;
+  const int vcol = tid - DP, ch = tid % DP, lane = tid % TL_WAVE;
+  if (tid < 2 * DP) {
+    // the decays: tokens 0 to 10 for those who convolve once, the others for those who do it twice
+    constexpr int SPLIT = 11;
+    const float rate = expf(a_log[h]);
+    float pre[SPLIT];
+    if (!a_per_head) {
+#pragma unroll
+      for (int i = 0; i < SPLIT; ++i) {
+        const int t = channel ? i : min(SPLIT + i, kCT - 1);
+        pre[i] = a[(int64_t)(tok0 + min(t, n - 1)) * a_stride + h * dim + min(ch, dim - 1)];
+      }
+    } else {
+      pre[0] = a[(int64_t)(tok0 + min(lane % kCT, n - 1)) * a_stride + h];
+    }
+    const float bias = dt_bias[a_per_head ? h : h * dim + min(ch, dim - 1)];
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) y[t] = 0.f;
+    if (ch < dim) conv((channel ? 0 : kv_heads * dim) + kh * dim + ch, y);
+    float(*const to)[LD] = channel ? qs : ks;
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) to[t][ch] = y[t];
+    if (a_per_head) {                   // a token's decay is worked out by one lane
+      const float g = lane < n ? expf(-rate * softplus(pre[0] + bias)) : 1.f;
+#pragma unroll
+      for (int i = 0; i < SPLIT; ++i) {
+        const int t = channel ? i : SPLIT + i;
+        const float gt = __uint_as_float(__builtin_amdgcn_ds_bpermute((t % kCT) * 4, __float_as_uint(g)));
+        if (t < kCT) gs[t][ch] = ch < dim ? gt : 1.f;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < SPLIT; ++i) {
+        const int t = channel ? i : SPLIT + i;
+        if (i >= kCT - SPLIT && !channel) break;
+        gs[t][ch] = t < n && ch < dim ? expf(-rate * softplus(pre[i] + bias)) : 1.f;
+      }
+    }
+  }
+  if (!channel) {
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) y[t] = 0.f;
+    if (vcol < vdim) conv(2 * kv_heads * dim + h * vdim + vcol, y);
+  }
+  if (tid < kCT)
+    beta[tid] = tid < n ? 1.f / (1.f + expf(-to_f32(p[(int64_t)(tok0 + tid) * p_stride + b_off + h]))) : 0.f;
+  __syncthreads();
+  // Unit vectors, sixteen threads a token.
+  const int l = tid % 16;
+  {
+    const int t = tid / 16;
+    f32x4 q4[DP / 64], k4[DP / 64];
+    float sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int i = 0; i < DP / 64; ++i) {
+      q4[i] = *(const f32x4*)&qs[t][i * 64 + l * 4];
+      k4[i] = *(const f32x4*)&ks[t][i * 64 + l * 4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sq = fmaf(q4[i][e], q4[i][e], sq);
+        sk = fmaf(k4[i][e], k4[i][e], sk);
+      }
+    }
+    sq = group_sum<16>(sq);
+    sk = group_sum<16>(sk);
+    const float rq = q_scale / sqrtf(sq + 1e-6f), rk = 1.f / sqrtf(sk + 1e-6f);
+#pragma unroll
+    for (int i = 0; i < DP / 64; ++i) {
+      *(f32x4*)&qs[t][i * 64 + l * 4] = q4[i] * rq;
+      *(f32x4*)&ks[t][i * 64 + l * 4] = k4[i] * rk;
+    }
+  }
+  __syncthreads();
+  // Columns s of A and B, sixteen threads a column: k_s, decayed from token to token, with every later token's k and q.  A
+  // wave's four columns begin at its first; which wave has the long ones changes from workgroup to workgroup.
+  const int s_first = (tid / TL_WAVE + (int)blockIdx.x) % 4 * 4, s = s_first + tid % TL_WAVE / 16;
+  float pa[kCT], pb[kCT];
+  {
+    f32x4 x[DP / 64];
+#pragma unroll
+    for (int i = 0; i < DP / 64; ++i) x[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) {
+      pa[t] = pb[t] = 0.f;
+      if (t >= s_first && t < n) {      // uniform
+        float ak[4] = {0.f, 0.f, 0.f, 0.f}, bq[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DP / 64; ++i) {
+          const f32x4 g4 = *(const f32x4*)&gs[t][i * 64 + l * 4], k4 = *(const f32x4*)&ks[t][i * 64 + l * 4],
+                      q4 = *(const f32x4*)&qs[t][i * 64 + l * 4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x[i][e] = t == s ? k4[e] : x[i][e] * g4[e];      // ahead of token s it is zero
+            ak[e] = fmaf(x[i][e], k4[e], ak[e]);
+            bq[e] = fmaf(x[i][e], q4[e], bq[e]);
+          }
+        }
+        pa[t] = (ak[0] + ak[1]) + (ak[2] + ak[3]);
+        pb[t] = (bq[0] + bq[1]) + (bq[2] + bq[3]);
+      }
+    }
+  }
+  {
+    const float at = scatter_sums(pa, l), bt = scatter_sums(pb, l);      // of token l
+    As[s][l] = l > s ? at : 0.f;
+    Bs[l][s] = l >= s ? bt : 0.f;
+  }
+  __syncthreads();
+  // W and U0, a column a thread: beta_t times x_t - sum A_ts w_s, summed in 64 bits (2 us of 46; in 32 the error against 64
+  // bits is 5 % above that of token by token, not below).
+  f32x4 *W = (f32x4*)item, *Q = W + 4 * DP, *K = Q + 4 * DP, *U0 = K + 4 * DP, *Bm = U0 + 4 * vp;
+  if (channel) {
+    // The products of decays in 64 bits: with one decay a head all channels would share their rounding errors, which token by
+    // token they do not.
+    double g = 1.0;
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) {
+      g *= (double)gs[t][tid];
+      y[t] = ks[t][tid] * (float)g;
+      qs[t][tid] *= (float)g;
+    }
+    ((float*)(Bm + kCT * kCT / 4))[tid] = (float)g;
+    g = 1.0;
+    f32x4 k4;
+#pragma unroll
+    for (int t = kCT - 1; t >= 0; --t) {
+      k4[t % 4] = ks[t][tid] * (float)g;
+      g *= (double)gs[t][tid];
+      if (t % 4 == 0) K[tid / 16 * 64 + t / 4 * 16 + tid % 16] = k4;
+    }
+  }
+  double z[kCT];
+#pragma unroll
+  for (int t = 0; t < kCT; ++t) z[t] = (double)y[t];
+#pragma unroll
+  for (int s0 = 0; s0 < kCT; ++s0) {
+    z[s0] *= (double)beta[s0];
+    y[s0] = (float)z[s0];
+#pragma unroll
+    for (int j = (s0 + 1) / 4; j < kCT / 4; ++j) {
+      const f32x4 a4 = *(const f32x4*)&As[s0][j * 4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (j * 4 + e > s0) z[j * 4 + e] = fma(-(double)a4[e], z[s0], z[j * 4 + e]);
+    }
+  }
+  if (channel) {
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) ks[t][tid] = y[t];
+  } else if (vcol < vp) {
+#pragma unroll
+    for (int i = 0; i < kCT / 4; ++i)
+      U0[vcol / 16 * 64 + i * 16 + vcol % 16] = f32x4{y[i * 4], y[i * 4 + 1], y[i * 4 + 2], y[i * 4 + 3]};
+  }
+  __syncthreads();
+  for (int e = tid; e < 4 * DP; e += kChunkThreads) {
+    const int row = e % 16, ch = e / 64 * 16 + e % 64 / 16 * 4;
+    W[e] = *(const f32x4*)&ks[row][ch];
+    Q[e] = *(const f32x4*)&qs[row][ch];
+  }
+  if (tid < kCT * kCT / 4) {
+    const int row = tid % 16, j = tid / 16 * 4;
+    Bm[tid] = *(const f32x4*)&Bs[row][j];
+  }
+}
+
+// A workgroup owns 16 value columns of one (request, head).  Wave rg < 4 keeps rows [rg * 16 NT, (rg + 1) * 16 NT) of S, as
+// results of matrix instructions, which are the second operand of the next ones as they are.  A chunk: its rows' part of
+// W S_0, left in LDS for the other three; its part of Q S_0, half of it ahead of the barrier and half behind, which hides
+// both ways through LDS; then u, of all four parts, and the update.  Wave 4 forms the outputs, a chunk later (by the waves in
+// turn they cost a chunk 0.38 of 1.05 us).  One barrier a chunk, which does not wait for the operands on their way: they come
+// straight into registers, AHEAD chunks ahead, and no load stands in a branch (the compiler would wait for all at its end).
+// Sums run in chains of two instructions, and what a chunk adds to S is summed by itself, so that the results are as close
+// to 64 bits as token by token.
+typedef unsigned int tl_u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kScanThreads = 5 * TL_WAVE;
+template <int NT, int AHEAD>
+__global__ __launch_bounds__(kScanThreads, AHEAD == 1 ? 5 : 3) void delta_chunk_scan_kernel(
+    const float* __restrict__ items, float* __restrict__ state, int64_t state_stride, const int32_t* __restrict__ cu_seqlens,
+    const int32_t* __restrict__ state_slots, float* __restrict__ out, int heads, int dim, int vdim) {
+  constexpr int DP = 64 * NT;
+  __shared__ f32x4 us[3][4][TL_WAVE], os[2][4][TL_WAVE];      // parts of chunk c: [c % 3], [c % 2]
+  const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid % TL_WAVE;
+  const int rg = __builtin_amdgcn_readfirstlane(tid / TL_WAVE), q = lane / 16, vt = blockIdx.z, col = vt * 16 + lane % 16;
+  const int t0 = cu_seqlens[r], t1 = cu_seqlens[r + 1];
+  if (t1 <= t0) return;                           // a padding request owns no state
+  const int chunks = (t1 - t0 + kCT - 1) / kCT, vp = (vdim + 31) / 32 * 32;
+  const int64_t size = chunk_floats(DP, vp), step = size * heads / 4;
+  const bool live = col < vdim;
+  const f32x4* item0 = (const f32x4*)(items + ((int64_t)chunk_place(t0, r) * heads + h) * size);
+  auto meet = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto u_of = [&](int slot) { return -((us[slot][0][lane] + us[slot][1][lane]) + (us[slot][2][lane] + us[slot][3][lane])); };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (rg == 4) {
+    const int row_bytes = heads * vdim * 4;
+    const f32x4* b_at = item0 + 12 * DP + 4 * vp + lane;
+    f32x4 b = b_at[0];
+    meet();
+    for (int c = 0; c < chunks; ++c) {
+      meet();
+      const f32x4 U = u_of(c % 3), o = (os[c % 2][0][lane] + os[c % 2][1][lane]) + (os[c % 2][2][lane] + os[c % 2][3][lane]);
+      f32x4 y = zero, y2 = zero;                    // transposed: four columns a lane
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        y = __builtin_amdgcn_mfma_f32_16x16x4f32(U[j], b[j], y, 0, 0, 0);
+        y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(U[j + 2], b[j + 2], y2, 0, 0, 0);
+      }
+      y = o + (y + y2);
+      b = b_at[step * min(c + 1, chunks - 1)];
+      // a buffer that ends with the request's last token of the chunk: what lies behind is not stored, without a branch
+      const int n = min(kCT, t1 - t0 - c * kCT);
+      const __amdgpu_buffer_rsrc_t rows =
+          __builtin_amdgcn_make_buffer_rsrc(out + ((int64_t)(t0 + c * kCT) * heads + h) * vdim, 0, (n - 1) * row_bytes + vdim * 4, 0x00020000);
+      const int at = lane % 16 * row_bytes + (vt * 16 + q * 4) * 4;
+      if (vdim % 4 == 0) {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(tl_u32x4, y), rows, vt * 16 + q * 4 < vdim ? at : -16, 0, 0);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[j]), rows, vt * 16 + q * 4 + j < vdim ? at + j * 4 : -4, 0, 0);
+      }
+    }
+    return;
+  }
+  float* S_mem = state + (int64_t)state_slots[r] * state_stride + (int64_t)h * dim * vdim;
+  f32x4 S[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)                    // clamped, so that all rows are requested together
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S[i][e] = S_mem[(int64_t)min((rg * NT + i) * 16 + q * 4 + e, dim - 1) * vdim + min(col, vdim - 1)];
+  struct Operands {
+    f32x4 w[NT], q[NT], k[NT], g[NT], u0;
+  };
+  Operands op[AHEAD];
+  // A chunk's numbers through a buffer of their own: one offset a lane for each kind, no address arithmetic in vector registers.
+  const int w_at = (rg * NT * TL_WAVE + lane) * 16, g_at = (12 * DP + 4 * vp + TL_WAVE + rg * NT * 4 + q) * 16,
+            u0_at = (12 * DP + vt * TL_WAVE + lane) * 16;
+  auto request = [&](Operands& x, int c) {        // (behind the last chunk: that one again)
+    const __amdgpu_buffer_rsrc_t from =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(item0 + step * min(c, chunks - 1)), 0, (int)size * 4, 0x00020000);
+    auto load = [&](int at, int more) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, at, more, 0)); };
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      x.w[i] = load(w_at + i * 1024, 0);
+      x.q[i] = load(w_at + i * 1024, 64 * DP);
+      x.k[i] = load(w_at + i * 1024, 128 * DP);
+      x.g[i] = load(g_at + i * 64, 0);
+    }
+    x.u0 = load(u0_at, 0);
+  };
+  request(op[0], 0);
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!live || (rg * NT + i) * 16 + q * 4 + e >= dim) S[i][e] = 0.f;
+  };
+  const float first_part = rg == 0 ? 1.f : 0.f;
+  auto chunk = [&](Operands& x, int c, int slot, auto ask) {
+    f32x4 y[NT][2], o[NT][2];
+    // instruction j of 16 rows i
+    auto part_u = [&](int i, int j) {
+      y[i][j % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[i][j], S[i][j], j < 2 ? zero : y[i][j % 2], 0, 0, 0);
+    };
+    auto part_o = [&](int i, int j) {             // transposed
+      o[i][j % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[i][j], x.q[i][j], j < 2 ? zero : o[i][j % 2], 0, 0, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) part_u(i, j);
+    if constexpr (NT == 2) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) part_o(0, j);
+    } else {
+      part_o(0, 0);
+      part_o(0, 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 u = y[0][0] + y[0][1];
+    if constexpr (NT == 2) u += y[1][0] + y[1][1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = fmaf(-first_part, x.u0[e], u[e]);
+    us[slot][rg][lane] = u;
+    meet();
+    const f32x4 p0 = us[slot][0][lane], p1 = us[slot][1][lane], p2 = us[slot][2][lane], p3 = us[slot][3][lane];
+    if constexpr (NT == 2) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) part_o(1, j);
+    } else {
+      part_o(0, 2);
+      part_o(0, 3);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const f32x4 U = -((p0 + p1) + (p2 + p3));
+    f32x4 add[NT], add2[NT];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        add[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][j], U[j], j == 0 ? zero : add[i], 0, 0, 0);
+        add2[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][j + 2], U[j + 2], j == 0 ? zero : add2[i], 0, 0, 0);
+      }
+    f32x4 os_ = o[0][0] + o[0][1];
+    if constexpr (NT == 2) os_ += o[1][0] + o[1][1];
+    os[c % 2][rg][lane] = os_;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[i][e] = fmaf(x.g[i][e], S[i][e], add[i][e] + add2[i][e]);
+    if constexpr (decltype(ask)::value) request(x, c + AHEAD);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (chunks == 1) {                              // a step's single tokens: nothing is asked for ahead
+    clear();
+    chunk(op[0], 0, 0, std::false_type{});
+  } else {
+#pragma unroll
+    for (int d = 1; d < AHEAD; ++d) request(op[d], d);
+    clear();
+    int c = 0, slot = 0;
+    auto next = [&]() { return slot = slot == 2 ? 0 : slot + 1; };
+    for (; c + AHEAD <= chunks; c += AHEAD) {
+#pragma unroll
+      for (int d = 0; d < AHEAD; ++d) {
+        chunk(op[d], c + d, slot, std::true_type{});
+        next();
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < AHEAD - 1; ++d)
+      if (c + d < chunks) {                       // (the whole workgroup)
+        chunk(op[d], c + d, slot, std::true_type{});
+        next();
+      }
+  }
+  meet();
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = (rg * NT + i) * 16 + q * 4 + e;
+      if (live && row < dim) S_mem[(int64_t)row * vdim + col] = S[i][e];
+    }
+}
+
 // z[t, h, :] = scale * w * o[t, h, :] / sqrt(mean(o[t, h, :]^2) + eps) * act(gate[t, h, :]); one wave per (t, h).
 // w is shared by the heads (w_head_stride 0) or each head's own (w_head_stride = vdim); act is the sigmoid
 // (gate_kind 0) or g * sigmoid(g) (gate_kind 1).
@@ -548,6 +999,45 @@ int tl_delta_recurrence(const float* qn, const float* kn, const float* vc, const
   else if (vec) TL_REC(32, true);
   else TL_REC(32, false);
 #undef TL_REC
+  return tl_launch_status();
+}
+
+// The whole of a step's recurrence in chunks: convolutions, unit vectors, decays, the recurrence over states in place.
+// tile_*: every request's tokens cut into chunks of at most 16, request after request (ntok 0: padding).  items: float32
+// [(n_tokens / 16 + n_requests + 1) * heads * tl_delta_chunk_floats(dim, vdim)].
+int64_t tl_delta_chunk_floats(int dim, int vdim) { return chunk_floats(dim <= 64 ? 64 : 128, (vdim + 31) / 32 * 32); }
+
+int tl_delta_chunks(const void* p, int64_t p_stride, int conv_off, int b_off, const float* a, int64_t a_stride,
+                    const float* conv_w, const float* a_log, const float* dt_bias, float* state, int64_t state_stride,
+                    int64_t saved_off, const int32_t* cu_seqlens, const int32_t* state_slots, const int32_t* tile_req,
+                    const int32_t* tile_tok0, const int32_t* tile_ntok, float* items, float* out, int n_tiles, int n_requests,
+                    int heads, int kv_heads, int dim, int vdim, int taps, float q_scale, int a_per_head, int dtype,
+                    hipStream_t stream) {
+  if (n_tiles <= 0 || n_requests <= 0) return TL_OK;
+  if (heads <= 0 || heads > 65535 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || dim > kChunkMaxDim || vdim <= 0 ||
+      vdim > kChunkMaxDim || taps < 1 || taps > kChunkTaps || ((uintptr_t)items & 15))
+    return TL_ERR_ARG;
+  dim3 g(n_tiles, heads), b(kChunkThreads), gs(n_requests, heads, (vdim + 15) / 16), bs(kScanThreads);
+  // Where every workgroup has a unit to itself only its own chain counts: operands two chunks ahead (one prompt of 2,047
+  // tokens, 16 heads of 128 x 128: 101 us, 138 one chunk ahead).  Beyond, registers for a second set cost waves (six
+  // prompts of 67 to 801: 108 us, 80 one ahead; 64 of 13: 83 and 59).
+  const bool few = (int64_t)n_requests * heads * ((vdim + 15) / 16) <= 256;
+#define TL_DELTA_CHUNK(DP)                                                                                               \
+  {                                                                                                                      \
+    TL_DISPATCH_T(dtype, hipLaunchKernelGGL((delta_chunk_kernel<T, DP>), g, b, 0, stream, (const T*)p, p_stride, conv_off, \
+                                            b_off, a, a_stride, conv_w, a_log, dt_bias, state, state_stride, saved_off,  \
+                                            cu_seqlens, state_slots, tile_req, tile_tok0, tile_ntok, items, heads,       \
+                                            kv_heads, dim, vdim, taps, q_scale, a_per_head);)                            \
+    if (few)                                                                                                             \
+      hipLaunchKernelGGL((delta_chunk_scan_kernel<DP / 64, 2>), gs, bs, 0, stream, items, state, state_stride, cu_seqlens, \
+                         state_slots, out, heads, dim, vdim);                                                            \
+    else                                                                                                                 \
+      hipLaunchKernelGGL((delta_chunk_scan_kernel<DP / 64, 1>), gs, bs, 0, stream, items, state, state_stride, cu_seqlens, \
+                         state_slots, out, heads, dim, vdim);                                                            \
+  }
+  if (dim <= 64) TL_DELTA_CHUNK(64)
+  else TL_DELTA_CHUNK(128)
+#undef TL_DELTA_CHUNK
   return tl_launch_status();
 }
 

@@ -1623,6 +1623,59 @@ def delta_recurrence(qn: torch.Tensor, kn: torch.Tensor, vc: torch.Tensor, beta:
     return out
 
 
+DELTA_CHUNK = 16                 # tokens of a chunk of the chunked form
+DELTA_CHUNK_MAX_DIM = 128        # its heads' channels and value columns
+DELTA_CHUNK_MAX_TAPS = 4
+
+
+def delta_chunks_pay(n_tokens: int, n_requests: int, dim: int, vdim: int, taps: int) -> bool:
+    """Whether a step's recurrence runs in chunks (`delta_chunks`) or token by token.  A request costs the chunks about 1 us
+    (16 heads of 128 x 128; its state goes through narrower pieces), token by token 0.6; a token 0.05 us against 0.05 and,
+    in the longest request, 0.37.  8 requests of 8, 16 and 32 tokens: 20, 24 and 31 us in chunks, 17, 21 and 36 by tokens;
+    40 of one token beside 3 of 32: 58 and 48; 64 of 13: 85 and 112; one of 48: 19 and 28; one of 2,047: 144 and 806."""
+    return (32 < dim <= DELTA_CHUNK_MAX_DIM and vdim <= DELTA_CHUNK_MAX_DIM and taps <= DELTA_CHUNK_MAX_TAPS
+            and n_tokens >= 6 * n_requests + 48)
+
+
+def delta_chunks(p: torch.Tensor, conv_off: int, b_off: int, a: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor,
+                 dt_bias: torch.Tensor, state: torch.Tensor, saved_off: int, cu_seqlens: torch.Tensor,
+                 state_slots: torch.Tensor, tiles, out: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int,
+                 taps: int, q_scale: float, decay_per_head: bool = False) -> torch.Tensor:
+    """What `delta_prepare` and `delta_recurrence` do (their arguments), chunk by chunk on the matrix cores, all float32.
+    tiles (req, tok0, ntok): every request's tokens cut into chunks of at most DELTA_CHUNK, request after request."""
+    req, tok0, ntok = tiles
+    _dev(p, a, conv_w, a_log, dt_bias, state, cu_seqlens, state_slots, req, tok0, ntok, out)
+    check_delta_sizes(heads, kv_heads, dim, vdim, taps)
+    _rows_2d(p, "projections")
+    _rows_2d(a, "decay pre-activations")
+    _i32(cu_seqlens, state_slots, req, tok0, ntok)
+    T, R, n_tiles = p.shape[0], state_slots.numel(), tok0.numel()
+    channels = 2 * kv_heads * dim + heads * vdim
+    _f32_vec(conv_w, channels * taps, "convolution taps")
+    _f32_vec(a_log, heads, "A_log")
+    n_decay = heads if decay_per_head else heads * dim
+    _f32_vec(dt_bias, n_decay, "dt_bias")
+    _f32_vec(out, T * heads * vdim, "delta_chunks output")
+    _need(max(dim, vdim) <= DELTA_CHUNK_MAX_DIM and taps <= DELTA_CHUNK_MAX_TAPS,
+          f"delta_chunks: heads of at most {DELTA_CHUNK_MAX_DIM} x {DELTA_CHUNK_MAX_DIM} and {DELTA_CHUNK_MAX_TAPS} taps")
+    _need(a.dtype == torch.float32 and a.shape[0] == T and a.shape[1] >= n_decay and conv_off >= 0
+          and conv_off + channels <= p.shape[1] and 0 <= b_off and b_off + heads <= p.shape[1]
+          and req.numel() == ntok.numel() == n_tiles > 0 and cu_seqlens.numel() == R + 1, "delta_chunks: shapes do not fit")
+    _need(state.dtype == torch.float32 and state.dim() == 2 and state.is_contiguous() and heads * dim * vdim <= saved_off
+          and saved_off + channels * (taps - 1) <= state.shape[1],
+          "delta_chunks: the state is contiguous float32 [slots, row] with room for the saved inputs behind the heads' states")
+    fn = _lib().tl_delta_chunk_floats
+    fn.restype = c_int64
+    items = scratch("delta_items", ((T // DELTA_CHUNK + R + 1) * heads * fn(c_int(dim), c_int(vdim)),), torch.float32, p.device)
+    _check(_lib().tl_delta_chunks(_ptr(p), c_int64(p.stride(0)), c_int(conv_off), c_int(b_off), _ptr(a), c_int64(a.stride(0)),
+                                  _ptr(conv_w), _ptr(a_log), _ptr(dt_bias), _ptr(state), c_int64(state.stride(0)),
+                                  c_int64(saved_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(req), _ptr(tok0), _ptr(ntok),
+                                  _ptr(items), _ptr(out), c_int(n_tiles), c_int(R), c_int(heads), c_int(kv_heads), c_int(dim),
+                                  c_int(vdim), c_int(taps), c_float(q_scale), c_int(1 if decay_per_head else 0), c_int(_dt(p)),
+                                  _stream()), "delta_chunks")
+    return out
+
+
 DELTA_DECODE_MAX_VDIM = 256      # a thread per value column in the one-kernel decode step
 DELTA_DECODE_MAX_TAPS = 4         # and its convolutions' inputs in registers
 

@@ -146,17 +146,23 @@ class ChannelDelta(Mixer):
                 ops.conv_state_update(p, 0, self.channels, state, self.state_size, ctx.cu_seqlens_q,
                                       ctx.state_slots, self.taps)
             return self._project_out(z, residual)
-        qn = ops.scratch("delta_q", (T * H * D,), torch.float32, dev)
-        kn = ops.scratch("delta_k", (T * H * D,), torch.float32, dev)
-        dec = ops.scratch("delta_decay", (T * H * D,), torch.float32, dev)
-        vc = ops.scratch("delta_v", (T * H * V,), torch.float32, dev)
-        beta = ops.scratch("delta_beta", (T * H,), torch.float32, dev)
-        ops.delta_prepare(p, 0, self.b_off, a, self.conv_w, self.a_log, self.dt_bias, state, self.state_size,
-                          ctx.req_of_token, ctx.cu_seqlens_q, ctx.state_slots, qn, kn, vc, beta, dec, H, KH, D, V,
-                          self.taps, D ** -0.5, self.per_head)
-        ops.conv_state_update(p, 0, self.channels, state, self.state_size, ctx.cu_seqlens_q, ctx.state_slots, self.taps)
         o = ops.scratch("delta_o", (T * H * V,), torch.float32, dev)
-        ops.delta_recurrence(qn, kn, vc, beta, dec, state, ctx.cu_seqlens_q, ctx.state_slots, o, H, D, V)
+        if ops.delta_chunks_pay(T, ctx.num_requests, D, V, self.taps):
+            ops.delta_chunks(p, 0, self.b_off, a, self.conv_w, self.a_log, self.dt_bias, state, self.state_size,
+                             ctx.cu_seqlens_q, ctx.state_slots, ctx.attention_tiles(ops.DELTA_CHUNK), o, H, KH, D, V,
+                             self.taps, D ** -0.5, self.per_head)
+            ops.conv_state_update(p, 0, self.channels, state, self.state_size, ctx.cu_seqlens_q, ctx.state_slots, self.taps)
+        else:
+            qn = ops.scratch("delta_q", (T * H * D,), torch.float32, dev)
+            kn = ops.scratch("delta_k", (T * H * D,), torch.float32, dev)
+            dec = ops.scratch("delta_decay", (T * H * D,), torch.float32, dev)
+            vc = ops.scratch("delta_v", (T * H * V,), torch.float32, dev)
+            beta = ops.scratch("delta_beta", (T * H,), torch.float32, dev)
+            ops.delta_prepare(p, 0, self.b_off, a, self.conv_w, self.a_log, self.dt_bias, state, self.state_size,
+                              ctx.req_of_token, ctx.cu_seqlens_q, ctx.state_slots, qn, kn, vc, beta, dec, H, KH, D, V,
+                              self.taps, D ** -0.5, self.per_head)
+            ops.conv_state_update(p, 0, self.channels, state, self.state_size, ctx.cu_seqlens_q, ctx.state_slots, self.taps)
+            ops.delta_recurrence(qn, kn, vc, beta, dec, state, ctx.cu_seqlens_q, ctx.state_slots, o, H, D, V)
         ops.head_norm_gate(o, self.w_norm, gate, z, H, V, self.eps, self.gate_kind)
         return self._project_out(z, residual)
 

@@ -629,3 +629,45 @@ def test_runs_of_an_experts_rows_through_the_tiled_product(T, top, E, N, K):
     ops.moe_combine_at(y.cuda(), pos, out, top, 0.5, out, sc.cuda())
     want = base.double() * sc.double()[:, None] + 0.5 * y.double()[where].reshape(T, top, N).sum(1)
     assert (out.double().cpu() - want).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("H,D,lens", [(3, 64, [40, 17, 0, 3, 1, 64, 16, 33, 15, 32]), (2, 37, [49, 1, 80]), (2, 100, [31, 2, 66]),
+                                      (5, 128, [130, 0, 16])])
+def test_time_mix_in_chunks(H, D, lens):
+    """The chunked form against the recurrence in 64 bits, around whole chunks of 16, with requests of one token and of none,
+    padding chunks, heads that are no whole tiles, from states that hold something and with decays down to nothing.  Bound: a
+    result sums at most 128 + 16 products in chains of four, a state is rounded twice a chunk, what enters a few times: less
+    than 30 roundings of 2^-24, 1.8e-6 of the largest."""
+    from tiny_llm_amd.engine.step import tile_lists
+    from tiny_llm_amd.kernels import ops
+    g = torch.Generator().manual_seed(D)
+    T, R, S = sum(lens), len(lens), H * D
+    slots = [int(s) for s in torch.randperm(R + 2, generator=g)[:R]]
+    x = torch.randn(T, 4 * S + 4, generator=g)
+    x[:, 3 * S:] = x[:, 3 * S:] * 2.0 - 1.0
+    w0, u = torch.randn(S, generator=g) * 0.5, torch.randn(S, generator=g)
+    floats = ops.time_mix_state_floats(H, D, D)
+    P = floats // (H * 4 * D)
+    state = torch.randn(R + 2, floats + 4, generator=g) * 0.5
+    rows = state[:, :floats].view(-1, H, 4, D, P).permute(0, 1, 4, 2, 3).reshape(-1, H, 4 * P, D)
+    rows[:, :, D:] = 0.0                                              # channels beyond the head's
+    state[:, :floats] = rows.view(-1, H, P, 4, D).permute(0, 1, 3, 4, 2).reshape(-1, floats)
+    cu = [sum(lens[:i]) for i in range(R + 1)]
+    r, k, v, w = (x[:, i * S:(i + 1) * S].double().view(T, H, D) for i in range(4))
+    w, uu = torch.exp(-torch.exp(w + w0.double().view(H, D))), u.double().view(H, D, 1)
+    want, S_all = torch.zeros(T, H, D, dtype=torch.float64), rows[:, :, :D].double().clone()
+    for i, slot in enumerate(slots):
+        for t in range(cu[i], cu[i + 1]):
+            kv = k[t][:, :, None] * v[t][:, None, :]
+            want[t] = ((S_all[slot] + uu * kv) * r[t][:, :, None]).sum(1)
+            S_all[slot] = w[t][:, :, None] * S_all[slot] + kv
+    dev = "cuda"
+    i32 = lambda y: torch.tensor(y, dtype=torch.int32, device=dev)  # noqa: E731
+    tiles = [i32(y + [0, 0]) for y in tile_lists(lens, ops.TIME_MIX_CHUNK)]      # two padding chunks behind
+    st, out = state.to(dev), torch.full((T * S,), float("nan"), device=dev)
+    ops.time_mix_chunks(x.to(dev), 0, S, 2 * S, 3 * S, w0.to(dev), u.to(dev), st, i32(cu), i32(slots), tiles, out, H, D, D)
+    assert (out.double().cpu().view(T, H, D) - want).abs().max() <= 1.8e-6 * want.abs().max()
+    got = st.cpu()[:, :floats].view(-1, H, 4, D, P).permute(0, 1, 4, 2, 3).reshape(-1, H, 4 * P, D)[:, :, :D]
+    assert (got.double() - S_all).abs().max() <= 1.8e-6 * S_all.abs().max()
+    idle = [s for s in range(R + 2) if s not in slots or lens[slots.index(s)] == 0]
+    assert torch.equal(st.cpu()[idle], state[idle]) and torch.equal(st.cpu()[:, floats:], state[:, floats:])

@@ -185,6 +185,35 @@ struct ConvRun {
   }
 };
 
+// Recurrences in chunks of 16 tokens (delta_rule.hip, time_mix.hip).  What a chunk leaves for the scan over a request's chunks
+// lies request after request: a request's chunks side by side from place t0 / 16 + r on, t0 its first row, as the r requests in
+// front have at most t0 / 16 + r of them.
+constexpr int kCT = 16;
+__host__ __device__ __forceinline__ int chunk_place(int t0, int r) { return t0 / kCT + r; }
+typedef unsigned int tl_u32x4 __attribute__((ext_vector_type(4)));
+
+// v[t] summed over a row of sixteen lanes, t = 0 .. 15: lane l of the row gets the sum of v[l].  Lanes exchange halves of
+// what they hold: 15 exchanges for sixteen sums.
+__device__ __forceinline__ float scatter_sums(float* v, int l) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float keep = l & 8 ? v[8 + i] : v[i], send = l & 8 ? v[i] : v[8 + i];
+    v[i] = keep + dpp_f32<TL_DPP_MIRROR>(send);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float keep = l & 4 ? v[4 + i] : v[i], send = l & 4 ? v[i] : v[4 + i];
+    v[i] = keep + dpp_f32<TL_DPP_HALF_MIRROR>(send);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float keep = l & 2 ? v[2 + i] : v[i], send = l & 2 ? v[i] : v[2 + i];
+    v[i] = keep + dpp_f32<TL_DPP_XOR2>(send);
+  }
+  const float keep = l & 1 ? v[1] : v[0], send = l & 1 ? v[0] : v[1];
+  return keep + dpp_f32<TL_DPP_XOR1>(send);
+}
+
 static inline int tl_launch_status() {
   return hipGetLastError() == hipSuccess ? TL_OK : TL_ERR_LAUNCH;
 }

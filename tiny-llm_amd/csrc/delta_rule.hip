@@ -304,7 +304,6 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
 // decays' functions; the second a chain of 0.75 us a chunk, of which the matrix instructions take a half.  Error against 64
 // bits (2-norm, 1,000 tokens, 128 x 128): one decay a channel 1.38e-7 and 1.44e-7 for two draws, token by token 1.46e-7 and
 // 1.55e-7; one a head 1.35e-7 and 1.38e-7, token by token 1.28e-7 and 1.39e-7; 64 x 64 1.53e-7 and 1.58e-7.
-constexpr int kCT = 16;                // tokens of a chunk
 constexpr int kChunkMaxDim = 128;      // channels and value columns a head may have here: a thread each
 constexpr int kChunkThreads = 256;
 constexpr int kChunkTaps = 4;
@@ -312,31 +311,7 @@ constexpr int kChunkTaps = 4;
 // What a (chunk, head) leaves for the scan, in floats: W, Q, K [dp / 16][64][4], U0 [vp / 16][64][4], B [64][4], G [dp].  A lane's
 // four numbers are what it holds of a matrix operand in four instructions of 16 x 16 x 4: of W and Q token l % 16, channels
 // 4 (l / 16) + j of sixteen; of K channel l % 16 of sixteen, tokens 4 (l / 16) + j; of U0 column l % 16, of B row l % 16, likewise.
-// A request's chunks lie side by side from place t0 / 16 + r on, t0 its first row: rows of at most t0 / 16 + r chunks lie in front.
-__host__ __device__ __forceinline__ int chunk_place(int t0, int r) { return t0 / kCT + r; }
 __host__ __device__ __forceinline__ int64_t chunk_floats(int dp, int vp) { return 3 * kCT * dp + kCT * vp + kCT * kCT + dp; }
-
-// v[t] summed over a row of sixteen lanes, t = 0 .. 15: lane l of the row gets the sum of v[l].  Lanes exchange halves of
-// what they hold: 15 exchanges for sixteen sums.
-__device__ __forceinline__ float scatter_sums(float* v, int l) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float keep = l & 8 ? v[8 + i] : v[i], send = l & 8 ? v[i] : v[8 + i];
-    v[i] = keep + dpp_f32<TL_DPP_MIRROR>(send);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float keep = l & 4 ? v[4 + i] : v[i], send = l & 4 ? v[i] : v[4 + i];
-    v[i] = keep + dpp_f32<TL_DPP_HALF_MIRROR>(send);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const float keep = l & 2 ? v[2 + i] : v[i], send = l & 2 ? v[i] : v[2 + i];
-    v[i] = keep + dpp_f32<TL_DPP_XOR2>(send);
-  }
-  const float keep = l & 1 ? v[1] : v[0], send = l & 1 ? v[0] : v[1];
-  return keep + dpp_f32<TL_DPP_XOR1>(send);
-}
 
 // One workgroup per (chunk, head).  Thread i < DP convolves q's channel i, i + DP k's; the others than the first DP also a value
 // column each.  The decays, the dearest functions here, are shared out so that both are equally busy.
@@ -561,7 +536,6 @@ __global__ __launch_bounds__(kChunkThreads) void delta_chunk_kernel(
 // straight into registers, AHEAD chunks ahead, and no load stands in a branch (the compiler would wait for all at its end).
 // Sums run in chains of two instructions, and what a chunk adds to S is summed by itself, so that the results are as close
 // to 64 bits as token by token.
-typedef unsigned int tl_u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kScanThreads = 5 * TL_WAVE;
 template <int NT, int AHEAD>
 __global__ __launch_bounds__(kScanThreads, AHEAD == 1 ? 5 : 3) void delta_chunk_scan_kernel(
@@ -569,8 +543,8 @@ __global__ __launch_bounds__(kScanThreads, AHEAD == 1 ? 5 : 3) void delta_chunk_
     const int32_t* __restrict__ state_slots, float* __restrict__ out, int heads, int dim, int vdim) {
   constexpr int DP = 64 * NT;
   __shared__ f32x4 us[3][4][TL_WAVE], os[2][4][TL_WAVE];      // parts of chunk c: [c % 3], [c % 2]
-  const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid % TL_WAVE;
-  const int rg = __builtin_amdgcn_readfirstlane(tid / TL_WAVE), q = lane / 16, vt = blockIdx.z, col = vt * 16 + lane % 16;
+  const int r = blockIdx.z, h = blockIdx.x, tid = threadIdx.x, lane = tid % TL_WAVE;
+  const int rg = __builtin_amdgcn_readfirstlane(tid / TL_WAVE), q = lane / 16, vt = blockIdx.y, col = vt * 16 + lane % 16;
   const int t0 = cu_seqlens[r], t1 = cu_seqlens[r + 1];
   if (t1 <= t0) return;                           // a padding request owns no state
   const int chunks = (t1 - t0 + kCT - 1) / kCT, vp = (vdim + 31) / 32 * 32;
@@ -1014,10 +988,12 @@ int tl_delta_chunks(const void* p, int64_t p_stride, int conv_off, int b_off, co
                     int heads, int kv_heads, int dim, int vdim, int taps, float q_scale, int a_per_head, int dtype,
                     hipStream_t stream) {
   if (n_tiles <= 0 || n_requests <= 0) return TL_OK;
-  if (heads <= 0 || heads > 65535 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || dim > kChunkMaxDim || vdim <= 0 ||
+  if (heads <= 0 || heads > 65535 || n_requests > 65535 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || dim > kChunkMaxDim || vdim <= 0 ||
       vdim > kChunkMaxDim || taps < 1 || taps > kChunkTaps || ((uintptr_t)items & 15))
     return TL_ERR_ARG;
-  dim3 g(n_tiles, heads), b(kChunkThreads), gs(n_requests, heads, (vdim + 15) / 16), bs(kScanThreads);
+  dim3 g(n_tiles, heads), b(kChunkThreads), gs(heads, (vdim + 15) / 16, n_requests), bs(kScanThreads);
+  // Heads first in the grid: the workgroups of the longest request are then spread over all XCDs (with requests first, eight
+  // of them, it had one), those of a head share one.
   // Where every workgroup has a unit to itself only its own chain counts: operands two chunks ahead (one prompt of 2,047
   // tokens, 16 heads of 128 x 128: 101 us, 138 one chunk ahead).  Beyond, registers for a second set cost waves (six
   // prompts of 67 to 801: 108 us, 80 one ahead; 64 of 13: 83 and 59).

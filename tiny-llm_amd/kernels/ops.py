@@ -1631,10 +1631,10 @@ DELTA_CHUNK_MAX_TAPS = 4
 def delta_chunks_pay(n_tokens: int, n_requests: int, dim: int, vdim: int, taps: int) -> bool:
     """Whether a step's recurrence runs in chunks (`delta_chunks`) or token by token.  A request costs the chunks about 1 us
     (16 heads of 128 x 128; its state goes through narrower pieces), token by token 0.6; a token 0.05 us against 0.05 and,
-    in the longest request, 0.37.  8 requests of 8, 16 and 32 tokens: 20, 24 and 31 us in chunks, 17, 21 and 36 by tokens;
-    40 of one token beside 3 of 32: 58 and 48; 64 of 13: 85 and 112; one of 48: 19 and 28; one of 2,047: 144 and 806."""
+    in the longest request, 0.37.  8 requests of 8, 16 and 32 tokens: 18, 20 and 35 us in chunks, 16, 21 and 34 by tokens,
+    24: 34 and 27; 40 of one token beside 3 of 32: 52 and 46; 64 of 13: 67 and 110; one of 48: 19 and 28; one of 2,047: 145 and 806."""
     return (32 < dim <= DELTA_CHUNK_MAX_DIM and vdim <= DELTA_CHUNK_MAX_DIM and taps <= DELTA_CHUNK_MAX_TAPS
-            and n_tokens >= 6 * n_requests + 48)
+            and n_tokens >= 20 * n_requests + 44)
 
 
 def delta_chunks(p: torch.Tensor, conv_off: int, b_off: int, a: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor,
@@ -2025,6 +2025,48 @@ def time_mix_recurrence(x: torch.Tensor, r_off: int, k_off: int, v_off: int, w_o
                                          c_int(w_off), _ptr(w0), _ptr(u), _ptr(state), c_int64(state.stride(0)),
                                          _ptr(cu_seqlens), _ptr(state_slots), _ptr(o), c_int(R), c_int(heads), c_int(dim),
                                          c_int(vdim), _stream()), "time_mix_recurrence")
+    return o
+
+
+TIME_MIX_CHUNK = 16              # tokens of a chunk of the chunked form
+TIME_MIX_CHUNK_MAX_DIM = 128     # its heads' channels and value columns
+
+
+def time_mix_chunks_pay(n_tokens: int, n_requests: int, dim: int, vdim: int) -> bool:
+    """Whether a step's recurrence runs in chunks (`time_mix_chunks`) or token by token.  32 heads of 64 x 64: 8 requests of
+    16 and 32 tokens 14 and 21 us in chunks, 9 and 16 by tokens; 64 of 13 and 16: 64 and 64, 43 and 45; 40 of one token beside 3
+    of 32: 49 and 21; one of 48, 64 and 2,047: 10, 11 and 110, 11, 14 and 460; six of 67 to 801 71 and 188."""
+    return 32 < dim <= TIME_MIX_CHUNK_MAX_DIM and vdim <= TIME_MIX_CHUNK_MAX_DIM and n_tokens >= 28 * n_requests + 36
+
+
+def time_mix_chunks(x: torch.Tensor, r_off: int, k_off: int, v_off: int, w_off: int, w0: torch.Tensor, u: torch.Tensor,
+                    state: torch.Tensor, cu_seqlens: torch.Tensor, state_slots: torch.Tensor, tiles, o: torch.Tensor,
+                    heads: int, dim: int, vdim: int) -> torch.Tensor:
+    """What `time_mix_recurrence` does (its arguments), chunk by chunk on the matrix cores, float32 as there.  tiles (req,
+    tok0, ntok): every request's tokens cut into chunks of at most TIME_MIX_CHUNK, request after request."""
+    req, tok0, ntok = tiles
+    _dev(x, w0, u, state, cu_seqlens, state_slots, req, tok0, ntok, o)
+    _rows_2d(x, "time_mix_chunks input")
+    T, R, n_tiles = x.shape[0], state_slots.numel(), tok0.numel()
+    _need(x.dtype == torch.float32, "time_mix_chunks: the input is float32")
+    _need(32 < dim <= TIME_MIX_CHUNK_MAX_DIM and 0 < vdim <= TIME_MIX_CHUNK_MAX_DIM and 0 < heads <= 65535,
+          f"time_mix_chunks: heads of 33 to {TIME_MIX_CHUNK_MAX_DIM} key channels")
+    for off, n in ((r_off, heads * dim), (k_off, heads * dim), (w_off, heads * dim), (v_off, heads * vdim)):
+        _need(0 <= off and off + n <= x.shape[1], "time_mix_chunks: a column range lies outside the input's rows")
+    _f32_vec(w0, heads * dim, "the decay's bias")
+    _f32_vec(u, heads * dim, "the bonus")
+    _f32_vec(o, T * heads * vdim, "time_mix_chunks output")
+    _need(state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1
+          and state.shape[1] >= time_mix_state_floats(heads, dim, vdim), "time_mix_chunks: state rows are too short")
+    _i32(cu_seqlens, state_slots, req, tok0, ntok)
+    _need(cu_seqlens.numel() == R + 1 and req.numel() == ntok.numel() == n_tiles > 0, "time_mix_chunks: shapes do not fit")
+    fn = _lib().tl_time_mix_chunk_floats
+    fn.restype = c_int64
+    items = scratch("time_mix_items", ((T // TIME_MIX_CHUNK + R + 1) * heads * fn(c_int(dim), c_int(vdim)),), torch.float32, x.device)
+    _check(_lib().tl_time_mix_chunks(_ptr(x), c_int64(x.stride(0)), c_int(r_off), c_int(k_off), c_int(v_off), c_int(w_off),
+                                     _ptr(w0), _ptr(u), _ptr(state), c_int64(state.stride(0)), _ptr(cu_seqlens),
+                                     _ptr(state_slots), _ptr(req), _ptr(tok0), _ptr(ntok), _ptr(items), _ptr(o), c_int(n_tiles),
+                                     c_int(R), c_int(heads), c_int(dim), c_int(vdim), _stream()), "time_mix_chunks")
     return o
 
 

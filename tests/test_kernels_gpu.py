@@ -1528,3 +1528,37 @@ def test_router_by_lanes_gives_the_bits_of_the_general_form(experts, top, groups
         assert torch.equal(ids[good], want_ids[good])
         assert torch.equal(wts[good].view(torch.int32), want_wts[good].view(torch.int32))
         assert wts[~good].isnan().all()
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 40, 64, 65, 130, 300, 1030])
+@pytest.mark.parametrize("F,K", [(33, 72), (1408, 2048), (704, 512)])
+def test_gated_epilogues_leave_the_bits_of_the_kernels_behind(M, F, K):
+    """The clamped unit and the gelu unit in a product's epilogue, over few rows, split inner sizes and tiles, against the same
+    product stored in bfloat16 and the units' own kernels: the same bits, infinities and NaN among them.  (At sizes where a stored
+    product of up to 8 rows takes eight columns a workgroup, whose sums run in another order, there is nothing to compare.)"""
+    k, g = ops(), torch.Generator().manual_seed(M + F)
+    a = (torch.randn(M, K, generator=g) * 2).to(torch.bfloat16).cuda()
+    gate, up = ((torch.randn(F, K, generator=g) / K ** 0.5 * 3).to(torch.bfloat16).cuda() for _ in range(2))
+    a[M // 2, 3] = float("inf")
+    if M > 4:
+        a[M // 4, 5] = float("nan")
+    bits = lambda x: torch.where(x.isnan(), torch.zeros_like(x), x).view(torch.int16)  # noqa: E731
+    same = lambda x, y: torch.equal(x.isnan(), y.isnan()) and torch.equal(bits(x), bits(y))  # noqa: E731
+    both, woven = torch.cat([gate, up]), torch.stack([gate, up], dim=1).reshape(2 * F, K).contiguous()
+    # the stored product of the woven columns: the same sums in the same columns, then put side by side for the kernels
+    gu = torch.empty(M, 2 * F, dtype=torch.bfloat16, device="cuda")
+    k.linear(a, woven, gu)
+    side = torch.cat([gu[:, 0::2], gu[:, 1::2]], dim=1).contiguous()
+    want, got = (torch.empty(M, F, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    k.clamped_glu(side, want, 1.7, 1.702, 1.0)
+    k.linear(a, woven, got, epilogue="clamped_glu", gate=(1.7, 1.702, 1.0))
+    assert same(got, want)
+    k.gelu_glu(side, want)
+    k.linear(a, woven, got, epilogue="gelu_glu")
+    assert same(got, want)
+    if K > 72:                      # and the columns' order changes no sum
+        stacked = torch.empty_like(gu)
+        k.linear(a, both, stacked)
+        assert same(stacked, side)
+    with pytest.raises(Exception):
+        k.linear(a.float(), woven.float(), want.float(), epilogue="gelu_glu")

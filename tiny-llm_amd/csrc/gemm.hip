@@ -53,6 +53,34 @@ __device__ __forceinline__ float swiglu_pair(float g, float u) { return g / (1.f
 __device__ __forceinline__ float swiglu_pair_fast(float g, float u) {
   return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g)) * u;
 }
+// The gated units that the bfloat16 products' epilogues form of interleaved (gate, up) columns: SiLU, from the float32 sums; the
+// clamped unit min(g, limit) sigmoid(alpha .) (clamp(u, -limit, limit) + shift) and gelu(g) u (tanh form), from sums rounded to
+// bfloat16: the bits that clamped_glu_kernel and gelu_glu_kernel make of a product's stored result.  Without those kernels a
+// layer of a decode step has a launch less, a prompt of 1,944 rows of 5,632 pairs 26 us (workload Lufazen 12.9 -> 12.6 ms).
+constexpr int kGateSilu = 0, kGateClamped = 1, kGateGelu = 2;
+struct Gate {
+  int kind = kGateSilu;
+  float limit = 0.f, alpha = 0.f, shift = 0.f;
+};
+// GATED: 1 SiLU, 2 one of the others (apart, so that SiLU products of few rows keep their registers: a decode step of them lost
+// 0.8 % to a choice at run time)
+template <int GATED>
+__device__ __forceinline__ float gated_pair(float g, float u, const Gate& gate) {
+  if constexpr (GATED == 1) return swiglu_pair_fast(g, u);
+  g = (float)(bf16_t)g;
+  u = (float)(bf16_t)u;
+  if (gate.kind == kGateClamped) {
+    g = fminf(g, gate.limit);
+    u = fminf(fmaxf(u, -gate.limit), gate.limit);
+    return g / (1.f + expf(-gate.alpha * g)) * (u + gate.shift);
+  }
+  return 0.5f * g * (1.f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
+}
+// Which gate an epilogue's number names (tl_linear_tile), and whether it names one
+static inline bool is_gated(int epilogue) { return epilogue == 1 || epilogue == 3 || epilogue == 4; }
+static inline Gate gate_of(int epilogue, float limit, float alpha, float shift) {
+  return Gate{epilogue == 3 ? kGateClamped : epilogue == 4 ? kGateGelu : kGateSilu, limit, alpha, shift};
+}
 
 // 16 bytes a lane from a buffer straight into LDS, side by side from `dst` on (the same for the whole wave; the
 // instruction takes its place from M0).  Written as an instruction block: given the builtin, the compiler waits for every
@@ -760,6 +788,7 @@ struct TileNorm {
   int group_rows = 0;
   const int32_t* tile_group = nullptr;
   int64_t group_stride = 0;
+  Gate gate;                          // a gated product's unit
   TileNorm() = default;
   TileNorm(const float* rs, int act_ = kActNone) : row_scale(rs), act(act_) {}
 };
@@ -785,7 +814,7 @@ struct GemmShape {
 constexpr int kTail = 0, kWhole = 1, kDirect = 2, kPhased = 3;
 // What is known of the residual where the epilogue is compiled (kNoResidual: none, or one of rows without whole vectors).
 constexpr int kNoResidual = 0, kResidual = 1, kAnyForm = 2;
-template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, int MODE>
+template <int BM, int BN, int WM, int WN, typename TO, int SWIGLU, int MODE>
 __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16_t* __restrict__ a,
                                                                       const bf16_t* __restrict__ w,
                                                                       TO* __restrict__ out,
@@ -1189,7 +1218,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   // of the next 32 rows is requested before these are stored: one 256 x 256 tile of 64 k takes its epilogue from 6.6 to 4.5 us,
   // with a residual from 9.2 to 6.0 (on a full chip from 31 to 15); 3,288 rows, 2,048 x 2,048 with a residual, 256 x 128
   // tiles: 41.3 -> 35.7 us.
-  constexpr bool TOGETHER = DIRECT || BM + BN > 256, NEXT = TOGETHER && sizeof(TO) == 4 && !SWIGLU;
+  constexpr bool TOGETHER = DIRECT || BM + BN > 256, NEXT = TOGETHER && sizeof(TO) == 4 && SWIGLU == 0;
   f32x4 res_next[NEXT ? 8 : 1];
   auto request_residual = [&](int i) {
     const int m = m0 + wm * S::TM + i * 32 + lane / 16, n = n0 + wn * S::TN + (lane % 16) * 4;
@@ -1291,11 +1320,11 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
           s4 = *(const f32x4*)(cstage + r * E_LD + col);
         }
         float v[4] = {s4[0] * rs, s4[1] * rs, s4[2] * rs, s4[3] * rs};
-        if constexpr (SWIGLU) {   // (gate, up, gate, up) -> two outputs; N is even and n a multiple of 4
+        if constexpr (SWIGLU != 0) {   // (gate, up, gate, up) -> two outputs; N is even and n a multiple of 4
           const int64_t oz = (int64_t)m * ldo + n / 2;
           if (n + 2 < N) {
             typedef TO to2 __attribute__((ext_vector_type(2)));
-            to2 sv = {from_f32<TO>(swiglu_pair_fast(v[0], v[1])), from_f32<TO>(swiglu_pair_fast(v[2], v[3]))};
+            to2 sv = {from_f32<TO>(gated_pair<SWIGLU>(v[0], v[1], nm.gate)), from_f32<TO>(gated_pair<SWIGLU>(v[2], v[3], nm.gate))};
             if (ldo % 2 == 0) {
               *(to2*)(out + oz) = sv;
             } else {
@@ -1303,7 +1332,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
               out[oz + 1] = sv[1];
             }
           } else {
-            out[oz] = from_f32<TO>(swiglu_pair_fast(v[0], v[1]));
+            out[oz] = from_f32<TO>(gated_pair<SWIGLU>(v[0], v[1], nm.gate));
           }
           continue;
         }
@@ -1319,7 +1348,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
           if constexpr (sizeof(TO) == 4) {
             f32x4 sv = {v[0], v[1], v[2], v[3]};
             *(f32x4*)((float*)out + o) = sv;
-            if constexpr (!SWIGLU) {
+            if constexpr (SWIGLU == 0) {
               if (nm.emit_operand) {      // uniform; N is a multiple of 64: the 16 lanes of a row are all here or none is
                 float wn[4];
                 if constexpr (TOGETHER) {
@@ -1368,7 +1397,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
   }
 }
 
-template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU, int MODE>
+template <int BM, int BN, int WM, int WN, typename TO, int SWIGLU, int MODE>
 static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, const float* residual,
                                  const TileNorm& row_scale, int M, int N, int K, int64_t lda, int64_t ldo,
                                  int k_per_split, hipStream_t stream) {
@@ -1382,7 +1411,7 @@ static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, cons
   }
   // a tile's rows are addressed with 32-bit byte offsets from its first row
   if ((int64_t)BM * lda * 2 >= 0x7fffffff || (int64_t)BN * K * 2 >= 0x7fffffff) return TL_ERR_ARG;
-  if (row_scale.emit_operand && (SWIGLU || sizeof(TO) != 4 || N % 64 || ldo % 4 || k_per_split > 0)) return TL_ERR_ARG;
+  if (row_scale.emit_operand && (SWIGLU != 0 || sizeof(TO) != 4 || N % 64 || ldo % 4 || k_per_split > 0)) return TL_ERR_ARG;
   if (row_scale.in_sumsq && k_per_split > 0) return TL_ERR_ARG;      // a split product has no epilogue of its own
   const int64_t splits = k_per_split > 0 ? (K + k_per_split - 1) / k_per_split : 1;
   const int64_t total = (int64_t)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits;
@@ -1390,7 +1419,7 @@ static int launch_gemm_bf16_mode(const bf16_t* a, const bf16_t* w, TO* out, cons
   if (grid > 0x7fffffff) return TL_ERR_ARG;
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, TO, SWIGLU, MODE>), dim3((unsigned)grid), dim3(S::THREADS),
                      S::smem_all(MODE >= kDirect), stream, a, w, out, residual, row_scale, M, N, K, lda, ldo, k_per_split);
-  static_assert(sizeof(TileNorm) <= 96, "passed by value");
+  static_assert(sizeof(TileNorm) <= 120, "passed by value");
   return TL_OK;
 }
 
@@ -1413,7 +1442,7 @@ static int tile_mode(int bm, int bn, int M, int N, int K, int k_per_split) {
   return K >= 4 * B_BK && (bm + bn == 384 || (bm + bn == 256 && alone)) ? kDirect : kWhole;
 }
 
-template <int BM, int BN, int WM, int WN, typename TO, bool SWIGLU>
+template <int BM, int BN, int WM, int WN, typename TO, int SWIGLU>
 static int launch_gemm_bf16(const bf16_t* a, const bf16_t* w, TO* out, const float* residual, const TileNorm& row_scale,
                             int M, int N, int K, int64_t lda, int64_t ldo, int k_per_split, hipStream_t stream) {
 #define TL_GEMM(MODE)                                                                                                  \
@@ -1466,7 +1495,7 @@ static int best_tile(int M, int N, int K, double* cost) {
   return best;
 }
 
-template <typename TO, bool SWIGLU>
+template <typename TO, int SWIGLU>
 static int launch_gemm_bf16_tile(int c, const bf16_t* a, const bf16_t* w, TO* out, const float* residual,
                                  const TileNorm& row_scale, int M, int N, int K, int64_t lda, int64_t ldo,
                                  int k_per_split, hipStream_t stream) {
@@ -1490,7 +1519,7 @@ static int launch_gemm_bf16_tile(int c, const bf16_t* a, const bf16_t* w, TO* ou
 // two parts: as many columns as fill the chip in whole rounds of the largest tile, and the rest
 // with whatever tile suits the rest; a single tile shape would leave the last round of
 // workgroups mostly empty (2048 x 11264: 352 tiles of 256 x 256 on 256 compute units).
-template <typename TO, bool SWIGLU>
+template <typename TO, int SWIGLU>
 static int launch_gemm_bf16_any(const bf16_t* a, const bf16_t* w, TO* out, const float* residual,
                                 const TileNorm& row_scale, int M, int N, int K, int64_t lda, int64_t ldo,
                                 int tile, int k_per_split, hipStream_t stream) {
@@ -1687,9 +1716,10 @@ struct ReduceArgs {
   bf16_t* emit_operand;
   float* emit_sumsq;
   int act = kActNone;       // bfloat16 output: applied before rounding
+  Gate gate;                // a gated product's unit
 };
 
-template <typename TO, bool SWIGLU>
+template <typename TO, int SWIGLU>
 __global__ __launch_bounds__(R_THREADS) void splitk_reduce_kernel(const ReduceArgs p) {
   __shared__ float red[R_THREADS / TL_WAVE];
   const int m = blockIdx.x, tid = threadIdx.x;
@@ -1702,7 +1732,7 @@ __global__ __launch_bounds__(R_THREADS) void splitk_reduce_kernel(const ReduceAr
     for (int q = tid; q < p.in_parts; q += R_THREADS) t += p.in_sumsq[(int64_t)m * p.in_parts + q];
   float scale = p.row_scale ? p.row_scale[m] : 1.f;
   float res[4] = {0.f, 0.f, 0.f, 0.f}, wn[4] = {0.f, 0.f, 0.f, 0.f};
-  if constexpr (!SWIGLU) {
+  if constexpr (SWIGLU == 0) {
     for (int e = 0; e < 4 && n + e < N; ++e) {
       if (p.residual) res[e] = p.residual[(int64_t)m * p.ldo + n + e];
       if (p.emit_operand)
@@ -1740,10 +1770,10 @@ __global__ __launch_bounds__(R_THREADS) void splitk_reduce_kernel(const ReduceAr
   TO* out = (TO*)p.out;
   float sq = 0.f;
   if (n < N) {
-    if constexpr (SWIGLU) {   // (gate, up, gate, up) -> two outputs; N is even and n a multiple of 4
-      out[(int64_t)m * p.ldo + n / 2] = from_f32<TO>(swiglu_pair_fast(v[0] * scale, v[1] * scale));
+    if constexpr (SWIGLU != 0) {   // (gate, up, gate, up) -> two outputs; N is even and n a multiple of 4
+      out[(int64_t)m * p.ldo + n / 2] = from_f32<TO>(gated_pair<SWIGLU>(v[0] * scale, v[1] * scale, p.gate));
       if (n + 2 < N)
-        out[(int64_t)m * p.ldo + n / 2 + 1] = from_f32<TO>(swiglu_pair_fast(v[2] * scale, v[3] * scale));
+        out[(int64_t)m * p.ldo + n / 2 + 1] = from_f32<TO>(gated_pair<SWIGLU>(v[2] * scale, v[3] * scale, p.gate));
     } else {
       for (int e = 0; e < 4 && n + e < N; ++e) {
         float x = v[e] * scale + res[e];
@@ -1848,6 +1878,7 @@ struct SkinnyArgs {
   // balanced round of workgroups out of a product whose column tiles do not divide by 256.
   int cols_wg = 0;
   int act = kActNone;       // bfloat16 output: applied before rounding
+  Gate gate;                // a gated product's unit
 };
 
 // One 8-wide k chunk of an activation row, as loaded (Raw) and as an MFMA operand.  With the norm
@@ -1917,7 +1948,7 @@ __device__ __forceinline__ bf16x8 skinny_operand(const SkinnyChunk<PRO_NORM>& c,
 // activation column j is row j % 8 at k offset (j / 8) * 32, and the wanted products are the two
 // diagonal blocks of the result, added in the epilogue.  One MFMA so covers 64 k, and a load
 // instruction reads whole 128-byte lines of 8 weight rows.
-template <int MT, int CT, bool DEEP, typename TO, int PRO, bool SWIGLU, bool HALF>
+template <int MT, int CT, bool DEEP, typename TO, int PRO, int SWIGLU, bool HALF>
 __device__ __forceinline__ void skinny_product(const SkinnyArgs& p) {
   static_assert(!HALF || (MT == 1 && CT == 1 && PRO == PRO_NONE && !SWIGLU), "HALF: one plain tile");
   constexpr int COLS = HALF ? 8 : S_COLS;          // columns of a tile that are outputs
@@ -2135,7 +2166,7 @@ __device__ __forceinline__ void skinny_product(const SkinnyArgs& p) {
       for (int wv = 0; wv < S_WAVES; ++wv) t += ss_part[wv * (MT * 16) + (tile / CT) * 16 + m_local];
       scale = 1.f / sqrtf(t / (float)K + p.eps);
     }
-    if constexpr (SWIGLU) {   // columns (2j, 2j+1) = (gate_j, up_j): even threads make one output of a pair
+    if constexpr (SWIGLU != 0) {   // columns (2j, 2j+1) = (gate_j, up_j): even threads make one output of a pair
       if ((nn & 1) || !valid) continue;
       float gv = 0.f, uv = 0.f;
 #pragma unroll
@@ -2143,7 +2174,7 @@ __device__ __forceinline__ void skinny_product(const SkinnyArgs& p) {
         gv += part[wv * TILES + tile][nn][m_local];
         uv += part[wv * TILES + tile][nn + 1][m_local];
       }
-      out[(int64_t)m * p.ldo + n / 2] = from_f32<TO>(swiglu_pair_fast(gv * scale, uv * scale));
+      out[(int64_t)m * p.ldo + n / 2] = from_f32<TO>(gated_pair<SWIGLU>(gv * scale, uv * scale, p.gate));
     } else {
       float v = 0.f;
 #pragma unroll
@@ -2177,7 +2208,7 @@ __device__ __forceinline__ void skinny_product(const SkinnyArgs& p) {
   }
 }
 
-template <int MT, int CT, bool DEEP, typename TO, int PRO, bool SWIGLU, bool HALF>
+template <int MT, int CT, bool DEEP, typename TO, int PRO, int SWIGLU, bool HALF>
 __global__ __launch_bounds__(S_THREADS) void gemm_skinny_bf16_kernel(const SkinnyArgs p) {
   skinny_product<MT, CT, DEEP, TO, PRO, SWIGLU, HALF>(p);
 }
@@ -2191,12 +2222,12 @@ struct SkinnySet {
 __global__ __launch_bounds__(S_THREADS) void gemm_skinny_set_kernel(const SkinnySet set) {
   const SkinnyArgs& p = set.p[blockIdx.y];
   if ((int)blockIdx.x * S_COLS >= p.N) return;
-  skinny_product<1, 1, false, float, PRO_NONE, false, false>(p);
+  skinny_product<1, 1, false, float, PRO_NONE, 0, false>(p);
 }
 
 // Column tiles per workgroup: every workgroup reads all M activation rows, so with more rows it
 // should own more columns, or the activations are read more often than the weights.
-template <int MT, int CT, bool DEEP, typename TO, int PRO, bool SWIGLU, bool HALF = false>
+template <int MT, int CT, bool DEEP, typename TO, int PRO, int SWIGLU, bool HALF = false>
 static int launch_skinny_deep(const SkinnyArgs& p, hipStream_t stream) {
   constexpr size_t smem = (size_t)S_WAVES * MT * CT * 16 * 17 * sizeof(float) + (size_t)(S_WAVES + 1) * MT * 16 * sizeof(float);
   static bool configured = false;
@@ -2237,7 +2268,7 @@ static int skinny_cols_wg_tiles(int N, int ct) {
 // units (measured: otherwise it is slower).
 static bool skinny_half(int M, int N, int K) { return M <= 8 && K >= 2048 && (N + 7) / 8 <= 256; }
 
-template <int MT, int CT, typename TO, int PRO, bool SWIGLU>
+template <int MT, int CT, typename TO, int PRO, int SWIGLU>
 static int launch_skinny_tile(const SkinnyArgs& p, hipStream_t stream) {
   if constexpr (MT * CT == 1 && PRO == PRO_NONE && !SWIGLU) {
     if (skinny_half(p.M, p.N, p.K)) {
@@ -2258,14 +2289,14 @@ static int launch_skinny_tile(const SkinnyArgs& p, hipStream_t stream) {
 
 // More column tiles only while at least 256 workgroups remain: fewer cannot pull the weights
 // through fast enough.
-template <int MT, typename TO, bool SWIGLU>
+template <int MT, typename TO, int SWIGLU>
 static int launch_skinny_rows(const SkinnyArgs& p, hipStream_t stream) {
   if (p.N >= 256 * 64) return launch_skinny_tile<MT, 4, TO, PRO_NONE, SWIGLU>(p, stream);
   if (p.N >= 256 * 32) return launch_skinny_tile<MT, 2, TO, PRO_NONE, SWIGLU>(p, stream);
   return launch_skinny_tile<MT, 1, TO, PRO_NONE, SWIGLU>(p, stream);
 }
 
-template <typename TO, int PRO, bool SWIGLU>
+template <typename TO, int PRO, int SWIGLU>
 static int launch_skinny(const SkinnyArgs& p, hipStream_t stream) {
   const int mt = (p.M + 15) / 16;
   if (mt == 1) {
@@ -2320,9 +2351,11 @@ static int launch_skinny(const SkinnyArgs& p, hipStream_t stream) {
 
 template <int PRO>
 static int launch_skinny_out(const SkinnyArgs& p, int out_dtype, bool swiglu, hipStream_t stream) {
-  if (out_dtype == 0 && !swiglu) return launch_skinny<float, PRO, false>(p, stream);
-  if (out_dtype == 1 && !swiglu) return launch_skinny<bf16_t, PRO, false>(p, stream);
-  if (out_dtype == 1 && swiglu) return launch_skinny<bf16_t, PRO, true>(p, stream);
+  if (out_dtype == 0 && !swiglu) return launch_skinny<float, PRO, 0>(p, stream);
+  if (out_dtype == 1 && !swiglu) return launch_skinny<bf16_t, PRO, 0>(p, stream);
+  if (out_dtype == 1 && p.gate.kind == kGateSilu) return launch_skinny<bf16_t, PRO, 1>(p, stream);
+  if constexpr (PRO == PRO_NONE)
+    if (out_dtype == 1) return launch_skinny<bf16_t, PRO, 2>(p, stream);
   return TL_ERR_ARG;
 }
 
@@ -2427,13 +2460,14 @@ int tl_norm_prescale_f32(const float* x, const float* norm_w, const int32_t* row
 // epilogue 1: SiLU-gate of interleaved columns, out[m, j] = silu(c[m, 2j]) * c[m, 2j+1], out is
 //             [M, N/2] of the input's type; N must be even; no residual.
 // epilogue 2 (bfloat16 in and out): out[m, n] = max(c[m, n], 0)^2; no residual.
+// epilogues 3 and 4 (bfloat16 in and out): as 1 with the clamped unit of limit, alpha and shift, and with gelu(gate) * up.
 // tile (bfloat16, M > 64): 0 lets the size decide; 1..4 force 256x256, 256x128, 128x128, 64x128.
 int tl_linear_tile(const void* a, const void* w, void* out, const float* residual, const float* row_scale, int M,
                    int N, int K, int64_t lda, int64_t ldo, int dtype, int out_dtype, int epilogue, int tile,
-                   hipStream_t stream) {
+                   float limit, float alpha, float shift, hipStream_t stream) {
   if (M <= 0) return TL_OK;
-  const bool swiglu = epilogue == 1;
-  if (N <= 0 || K <= 0 || lda < K || ldo < (swiglu ? N / 2 : N) || epilogue < 0 || epilogue > 2 || tile < 0 ||
+  const bool swiglu = is_gated(epilogue);
+  if (N <= 0 || K <= 0 || lda < K || ldo < (swiglu ? N / 2 : N) || epilogue < 0 || epilogue > 4 || (dtype == 0 && epilogue > 2) || tile < 0 ||
       tile > 4)
     return TL_ERR_ARG;
   if (swiglu && ((N & 1) || residual || out_dtype != dtype)) return TL_ERR_ARG;
@@ -2557,18 +2591,24 @@ int tl_linear_tile(const void* a, const void* w, void* out, const float* residua
     if (M <= 64) {
       SkinnyArgs p{a, (const bf16_t*)w, out, residual, nullptr, nullptr, row_scale, 0.f, 0, M, N, K, lda, ldo};
       p.act = act;
+      p.gate = gate_of(epilogue, limit, alpha, shift);
       const int rc = launch_skinny_out<PRO_NONE>(p, out_dtype, swiglu, stream);
       if (rc != TL_OK) return rc;
     } else {
       int rc;
-      if (swiglu)
-        rc = launch_gemm_bf16_any<bf16_t, true>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual, row_scale,
+      TileNorm gated(row_scale);
+      gated.gate = gate_of(epilogue, limit, alpha, shift);
+      if (swiglu && gated.gate.kind != kGateSilu)
+        rc = launch_gemm_bf16_any<bf16_t, 2>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual, gated, M, N, K, lda, ldo,
+                                             tile, 0, stream);
+      else if (swiglu)
+        rc = launch_gemm_bf16_any<bf16_t, 1>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual, gated,
                                                 M, N, K, lda, ldo, tile, 0, stream);
       else if (out_dtype == 0)
-        rc = launch_gemm_bf16_any<float, false>((const bf16_t*)a, (const bf16_t*)w, (float*)out, residual, row_scale,
+        rc = launch_gemm_bf16_any<float, 0>((const bf16_t*)a, (const bf16_t*)w, (float*)out, residual, row_scale,
                                                 M, N, K, lda, ldo, tile, 0, stream);
       else
-        rc = launch_gemm_bf16_any<bf16_t, false>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual,
+        rc = launch_gemm_bf16_any<bf16_t, 0>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual,
                                                  TileNorm(row_scale, act), M, N, K, lda, ldo, tile, 0, stream);
       if (rc != TL_OK) return rc;
     }
@@ -2581,7 +2621,7 @@ int tl_linear_tile(const void* a, const void* w, void* out, const float* residua
 int tl_linear(const void* a, const void* w, void* out, const float* residual, const float* row_scale, int M,
               int N, int K, int64_t lda, int64_t ldo, int dtype, int out_dtype, int epilogue,
               hipStream_t stream) {
-  return tl_linear_tile(a, w, out, residual, row_scale, M, N, K, lda, ldo, dtype, out_dtype, epilogue, 0, stream);
+  return tl_linear_tile(a, w, out, residual, row_scale, M, N, K, lda, ldo, dtype, out_dtype, epilogue, 0, 0.f, 0.f, 0.f, stream);
 }
 
 // `count` products of at most 16 rows, one inner size: out[i] (float32 [M, n[i]], rows ldo[i] apart) = a[i] @ w[i]^T,
@@ -2643,13 +2683,13 @@ int tl_linear_handoff(const void* a, const void* w, void* out, const float* resi
     }
     int rc;
     if (swiglu)
-      rc = launch_gemm_bf16_any<bf16_t, true>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual, nm, M, N, K,
+      rc = launch_gemm_bf16_any<bf16_t, 1>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual, nm, M, N, K,
                                               lda, ldo, 0, 0, stream);
     else if (out_dtype == 0)
-      rc = launch_gemm_bf16_any<float, false>((const bf16_t*)a, (const bf16_t*)w, (float*)out, residual, nm, M, N, K,
+      rc = launch_gemm_bf16_any<float, 0>((const bf16_t*)a, (const bf16_t*)w, (float*)out, residual, nm, M, N, K,
                                               lda, ldo, 0, 0, stream);
     else
-      rc = launch_gemm_bf16_any<bf16_t, false>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual, nm, M, N, K,
+      rc = launch_gemm_bf16_any<bf16_t, 0>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, residual, nm, M, N, K,
                                                lda, ldo, 0, 0, stream);
     if (rc != TL_OK) return rc;
     return tl_launch_status();
@@ -2688,13 +2728,13 @@ int tl_linear_grouped(const void* a, const void* w, void* out, const int32_t* ti
   nm.group_stride = (int64_t)N * K;
   int rc;
   if (swiglu)
-    rc = launch_gemm_bf16_any<bf16_t, true>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, nullptr, nm, M, N, K, lda,
+    rc = launch_gemm_bf16_any<bf16_t, 1>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, nullptr, nm, M, N, K, lda,
                                             ldo, 0, 0, stream);
   else if (out_dtype == 0)
-    rc = launch_gemm_bf16_any<float, false>((const bf16_t*)a, (const bf16_t*)w, (float*)out, nullptr, nm, M, N, K, lda,
+    rc = launch_gemm_bf16_any<float, 0>((const bf16_t*)a, (const bf16_t*)w, (float*)out, nullptr, nm, M, N, K, lda,
                                             ldo, 0, 0, stream);
   else
-    rc = launch_gemm_bf16_any<bf16_t, false>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, nullptr, nm, M, N, K, lda,
+    rc = launch_gemm_bf16_any<bf16_t, 0>((const bf16_t*)a, (const bf16_t*)w, (bf16_t*)out, nullptr, nm, M, N, K, lda,
                                              ldo, 0, 0, stream);
   if (rc != TL_OK) return rc;
   return tl_launch_status();
@@ -2744,10 +2784,11 @@ int tl_splitk_plan(int M, int N, int K) {
 int tl_linear_splitk(const void* a, const void* w, void* out, const float* residual, const float* row_scale,
                      const float* in_sumsq, int in_parts, float in_eps, int in_width, const void* emit_w,
                      int emit_w_dtype, void* emit_operand, float* emit_sumsq, int M, int N, int K, int64_t lda,
-                     int64_t ldo, int out_dtype, int epilogue, float* workspace, hipStream_t stream) {
-  const bool swiglu = epilogue == 1;
+                     int64_t ldo, int out_dtype, int epilogue, float limit, float alpha, float shift, float* workspace,
+                     hipStream_t stream) {
+  const bool swiglu = is_gated(epilogue);
   if (M <= 0 || N <= 0 || K <= 0 || K % 8 || lda % 8 || lda < K || ldo < (swiglu ? N / 2 : N) || epilogue < 0 ||
-      epilogue > 2 || (out_dtype != 0 && out_dtype != 1) || !workspace)
+      epilogue > 4 || (out_dtype != 0 && out_dtype != 1) || !workspace)
     return TL_ERR_ARG;
   if (swiglu && ((N & 1) || residual || out_dtype != 1)) return TL_ERR_ARG;
   const int act = epilogue == 2 ? kActRelu2 : kActNone;
@@ -2773,20 +2814,22 @@ int tl_linear_splitk(const void* a, const void* w, void* out, const float* resid
     hipLaunchKernelGGL(gemm_oneshot_bf16_kernel, dim3((N + O_BN - 1) / O_BN, splits, (M + O_BM - 1) / O_BM), dim3(O_THREADS), smem, stream,
                        (const bf16_t*)a, (const bf16_t*)w, workspace, M, N, K, lda, slabs);
   } else {
-    rc = launch_gemm_bf16_any<float, false>((const bf16_t*)a, (const bf16_t*)w, workspace, nullptr, nullptr, M, N, K, lda,
+    rc = launch_gemm_bf16_any<float, 0>((const bf16_t*)a, (const bf16_t*)w, workspace, nullptr, nullptr, M, N, K, lda,
                                             N, tile, kps, stream);
   }
   if (rc != TL_OK) return rc;
   ReduceArgs p{workspace, splits, M, N, out, ldo, residual, row_scale, in_sumsq, in_parts, in_width, in_eps, emit_w,
-               emit_w_dtype == 0 ? 1 : 0, (bf16_t*)emit_operand, emit_sumsq, act};
+               emit_w_dtype == 0 ? 1 : 0, (bf16_t*)emit_operand, emit_sumsq, act, gate_of(epilogue, limit, alpha, shift)};
   if (M > 65535) return TL_ERR_ARG;
   dim3 g(M, (N + R_CHUNK - 1) / R_CHUNK), b(R_THREADS);
-  if (swiglu)
-    hipLaunchKernelGGL((splitk_reduce_kernel<bf16_t, true>), g, b, 0, stream, p);
+  if (swiglu && p.gate.kind != kGateSilu)
+    hipLaunchKernelGGL((splitk_reduce_kernel<bf16_t, 2>), g, b, 0, stream, p);
+  else if (swiglu)
+    hipLaunchKernelGGL((splitk_reduce_kernel<bf16_t, 1>), g, b, 0, stream, p);
   else if (out_dtype == 0)
-    hipLaunchKernelGGL((splitk_reduce_kernel<float, false>), g, b, 0, stream, p);
+    hipLaunchKernelGGL((splitk_reduce_kernel<float, 0>), g, b, 0, stream, p);
   else
-    hipLaunchKernelGGL((splitk_reduce_kernel<bf16_t, false>), g, b, 0, stream, p);
+    hipLaunchKernelGGL((splitk_reduce_kernel<bf16_t, 0>), g, b, 0, stream, p);
   return tl_launch_status();
 }
 

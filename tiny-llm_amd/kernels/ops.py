@@ -223,11 +223,13 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor
 
 
 def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual: Optional[torch.Tensor] = None,
-           epilogue: Optional[str] = None, row_scale: Optional[torch.Tensor] = None, tile: int = 0) -> torch.Tensor:
+           epilogue: Optional[str] = None, row_scale: Optional[torch.Tensor] = None, tile: int = 0,
+           gate=(0.0, 0.0, 0.0)) -> torch.Tensor:
     """out = a @ w.T (+ residual).  a [M, K], w [N, K] share an element type; out [M, N] is that
     type or float32; residual float32 with out's strides.  epilogue="swiglu": the N columns are
     interleaved (gate_j, up_j) pairs and out [M, N/2] = silu(gate) * up, computed from the float32
-    accumulators; epilogue="relu2" (bfloat16 in and out, no residual): out = max(., 0)^2 likewise.  row_scale [M] (float32) multiplies the rows of the product first.
+    accumulators; "clamped_glu" and "gelu_glu" (bfloat16) likewise, with the units of `clamped_glu` (its limit, alpha and shift
+    in `gate`) and `gelu_glu`; epilogue="relu2" (bfloat16 in and out, no residual): out = max(., 0)^2 likewise.  row_scale [M] (float32) multiplies the rows of the product first.
     tile: 0 lets the sizes choose the tile of the bfloat16 product for more than 64 rows; 1 to 4
     force 256x256, 256x128, 128x128, 64x128 (tests and tuning)."""
     _dev(a, w, out, residual, row_scale)
@@ -235,8 +237,8 @@ def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual: Option
     _rows_2d(out, "linear output")
     M, K = a.shape
     N = w.shape[0]
-    code = EPILOGUES["relu2"] if epilogue == "relu2" else _epilogue(epilogue)
-    swiglu = code == EPILOGUES["swiglu"]
+    code = EPILOGUES[epilogue] if epilogue in ("relu2", *GATED_EPILOGUES) else _epilogue(epilogue)
+    swiglu = epilogue in GATED_EPILOGUES
     if not (w.dim() == 2 and w.is_contiguous() and w.shape[1] == K):
         _fail(f"weight must be contiguous [N, {K}]")
     if not (a.dtype == w.dtype):
@@ -244,6 +246,8 @@ def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual: Option
     dt, odt = _dt(a), _dt(out)
     if epilogue == "relu2" and not (dt == odt == 1 and residual is None):
         _fail("the squared-relu epilogue takes and leaves bfloat16, without a residual")
+    if code > EPILOGUES["relu2"] and dt != 1:
+        _fail(f"the {epilogue} epilogue takes and leaves bfloat16")
     if swiglu:
         if not (N % 2 == 0 and tuple(out.shape) == (M, N // 2) and odt == dt and residual is None):
             _fail(f"the SiLU-gate epilogue writes [{M}, {N // 2}] of the input's type and takes no residual")
@@ -269,14 +273,15 @@ def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual: Option
     if dt == 1 and tile == 0 and M > 16:
         splits = split_k(M, N, K)
         if splits > 1:
-            return _linear_split(a, w, out, residual, code, row_scale, None, 0, 0.0, 0, None, splits)
+            return _linear_split(a, w, out, residual, code, row_scale, None, 0, 0.0, 0, None, splits, gate)
     _check(_lib().tl_linear_tile(_ptr(a, al), _ptr(w, al), _ptr(out, ao), _ptr(residual, ao), _ptr(row_scale),
                                  c_int(M), c_int(N), c_int(K), c_int64(a.stride(0)), c_int64(out.stride(0)), c_int(dt),
-                                 c_int(odt), c_int(code), c_int(tile), _stream()), "linear")
+                                 c_int(odt), c_int(code), c_int(tile), *(c_float(x) for x in gate), _stream()), "linear")
     return out
 
 
-EPILOGUES = {None: 0, "swiglu": 1, "relu2": 2}      # what `linear` does to its sums, by the number the kernels take
+GATED_EPILOGUES = ("swiglu", "clamped_glu", "gelu_glu")
+EPILOGUES = {None: 0, "swiglu": 1, "relu2": 2, "clamped_glu": 3, "gelu_glu": 4}      # what `linear` does to its sums, by the number the kernels take
 
 
 def _epilogue(name: Optional[str]) -> int:
@@ -481,7 +486,8 @@ def handoff_parts(rows: int, width: int, inner: int) -> int:
 _PARTS: dict = {}
 
 
-def _linear_split(a, w, out, residual, swiglu, row_scale, sumsq_in, parts, eps, width, emit, splits) -> torch.Tensor:
+def _linear_split(a, w, out, residual, swiglu, row_scale, sumsq_in, parts, eps, width, emit, splits,
+                  gate=(0.0, 0.0, 0.0)) -> torch.Tensor:
     """Partial products into a workspace, then one kernel that adds them and applies the epilogue."""
     M, K = a.shape
     N = w.shape[0]
@@ -491,7 +497,7 @@ def _linear_split(a, w, out, residual, swiglu, row_scale, sumsq_in, parts, eps, 
         _ptr(a, 16), _ptr(w, 16), _ptr(out), _ptr(residual), _ptr(row_scale), _ptr(sumsq_in), c_int(parts),
         c_float(eps), c_int(width), _ptr(emit_w), c_int(_dt(emit_w) if emit_w is not None else 0), _ptr(emit_op),
         _ptr(emit_sq), c_int(M), c_int(N), c_int(K), c_int64(a.stride(0)), c_int64(out.stride(0)), c_int(_dt(out)),
-        c_int(swiglu), _ptr(work, 16), _stream()), "linear_splitk")
+        c_int(swiglu), *(c_float(x) for x in gate), _ptr(work, 16), _stream()), "linear_splitk")
     return out
 
 

@@ -17,6 +17,11 @@ from .norm import LazyNorm
 from .base import FeedForward, WeightSpec, project_into_residual, register_feed_forward
 
 
+def _interleaved(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    """Rows (gate_0, up_0, gate_1, up_1, ...): a product's epilogue sees each pair side by side and writes the gated unit."""
+    return torch.stack([gate, up], dim=1).reshape(2 * gate.shape[0], gate.shape[1]).contiguous()
+
+
 class SwiGLU(FeedForward):
     graph_safe = True
     accepts_lazy_norm = True
@@ -39,10 +44,7 @@ class SwiGLU(FeedForward):
     def bind(self, tensors: Dict[str, torch.Tensor]) -> None:
         p = self.prefix
         gate, up = tensors[f"{p}.gate_proj.weight"], tensors[f"{p}.up_proj.weight"]
-        # rows interleaved (gate_0, up_0, gate_1, up_1, ...): a product's epilogue then sees each
-        # pair side by side and writes silu(gate) * up directly
-        self.w_gate_up = torch.stack([gate, up], dim=1).reshape(2 * self.intermediate_size,
-                                                                self.hidden_size).contiguous()
+        self.w_gate_up = _interleaved(gate, up)
         self.w_down = tensors[f"{p}.down_proj.weight"].contiguous()
 
     def forward(self, h, ctx, residual, next_norm=None):
@@ -58,8 +60,9 @@ class SwiGLU(FeedForward):
 
 class ClampedGLU(FeedForward):
     """down(g * sigmoid(alpha * g) * (u + shift)) with g = min(gate(h), limit) and
-    u = clamp(up(h), -limit, limit).  Gate and up weights are stacked on load into one [2F, H]
-    matrix (one product); the activation runs on its result in the engine's element type.
+    u = clamp(up(h), -limit, limit).  Gate and up weights make one [2F, H] matrix on load (one product).  In bfloat16 their
+    rows are interleaved and the activation rides in the product's epilogue, on sums rounded to bfloat16; in float32 they are
+    stacked and it runs on the result.
 
     `names`: the tensors' names below the prefix, (gate, up, down).  With `residual=None` the
     result is returned by itself in float32 (a block that norms the sublayer's output adds it)."""
@@ -86,23 +89,28 @@ class ClampedGLU(FeedForward):
 
     def bind(self, tensors: Dict[str, torch.Tensor]) -> None:
         gate, up, down = self.names
-        self.w_gate_up = torch.cat([tensors[gate], tensors[up]], dim=0).contiguous()
+        self.w_gate_up = (_interleaved(tensors[gate], tensors[up]) if self.dtype == torch.bfloat16
+                          else torch.cat([tensors[gate], tensors[up]], dim=0).contiguous())
         self.w_down = tensors[down].contiguous()
 
     def forward(self, h, ctx, residual):
         T, dev = h.shape[0], h.device
-        gu = ops.scratch("ffn_gate_up", (T, 2 * self.intermediate_size), self.dtype, dev)
-        ops.linear(h, self.w_gate_up, gu)
         z = ops.scratch("ffn_gated", (T, self.intermediate_size), self.dtype, dev)
-        ops.clamped_glu(gu, z, self.limit, self.alpha, self.shift)
+        if self.dtype == torch.bfloat16:
+            ops.linear(h, self.w_gate_up, z, epilogue="clamped_glu", gate=(self.limit, self.alpha, self.shift))
+        else:
+            gu = ops.scratch("ffn_gate_up", (T, 2 * self.intermediate_size), self.dtype, dev)
+            ops.linear(h, self.w_gate_up, gu)
+            ops.clamped_glu(gu, z, self.limit, self.alpha, self.shift)
         if residual is None:
             return ops.linear(z, self.w_down, ops.scratch("sublayer_out", (T, self.hidden_size), torch.float32, dev))
         return ops.linear(z, self.w_down, residual, residual)
 
 
 class GeluGLU(FeedForward):
-    """down(gelu(gate(h)) * up(h)), gelu in its tanh form.  Gate and up weights are stacked on load into
-    one [2F, H] matrix (one product); the activation runs on its result in the engine's element type.
+    """down(gelu(gate(h)) * up(h)), gelu in its tanh form.  Gate and up weights make one [2F, H] matrix on load (one
+    product).  In bfloat16 their rows are interleaved and the activation rides in the product's epilogue, on sums rounded to
+    bfloat16; in float32 they are stacked and it runs on the result.
     `names`: the tensors' names below the prefix, (gate, up, down).  With `residual=None` the result is
     returned by itself in float32."""
     graph_safe = True
@@ -125,15 +133,19 @@ class GeluGLU(FeedForward):
 
     def bind(self, tensors: Dict[str, torch.Tensor]) -> None:
         gate, up, down = self.names
-        self.w_gate_up = torch.cat([tensors[gate], tensors[up]], dim=0).contiguous()
+        self.w_gate_up = (_interleaved(tensors[gate], tensors[up]) if self.dtype == torch.bfloat16
+                          else torch.cat([tensors[gate], tensors[up]], dim=0).contiguous())
         self.w_down = tensors[down].contiguous()
 
     def forward(self, h, ctx, residual):
         T, dev = h.shape[0], h.device
-        gu = ops.scratch("ffn_gate_up", (T, 2 * self.intermediate_size), self.dtype, dev)
-        ops.linear(h, self.w_gate_up, gu)
         z = ops.scratch("ffn_gated", (T, self.intermediate_size), self.dtype, dev)
-        ops.gelu_glu(gu, z)
+        if self.dtype == torch.bfloat16:
+            ops.linear(h, self.w_gate_up, z, epilogue="gelu_glu")
+        else:
+            gu = ops.scratch("ffn_gate_up", (T, 2 * self.intermediate_size), self.dtype, dev)
+            ops.linear(h, self.w_gate_up, gu)
+            ops.gelu_glu(gu, z)
         if residual is None:
             return ops.linear(z, self.w_down, ops.scratch("sublayer_out", (T, self.hidden_size), torch.float32, dev))
         return ops.linear(z, self.w_down, residual, residual)

@@ -651,3 +651,40 @@ def test_latent_decode_splits_and_sizes(C, R, H):
             ops.latent_flash(qa, lat, rope[:, :, :R].contiguous() if R else None, table, None, pos, out, scale, gate, splits, part,
                              window=window, sinks=sinks)
             assert ((out.double() - want).abs() <= 2.0 ** -7 * size + 1e-6).all(), (window, splits)
+
+
+@pytest.mark.parametrize("H,window", [(16, 0), (16, 100), (4, 33), (20, 0)])
+def test_latent_prefill_over_every_page_size(H, window):
+    """Latents of 512 with 64 rotated dims, whose rows a wave fetches whole: the same keys in pages of one, of powers of two and
+    of other sizes give the same bits, and these agree with attention in 64 bits.  Bound: probabilities are rounded to bfloat16
+    (2^-9 each, of a weighted mean of latents below 5), the result once more."""
+    from tiny_llm_amd.engine.step import tile_lists
+    from tiny_llm_amd.kernels import ops
+    g = torch.Generator().manual_seed(H + window)
+    lens, ctx, C, R = [70, 1, 33], [5, 90, 0], 512, 64
+    T, ends = sum(lens), [a + b for a, b in zip(lens, ctx)]
+    keys = [torch.randn(n, C + R, generator=g).to(torch.bfloat16) for n in ends]
+    qa = torch.randn(T, H, C + R, generator=g) * 0.5
+    pos = torch.cat([torch.arange(c, c + n) for c, n in zip(ctx, lens)])
+    want, at = torch.zeros(T, H, C, dtype=torch.float64), 0
+    for k, n, c in zip(keys, lens, ctx):
+        s = torch.einsum("thd,kd->thk", qa[at:at + n].double(), k.double()) * 0.05
+        i, j = torch.arange(c, c + n)[:, None], torch.arange(c + n)[None, :]
+        s = s.masked_fill(~((j <= i) & ((j > i - window) if window else True))[:, None, :], float("-inf"))
+        want[at:at + n] = torch.einsum("thk,kd->thd", torch.softmax(s, -1), k[:, :C].double())
+        at += n
+    first = None
+    tiles = [torch.tensor(x, dtype=torch.int32).cuda() for x in tile_lists(lens, 4 * (16 // min(H, 16)))]
+    for bs in (64, 1, 4, 16, 24, 48):
+        per = -(-max(ends) // bs)
+        order = (torch.randperm(3 * per, generator=g) + 1).to(torch.int32).view(3, per)
+        latent, rope = (torch.full((3 * per + 1, bs, n), float("nan"), dtype=torch.bfloat16) for n in (C, R))
+        for r, k in enumerate(keys):
+            for j in range(k.shape[0]):
+                latent[order[r, j // bs], j % bs], rope[order[r, j // bs], j % bs] = k[j, :C], k[j, C:]
+        out = torch.empty(T, H, C, dtype=torch.bfloat16, device="cuda")
+        ops.latent_prefill(qa.cuda(), latent.cuda(), rope.cuda(), order.cuda(), tiles, pos.to(torch.int32).cuda(), out, 0.05, None, window)
+        if first is None:
+            first = out
+            assert (out.double().cpu() - want).abs().max() <= 5 * 2.0 ** -8
+        assert torch.equal(out, first), bs

@@ -418,21 +418,22 @@ __global__ __launch_bounds__(LF_WAVES * TL_WAVE) void latent_flash_bf16_kernel(
 // LDS.  A wave keeps its own (max, sum, output): nothing is merged.
 // What bounds it is what a SIMD's one wave issues per 32 keys: 72 matrix instructions for the scores in four sums, 32
 // for the values (both halves of the keys in one operand, in the order in which the scores leave the registers), and
-// the output's rescaling only where a maximum rose.  2,048 tokens of 16 heads: 707 -> 496 us, in a window of 512 tokens
-// 271 -> 209 us (half the keys an instruction and every output rescaled, before).  The form for other sizes takes every
+// the output's rescaling only where a maximum rose.  2,048 tokens of 16 heads: 707 -> 496 -> 347 us, in a window of 512 tokens
+// 271 -> 207 -> 146 us (half the keys an instruction and every output rescaled, before).  The form for other sizes takes every
 // register there is and keeps 12 values in scratch: 2,048 tokens, latents of 496 with 64 rotated dims 698 -> 621 us, of
 // 256 with 64 551 -> 474, of 64 with 32 414 -> 343; ten sizes in six shapes of step took 0.80 to 0.99 of the time before.
 constexpr int LP_KEYS = 32;         // keys a staged tile holds (two 16-key tiles of the products)
 constexpr int LP_NPF = 9;           // 16-byte pieces of a staged tile a thread fetches: 32 * 72 / 256
-// WHOLE: as in latent_flash_bf16_kernel.
-template <bool WHOLE>
+// WHOLE: as in latent_flash_bf16_kernel; SHIFT (with it): pages of a power of two of keys (2,048 tokens 347 us, 388 with the choice
+// at run time).
+template <bool WHOLE, bool SHIFT>
 __global__ __launch_bounds__(LF_WAVES * TL_WAVE) void latent_prefill_bf16_kernel(
     const float* __restrict__ qa, const bf16_t* __restrict__ latent, const bf16_t* __restrict__ rope,
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ tile_req,
     const int32_t* __restrict__ tile_tok0, const int32_t* __restrict__ tile_ntok,
     const int32_t* __restrict__ positions, const bf16_t* __restrict__ gate, int64_t gate_stride,
-    bf16_t* __restrict__ out, int heads, int tpt, int kv_rank_, int rot_, int block_size, float scale, int window,
-    const float* __restrict__ sinks) {
+    bf16_t* __restrict__ out, int heads, int tpt, int kv_rank_, int rot_, int block_size, int page_shift, float scale,
+    int window, const float* __restrict__ sinks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lf_smem[];
   const int tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE, g = lane / 16, c = lane % 16;
   const int tile = blockIdx.x, head0 = blockIdx.y * 16;
@@ -485,25 +486,52 @@ __global__ __launch_bounds__(LF_WAVES * TL_WAVE) void latent_prefill_bf16_kernel
   }
   // A staged tile is fetched in pieces: piece f is row f / CPR, dims 8 (f % CPR) ...  The pages of a
   // tile are looked up an iteration before its rows are requested, so that a request never begins
-  // with a round trip of its own.
+  // with a round trip of its own.  WHOLE: a wave fetches eight whole rows, a lane one piece of each latent (their pages and
+  // addresses are scalars) and one piece of a row's rotated dims; with pieces dealt out over all threads every piece had its
+  // own page, quotients by the page size and a branch, 1,944 tokens of six requests in a window of 512 took 146 us, now 106; one
+  // prompt of 2,048 497 and 347, of 100 29 and 24 (16 heads); pages of 48 keys, which are no shift, 170 and 133 (370 tokens of 20 heads).
+  static_assert(!WHOLE || (LF_MAXDT * 16 == TL_WAVE * 8 && LF_MAXKS * 32 - LF_MAXDT * 16 == 64 && LP_KEYS == 8 * LF_WAVES && LP_NPF == 9),
+                "a latent is a wave's pieces, a row's rotated dims are eight");
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  // keys beyond the end, and keys every window has left (their pages may be given back), read a row that exists
+  auto key_at = [&](int k) { return max(min(k, kv_end - 1), kv_first); };
+  auto page_of = [&](int key) { return SHIFT ? key >> page_shift : key / block_size; };
   bf16x8 pf[LP_NPF];
   int page[LP_NPF];
   auto lookup = [&](int kt) {
+    if constexpr (WHOLE) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) page[j] = bt[page_of(key_at(kt * LP_KEYS + wv * 8 + j))];
+      page[8] = bt[page_of(key_at(kt * LP_KEYS + wv * 8 + lane / 8))];
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < LP_NPF; ++j) {
       const int f = tid + j * LF_WAVES * TL_WAVE;
-      // keys beyond the end, and keys every window has left (their pages may be given back), read a row that exists
-      const int key = max(min(kt * LP_KEYS + min(f / CPR, LP_KEYS - 1), kv_end - 1), kv_first);
-      page[j] = bt[key / block_size];
+      page[j] = bt[key_at(kt * LP_KEYS + min(f / CPR, LP_KEYS - 1)) / block_size];
     }
   };
   auto fetch = [&](int kt) {
+    if constexpr (WHOLE) {
+      auto slot_of = [&](int page_id, int key) {
+        return SHIFT ? ((int64_t)page_id << page_shift) + (key & (block_size - 1))
+                     : (int64_t)page_id * block_size + (key - page_of(key) * block_size);
+      };
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int64_t slot = slot_of(page[j], key_at(kt * LP_KEYS + wv * 8 + j));
+        pf[j] = ((const bf16x8*)(latent + slot * (LF_MAXDT * 16)))[lane];
+      }
+      const int64_t slot = slot_of(page[8], key_at(kt * LP_KEYS + wv * 8 + lane / 8));
+      pf[8] = ((const bf16x8*)(rope + slot * 64))[lane % 8];
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < LP_NPF; ++j) {
       const int f = tid + j * LF_WAVES * TL_WAVE;
       if (f < LP_KEYS * CPR) {
         const int row = f / CPR, d0 = (f - row * CPR) * 8;
-        const int key = max(min(kt * LP_KEYS + row, kv_end - 1), kv_first);
+        const int key = key_at(kt * LP_KEYS + row);
         const int64_t slot = (int64_t)page[j] * block_size + (key % block_size);
         if (d0 < kv_rank) pf[j] = *(const bf16x8*)(latent + slot * kv_rank + d0);
         else if (d0 - kv_rank < rot) pf[j] = *(const bf16x8*)(rope + slot * rot + (d0 - kv_rank));
@@ -512,6 +540,12 @@ __global__ __launch_bounds__(LF_WAVES * TL_WAVE) void latent_prefill_bf16_kernel
     }
   };
   auto stage = [&](bf16_t* buf) {
+    if constexpr (WHOLE) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) *(bf16x8*)(buf + (wv * 8 + j) * KSTR + lane * 8) = pf[j];
+      *(bf16x8*)(buf + (wv * 8 + lane / 8) * KSTR + LF_MAXDT * 16 + lane % 8 * 8) = pf[8];
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < LP_NPF; ++j) {
       const int f = tid + j * LF_WAVES * TL_WAVE;
@@ -966,18 +1000,22 @@ int tl_latent_prefill(const float* qa, const void* latent, const void* rope, con
   const int WP = (kv_rank + rot + 31) / 32 * 32;
   // two staged tiles and the four waves' lower query terms: at most 150 KB (the default limit is 64 KB)
   const size_t lds = (size_t)(2 * LP_KEYS + LF_WAVES * 16) * (WP + LF_PAD) * 2;
+  const int log2 = 31 - __builtin_clz((unsigned)block_size), page_shift = (1 << log2) == block_size ? log2 : -1;
   const bool whole = kv_rank == 16 * LF_MAXDT && rot == 32 * LF_MAXKS - 16 * LF_MAXDT;
-  const auto kernel = whole ? latent_prefill_bf16_kernel<true> : latent_prefill_bf16_kernel<false>;
-  static int granted[2] = {0, 0};
-  if ((int)lds > granted[whole]) {
+  const int form = !whole ? 0 : page_shift < 0 ? 1 : 2;
+  const auto kernel = form == 0   ? latent_prefill_bf16_kernel<false, false>
+                      : form == 1 ? latent_prefill_bf16_kernel<true, false>
+                                  : latent_prefill_bf16_kernel<true, true>;
+  static int granted[3] = {0, 0, 0};
+  if ((int)lds > granted[form]) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return TL_ERR_LAUNCH;
-    granted[whole] = (int)lds;
+    granted[form] = (int)lds;
   }
   dim3 g(n_tiles, (heads + 15) / 16), b(LF_WAVES * TL_WAVE);
   hipLaunchKernelGGL(kernel, g, b, lds, stream, qa, (const bf16_t*)latent, (const bf16_t*)rope, block_tables, max_blocks,
                      tile_req, tile_tok0, tile_ntok, positions, (const bf16_t*)gate, gate_stride, (bf16_t*)out, heads, tpt,
-                     kv_rank, rot, block_size, scale, window, sinks);
+                     kv_rank, rot, block_size, page_shift, scale, window, sinks);
   return tl_launch_status();
 }
 

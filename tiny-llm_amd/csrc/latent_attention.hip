@@ -804,17 +804,19 @@ __global__ __launch_bounds__(kThreads) void head_products_kernel(const TI* __res
 // 2 x 2 tiles of v_mfma_f32_16x16x32_bf16; both operands go straight from memory into registers (a
 // lane's eight consecutive k of one row).  The product is computed transposed (columns as the
 // instruction's rows), so a lane ends with four consecutive output columns of one row.
-// STEPS: k steps of 32 whose operands are requested together, each with a sum of its own.  With few rows the kernel is its
+// A lane's four results leave as one vector where rows and heads allow it: 1,944 rows of 16 heads, 128 -> 512, 54.8 -> 34.8 us
+// (as scalars every store was 64 pieces of four bytes), 512 -> 128 in bfloat16 36.4 -> 32.0.
+// STEPS: k steps of 32 whose operands are requested together; SUMS of them, one after the other.  With few rows the kernel is its
 // round trips to memory and takes four: 6 rows of 16 heads, 512 -> 128, 7.0 us one by one and 6.1 so.  Four sums also keep its
 // error where the kernel of few rows has it (5.7e-8 of the result against 64 bits; in one sum 8.5e-8).  Many rows find
-// their operands in the caches and lose waves by it: 64 rows of 16 heads, 128 -> 512, 6.1 us by one step and 6.3 by four.
+// their operands in the caches and lose waves by it: 64 rows of 16 heads, 128 -> 512, 6.1 us by one step and 6.3 by four; 1,944 rows 34.8 and 34.0.
 constexpr int kHeadFewRows = 32;
-template <typename TO, int STEPS>
+template <typename TO, int STEPS, int SUMS>
 __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* __restrict__ in, int64_t in_stride,
                                                                   int in_head_width, const bf16_t* __restrict__ w,
                                                                   TO* __restrict__ out, int64_t out_stride,
                                                                   int out_head_width, int n_rows, int inner, int cols,
-                                                                  const bf16_t* __restrict__ gate, int64_t gate_stride) {
+                                                                  const bf16_t* __restrict__ gate, int64_t gate_stride, int whole) {
   const int h = blockIdx.x, wave = threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE, g = lane / 16, c = lane % 16;
   const int col0 = blockIdx.y * 64 + (wave & 1) * 32, row0 = blockIdx.z * 64 + (wave >> 1) * 32;
   if (col0 >= cols || row0 >= n_rows) return;
@@ -825,9 +827,9 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
     wp[a] = w + ((int64_t)h * cols + min(col0 + a * 16 + c, cols - 1)) * inner;
     xp[a] = in + (int64_t)min(row0 + a * 16 + c, n_rows - 1) * in_stride + (int64_t)h * in_head_width;
   }
-  f32x4 sum[STEPS][2][2];
+  f32x4 sum[SUMS][2][2];
 #pragma unroll
-  for (int p = 0; p < STEPS; ++p)
+  for (int p = 0; p < SUMS; ++p)
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -851,7 +853,7 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
         for (int a = 0; a < 2; ++a)
 #pragma unroll
           for (int b = 0; b < 2; ++b)
-            sum[u][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][a], xb[u][b], sum[u][a][b], 0, 0, 0);
+            sum[u % SUMS][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][a], xb[u][b], sum[u % SUMS][a][b], 0, 0, 0);
       }
   }
   f32x4 acc[2][2];
@@ -859,7 +861,7 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      if constexpr (STEPS == 4) acc[a][b] = (sum[0][a][b] + sum[1][a][b]) + (sum[2][a][b] + sum[3][a][b]);
+      if constexpr (SUMS == 4) acc[a][b] = (sum[0][a][b] + sum[1][a][b]) + (sum[2][a][b] + sum[3][a][b]);
       else acc[a][b] = sum[0][a][b];
     }
   // acc[a][b][i] = out[row0 + b*16 + c][col0 + a*16 + g*4 + i]
@@ -871,6 +873,18 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
     for (int a = 0; a < 2; ++a) {
       const int n = col0 + a * 16 + g * 4;
       TO* dst = out + (int64_t)row * out_stride + (int64_t)h * out_head_width + n;
+      if (whole && n < cols) {                    // four columns together (as scalars each is a piece of its own)
+        typedef TO to4 __attribute__((ext_vector_type(4)));
+        to4 v4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v = acc[a][b][i];
+          if (gate) v /= 1.f + expf(-(float)gate[(int64_t)row * gate_stride + (int64_t)h * cols + n + i]);
+          v4[i] = from_f32<TO>(v);
+        }
+        *(to4*)dst = v4;
+        continue;
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (n + i < cols) {
@@ -1054,16 +1068,19 @@ int tl_head_gemm(const void* in, int64_t in_stride, int in_head_width, const voi
     return TL_ERR_ARG;
   dim3 g(heads, (cols + 63) / 64, (n_rows + 63) / 64), b(kThreads);
   const bool few = n_rows <= kHeadFewRows;
-  if (out_dtype == 0)
-    hipLaunchKernelGGL((few ? head_gemm_bf16_kernel<float, 4> : head_gemm_bf16_kernel<float, 1>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width,
-                       (const bf16_t*)w, (float*)out, out_stride, out_head_width, n_rows, inner, cols,
-                       (const bf16_t*)gate, gate_stride);
-  else if (out_dtype == 1)
-    hipLaunchKernelGGL((few ? head_gemm_bf16_kernel<bf16_t, 4> : head_gemm_bf16_kernel<bf16_t, 1>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width,
-                       (const bf16_t*)w, (bf16_t*)out, out_stride, out_head_width, n_rows, inner, cols,
-                       (const bf16_t*)gate, gate_stride);
-  else
-    return TL_ERR_ARG;
+  const int size = out_dtype == 0 ? 4 : 2;
+  // results leave four columns at a time where rows, heads and the buffer are whole vectors of them
+  const int whole = cols % 4 == 0 && out_stride % 4 == 0 && out_head_width % 4 == 0 && (uintptr_t)out % (4 * size) == 0;
+#define TL_HEAD_GEMM(TO, STEPS, SUMS)                                                                                   \
+  hipLaunchKernelGGL((head_gemm_bf16_kernel<TO, STEPS, SUMS>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width, \
+                     (const bf16_t*)w, (TO*)out, out_stride, out_head_width, n_rows, inner, cols, (const bf16_t*)gate,   \
+                     gate_stride, whole)
+  if (out_dtype == 0 && few) TL_HEAD_GEMM(float, 4, 4);
+  else if (out_dtype == 0) TL_HEAD_GEMM(float, 1, 1);
+  else if (out_dtype == 1 && few) TL_HEAD_GEMM(bf16_t, 4, 4);
+  else if (out_dtype == 1) TL_HEAD_GEMM(bf16_t, 1, 1);
+  else return TL_ERR_ARG;
+#undef TL_HEAD_GEMM
   return tl_launch_status();
 }
 

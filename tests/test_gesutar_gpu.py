@@ -603,6 +603,40 @@ def test_latent_prepare_without_a_query_latent_and_rotate_into(dtype, pairing):
     assert (qa[:, :, C:].double().cpu() - want_q).abs().max() < 1e-5 and float(qa[:, :, :C].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("T,H,K,N,R,rd", [(1, 3, 24, 40, 8, 4), (6, 16, 128, 512, 64, 64), (33, 2, 40, 33, 8, 8), (64, 2, 64, 64, 72, 2),
+                                          (65, 5, 32, 65, 16, 6), (200, 1, 8, 16, 296, 296)])
+def test_rotation_and_gate_that_ride_in_the_heads_products(T, H, K, N, R, rd):
+    """The rotation of a query's other dims within the launch of its product, and the gate within the values' product, against the
+    launches of their own: the same bits."""
+    from tiny_llm_amd.kernels import ops
+    from tiny_llm_amd.parts.rotary import angle_tables
+    g = torch.Generator().manual_seed(T + R)
+    cos, sin = angle_tables(rd, 500.0, 512, "cuda")
+    positions = torch.randint(0, 512, (T,), generator=g).to(torch.int32).cuda()
+    q = torch.randn(T, H * (K + R) + 8, generator=g).to(torch.bfloat16).cuda()
+    q = torch.nn.functional.pad(q, (0, -q.shape[1] % 8))
+    q3 = q[:, :H * (K + R)].unflatten(1, (H, K + R))
+    w = (torch.randn(H, N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+    for pairing in ("interleaved", "half"):
+        one, two = torch.full((2, T, H, N + R), float("nan"), device="cuda")
+        ops.head_gemm(q3[:, :, :K], w, one[:, :, :N])
+        ops.rotate_into(q, H, K + R, K, R, rd, positions, cos, sin, one, N, pairing)
+        ops.head_gemm(q3[:, :, :K], w, two[:, :, :N], rotate=(q, H, K + R, K, R, rd, positions, cos, sin, two, N, pairing))
+        assert not torch.isnan(one).any() and torch.equal(one, two)
+    heads = (torch.arange(T * H, dtype=torch.int32) % H).reshape(-1, 1).cuda()
+    for dtype in (torch.bfloat16, torch.float32):
+        x = torch.randn(T * H, K, generator=g).to(dtype).cuda()
+        w = (torch.randn(H, N, K, generator=g) / K ** 0.5).to(dtype).cuda()
+        gate = torch.randn(T, H * N + 16, generator=g).to(dtype).cuda()[:, 8:8 + H * N]
+        one, two = torch.empty(2, T * H, N, dtype=dtype, device="cuda")
+        ops.table_moe_up(x, w, None, heads, one)
+        ops.gate_rows(one.view(T, H * N), gate, one.view(T, H * N))
+        ops.table_moe_up(x, w, None, heads, two, gate=gate)
+        assert torch.equal(one, two)
+        with pytest.raises(ops.KernelError):
+            ops.table_moe_up(x, w, None, heads, two, "relu2", gate=gate)
+
+
 def test_gate_and_activation_rows():
     from tiny_llm_amd.kernels import ops
     g = torch.Generator().manual_seed(0)

@@ -70,27 +70,41 @@ __global__ void latent_prepare_kernel(const T* __restrict__ d, int64_t d_stride,
 // of them rotated by the angle table's row positions[t] (pair i is (i, i + rdims/2), or (2i, 2i + 1) when
 // `interleaved`).
 template <typename T>
-__global__ void rotate_into_kernel(const T* __restrict__ q, int64_t q_stride, int head_width, int in_off, int rot,
-                                   int rdims, int heads, const int32_t* __restrict__ positions, const float* __restrict__ cos_t,
-                                   const float* __restrict__ sin_t, float* __restrict__ out, int out_width,
-                                   int out_off, int interleaved) {
-  const int t = blockIdx.x;
-  const int half = rdims / 2, rest = rot - rdims, per_head = half + rest;
-  const int pos = positions[t];
-  for (int e = threadIdx.x; e < heads * per_head; e += kThreads) {
-    const int h = e / per_head, i = e - h * per_head;
+struct Rotate {
+  const T* q;
+  int64_t q_stride;
+  int head_width, in_off, rot, rdims, heads;
+  const int32_t* positions;
+  const float *cos_t, *sin_t;
+  float* out;
+  int out_width, out_off, interleaved;
+
+  __host__ __device__ int per_head() const { return rdims / 2 + rot - rdims; }     // pieces of work of a head
+  __device__ void piece(int t, int h, int i) const {
+    const int half = rdims / 2;
     const T* src = q + (int64_t)t * q_stride + (int64_t)h * head_width + in_off;
     float* dst = out + ((int64_t)t * heads + h) * out_width + out_off;
     if (i >= half) {
       dst[rdims + i - half] = to_f32(src[rdims + i - half]);
-      continue;
+      return;
     }
+    const int pos = positions[t];
     const float c = cos_t[(int64_t)pos * half + i], s = sin_t[(int64_t)pos * half + i];
     const int a = interleaved ? 2 * i : i, b = interleaved ? 2 * i + 1 : half + i;
     const float u = to_f32(src[a]), v = to_f32(src[b]);
     dst[a] = u * c - v * s;
     dst[b] = v * c + u * s;
   }
+  bool fits() const {
+    return rot > 0 && rdims >= 0 && rdims % 2 == 0 && rdims <= rot && heads > 0 && in_off >= 0 && in_off + rot <= head_width &&
+           out_off >= 0 && out_off + rot <= out_width && (interleaved == 0 || interleaved == 1);
+  }
+};
+
+template <typename T>
+__global__ void rotate_into_kernel(Rotate<T> r) {
+  const int per_head = r.per_head();
+  for (int e = threadIdx.x; e < r.heads * per_head; e += kThreads) r.piece(blockIdx.x, e / per_head, e % per_head);
 }
 
 // One wave64 per (token, head).  Lanes split the keys of a 64-key tile for the scores and the
@@ -810,13 +824,24 @@ __global__ __launch_bounds__(kThreads) void head_products_kernel(const TI* __res
 // round trips to memory and takes four: 6 rows of 16 heads, 512 -> 128, 7.0 us one by one and 6.1 so.  Four sums also keep its
 // error where the kernel of few rows has it (5.7e-8 of the result against 64 bits; in one sum 8.5e-8).  Many rows find
 // their operands in the caches and lose waves by it: 64 rows of 16 heads, 128 -> 512, 6.1 us by one step and 6.3 by four; 1,944 rows 34.8 and 34.0.
+// ROTATE: the last workgroup along the columns rotates the other dims of its head and rows, which a query's product leaves beside its
+// results: it needs nothing of the product, and took 3.0 us as a launch of its own for 6 rows of 16 heads, 6.0 for 1,944.
 constexpr int kHeadFewRows = 32;
-template <typename TO, int STEPS, int SUMS>
+template <typename TO, int STEPS, int SUMS, bool ROTATE>
 __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* __restrict__ in, int64_t in_stride,
                                                                   int in_head_width, const bf16_t* __restrict__ w,
                                                                   TO* __restrict__ out, int64_t out_stride,
                                                                   int out_head_width, int n_rows, int inner, int cols,
-                                                                  const bf16_t* __restrict__ gate, int64_t gate_stride, int whole) {
+                                                                  const bf16_t* __restrict__ gate, int64_t gate_stride, int whole,
+                                                                  Rotate<bf16_t> rotate) {
+  if constexpr (ROTATE) {
+    if (blockIdx.y == gridDim.y - 1) {
+      const int first = blockIdx.z * 64, per_head = rotate.per_head();
+      for (int e = threadIdx.x; e < min(64, n_rows - first) * per_head; e += kThreads)
+        rotate.piece(first + e / per_head, blockIdx.x, e % per_head);
+      return;
+    }
+  }
   const int h = blockIdx.x, wave = threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE, g = lane / 16, c = lane % 16;
   const int col0 = blockIdx.y * 64 + (wave & 1) * 32, row0 = blockIdx.z * 64 + (wave >> 1) * 32;
   if (col0 >= cols || row0 >= n_rows) return;
@@ -939,12 +964,10 @@ int tl_rotate_into(const void* q, int64_t q_stride, int head_width, int in_off, 
                    const int32_t* positions, const float* cos_t, const float* sin_t, float* out, int out_width,
                    int out_off, int n_tokens, int interleaved, int dtype, hipStream_t stream) {
   if (n_tokens <= 0 || rot == 0) return TL_OK;
-  if (rot < 0 || rdims < 0 || rdims % 2 || rdims > rot || heads <= 0 || in_off + rot > head_width ||
-      out_off + rot > out_width || (interleaved != 0 && interleaved != 1))
-    return TL_ERR_ARG;
-  TL_DISPATCH_T(dtype, hipLaunchKernelGGL(rotate_into_kernel<T>, dim3(n_tokens), dim3(kThreads), 0, stream,
-                                          (const T*)q, q_stride, head_width, in_off, rot, rdims, heads, positions, cos_t,
-                                          sin_t, out, out_width, out_off, interleaved);)
+  TL_DISPATCH_T(dtype, const Rotate<T> r = {(const T*)q, q_stride, head_width, in_off, rot, rdims, heads, positions, cos_t, sin_t, out,
+                                            out_width, out_off, interleaved};
+                if (!r.fits()) return TL_ERR_ARG;
+                hipLaunchKernelGGL(rotate_into_kernel<T>, dim3(n_tokens), dim3(kThreads), 0, stream, r);)
   return tl_launch_status();
 }
 
@@ -1058,27 +1081,35 @@ int tl_head_products(const void* in, int64_t in_stride, int in_head_width, const
   return tl_launch_status();
 }
 
-// bfloat16, many rows: w [heads, cols, inner]; inner a multiple of 8, operands 16-byte aligned.
+// bfloat16, many rows: w [heads, cols, inner]; inner a multiple of 8, operands 16-byte aligned.  rot > 0 (float32 results): the launch
+// also rotates the `rot` dims at rot_in of the rows of q into rot_out, as tl_rotate_into does.
 int tl_head_gemm(const void* in, int64_t in_stride, int in_head_width, const void* w, void* out, int64_t out_stride,
                  int out_head_width, int n_rows, int heads, int inner, int cols, const void* gate, int64_t gate_stride,
-                 int out_dtype, hipStream_t stream) {
+                 int out_dtype, int rot, const void* q, int64_t q_stride, int head_width, int rot_in, int rdims,
+                 const int32_t* positions, const float* cos_t, const float* sin_t, float* rot_out, int rot_width, int rot_off,
+                 int interleaved, hipStream_t stream) {
   if (n_rows <= 0) return TL_OK;
+  const Rotate<bf16_t> rotate = {(const bf16_t*)q, q_stride, head_width, rot_in, rot, rdims, heads, positions, cos_t, sin_t, rot_out,
+                                 rot_width, rot_off, interleaved};
+  if (rot && (out_dtype != 0 || !rotate.fits())) return TL_ERR_ARG;
   if (heads <= 0 || inner <= 0 || inner % 8 || cols <= 0 || inner > in_head_width || cols > out_head_width ||
-      in_stride % 8 || in_head_width % 8 || (n_rows + 63) / 64 > 65535 || (cols + 63) / 64 > 65535)
+      in_stride % 8 || in_head_width % 8 || (n_rows + 63) / 64 > 65535 || (cols + 63) / 64 >= 65535)
     return TL_ERR_ARG;
-  dim3 g(heads, (cols + 63) / 64, (n_rows + 63) / 64), b(kThreads);
+  dim3 g(heads, (cols + 63) / 64 + (rot ? 1 : 0), (n_rows + 63) / 64), b(kThreads);
   const bool few = n_rows <= kHeadFewRows;
   const int size = out_dtype == 0 ? 4 : 2;
   // results leave four columns at a time where rows, heads and the buffer are whole vectors of them
   const int whole = cols % 4 == 0 && out_stride % 4 == 0 && out_head_width % 4 == 0 && (uintptr_t)out % (4 * size) == 0;
-#define TL_HEAD_GEMM(TO, STEPS, SUMS)                                                                                   \
-  hipLaunchKernelGGL((head_gemm_bf16_kernel<TO, STEPS, SUMS>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width, \
+#define TL_HEAD_GEMM(TO, STEPS, SUMS, ROTATE)                                                                           \
+  hipLaunchKernelGGL((head_gemm_bf16_kernel<TO, STEPS, SUMS, ROTATE>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width, \
                      (const bf16_t*)w, (TO*)out, out_stride, out_head_width, n_rows, inner, cols, (const bf16_t*)gate,   \
-                     gate_stride, whole)
-  if (out_dtype == 0 && few) TL_HEAD_GEMM(float, 4, 4);
-  else if (out_dtype == 0) TL_HEAD_GEMM(float, 1, 1);
-  else if (out_dtype == 1 && few) TL_HEAD_GEMM(bf16_t, 4, 4);
-  else if (out_dtype == 1) TL_HEAD_GEMM(bf16_t, 1, 1);
+                     gate_stride, whole, rotate)
+  if (rot && few) TL_HEAD_GEMM(float, 4, 4, true);
+  else if (rot) TL_HEAD_GEMM(float, 1, 1, true);
+  else if (out_dtype == 0 && few) TL_HEAD_GEMM(float, 4, 4, false);
+  else if (out_dtype == 0) TL_HEAD_GEMM(float, 1, 1, false);
+  else if (out_dtype == 1 && few) TL_HEAD_GEMM(bf16_t, 4, 4, false);
+  else if (out_dtype == 1) TL_HEAD_GEMM(bf16_t, 1, 1, false);
   else return TL_ERR_ARG;
 #undef TL_HEAD_GEMM
   return tl_launch_status();

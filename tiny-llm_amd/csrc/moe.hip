@@ -126,14 +126,16 @@ __device__ __forceinline__ float activate(float v, int act) {
 
 // out[t * top + j, n] = act(sum_k a[t, k] * w[e(t, j)][n, k]); with the gated activation an expert's N rows are
 // (gate_0, up_0, gate_1, up_1, ...) and out[t * top + j, n] = silu(gate_n) * up_n for n < N / 2, formed from the
-// float32 sums (a wave's four dot products are then two gates and their two ups).
+// float32 sums (a wave's four dot products are then two gates and their two ups).  gate (optional, no activation): `per_gate` rows of
+// results lie beside one row of the gate, and what would be stored is multiplied by its sigmoid (a launch of its own took 2.5 us for 6 rows of 2,048).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void table_moe_up_kernel(const T* __restrict__ a, int64_t a_stride,
                                                                 const T* __restrict__ w,
                                                                 const int32_t* __restrict__ tokens,
                                                                 const int32_t* __restrict__ table, T* __restrict__ out,
                                                                 int top, int experts, int vocab, int N, int K, int act,
-                                                                int kCols) {
+                                                                int kCols, const T* __restrict__ gate, int64_t gate_stride,
+                                                                int per_gate) {
   const int row = blockIdx.x, t = row / top, j = row - t * top;
   const int wave = threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE;
   const int e = expert_of(tokens, table, t, j, top, vocab, experts);
@@ -161,7 +163,11 @@ __global__ __launch_bounds__(kThreads) void table_moe_up_kernel(const T* __restr
     for (int c = 0; c < 4; ++c) wr[c] = we + (int64_t)min(n + c, N - 1) * K;
     float v[4];
     dot_lanes4(arow, wr, K, lane, v);
-    if (lane < 4 && n + lane < N) out[(int64_t)row * N + n + lane] = from_f32<T>(activate(v[lane], act));
+    if (lane < 4 && n + lane < N) {
+      T y = from_f32<T>(activate(v[lane], act));
+      if (gate) y = from_f32<T>(to_f32(y) / (1.f + expf(-to_f32(gate[row / per_gate * gate_stride + (int64_t)(row % per_gate) * N + n + lane]))));
+      out[(int64_t)row * N + n + lane] = y;
+    }
   }
 }
 
@@ -892,9 +898,13 @@ int tl_table_moe_by_expert(int down, int n_tokens, int top, int N, int K, int ac
 
 // a: [n_tokens, K] (row stride a_stride); w: [experts, N, K]; table: int32 [vocab, top], looked up by tokens[t], or
 // (tokens null) by t itself; out: [n_tokens * top, N], with the activation `act` (0 none, 1 squared relu) applied.
+// gate (or null; no activation): [n_tokens * top / per_gate, per_gate * N], the results are multiplied by its sigmoid.
 int tl_table_moe_up(const void* a, int64_t a_stride, const void* w, const int32_t* tokens, const int32_t* table, void* out,
-                    int n_tokens, int top, int experts, int vocab, int N, int K, int act, int dtype, hipStream_t stream) {
+                    int n_tokens, int top, int experts, int vocab, int N, int K, int act, const void* gate, int64_t gate_stride,
+                    int per_gate, int dtype, hipStream_t stream) {
   if (n_tokens <= 0) return TL_OK;
+  if (gate && (act != kActNone || per_gate <= 0 || (int64_t)n_tokens * top % per_gate || gate_stride < (int64_t)per_gate * N))
+    return TL_ERR_ARG;
   if (top <= 0 || experts <= 0 || vocab <= 0 || N <= 0 || K <= 0 || a_stride < K || !a || !w || !table || !out ||
       (act != kActNone && act != kActRelu2 && act != kActSiluGate) || (act == kActSiluGate && (N & 1)) ||
       (!tokens && vocab < n_tokens) || (int64_t)n_tokens * top > 0x7fffffff || (N + kColsFew - 1) / kColsFew > 65535)
@@ -902,7 +912,7 @@ int tl_table_moe_up(const void* a, int64_t a_stride, const void* w, const int32_
   const int kCols = (int64_t)n_tokens * top <= kFewRows ? kColsFew : kColsWide;
   const int n_out = act == kActSiluGate ? N / 2 : N;      // output columns
   dim3 g(n_tokens * top, (n_out + kCols - 1) / kCols), b(kThreads);
-  const int nit = shared_up_pays(N, K, act) ? shared_vectors((int64_t)n_tokens * top, K, dtype, a_stride, a, w) : 0;
+  const int nit = !gate && shared_up_pays(N, K, act) ? shared_vectors((int64_t)n_tokens * top, K, dtype, a_stride, a, w) : 0;
   if (nit) {
     const int cols = (act == kActSiluGate ? 2 : 4) * kWaves;
     g = dim3(n_tokens * top < experts ? n_tokens * top : experts, (n_out + cols - 1) / cols);
@@ -918,10 +928,10 @@ int tl_table_moe_up(const void* a, int64_t a_stride, const void* w, const int32_
   }
   if (dtype == 0)
     hipLaunchKernelGGL(table_moe_up_kernel<float>, g, b, 0, stream, (const float*)a, a_stride, (const float*)w, tokens,
-                       table, (float*)out, top, experts, vocab, N, K, act, kCols);
+                       table, (float*)out, top, experts, vocab, N, K, act, kCols, (const float*)gate, gate_stride, per_gate);
   else if (dtype == 1)
     hipLaunchKernelGGL(table_moe_up_kernel<bf16_t>, g, b, 0, stream, (const bf16_t*)a, a_stride, (const bf16_t*)w, tokens,
-                       table, (bf16_t*)out, top, experts, vocab, N, K, act, kCols);
+                       table, (bf16_t*)out, top, experts, vocab, N, K, act, kCols, (const bf16_t*)gate, gate_stride, per_gate);
   else
     return TL_ERR_ARG;
   return tl_launch_status();

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -1304,13 +1304,7 @@ def latent_prepare(d: torch.Tensor, q_off: int, q_rank: int, w_q: Optional[torch
                                     c_int(ROPE_PAIRINGS.index(pairing)), c_int(_dt(d)), _stream()), "latent_prepare")
 
 
-def rotate_into(q: torch.Tensor, heads: int, head_width: int, in_off: int, rot: int, rdims: int,
-                positions: torch.Tensor,
-                cos: torch.Tensor, sin: torch.Tensor, out: torch.Tensor, out_off: int,
-                pairing: str = "half") -> torch.Tensor:
-    """out[t, h, out_off : out_off + rot] (float32) = the dims in_off : in_off + rot of head h of
-    row t of q, the first `rdims` of them rotated by the angle tables' row positions[t] (pairs
-    (i, i + rdims/2), or (2i, 2i + 1) with pairing "interleaved"), the others as they are."""
+def _rotation_fits(q, heads, head_width, rot, rdims, positions, cos, sin, out, pairing) -> None:
     _dev(q, positions, cos, sin, out)
     _need(pairing in ROPE_PAIRINGS, f"rotate_into: pairing {pairing!r} is not built")
     _rows_2d(q, "rotate_into input")
@@ -1322,6 +1316,17 @@ def rotate_into(q: torch.Tensor, heads: int, head_width: int, in_off: int, rot: 
             and sin.is_contiguous() and cos.shape == sin.shape and cos.shape[1] == rdims // 2
             and 0 < rdims <= rot and rdims % 2 == 0):
         _fail("rotate_into: shapes do not fit")
+
+
+def rotate_into(q: torch.Tensor, heads: int, head_width: int, in_off: int, rot: int, rdims: int,
+                positions: torch.Tensor,
+                cos: torch.Tensor, sin: torch.Tensor, out: torch.Tensor, out_off: int,
+                pairing: str = "half") -> torch.Tensor:
+    """out[t, h, out_off : out_off + rot] (float32) = the dims in_off : in_off + rot of head h of
+    row t of q, the first `rdims` of them rotated by the angle tables' row positions[t] (pairs
+    (i, i + rdims/2), or (2i, 2i + 1) with pairing "interleaved"), the others as they are."""
+    _rotation_fits(q, heads, head_width, rot, rdims, positions, cos, sin, out, pairing)
+    T = q.shape[0]
     _check(_lib().tl_rotate_into(_ptr(q), c_int64(q.stride(0)), c_int(head_width), c_int(in_off), c_int(rot),
                                  c_int(rdims), c_int(heads), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(out), c_int(out.shape[2]),
                                  c_int(out_off), c_int(T), c_int(ROPE_PAIRINGS.index(pairing)), c_int(_dt(q)), _stream()),
@@ -1516,10 +1521,12 @@ def head_products(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Opt
     return out
 
 
-def head_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+def head_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Optional[torch.Tensor] = None,
+              rotate: Optional[Tuple] = None) -> torch.Tensor:
     """out[t, h, :] = w[h] x[t, h, :] for every head in one launch on the matrix cores (bfloat16, any
     number of rows): x [T, heads, inner] and out [T, heads, cols] may be views into wider rows; w
-    [heads, cols, inner] contiguous; out bfloat16 or float32.  gate: as in `head_products`."""
+    [heads, cols, inner] contiguous; out bfloat16 or float32.  gate: as in `head_products`.  rotate (with float32 out): the
+    arguments of a `rotate_into` over the same rows and heads, which the launch then does as well."""
     _dev(x, w, out)
     T, H = x.shape[0], x.shape[1]
     cols, inner = w.shape[1], w.shape[2]
@@ -1529,10 +1536,19 @@ def head_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Optiona
             and tuple(out.shape[:2]) == (T, H) and x.shape[2] == inner and out.shape[2] == cols and inner % 8 == 0
             and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and out.dtype in (torch.bfloat16, torch.float32)):
         _fail("head_gemm: bfloat16 x [T, heads, inner] (inner and strides multiples of 8), w [heads, cols, inner], out [T, heads, cols]")
+    turn = (c_int(0), _ptr(None), c_int64(0), c_int(0), c_int(0), c_int(0), _ptr(None), _ptr(None), _ptr(None), _ptr(None), c_int(0),
+            c_int(0), c_int(0))
+    if rotate is not None:
+        q, heads, head_width, in_off, rot, rdims, positions, cos, sin, wide, wide_off, pairing = rotate
+        _rotation_fits(q, heads, head_width, rot, rdims, positions, cos, sin, wide, pairing)
+        _need(q.dtype == torch.bfloat16 and out.dtype == torch.float32 and heads == H and q.shape[0] == T,
+              "head_gemm: what is rotated is bfloat16, of the product's rows and heads, beside a float32 product")
+        turn = (c_int(rot), _ptr(q), c_int64(q.stride(0)), c_int(head_width), c_int(in_off), c_int(rdims), _ptr(positions), _ptr(cos),
+                _ptr(sin), _ptr(wide), c_int(wide.shape[2]), c_int(wide_off), c_int(ROPE_PAIRINGS.index(pairing)))
     _check(_lib().tl_head_gemm(_ptr(x, 16), c_int64(x.stride(0)), c_int(x.stride(1)), _ptr(w, 16), _ptr(out),
                                c_int64(out.stride(0)), c_int(out.stride(1)), c_int(T), c_int(H), c_int(inner),
                                c_int(cols), _ptr(gate), c_int64(gate.stride(0) if gate is not None else 0),
-                               c_int(_dt(out)), _stream()), "head_gemm")
+                               c_int(_dt(out)), *turn, _stream()), "head_gemm")
     return out
 
 
@@ -2191,12 +2207,13 @@ MOE_GATED = "swiglu"                         # `table_moe_up` only: an expert's 
 
 
 def table_moe_up(a: torch.Tensor, w: torch.Tensor, tokens: Optional[torch.Tensor], table: torch.Tensor, out: torch.Tensor,
-                 act: Optional[str] = None) -> torch.Tensor:
+                 act: Optional[str] = None, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[t * top + j] = act(w[table[tokens[t], j]] @ a[t]); a [T, K], w [E, N, K] of one type, table int32 [vocab, top],
     out contiguous [T * top, N].  tokens None: the table has a row per row of a (the experts a router chose).
     act None, "relu2" (the square of max(., 0)) or "swiglu": an expert's N rows are (gate_0, up_0, gate_1, up_1, ...) and
-    out [T * top, N / 2] = silu(gate) * up, formed from the float32 sums."""
-    _dev(a, w, tokens, table, out)
+    out [T * top, N / 2] = silu(gate) * up, formed from the float32 sums.  gate (without act): of a's type and as many elements as
+    out, a row for every so many rows of out; out is multiplied by its sigmoid, as `gate_rows` would."""
+    _dev(a, w, tokens, table, out, gate)
     _need(act in MOE_ACTIVATIONS or act == MOE_GATED, f"table_moe_up: activation {act!r} is not built")
     _rows_2d(a, "table_moe_up input")
     T, K = a.shape
@@ -2212,9 +2229,15 @@ def table_moe_up(a: torch.Tensor, w: torch.Tensor, tokens: Optional[torch.Tensor
         _need(tokens.numel() == T, "table_moe_up: one token id per row")
     else:
         _need(V >= T and table.is_contiguous(), "table_moe_up: without token ids the table has a row per row of the input")
+    if gate is not None:
+        _rows_2d(gate, "table_moe_up gate")
+        _need(act is None and gate.dtype == a.dtype and gate.shape[1] % N == 0 and gate.shape[0] * gate.shape[1] == T * top * N,
+              "table_moe_up: the gate is of the input's type, holds whole rows of the output, as many as there are, and allows no activation")
     _check(_lib().tl_table_moe_up(_ptr(a), c_int64(a.stride(0)), _ptr(w), _ptr(tokens), _ptr(table), _ptr(out), c_int(T),
                                   c_int(top), c_int(E), c_int(V), c_int(N), c_int(K),
-                                  c_int(2 if act == MOE_GATED else MOE_ACTIVATIONS[act]), c_int(_dt(a)), _stream()),
+                                  c_int(2 if act == MOE_GATED else MOE_ACTIVATIONS[act]), _ptr(gate),
+                                  c_int64(gate.stride(0) if gate is not None else 0),
+                                  c_int(gate.shape[1] // N if gate is not None else 1), c_int(_dt(a)), _stream()),
            "table_moe_up")
     return out
 

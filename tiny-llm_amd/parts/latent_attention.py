@@ -187,15 +187,17 @@ class LatentAttention(Mixer):
         few = T <= ops.HEAD_PRODUCT_ROWS and max(D, KR) <= ops.HEAD_PRODUCT_INNER
         gemm = self.dtype == torch.bfloat16 and q.stride(0) % 8 == 0     # one launch on the matrix cores
         many = gemm and not few
+        rotate = (q, H, D + R, D, R, self.rdims, ctx.positions, cos, sin, qa, KR, self.pairing) if R else None
         if few and self.keys_by_rows:
             ops.head_products(q3[:, :, :D], self.w_uk_few, qa[:, :, :KR])
         elif gemm:
-            ops.head_gemm(q3[:, :, :D], self.w_uk_t, qa[:, :, :KR])
+            ops.head_gemm(q3[:, :, :D], self.w_uk_t, qa[:, :, :KR], rotate=rotate)      # the rotation rides in the product
+            rotate = None
         else:
             for n in range(H):
                 ops.linear(q3[:, n, :D], self.w_uk_t[n], qa2[:, n * (KR + R):n * (KR + R) + KR])
-        if R:
-            ops.rotate_into(q, H, D + R, D, R, self.rdims, ctx.positions, cos, sin, qa, KR, self.pairing)
+        if rotate is not None:
+            ops.rotate_into(*rotate)
         mix = ops.scratch("latent_mix", (T, H, KR), self.dtype, dev)
         gate = down[:, self.g_off:self.g_off + H] if self.gate == "head" else None
         extra = dict(window=self.window, sinks=self.sinks)
@@ -233,9 +235,7 @@ class LatentAttention(Mixer):
         if few and KR >= 256:
             # a long inner size and few columns a head: a wave a group of four columns of one (token, head), its lanes
             # striding over the latent, fills the chip where a workgroup per 64 columns of a head leaves it idle
-            ops.table_moe_up(mix.view(T * H, KR), self.w_uv.view(H, V, KR), None, self.head_of_row, o.view(T * H, V))
-            if gate is not None:
-                ops.gate_rows(o, gate, o)
+            ops.table_moe_up(mix.view(T * H, KR), self.w_uv.view(H, V, KR), None, self.head_of_row, o.view(T * H, V), gate=gate)
         elif few:
             ops.head_products(mix, self.w_uv_few, o.view(T, H, V), gate)      # the gate rides in the product
         elif many:

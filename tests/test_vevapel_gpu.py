@@ -816,3 +816,51 @@ def test_delta_rule_in_chunks(dtype, H, G, D, V, taps, per_head, lens):
     assert (st.double().cpu() - S_all)[:, :H * D * V].abs().max() <= 2.4e-6 * S_all.abs().max()
     idle = [s for s in range(R + 2) if s not in slots or lens[slots.index(s)] == 0]
     assert torch.equal(st.cpu()[idle], state[idle]) and torch.equal(st.cpu()[:, H * D * V:], state[:, H * D * V:])
+
+
+@pytest.mark.parametrize("H,G,D,V,taps,lens", [(3, 3, 128, 128, 4, [40, 17, 33]), (4, 2, 64, 48, 4, [15, 31, 50]), (2, 1, 100, 37, 4, [49, 96])])
+def test_delta_rule_in_chunks_keeps_what_is_not_finite_behind_its_token(H, G, D, V, taps, lens):
+    """A NaN or an infinity in one token's q, k, v, beta or decay: what comes before the token, and every other request, keeps its
+    bits, and the same results and states are not finite as token by token."""
+    from tiny_llm_amd.engine.step import tile_lists
+    from tiny_llm_amd.kernels import ops
+    g = torch.Generator().manual_seed(D)
+    T, R, C = sum(lens), len(lens), 2 * G * D + H * V
+    p, a = torch.randn(T, C + H, generator=g), torch.randn(T, H * D, generator=g)
+    w, a_log = (torch.randn(C, taps, generator=g) * 0.5).cuda(), (torch.randn(H, generator=g) * 0.5).cuda()
+    dt_bias = (torch.randn(H * D, generator=g) - 2).cuda()
+    state = torch.randn(R, H * D * V + C * (taps - 1), generator=g) * 0.3
+    cu = [sum(lens[:i]) for i in range(R + 1)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    tiles, where, slots = [i32(x) for x in tile_lists(lens, ops.DELTA_CHUNK)], i32(cu), i32(list(range(R)))
+    rot = i32([r for r, n in enumerate(lens) for _ in range(n)])
+
+    def run(p, a, chunks):
+        p, a, st, out = p.cuda(), a.cuda(), state.cuda(), torch.full((T * H * V,), float("nan"), device="cuda")
+        if chunks:
+            ops.delta_chunks(p, 0, C, a, w, a_log, dt_bias, st, H * D * V, where, slots, tiles, out, H, G, D, V, taps, D ** -0.5)
+        else:
+            q, k, decay = torch.empty(3, T * H * D, device="cuda")
+            v, beta = torch.empty(T * H * V, device="cuda"), torch.empty(T * H, device="cuda")
+            ops.delta_prepare(p, 0, C, a, w, a_log, dt_bias, st, H * D * V, rot, where, slots, q, k, v, beta, decay, H, G, D, V, taps, D ** -0.5)
+            ops.delta_recurrence(q, k, v, beta, decay, st, where, slots, out, H, D, V)
+        return out.cpu().view(T, H * V), st.cpu()[:, :H * D * V]
+
+    clean, clean_state = run(p, a, True)
+    assert clean.isfinite().all()
+    for r, at in ((0, 7), (1, 14), (R - 1, lens[-1] - 1), (R - 1, lens[-1] - 2), (R - 1, 30)):
+        t = cu[r] + at
+        for value in (float("nan"), float("inf")):
+            for what, col in (("q", D // 2), ("k", G * D + 3), ("v", 2 * G * D + V + 5), ("beta", C + H - 1), ("decay", D + 1)):
+                if (what, value) in (("beta", float("inf")), ("decay", float("inf"))):
+                    continue                      # an open gate and a decay of nothing are finite
+                p2, a2 = p.clone(), a.clone()
+                (a2 if what == "decay" else p2)[t, col] = value
+                got, got_state = run(p2, a2, True)
+                want, want_state = run(p2, a2, False)
+                assert not want.isfinite().all()
+                assert torch.equal(got[:t], clean[:t]) and torch.equal(got[cu[r + 1]:], clean[cu[r + 1]:]), (r, at, what, value)
+                assert torch.equal(got.isfinite(), want.isfinite()), (r, at, what, value)
+                assert torch.equal(got_state.isfinite(), want_state.isfinite()), (r, at, what, value)
+                others = [i for i in range(R) if i != r]
+                assert torch.equal(got_state[others], clean_state[others])

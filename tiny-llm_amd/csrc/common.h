@@ -192,6 +192,32 @@ constexpr int kCT = 16;
 __host__ __device__ __forceinline__ int chunk_place(int t0, int r) { return t0 / kCT + r; }
 typedef unsigned int tl_u32x4 __attribute__((ext_vector_type(4)));
 
+// A product of a chunk's own: tokens in front of token s meet it with a zero, and zero times a number that is not finite is none.
+// hides_not_finite: x's numbers that are not finite become zero; true if the wave has any (uniform).  add_not_finite then adds them,
+// once the product has been made without them, where they belong.  x[j]: column lane % 16, token 4 (lane / 16) + j; b[j]: token
+// lane % 16 of the results, token 4 (lane / 16) + j of x; y: token lane % 16, columns 4 (lane / 16) + e.
+__device__ __forceinline__ bool hides_not_finite(f32x4& x) {
+  const float size = (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3]));
+  if (__builtin_amdgcn_ballot_w64(!(size < INFINITY)) == 0) return false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = fabsf(x[j]) < INFINITY ? x[j] : 0.f;
+  return true;
+}
+__device__ __forceinline__ void add_not_finite(f32x4& y, const f32x4& x, const f32x4& b, int lane) {
+  auto from = [](float v, int l) { return __uint_as_float(__builtin_amdgcn_ds_bpermute(l * 4, __float_as_uint(v))); };
+#pragma unroll 1
+  for (int s4 = 0; s4 < kCT; s4 += 4)             // tokens s4 + j
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float bs = from(b[j], s4 * 4 + lane % 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float xs = from(x[j], s4 * 4 + lane / 16 * 4 + e);
+        if (s4 + j <= lane % 16 && !(fabsf(xs) < INFINITY)) y[e] = fmaf(bs, xs, y[e]);
+      }
+    }
+}
+
 // v[t] summed over a row of sixteen lanes, t = 0 .. 15: lane l of the row gets the sum of v[l].  Lanes exchange halves of
 // what they hold: 15 exchanges for sixteen sums.
 __device__ __forceinline__ float scatter_sums(float* v, int l) {

@@ -297,8 +297,8 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
 // A, B and the solution of the first line for u = U0 - W S_0 (W and U0 by forward substitution, row by row as the recurrence
 // goes) do not depend on the state: delta_chunk_kernel makes them for all chunks at once.  What is left for
 // delta_chunk_scan_kernel to do in order are three products of 16 x dim (x vdim columns) a chunk.  Products of decays are
-// taken of the decays themselves (none exceeds one), never as quotients, so decays near zero lose nothing.  Within its chunk
-// a number that is not finite reaches the request's tokens ahead of it too.
+// taken of the decays themselves (none exceeds one), never as quotients, so decays near zero lose nothing.  A number
+// that is not finite reaches no token ahead of its own: B's zeros never meet it.
 // 1,944 tokens of six requests, the longest 801, 16 heads of 128 x 128: convolutions and decays 97 us and the recurrence 299,
 // now 46 and 79; one request of 2,047 tokens 102 and 704, now 45 and 101.  What bounds them: the first its convolutions' and
 // decays' functions; the second a chain of 0.75 us a chunk, of which the matrix instructions take a half.  Error against 64
@@ -565,14 +565,16 @@ __global__ __launch_bounds__(kScanThreads, AHEAD == 1 ? 5 : 3) void delta_chunk_
     meet();
     for (int c = 0; c < chunks; ++c) {
       meet();
-      const f32x4 U = u_of(c % 3), o = (os[c % 2][0][lane] + os[c % 2][1][lane]) + (os[c % 2][2][lane] + os[c % 2][3][lane]);
-      f32x4 y = zero, y2 = zero;                    // transposed: four columns a lane
+      const f32x4 u = u_of(c % 3), o = (os[c % 2][0][lane] + os[c % 2][1][lane]) + (os[c % 2][2][lane] + os[c % 2][3][lane]);
+      f32x4 U = u, y = zero, y2 = zero;             // transposed: four columns a lane
+      const bool hidden = hides_not_finite(U);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         y = __builtin_amdgcn_mfma_f32_16x16x4f32(U[j], b[j], y, 0, 0, 0);
         y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(U[j + 2], b[j + 2], y2, 0, 0, 0);
       }
       y = o + (y + y2);
+      if (hidden) add_not_finite(y, u, b, lane);
       b = b_at[step * min(c + 1, chunks - 1)];
       // a buffer that ends with the request's last token of the chunk: what lies behind is not stored, without a branch
       const int n = min(kCT, t1 - t0 - c * kCT);

@@ -818,10 +818,12 @@ def test_delta_rule_in_chunks(dtype, H, G, D, V, taps, per_head, lens):
     assert torch.equal(st.cpu()[idle], state[idle]) and torch.equal(st.cpu()[:, H * D * V:], state[:, H * D * V:])
 
 
-@pytest.mark.parametrize("H,G,D,V,taps,lens", [(3, 3, 128, 128, 4, [40, 17, 33]), (4, 2, 64, 48, 4, [15, 31, 50]), (2, 1, 100, 37, 4, [49, 96])])
+@pytest.mark.parametrize("H,G,D,V,taps,lens", [(3, 3, 128, 128, 4, [40, 17, 33]), (4, 2, 64, 48, 4, [15, 31, 50]), (2, 1, 100, 37, 4, [49, 96]),
+                                               (2, 1, 64, 64, 3, [40, 33]), (2, 2, 128, 64, 2, [16, 40]), (2, 2, 64, 64, 1, [16, 34])])
 def test_delta_rule_in_chunks_keeps_what_is_not_finite_behind_its_token(H, G, D, V, taps, lens):
     """A NaN or an infinity in one token's q, k, v, beta or decay: what comes before the token, and every other request, keeps its
-    bits, and the same results and states are not finite as token by token."""
+    bits, and the same results and states are not finite as token by token (an input that is behind the convolution's reach among
+    those that are)."""
     from tiny_llm_amd.engine.step import tile_lists
     from tiny_llm_amd.kernels import ops
     g = torch.Generator().manual_seed(D)

@@ -353,12 +353,15 @@ __global__ __launch_bounds__(kChunkThreads) void delta_chunk_kernel(
       for (int j = 0; j < BACK; ++j) x[j] = j >= kChunkTaps - taps ? sv[j - (kChunkTaps - taps)] : 0.f;
     }
 #pragma unroll
-    for (int t = 0; t < kCT; ++t) {
-      float acc = 0.f;
+    for (int t = 0; t < kCT; ++t) y[t] = 0.f;
 #pragma unroll
-      for (int j = 0; j < kChunkTaps; ++j) acc = fmaf(wt[j], x[t + j], acc);
-      y[t] = t < n ? silu(acc) : 0.f;
-    }
+    for (int j = 0; j < kChunkTaps; ++j)
+      if (j >= kChunkTaps - taps) {       // uniform: an input that no tap meets may be anything
+#pragma unroll
+        for (int t = 0; t < kCT; ++t) y[t] = fmaf(wt[j], x[t + j], y[t]);
+      }
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) y[t] = t < n ? silu(y[t]) : 0.f;
   };
   float y[kCT];
   const bool channel = tid < DP;

@@ -671,3 +671,46 @@ def test_time_mix_in_chunks(H, D, lens):
     assert (got.double() - S_all).abs().max() <= 1.8e-6 * S_all.abs().max()
     idle = [s for s in range(R + 2) if s not in slots or lens[slots.index(s)] == 0]
     assert torch.equal(st.cpu()[idle], state[idle]) and torch.equal(st.cpu()[:, floats:], state[:, floats:])
+
+
+@pytest.mark.parametrize("H,D,lens", [(3, 64, [40, 17, 33]), (2, 100, [15, 31, 50]), (2, 128, [16, 34])])
+def test_time_mix_in_chunks_keeps_what_is_not_finite_behind_its_token(H, D, lens):
+    """A NaN or an infinity in one token's r, k, v or decay: what comes before the token, and every other request, keeps its bits,
+    and the same results and states are not finite as token by token."""
+    from tiny_llm_amd.engine.step import tile_lists
+    from tiny_llm_amd.kernels import ops
+    g = torch.Generator().manual_seed(D)
+    T, R, S = sum(lens), len(lens), H * D
+    x, w0, u = torch.randn(T, 4 * S, generator=g), torch.randn(S, generator=g) * 0.5, torch.randn(S, generator=g)
+    state = torch.zeros(R, ops.time_mix_state_floats(H, D, D))
+    cu = [sum(lens[:i]) for i in range(R + 1)]
+    i32 = lambda y: torch.tensor(y, dtype=torch.int32, device="cuda")  # noqa: E731
+    tiles, where, slots = [i32(y) for y in tile_lists(lens, ops.TIME_MIX_CHUNK)], i32(cu), i32(list(range(R)))
+
+    def run(x, chunks):
+        st, out = state.cuda(), torch.full((T * S,), float("nan"), device="cuda")
+        args = (x.cuda(), 0, S, 2 * S, 3 * S, w0.cuda(), u.cuda(), st, where, slots)
+        if chunks:
+            ops.time_mix_chunks(*args, tiles, out, H, D, D)
+        else:
+            ops.time_mix_recurrence(*args, out, H, D, D)
+        return out.cpu().view(T, S), st.cpu()
+
+    clean, clean_state = run(x, True)
+    assert clean.isfinite().all()
+    for r, at in ((0, 7), (1, 14), (R - 1, lens[-1] - 1), (R - 1, lens[-1] - 2), (R - 1, 30)):
+        t = cu[r] + at
+        for value in (float("nan"), float("inf")):
+            for what, col in (("r", D // 2), ("k", S + 3), ("v", 2 * S + D + 5), ("decay", 3 * S + D + 1)):
+                if (what, value) == ("decay", float("inf")):
+                    continue                      # a decay to nothing is finite
+                x2 = x.clone()
+                x2[t, col] = value
+                got, got_state = run(x2, True)
+                want, want_state = run(x2, False)
+                assert not (want.isfinite().all() and want_state.isfinite().all())
+                assert torch.equal(got[:t], clean[:t]) and torch.equal(got[cu[r + 1]:], clean[cu[r + 1]:]), (r, at, what, value)
+                assert torch.equal(got.isfinite(), want.isfinite()), (r, at, what, value)
+                assert torch.equal(got_state.isfinite(), want_state.isfinite()), (r, at, what, value)
+                others = [i for i in range(R) if i != r]
+                assert torch.equal(got_state[others], clean_state[others])

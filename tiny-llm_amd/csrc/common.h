@@ -198,10 +198,9 @@ typedef unsigned int tl_u32x4 __attribute__((ext_vector_type(4)));
 // lane % 16 of the results, token 4 (lane / 16) + j of x; y: token lane % 16, columns 4 (lane / 16) + e.
 __device__ __forceinline__ bool hides_not_finite(f32x4& x) {
   const float size = (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3]));
-  if (__builtin_amdgcn_ballot_w64(!(size < INFINITY)) == 0) return false;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) x[j] = fabsf(x[j]) < INFINITY ? x[j] : 0.f;
-  return true;
+  for (int j = 0; j < 4; ++j) x[j] = fabsf(x[j]) < INFINITY ? x[j] : 0.f;      // (without a branch: products would move behind it)
+  return __builtin_amdgcn_ballot_w64(!(size < INFINITY)) != 0;
 }
 __device__ __forceinline__ void add_not_finite(f32x4& y, const f32x4& x, const f32x4& b, int lane) {
   auto from = [](float v, int l) { return __uint_as_float(__builtin_amdgcn_ds_bpermute(l * 4, __float_as_uint(v))); };

@@ -189,10 +189,11 @@ __global__ __launch_bounds__(kThreads) void time_mix_recurrence_kernel(
 //     S   = diag(P_16) S_0 + sum_s (w_(s+1) .. w_16 k_s) v_s^T
 // B and the decayed r and k (Q and K) do not depend on the state: time_mix_chunk_kernel makes them for all chunks at once, and
 // time_mix_scan_kernel walks a request's chunks.  Products of decays are taken of the decays themselves, never as quotients,
-// along a chunk in 64 bits, and so are B's sums; all else is float32.
-// 1,944 tokens of six requests, the longest 801, 32 heads of 64 x 64: 188 us token by token, now 36 and 35; one request of 2,047
-// tokens 460, now 35 and 75; heads of 128 x 128, half as many, 280, now 37 and 53.  The first kernel is bound by its vector
-// instructions, the second by a chain of 0.55 us a chunk.  Error against 64 bits (2-norm, 700 to 1,000 tokens): 9.1e-8, token
+// along a chunk in 64 bits, and so are B's sums; all else is float32.  A number that is not finite reaches no token ahead of its
+// own: B's zeros never meet it.
+// 1,944 tokens of six requests, the longest 801, 32 heads of 64 x 64: 188 us token by token, now 36 and 28; one request of 2,047
+// tokens 460, now 35 and 52; heads of 128 x 128, half as many, 280, now 37 and 48.  The first kernel is bound by its vector
+// instructions, the second by a chain of 0.4 us a chunk.  Error against 64 bits (2-norm, 700 to 1,000 tokens): 9.1e-8, token
 // by token 9.5e-8; 128 x 128 9.2e-8 and 1.01e-7 (with B in float32 1.02e-7 and 1.05e-7, 8 us less).
 constexpr int kMaxChunkDim = 128;      // channels and value columns a head may have here
 
@@ -344,17 +345,34 @@ __global__ __launch_bounds__(kScanThreads) void time_mix_scan_kernel(
   if (rg == 4) {
     const int row_bytes = heads * vdim * 4, b_at = (8 * DP + 4 * vp + lane) * 16;
     const int to = lane % 16 * row_bytes + (vt * 16 + q * 4) * 4;
-    __amdgpu_buffer_rsrc_t from = buffer(0);
-    f32x4 v = load(from, v_at, 0), b = load(from, b_at, 0);
-    for (int c = 0; c < chunks; ++c) {
-      f32x4 own[4];
+    struct Own {
+      f32x4 v, b;
+    };
+    auto request = [&](Own& x, int c) {
+      const __amdgpu_buffer_rsrc_t from = buffer(c);
+      x.v = load(from, v_at, 0);
+      x.b = load(from, b_at, 0);
+    };
+    // Two chunks ahead: with one, what is done here between a chunk's values and the next request is on the way of every chunk
+    // (2,047 tokens of 32 heads of 64 x 64, both kernels: 110 us with the products alone there, 120 with the look for numbers
+    // that are not finite as well, 87 so).
+    Own op[2];
+    request(op[0], 0);
+    request(op[1], 1);
+    auto chunk = [&](Own& x, int c) {
+      f32x4 own[4], v = x.v;
+      const bool hidden = hides_not_finite(v);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], b[j], zero, 0, 0, 0);
-      from = buffer(c + 1);
-      v = load(from, v_at, 0);
-      b = load(from, b_at, 0);
+      for (int j = 0; j < 4; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], x.b[j], zero, 0, 0, 0);
+      request(x, c + 2);
+      __builtin_amdgcn_sched_barrier(0);
       meet();
-      const f32x4 y = ((os[c % 2][0][lane] + os[c % 2][1][lane]) + (os[c % 2][2][lane] + os[c % 2][3][lane])) + ((own[0] + own[1]) + (own[2] + own[3]));
+      f32x4 y = ((os[c % 2][0][lane] + os[c % 2][1][lane]) + (os[c % 2][2][lane] + os[c % 2][3][lane])) + ((own[0] + own[1]) + (own[2] + own[3]));
+      if (hidden) {                               // v and b once more: to keep them would cost registers and copies in every chunk
+        Own again;
+        request(again, c);
+        add_not_finite(y, again.v, again.b, lane);
+      }
       // a buffer that ends with the request's last token of the chunk: what lies behind is not stored, without a branch
       const int n = min(kCT, t1 - t0 - c * kCT);
       const __amdgpu_buffer_rsrc_t rows =
@@ -366,7 +384,13 @@ __global__ __launch_bounds__(kScanThreads) void time_mix_scan_kernel(
         for (int j = 0; j < 4; ++j)
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[j]), rows, vt * 16 + q * 4 + j < vdim ? to + j * 4 : -4, 0, 0);
       }
+    };
+    int c = 0;
+    for (; c + 2 <= chunks; c += 2) {
+      chunk(op[0], c);
+      chunk(op[1], c + 1);
     }
+    if (c < chunks) chunk(op[0], c);
     return;
   }
   float* Sg = state + (int64_t)slots[r] * state_stride + ((int64_t)h * kSlice * vdim + min(col, vdim - 1)) * P + rg * NT * 4 + q;

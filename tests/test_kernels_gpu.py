@@ -1531,11 +1531,11 @@ def test_router_by_lanes_gives_the_bits_of_the_general_form(experts, top, groups
 
 
 @pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 40, 64, 65, 130, 300, 1030])
-@pytest.mark.parametrize("F,K", [(33, 72), (1408, 2048), (704, 512)])
+@pytest.mark.parametrize("F,K", [(33, 72), (1408, 2048), (704, 512), (1024, 2048), (333, 4104)])
 def test_gated_epilogues_leave_the_bits_of_the_kernels_behind(M, F, K):
     """The clamped unit and the gelu unit in a product's epilogue, over few rows, split inner sizes and tiles, against the same
-    product stored in bfloat16 and the units' own kernels: the same bits, infinities and NaN among them.  (At sizes where a stored
-    product of up to 8 rows takes eight columns a workgroup, whose sums run in another order, there is nothing to compare.)"""
+    product stored in bfloat16 and the units' own kernels: the same bits, infinities and NaN among them, also where a product of up
+    to 8 rows takes eight columns a workgroup (inner sizes from 2,048 on, up to 2,048 columns)."""
     k, g = ops(), torch.Generator().manual_seed(M + F)
     a = (torch.randn(M, K, generator=g) * 2).to(torch.bfloat16).cuda()
     gate, up = ((torch.randn(F, K, generator=g) / K ** 0.5 * 3).to(torch.bfloat16).cuda() for _ in range(2))

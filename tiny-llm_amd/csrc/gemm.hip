@@ -1941,7 +1941,7 @@ __device__ __forceinline__ bf16x8 skinny_operand(const SkinnyChunk<PRO_NORM>& c,
 // DEEP: two register stages also with one tile, for long inner sizes, where a wave works through
 // several stages and the chain of their memory round trips sets the kernel's duration.
 //
-// HALF (at most 8 activation rows, one tile, no prologue): a workgroup owns 8 columns only, so that
+// HALF (at most 8 activation rows, one tile, no prologue, no SiLU-gate): a workgroup owns 8 columns only, so that
 // a matrix with few rows still gives every compute unit a workgroup; what a workgroup can have in
 // flight, not the memory system, bounds these kernels.  The 16 x 16 MFMA tile is then used as two
 // 8 x 8 tiles that split k: weight row i of the operand is column i % 8 at k offset (i / 8) * 32,
@@ -1950,7 +1950,7 @@ __device__ __forceinline__ bf16x8 skinny_operand(const SkinnyChunk<PRO_NORM>& c,
 // instruction reads whole 128-byte lines of 8 weight rows.
 template <int MT, int CT, bool DEEP, typename TO, int PRO, int SWIGLU, bool HALF>
 __device__ __forceinline__ void skinny_product(const SkinnyArgs& p) {
-  static_assert(!HALF || (MT == 1 && CT == 1 && PRO == PRO_NONE && !SWIGLU), "HALF: one plain tile");
+  static_assert(!HALF || (MT == 1 && CT == 1 && PRO == PRO_NONE && SWIGLU != 1), "HALF: one plain tile");
   constexpr int COLS = HALF ? 8 : S_COLS;          // columns of a tile that are outputs
   constexpr int KW = HALF ? 64 : 32;               // k covered by one MFMA
   constexpr int KBLK = 4 * KW;                     // k covered by a block of four MFMAs
@@ -2173,6 +2173,10 @@ __device__ __forceinline__ void skinny_product(const SkinnyArgs& p) {
       for (int wv = 0; wv < S_WAVES; ++wv) {
         gv += part[wv * TILES + tile][nn][m_local];
         uv += part[wv * TILES + tile][nn + 1][m_local];
+        if constexpr (HALF) {
+          gv += part[wv * TILES + tile][nn + 8][m_local + 8];
+          uv += part[wv * TILES + tile][nn + 9][m_local + 8];
+        }
       }
       out[(int64_t)m * p.ldo + n / 2] = from_f32<TO>(gated_pair<SWIGLU>(gv * scale, uv * scale, p.gate));
     } else {
@@ -2265,12 +2269,14 @@ static int skinny_cols_wg_tiles(int N, int ct) {
 
 // 8 columns a workgroup: for at most 8 rows and an inner size that gives every wave at least
 // one block of four MFMAs, where that still gives no more workgroups than there are compute
-// units (measured: otherwise it is slower).
+// units (measured: otherwise it is slower).  With the clamped and the gelu unit too, whose stored products took it: their bits, and
+// 6 rows by 512 pairs of inner size 4,096 8.6 us in 16 columns, 6.3 so (stored, with the unit's own kernel, 7.8); 1,024 pairs 7.5 and
+// 7.6 (9.3).  SiLU products keep the order of sums that they have always had.
 static bool skinny_half(int M, int N, int K) { return M <= 8 && K >= 2048 && (N + 7) / 8 <= 256; }
 
 template <int MT, int CT, typename TO, int PRO, int SWIGLU>
 static int launch_skinny_tile(const SkinnyArgs& p, hipStream_t stream) {
-  if constexpr (MT * CT == 1 && PRO == PRO_NONE && !SWIGLU) {
+  if constexpr (MT * CT == 1 && PRO == PRO_NONE && SWIGLU != 1) {
     if (skinny_half(p.M, p.N, p.K)) {
       if (p.K > 4096) return launch_skinny_deep<MT, CT, true, TO, PRO, SWIGLU, true>(p, stream);
       return launch_skinny_deep<MT, CT, false, TO, PRO, SWIGLU, true>(p, stream);

@@ -2,6 +2,7 @@
 (tests/plain_fofapel.py): each mechanism alone, every way of cutting the work, pages and state slots
 used again, captured steps, long decoding, generation through the entry point, and keys that a
 crafted query singles out at the places where an index can be off by one."""
+import copy
 import json
 import os
 import subprocess
@@ -714,3 +715,22 @@ def test_time_mix_in_chunks_keeps_what_is_not_finite_behind_its_token(H, D, lens
                 assert torch.equal(got_state.isfinite(), want_state.isfinite()), (r, at, what, value)
                 others = [i for i in range(R) if i != r]
                 assert torch.equal(got_state[others], clean_state[others])
+
+
+def test_float32_rows_have_the_same_bits_in_every_step(tmp_path):
+    """float32, heads of 64: requests of up to 200 tokens alone and whole, then all in one step, in portions, with their tails one
+    by one and beside each other, eagerly and captured: every row's logits bit for bit the same."""
+    cfg, block = copy.deepcopy(CONFIGS["A"])
+    for layer in cfg["layers"]:
+        layer["mixer"]["right"]["dim"] = 64
+    folder, _ = make_folder(tmp_path, cfg, seed=11)
+    reqs = {f"r{i}": random_tokens(n, cfg["vocab"], 100 * i) for i, n in enumerate([70, 133, 33, 200, 97, 64, 8, 1])}
+    runner = make_runner(folder, "float32", block, 1024, max_seqs=8)
+    whole = [{"id": rid, "tokens": toks, "want": list(range(len(toks)))} for rid, toks in reqs.items()]
+    rows = lambda steps, out: {at: out[s][i] for s, where in traces.rows_of(steps).items() for i, at in enumerate(where)}  # noqa: E731
+    alone = rows(traces.whole(reqs), replay(runner, traces.whole(reqs)))
+    for steps in ([{"step": 0, "entries": whole, "end": list(reqs)}], traces.portions(reqs), traces.tail_one_by_one(reqs),
+                  traces.mixed(reqs, seed=0)[0]):
+        for use_graph in (False, True, True):
+            got = rows(steps, replay(runner, steps, use_graph))
+            assert set(got) == set(alone) and all(torch.equal(got[at], alone[at]) for at in alone)

@@ -2,6 +2,7 @@
 (tests/plain_vevapel.py): each mechanism alone, every way of cutting the work, pages and state slots
 used again, captured steps, long decoding, generation through the entry point, and keys that a
 crafted query singles out at the places where an index can be off by one."""
+import copy
 import json
 import os
 import subprocess
@@ -866,3 +867,22 @@ def test_delta_rule_in_chunks_keeps_what_is_not_finite_behind_its_token(H, G, D,
                 assert torch.equal(got_state.isfinite(), want_state.isfinite()), (r, at, what, value)
                 others = [i for i in range(R) if i != r]
                 assert torch.equal(got_state[others], clean_state[others])
+
+
+def test_float32_prompts_have_the_same_bits_alone_and_in_one_step(tmp_path):
+    """float32, recurrent heads of 64 x 64: prompts of 33 to 200 tokens alone, then all in one step, then beside decoded tokens of
+    two of them: every row of a prompt bit for bit the same."""
+    cfg, block = copy.deepcopy(CONFIGS["A"])
+    for layer in cfg["layers"]:
+        if "conv" in layer["mixer"]:
+            layer["mixer"]["dim"] = layer["mixer"]["vdim"] = 64
+    folder, _ = make_folder(tmp_path, cfg, seed=11)
+    reqs = {f"r{i}": random_tokens(n, cfg["vocab"], 100 * i) for i, n in enumerate([70, 133, 33, 200, 97, 64])}
+    runner = make_runner(folder, "float32", block, 1024, max_seqs=6)
+    whole = [{"id": rid, "tokens": toks, "want": list(range(len(toks)))} for rid, toks in reqs.items()]
+    alone = replay(runner, traces.whole(reqs))
+    together = replay(runner, [{"step": 0, "entries": whole, "end": list(reqs)}])
+    assert torch.equal(together[0], torch.cat([alone[i] for i in range(6)]))
+    beside = [{"step": 0, "entries": whole[:2], "end": []},
+              {"step": 1, "entries": [{"id": e["id"], "tokens": [5], "want": []} for e in whole[:2]] + whole[2:], "end": list(reqs)}]
+    assert torch.equal(replay(runner, beside)[1], torch.cat([alone[i] for i in range(2, 6)]))

@@ -147,7 +147,8 @@ class ChannelDelta(Mixer):
                                       ctx.state_slots, self.taps)
             return self._project_out(z, residual)
         o = ops.scratch("delta_o", (T * H * V,), torch.float32, dev)
-        if ops.delta_chunks_pay(T, ctx.num_requests, D, V, self.taps):
+        # In float32 a row's bits do not depend on what else its step holds, so every step goes token by token there.
+        if self.dtype == torch.bfloat16 and ops.delta_chunks_pay(T, ctx.num_requests, D, V, self.taps):
             ops.delta_chunks(p, 0, self.b_off, a, self.conv_w, self.a_log, self.dt_bias, state, self.state_size,
                              ctx.cu_seqlens_q, ctx.state_slots, ctx.attention_tiles(ops.DELTA_CHUNK), o, H, KH, D, V,
                              self.taps, D ** -0.5, self.per_head)

@@ -101,7 +101,8 @@ class TimeMix(Mixer):
         act = ops.tanh_rows(low, ops.scratch("time_mix_low_act", (T, self.rank), self.dtype, dev))
         ops.linear(act, self.w2, x[:, 3 * seg:3 * seg + S])
         o = ops.scratch("time_mix_o", (T * S,), torch.float32, dev)
-        if not single and ops.time_mix_chunks_pay(T, ctx.num_requests, self.head_dim, self.head_dim):
+        # In float32 a row's bits do not depend on what else its step holds, so every step goes token by token there.
+        if self.dtype == torch.bfloat16 and not single and ops.time_mix_chunks_pay(T, ctx.num_requests, self.head_dim, self.head_dim):
             ops.time_mix_chunks(x, 0, seg, 2 * seg, 3 * seg, self.w0, self.u, state, ctx.cu_seqlens_q, ctx.state_slots,
                                 ctx.attention_tiles(ops.TIME_MIX_CHUNK), o, self.num_heads, self.head_dim, self.head_dim)
         else:

@@ -135,3 +135,37 @@ def test_tiles_through_registers_and_few_rows_of_tiles_stand_in_columns(tiles_m)
     columns = [(m, n) for n in range(5) for m in range(tiles_m)]
     assert _places(tiles_m, 5, 0) == columns
     assert (_places(tiles_m, 5, 1) == columns) == (tiles_m < 8)
+
+
+def test_time_mix_runs_in_chunks_where_its_longest_portion_pays_for_them():
+    """The steps beside the rule, and sizes that the chunks do not take."""
+    pays = lambda lens, heads=32, dim=64: ops.time_mix_chunks_pay(sum(lens), len(lens), max(lens), heads, dim, dim)  # noqa: E731
+    for lens in ([48] * 8, [48] * 64, [30] * 32, [31] * 16, [1] * 40 + [32] * 3, [1] * 64, [1]):      # chunks took 1.1 to 2.2 times as long
+        assert not pays(lens), lens
+    for lens in ([64], [2047], [67, 801, 143, 411, 205, 317], [1] * 8 + [512], [1] * 64 + [512], [1] * 64 + [1024]):
+        assert pays(lens), lens
+    assert pays([24] * 16, 16, 128) and pays([31] * 16, 16, 128) and not pays([24] * 8, 8, 128) and not pays([1] * 256, 16, 128)
+    assert not pays([2047], 16, 32) and not pays([2047], 16, 129)
+
+
+def test_a_step_is_known_by_the_forms_its_parts_choose():
+    """Parts that choose a form by a step's own sizes are asked, those within a parallel mixer too, and no others."""
+    from tiny_llm_amd.engine.step import StepContext, StepSizes
+    from tiny_llm_amd.models.decoder import Decoder
+    from tiny_llm_amd.parts import base, parallel
+
+    class ByLength(base.Mixer):
+        def form(self, sizes):
+            return sizes.longest > 10
+
+    plain, chooses = base.Mixer("a", None, None), ByLength("b", None, None)
+    side = object.__new__(parallel.ParallelMixer)
+    side.branches = [plain, chooses]
+    d = object.__new__(Decoder)
+    d._formed, d.parts = None, lambda: [plain, chooses, plain, side]
+    assert d.forms(StepSizes(40, 4, 10)) == (False, (None, False)) and d.forms(StepSizes(40, 2, 30)) == (True, (None, True))
+    d._formed, d.parts = None, lambda: [plain]
+    assert d.forms(StepSizes(40, 4, 10)) == ()
+    bare = dict.fromkeys(("tokens", "positions", "req_of_token", "cu_seqlens_q", "seq_lens", "state_slots", "logit_rows", "block_tables", "slot_mappings"))
+    assert StepContext(num_tokens=9, num_requests=2, max_q_len=8, **bare).sizes == (9, 2, 8)
+    assert StepContext(num_tokens=16, num_requests=2, max_q_len=16, sizes=StepSizes(9, 2, 8), **bare).sizes == (9, 2, 8)

@@ -16,7 +16,8 @@ separators (tiny_llm/ops/details.hpp:19-36).
 
 A step runs eagerly or as a HIP graph.  A graph is captured per shape of step:
 decode-only steps by (requests, bound on the context), other steps by capacities
-(tokens, requests, wanted rows) to which the step is padded: padding tokens write
+(tokens, requests, wanted rows) to which the step is padded, and by what the model's parts
+choose by the step's own sizes (`Part.form`): padding tokens write
 no cache slot, padding query tiles hold no token, padding rows of the output are
 dropped.  Eager and captured steps share the layout routine, the model code and
 the sampler; a captured step only has its sizes rounded up and its buffers static.
@@ -28,7 +29,7 @@ from __future__ import annotations
 import gc
 from collections import OrderedDict
 from dataclasses import dataclass, field
-from typing import Dict, Hashable, List, Optional, Sequence, Tuple
+from typing import Dict, Hashable, List, NamedTuple, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -56,6 +57,13 @@ class SampleSpec:
     counter: int = 0
 
 
+class StepSizes(NamedTuple):
+    """What a step brings, padding left out."""
+    tokens: int
+    requests: int
+    longest: int                    # the most tokens one of its requests brings
+
+
 @dataclass
 class StepContext:
     """Who is in the batch and where each token sits; device tensors are int32.
@@ -78,11 +86,18 @@ class StepContext:
     slots_host: List[int] = field(default_factory=list)
     max_q_len: int = 0
     max_seq_len: int = 0
+    # by what a part chooses between forms of its work (`Part.form`): of a captured step, those of the step it was made
+    # for, and it is replayed for steps of the same forms only
+    sizes: Optional[StepSizes] = None
     block_size: int = 0
     static: bool = False            # a captured step: nothing may be built on the host any more
     logits_all_rows: bool = False   # logit_rows is 0, 1, 2, ...: every token's logits, in order (no gather needed)
     _tiles: Dict[int, tuple] = field(default_factory=dict)
     _on_new_width = None            # told when a tile width is asked for the first time
+
+    def __post_init__(self):
+        if self.sizes is None:
+            self.sizes = StepSizes(self.num_tokens, self.num_requests, self.max_q_len)
 
     @property
     def decode_only(self) -> bool:
@@ -541,6 +556,7 @@ class ModelRunner:
                 bound = max(bound, max(new_lens))
                 key = ("decode", R, bound, samples is not None)
                 caps = (R, R, R, 1, bound)
+                sizes = StepSizes(R, R, 1)
             else:
                 T_cap = token_capacity(T, self.max_tokens)
                 R_cap = min(power_of_two_at_least(R), max(self.cache.max_seqs, R))
@@ -548,11 +564,12 @@ class ModelRunner:
                 n_cap = R_cap if n_out <= R_cap and samples is not None else T_cap
                 # the bound on the context decides whether attention shares a tile's keys out
                 bound = max(min(max(512, power_of_two_at_least(max(new_lens))), max(self.max_model_len, 1)), max(new_lens))
-                key = ("mixed", T_cap, R_cap, n_cap, bound, samples is not None)
+                sizes = StepSizes(T, R, max(len(r.tokens) for r in rows))
+                key = ("mixed", T_cap, R_cap, n_cap, bound, samples is not None, self.decoder.forms(sizes))
                 caps = (T_cap, R_cap, n_cap, T_cap, bound)
             sg = self._step_graph(key)
             if sg is None:
-                sg = self._graphs[key] = StepGraph(self, *caps, sampling=samples is not None)
+                sg = self._graphs[key] = StepGraph(self, *caps, sampling=samples is not None, sizes=sizes)
                 while len(self._graphs) > self.MAX_STEP_SHAPES:
                     self._graphs.popitem(last=False)        # no capture is under way here: it may be released
             logits, toks = sg.run(rows, samples, n_out)
@@ -577,7 +594,7 @@ class ModelRunner:
 class StepGraph:
     """Static buffers and the captured HIP graph of steps of one shape: capacities of T tokens,
     R requests and n_out wanted rows, `max_q_len` 1 (decode: row i is request i) or more, contexts
-    within `max_seq_len`.
+    within `max_seq_len`, the forms that the parts choose by `sizes`.
 
     The block-table width is fixed at its maximum.  The first run of a shape executes eagerly on the
     static buffers (kernels configure themselves, the workspace grows, the tile widths the kernels
@@ -586,8 +603,9 @@ class StepGraph:
     (a part asks for something that was not laid out) keeps running eagerly."""
 
     def __init__(self, runner: ModelRunner, T: int, R: int, n_out: int, max_q_len: int, max_seq_len: int,
-                 sampling: bool):
+                 sampling: bool, sizes: StepSizes):
         self.runner = runner
+        self.sizes = sizes
         self.T, self.R, self.n_out = T, R, n_out
         self.max_q_len, self.max_seq_len, self.sampling = max_q_len, max_seq_len, sampling
         self.graph: Optional[torch.cuda.CUDAGraph] = None
@@ -611,7 +629,7 @@ class StepGraph:
         self.dev = torch.zeros(self.layout.total, dtype=torch.int32, device=runner.device)
         self.np = self.host.numpy()
         self.ctx = self.layout.context(self.dev, cm.block_size, q_lens=[], context_lens=[], slots_host=[],
-                                       max_q_len=self.max_q_len, max_seq_len=self.max_seq_len)
+                                       max_q_len=self.max_q_len, max_seq_len=self.max_seq_len, sizes=self.sizes)
         # decode with a wanted row per request: row i of the logits is token i (padding rows, which would
         # point at row 0, are dropped by the caller either way), so the head needs no gather of rows
         self.ctx.logits_all_rows = self.max_q_len == 1 and self.n_out == self.R == self.T

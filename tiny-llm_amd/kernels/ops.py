@@ -2054,11 +2054,20 @@ TIME_MIX_CHUNK = 16              # tokens of a chunk of the chunked form
 TIME_MIX_CHUNK_MAX_DIM = 128     # its heads' channels and value columns
 
 
-def time_mix_chunks_pay(n_tokens: int, n_requests: int, dim: int, vdim: int) -> bool:
-    """Whether a step's recurrence runs in chunks (`time_mix_chunks`) or token by token.  32 heads of 64 x 64: 8 requests of
-    16 and 32 tokens 14 and 21 us in chunks, 9 and 16 by tokens; 64 of 13 and 16: 64 and 64, 43 and 45; 40 of one token beside 3
-    of 32: 49 and 21; one of 48, 64 and 2,047: 10, 11 and 110, 11, 14 and 460; six of 67 to 801 71 and 188."""
-    return 32 < dim <= TIME_MIX_CHUNK_MAX_DIM and vdim <= TIME_MIX_CHUNK_MAX_DIM and n_tokens >= 28 * n_requests + 36
+def time_mix_chunks_pay(n_tokens: int, n_requests: int, longest: int, heads: int, dim: int, vdim: int) -> bool:
+    """Whether a step's recurrence runs in chunks (`time_mix_chunks`) or token by token.  Token by token it is a chain of 0.2 us a
+    token of the longest request (0.3 with heads of 128), in chunks of 0.02; a request costs chunks more, whose two kernels
+    both go through its 16-token pieces (0.75 us against 0.3, 16 heads of 64 x 64; its state moves in narrower pieces), and
+    with heads of 128 a token of any request costs them 0.05 us less.  1,002 steps (1 to 256 requests: equal portions, one or two
+    portions beside single tokens, any mix; 1 to 64 heads of 33 to 128): the sum of what the choice loses against the better
+    form is 0.2 % of their times, and in three of them chunks are chosen where they are more than 3 % slower (5, 4 and 18 %).
+    32 heads of 64 x 64, chunks and tokens: 8 requests of 48 tokens 26 and 21 us, 64 of 48 119 and 108, one of 64 12 and 15, of
+    2,047 89 and 459, six of 67 to 801 65 and 184, 8 and 64 single tokens beside a portion of 512 44 and 119, 86 and 134."""
+    if not (32 < dim <= TIME_MIX_CHUNK_MAX_DIM and vdim <= TIME_MIX_CHUNK_MAX_DIM):
+        return False
+    if dim <= 64:
+        return 16 * (longest - 36) >= 3 * heads * n_requests
+    return 16 * (longest - 64) >= heads * (4.5 * n_requests - 0.3 * n_tokens)
 
 
 def time_mix_chunks(x: torch.Tensor, r_off: int, k_off: int, v_off: int, w_off: int, w0: torch.Tensor, u: torch.Tensor,

@@ -74,6 +74,7 @@ class Decoder:
         self.states: List[Dict[str, torch.Tensor]] = [{} for _ in spec.plan]
         self.embedding_state: Optional[torch.Tensor] = None     # if the embedding keeps per-request state
         self._graph_safe: Optional[bool] = None
+        self._formed: Optional[List[Part]] = None
         self._graph_runs: Optional[List[tuple]] = None
 
     # ---------------------------------------------------------------- declarations
@@ -94,6 +95,12 @@ class Decoder:
             parts += [getattr(p, "position", None) for p in parts]
             self._graph_safe = all(p.graph_safe for p in parts if p is not None)
         return self._graph_safe
+
+    def forms(self, sizes) -> tuple:
+        """What the parts choose by a step's own sizes (`Part.form`); empty where none does."""
+        if self._formed is None:
+            self._formed = [p for p in self.parts() if type(p).form is not Part.form]
+        return tuple(p.form(sizes) for p in self._formed)
 
     def weight_specs(self) -> List[WeightSpec]:
         specs: List[WeightSpec] = []

@@ -23,7 +23,7 @@ Calling conventions
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Any, Callable, Dict, List, Optional, Tuple
+from typing import Any, Callable, Dict, Hashable, List, Optional, Tuple
 
 import torch
 
@@ -133,6 +133,12 @@ class Part:
 
     def state_spec(self) -> Optional[StateSpec]:
         """Per-request memory of fixed size this part needs (None: none)."""
+        return None
+
+    def form(self, sizes) -> Hashable:
+        """What this part chooses by a step's own sizes (`sizes.tokens`, `sizes.requests`, `sizes.longest`) and not by the
+        capacities of the step it runs in, as `forward` does by `ctx.sizes`.  A captured step is replayed only for steps for
+        which every part's answer is that of the step it was captured for."""
         return None
 
 

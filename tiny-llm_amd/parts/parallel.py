@@ -59,6 +59,9 @@ class ParallelMixer(Mixer):
         parts = list(self.branches) + [getattr(m, "position", None) for m in self.branches]
         return all(p.graph_safe for p in parts if p is not None)
 
+    def form(self, sizes):
+        return tuple(m.form(sizes) for m in self.branches)
+
     def weights(self) -> List[WeightSpec]:
         return [w for m in self.branches for w in m.weights()]
 

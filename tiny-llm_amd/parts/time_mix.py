@@ -80,6 +80,12 @@ class TimeMix(Mixer):
         # [S in the recurrence kernel's layout | the last token's h], rows a multiple of four floats
         return StateSpec((-(-(self.s_floats + self.hidden_size) // 4) * 4,), torch.float32)
 
+    def form(self, sizes):
+        """Whether the recurrence runs in chunks.  In float32 a row's bits do not depend on what else its step holds, so every
+        step goes token by token there."""
+        return self.dtype == torch.bfloat16 and ops.time_mix_chunks_pay(sizes.tokens, sizes.requests, sizes.longest, self.num_heads,
+                                                                        self.head_dim, self.head_dim)
+
     def forward(self, h, ctx, cache, state, residual):
         T, dev, S, seg = h.shape[0], h.device, self.size, self.seg
         mixes = ops.scratch("shift_mixes", (len(self.MIXES), T, self.hidden_size), self.dtype, dev)
@@ -101,8 +107,7 @@ class TimeMix(Mixer):
         act = ops.tanh_rows(low, ops.scratch("time_mix_low_act", (T, self.rank), self.dtype, dev))
         ops.linear(act, self.w2, x[:, 3 * seg:3 * seg + S])
         o = ops.scratch("time_mix_o", (T * S,), torch.float32, dev)
-        # In float32 a row's bits do not depend on what else its step holds, so every step goes token by token there.
-        if self.dtype == torch.bfloat16 and not single and ops.time_mix_chunks_pay(T, ctx.num_requests, self.head_dim, self.head_dim):
+        if not single and self.form(ctx.sizes):
             ops.time_mix_chunks(x, 0, seg, 2 * seg, 3 * seg, self.w0, self.u, state, ctx.cu_seqlens_q, ctx.state_slots,
                                 ctx.attention_tiles(ops.TIME_MIX_CHUNK), o, self.num_heads, self.head_dim, self.head_dim)
         else:

@@ -524,3 +524,30 @@ def test_float32_prompts_have_the_same_bits_alone_and_in_one_step(tmp_path):
     beside = [{"step": 0, "entries": whole[:2], "end": []},
               {"step": 1, "entries": [{"id": e["id"], "tokens": [5], "want": []} for e in whole[:2]] + whole[2:], "end": list(reqs)}]
     assert torch.equal(replay(runner, beside)[1], torch.cat([alone[i] for i in range(2, 6)]))
+
+
+def test_steps_of_one_size_take_the_form_their_longest_portion_pays_for(tmp_path, monkeypatch):
+    """bfloat16, recurrent heads of 64 x 64: 64 tokens of four requests as equal portions and as one portion of 61 beside single
+    tokens, which have the same capacities: the delta rule runs token by token in the first and in chunks in the second, eagerly,
+    captured and replayed, and gives the plain model's logits each time."""
+    from tiny_llm_amd.engine.step import StepEntry
+    from tiny_llm_amd.kernels import ops
+    cfg, ranks, block = copy.deepcopy(CONFIGS["delta"])
+    for layer in cfg["layers"]:
+        layer["mixer"]["dim"] = layer["mixer"]["vdim"] = 64
+    folder, w = make_folder(tmp_path, cfg, ranks, seed=11, store=torch.bfloat16, sharpen=1.0)
+    reqs = [random_tokens(61, cfg["vocab"], 100 * i) for i in range(4)]
+    ref = [plain.forward(cfg, rounded(w), toks) for toks in reqs]
+    runner = make_runner(folder, "bfloat16", block, 1024)
+    took = []
+    for name in ("delta_chunks", "delta_recurrence"):
+        monkeypatch.setattr(ops, name, lambda *a, _name=name, _op=getattr(ops, name), **kw: (took.append(_name), _op(*a, **kw))[1])
+    for turn in range(4):                                   # eager, eager on the static buffers, captured, replayed
+        for lens, form in (([16, 16, 16, 16], "delta_recurrence"), ([1, 61, 1, 1], "delta_chunks")):
+            took.clear()
+            got = runner.step([StepEntry(str(i), reqs[i][:n], [n - 1]) for i, n in enumerate(lens)], use_graph=turn > 0).cpu()
+            assert set(took) == ({form} if turn < 3 else set()), (turn, lens, took)
+            for i, n in enumerate(lens):
+                assert row_err(got[i], ref[i][n - 1]) < TOL["bfloat16"], (turn, lens, i)
+                runner.finish(str(i))
+    assert len(runner._graphs) == 2 and all(g.graph is not None for g in runner._graphs.values())

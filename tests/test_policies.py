@@ -169,3 +169,15 @@ def test_a_step_is_known_by_the_forms_its_parts_choose():
     bare = dict.fromkeys(("tokens", "positions", "req_of_token", "cu_seqlens_q", "seq_lens", "state_slots", "logit_rows", "block_tables", "slot_mappings"))
     assert StepContext(num_tokens=9, num_requests=2, max_q_len=8, **bare).sizes == (9, 2, 8)
     assert StepContext(num_tokens=16, num_requests=2, max_q_len=16, sizes=StepSizes(9, 2, 8), **bare).sizes == (9, 2, 8)
+
+
+def test_the_delta_rule_runs_in_chunks_where_its_longest_portion_pays_for_them():
+    """The steps beside the rule, and sizes that the chunks do not take."""
+    pays = lambda lens, heads=16, dim=128, vdim=128, taps=4: ops.delta_chunks_pay(sum(lens), len(lens), max(lens), heads, dim, vdim, taps)  # noqa: E731
+    for lens in ([8] * 8, [24] * 8, [16], [1] * 40 + [32] * 3, [1] * 64, [1] * 256, [1]):
+        assert not pays(lens), lens
+    for lens in ([32] * 8, [48] * 8, [13] * 64, [48] * 64, [48], [2047], [67, 801, 143, 411, 205, 317], [1] * 8 + [128], [1] * 16 + [256],
+                 [1] * 40 + [512], [1] * 64 + [512], [1] * 64 + [1024]):
+        assert pays(lens), lens
+    assert not pays([1] * 239 + [62], 32, 48, 64) and not pays([1] * 94 + [43], 64, 33, 33)
+    assert not pays([2047], dim=32) and not pays([2047], dim=129) and not pays([2047], vdim=129) and not pays([2047], taps=5)

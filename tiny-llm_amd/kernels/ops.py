@@ -1650,13 +1650,18 @@ DELTA_CHUNK_MAX_DIM = 128        # its heads' channels and value columns
 DELTA_CHUNK_MAX_TAPS = 4
 
 
-def delta_chunks_pay(n_tokens: int, n_requests: int, dim: int, vdim: int, taps: int) -> bool:
-    """Whether a step's recurrence runs in chunks (`delta_chunks`) or token by token.  A request costs the chunks about 1 us
-    (16 heads of 128 x 128; its state goes through narrower pieces), token by token 0.6; a token 0.05 us against 0.05 and,
-    in the longest request, 0.37.  8 requests of 8, 16 and 32 tokens: 18, 20 and 35 us in chunks, 16, 21 and 34 by tokens,
-    24: 34 and 27; 40 of one token beside 3 of 32: 52 and 46; 64 of 13: 67 and 110; one of 48: 19 and 28; one of 2,047: 145 and 806."""
+def delta_chunks_pay(n_tokens: int, n_requests: int, longest: int, heads: int, dim: int, vdim: int, taps: int) -> bool:
+    """Whether a step's recurrence runs in chunks (`delta_chunks`) or token by token.  Token by token it is a chain of 0.38 us a
+    token of the longest request (16 heads of 128 x 128; 0.3 with heads of 64), in chunks of 0.06; a request costs chunks more (0.95 us
+    against 0.65; its state goes through narrower pieces), every 16 tokens of it one more piece, and a token of any request a
+    little less.  978 steps (1 to 256 requests: equal portions, one or two portions beside single tokens, any mix; 1 to 64 heads of
+    33 to 128 by 16 to 128): the sum of what the choice loses against the better form is 0.3 % of their times, and in three of them
+    chunks are chosen where they are more than 3 % slower (5, 4 and 4 %).  16 heads of 128 x 128, chunks and tokens: 8 requests of 8,
+    16, 24, 32 and 48 tokens 22 and 17 us, 24 and 23, 35 and 30, 36 and 39, 42 and 52; 64 of 13 and 48 69 and 108, 232 and 319; one
+    of 16, 48 and 2,047 18 and 15, 21 and 27, 146 and 803; six of 67 to 801 120 and 402; 40 single tokens beside 3 of 32, beside one
+    of 128 and of 512 56 and 50, 62 and 83, 104 and 250."""
     return (32 < dim <= DELTA_CHUNK_MAX_DIM and vdim <= DELTA_CHUNK_MAX_DIM and taps <= DELTA_CHUNK_MAX_TAPS
-            and n_tokens >= 20 * n_requests + 44)
+            and 16 * (longest - 40) >= heads * (0.6 * n_requests - 0.1 * n_tokens))
 
 
 def delta_chunks(p: torch.Tensor, conv_off: int, b_off: int, a: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor,

@@ -121,6 +121,12 @@ class ChannelDelta(Mixer):
         return StateSpec((-(-(self.state_size + self.channels * (self.taps - 1)) // 4) * 4,), torch.float32)
 
     # --------------------------------------------------------------------- compute
+    def form(self, sizes):
+        """Whether the recurrence runs in chunks.  In float32 a row's bits do not depend on what else its step holds, so every
+        step goes token by token there."""
+        return self.dtype == torch.bfloat16 and ops.delta_chunks_pay(sizes.tokens, sizes.requests, sizes.longest, self.num_heads,
+                                                                     self.head_dim, self.value_dim, self.taps)
+
     def forward(self, h, ctx, cache, state, residual):
         T, dev = h.shape[0], h.device
         H, KH, D, V = self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim
@@ -147,8 +153,7 @@ class ChannelDelta(Mixer):
                                       ctx.state_slots, self.taps)
             return self._project_out(z, residual)
         o = ops.scratch("delta_o", (T * H * V,), torch.float32, dev)
-        # In float32 a row's bits do not depend on what else its step holds, so every step goes token by token there.
-        if self.dtype == torch.bfloat16 and ops.delta_chunks_pay(T, ctx.num_requests, D, V, self.taps):
+        if self.dtype == torch.bfloat16 and self.form(ctx.sizes):
             ops.delta_chunks(p, 0, self.b_off, a, self.conv_w, self.a_log, self.dt_bias, state, self.state_size,
                              ctx.cu_seqlens_q, ctx.state_slots, ctx.attention_tiles(ops.DELTA_CHUNK), o, H, KH, D, V,
                              self.taps, D ** -0.5, self.per_head)

@@ -1562,3 +1562,14 @@ def test_gated_epilogues_leave_the_bits_of_the_kernels_behind(M, F, K):
         assert same(stacked, side)
     with pytest.raises(Exception):
         k.linear(a.float(), woven.float(), want.float(), epilogue="gelu_glu")
+
+
+def test_the_clamped_epilogue_is_told_its_limit():
+    """Without a limit the product is refused: every gate would be clamped to nothing."""
+    from tiny_llm_amd.kernels import KernelError
+    k = ops()
+    a, w, z = (torch.zeros(*shape, dtype=torch.bfloat16, device="cuda") for shape in ((4, 64), (32, 64), (4, 16)))
+    with pytest.raises(KernelError):
+        k.linear(a, w, z, epilogue="clamped_glu")
+    for epilogue, gate in (("clamped_glu", (0.0, 0.0, 0.0)), ("gelu_glu", None), ("swiglu", None)):
+        assert torch.equal(k.linear(a, w, z.fill_(1.0), epilogue=epilogue, gate=gate), torch.zeros_like(z))

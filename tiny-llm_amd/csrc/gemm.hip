@@ -2627,6 +2627,7 @@ int tl_linear_tile(const void* a, const void* w, void* out, const float* residua
 int tl_linear(const void* a, const void* w, void* out, const float* residual, const float* row_scale, int M,
               int N, int K, int64_t lda, int64_t ldo, int dtype, int out_dtype, int epilogue,
               hipStream_t stream) {
+  if (epilogue == 3) return TL_ERR_ARG;      // its limit has no place here
   return tl_linear_tile(a, w, out, residual, row_scale, M, N, K, lda, ldo, dtype, out_dtype, epilogue, 0, 0.f, 0.f, 0.f, stream);
 }
 

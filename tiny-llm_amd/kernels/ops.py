@@ -224,7 +224,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor
 
 def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual: Optional[torch.Tensor] = None,
            epilogue: Optional[str] = None, row_scale: Optional[torch.Tensor] = None, tile: int = 0,
-           gate=(0.0, 0.0, 0.0)) -> torch.Tensor:
+           gate: Optional[Tuple[float, float, float]] = None) -> torch.Tensor:
     """out = a @ w.T (+ residual).  a [M, K], w [N, K] share an element type; out [M, N] is that
     type or float32; residual float32 with out's strides.  epilogue="swiglu": the N columns are
     interleaved (gate_j, up_j) pairs and out [M, N/2] = silu(gate) * up, computed from the float32
@@ -248,6 +248,9 @@ def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual: Option
         _fail("the squared-relu epilogue takes and leaves bfloat16, without a residual")
     if code > EPILOGUES["relu2"] and dt != 1:
         _fail(f"the {epilogue} epilogue takes and leaves bfloat16")
+    if epilogue == "clamped_glu" and gate is None:
+        _fail("the clamped_glu epilogue takes its limit, alpha and shift in `gate`")
+    gate = gate or (0.0, 0.0, 0.0)
     if swiglu:
         if not (N % 2 == 0 and tuple(out.shape) == (M, N // 2) and odt == dt and residual is None):
             _fail(f"the SiLU-gate epilogue writes [{M}, {N // 2}] of the input's type and takes no residual")

@@ -637,6 +637,34 @@ def test_rotation_and_gate_that_ride_in_the_heads_products(T, H, K, N, R, rd):
             ops.table_moe_up(x, w, None, heads, two, "relu2", gate=gate)
 
 
+def test_a_rotation_that_rides_in_a_product_writes_other_columns():
+    """Product and rotation of one launch run in no order: a call in which they meet is refused, one buffer or two apart are not."""
+    from tiny_llm_amd.kernels import ops
+    from tiny_llm_amd.parts.rotary import angle_tables
+    T, H, K, N, R = 5, 3, 24, 40, 8
+    cos, sin = angle_tables(R, 500.0, 512, "cuda")
+    positions = torch.arange(T, dtype=torch.int32, device="cuda")
+    q = torch.randn(T, H * (K + R), device="cuda").to(torch.bfloat16)
+    w = torch.randn(H, N, K, device="cuda").to(torch.bfloat16)
+    store = torch.zeros(2, T, H, N + R, device="cuda")
+    wide, other = store
+
+    def both(out, off):
+        ops.head_gemm(q.view(T, H, K + R)[:, :, :K], w, out, rotate=(q, H, K + R, K, R, R, positions, cos, sin, wide, off, "half"))
+
+    for out, off in ((wide[:, :, :N], N - 1), (wide[:, :, R:], 1), (wide[:, :, 4:4 + N], 0), (wide.view(-1)[:T * H * N].view(T, H, N), N),
+                     (store.view(-1)[T * H * (N + R) - N:][:T * H * N].view(T, H, N), N)):
+        with pytest.raises(ops.KernelError):
+            both(out, off)
+    assert not store.any()
+    both(wide[:, :, :N], N)
+    both(other[:, :, R:], N)
+    assert torch.equal(wide[:, :, :N], other[:, :, R:]) and wide.any() and not other[:, :, :R].any()
+    wide.zero_()
+    both(wide[:, :, R:], 0)
+    assert torch.equal(wide[:, :, R:], other[:, :, R:])
+
+
 def test_gate_and_activation_rows():
     from tiny_llm_amd.kernels import ops
     g = torch.Generator().manual_seed(0)

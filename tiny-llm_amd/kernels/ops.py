@@ -1546,6 +1546,12 @@ def head_gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Optiona
         _rotation_fits(q, heads, head_width, rot, rdims, positions, cos, sin, wide, pairing)
         _need(q.dtype == torch.bfloat16 and out.dtype == torch.float32 and heads == H and q.shape[0] == T,
               "head_gemm: what is rotated is bfloat16, of the product's rows and heads, beside a float32 product")
+        # both are written by one launch, in no order: within one buffer the columns of a head lie apart
+        at = (out.data_ptr() - wide.data_ptr()) // 4
+        if T and at < wide.numel() and at + (T - 1) * out.stride(0) + (H - 1) * out.stride(1) + cols > 0:
+            _need(out.stride(0) == wide.stride(0) and out.stride(1) == wide.stride(1) and 0 <= at < wide.shape[2]
+                  and at + cols <= wide.shape[2] and (at + cols <= wide_off or wide_off + rot <= at),
+                  "head_gemm: the product and what is rotated are written to the same columns")
         turn = (c_int(rot), _ptr(q), c_int64(q.stride(0)), c_int(head_width), c_int(in_off), c_int(rdims), _ptr(positions), _ptr(cos),
                 _ptr(sin), _ptr(wide), c_int(wide.shape[2]), c_int(wide_off), c_int(ROPE_PAIRINGS.index(pairing)))
     _check(_lib().tl_head_gemm(_ptr(x, 16), c_int64(x.stride(0)), c_int(x.stride(1)), _ptr(w, 16), _ptr(out),

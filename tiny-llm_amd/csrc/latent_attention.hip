@@ -820,14 +820,15 @@ __global__ __launch_bounds__(kThreads) void head_products_kernel(const TI* __res
 // instruction's rows), so a lane ends with four consecutive output columns of one row.
 // A lane's four results leave as one vector where rows and heads allow it: 1,944 rows of 16 heads, 128 -> 512, 54.8 -> 34.8 us
 // (as scalars every store was 64 pieces of four bytes), 512 -> 128 in bfloat16 36.4 -> 32.0.
-// STEPS: k steps of 32 whose operands are requested together; SUMS of them, one after the other.  With few rows the kernel is its
+// STEPS: k steps of 32 whose operands are requested together, each with a sum of its own.  With few rows the kernel is its
 // round trips to memory and takes four: 6 rows of 16 heads, 512 -> 128, 7.0 us one by one and 6.1 so.  Four sums also keep its
 // error where the kernel of few rows has it (5.7e-8 of the result against 64 bits; in one sum 8.5e-8).  Many rows find
-// their operands in the caches and lose waves by it: 64 rows of 16 heads, 128 -> 512, 6.1 us by one step and 6.3 by four; 1,944 rows 34.8 and 34.0.
+// their operands in the caches and lose waves by it: 16 heads, 128 -> 512, by one step and by four, 64 rows 4.6 and 4.9 us, 300
+// rows 9.0 and 9.3, from 700 on the same (1,944 rows 34.6 and 34.7); 512 -> 128 64 rows 9.5 and 10.0, 1,944 32.1 and 31.8.
 // ROTATE: the last workgroup along the columns rotates the other dims of its head and rows, which a query's product leaves beside its
 // results: it needs nothing of the product, and took 3.0 us as a launch of its own for 6 rows of 16 heads, 6.0 for 1,944.
 constexpr int kHeadFewRows = 32;
-template <typename TO, int STEPS, int SUMS, bool ROTATE>
+template <typename TO, int STEPS, bool ROTATE>
 __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* __restrict__ in, int64_t in_stride,
                                                                   int in_head_width, const bf16_t* __restrict__ w,
                                                                   TO* __restrict__ out, int64_t out_stride,
@@ -852,9 +853,9 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
     wp[a] = w + ((int64_t)h * cols + min(col0 + a * 16 + c, cols - 1)) * inner;
     xp[a] = in + (int64_t)min(row0 + a * 16 + c, n_rows - 1) * in_stride + (int64_t)h * in_head_width;
   }
-  f32x4 sum[SUMS][2][2];
+  f32x4 sum[STEPS][2][2];
 #pragma unroll
-  for (int p = 0; p < SUMS; ++p)
+  for (int p = 0; p < STEPS; ++p)
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -878,7 +879,7 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
         for (int a = 0; a < 2; ++a)
 #pragma unroll
           for (int b = 0; b < 2; ++b)
-            sum[u % SUMS][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][a], xb[u][b], sum[u % SUMS][a][b], 0, 0, 0);
+            sum[u][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u][a], xb[u][b], sum[u][a][b], 0, 0, 0);
       }
   }
   f32x4 acc[2][2];
@@ -886,7 +887,7 @@ __global__ __launch_bounds__(kThreads) void head_gemm_bf16_kernel(const bf16_t* 
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      if constexpr (SUMS == 4) acc[a][b] = (sum[0][a][b] + sum[1][a][b]) + (sum[2][a][b] + sum[3][a][b]);
+      if constexpr (STEPS == 4) acc[a][b] = (sum[0][a][b] + sum[1][a][b]) + (sum[2][a][b] + sum[3][a][b]);
       else acc[a][b] = sum[0][a][b];
     }
   // acc[a][b][i] = out[row0 + b*16 + c][col0 + a*16 + g*4 + i]
@@ -1100,16 +1101,16 @@ int tl_head_gemm(const void* in, int64_t in_stride, int in_head_width, const voi
   const int size = out_dtype == 0 ? 4 : 2;
   // results leave four columns at a time where rows, heads and the buffer are whole vectors of them
   const int whole = cols % 4 == 0 && out_stride % 4 == 0 && out_head_width % 4 == 0 && (uintptr_t)out % (4 * size) == 0;
-#define TL_HEAD_GEMM(TO, STEPS, SUMS, ROTATE)                                                                           \
-  hipLaunchKernelGGL((head_gemm_bf16_kernel<TO, STEPS, SUMS, ROTATE>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width, \
+#define TL_HEAD_GEMM(TO, STEPS, ROTATE)                                                                                 \
+  hipLaunchKernelGGL((head_gemm_bf16_kernel<TO, STEPS, ROTATE>), g, b, 0, stream, (const bf16_t*)in, in_stride, in_head_width, \
                      (const bf16_t*)w, (TO*)out, out_stride, out_head_width, n_rows, inner, cols, (const bf16_t*)gate,   \
                      gate_stride, whole, rotate)
-  if (rot && few) TL_HEAD_GEMM(float, 4, 4, true);
-  else if (rot) TL_HEAD_GEMM(float, 1, 1, true);
-  else if (out_dtype == 0 && few) TL_HEAD_GEMM(float, 4, 4, false);
-  else if (out_dtype == 0) TL_HEAD_GEMM(float, 1, 1, false);
-  else if (out_dtype == 1 && few) TL_HEAD_GEMM(bf16_t, 4, 4, false);
-  else if (out_dtype == 1) TL_HEAD_GEMM(bf16_t, 1, 1, false);
+  if (rot && few) TL_HEAD_GEMM(float, 4, true);
+  else if (rot) TL_HEAD_GEMM(float, 1, true);
+  else if (out_dtype == 0 && few) TL_HEAD_GEMM(float, 4, false);
+  else if (out_dtype == 0) TL_HEAD_GEMM(float, 1, false);
+  else if (out_dtype == 1 && few) TL_HEAD_GEMM(bf16_t, 4, false);
+  else if (out_dtype == 1) TL_HEAD_GEMM(bf16_t, 1, false);
   else return TL_ERR_ARG;
 #undef TL_HEAD_GEMM
   return tl_launch_status();

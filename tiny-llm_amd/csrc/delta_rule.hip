@@ -299,11 +299,12 @@ __global__ __launch_bounds__(kRecThreads) void delta_recurrence_kernel(
 // delta_chunk_scan_kernel to do in order are three products of 16 x dim (x vdim columns) a chunk.  Products of decays are
 // taken of the decays themselves (none exceeds one), never as quotients, so decays near zero lose nothing.  A number
 // that is not finite reaches no token ahead of its own: B's zeros never meet it.
-// 1,944 tokens of six requests, the longest 801, 16 heads of 128 x 128: convolutions and decays 97 us and the recurrence 299,
-// now 46 and 79; one request of 2,047 tokens 102 and 704, now 45 and 101.  What bounds them: the first its convolutions' and
-// decays' functions; the second a chain of 0.75 us a chunk, of which the matrix instructions take a half.  Error against 64
-// bits (2-norm, 1,000 tokens, 128 x 128): one decay a channel 1.38e-7 and 1.44e-7 for two draws, token by token 1.46e-7 and
-// 1.55e-7; one a head 1.35e-7 and 1.38e-7, token by token 1.28e-7 and 1.39e-7; 64 x 64 1.53e-7 and 1.58e-7.
+// 1,944 tokens of six requests, the longest 801, 16 heads of 128 x 128: convolutions and decays 98 us and the recurrence 311,
+// now 52 and 74; one request of 2,047 tokens 103 and 700, now 50 and 102.  What bounds them: the first its convolutions' and
+// decays' functions; the second a chain of 0.8 us a chunk, of which the matrix instructions take a half.  Error against 64
+// bits (2-norm, 1,000 tokens of 8 heads, mean of 16 draws, in chunks and token by token): of the results with one decay a channel
+// 1.40e-7 and 1.45e-7 (64 x 64 1.54e-7 and 1.58e-7), with one a head 1.42e-7 and 1.41e-7 (1.52e-7 and 1.51e-7), of the states
+// 1.59e-7 and 1.85e-7 (1.49e-7 and 1.65e-7), 1.54e-7 and 1.70e-7 (1.44e-7 and 1.51e-7).
 constexpr int kChunkMaxDim = 128;      // channels and value columns a head may have here: a thread each
 constexpr int kChunkThreads = 256;
 constexpr int kChunkTaps = 4;
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(kChunkThreads) void delta_chunk_kernel(
     Bs[l][s] = l >= s ? bt : 0.f;
   }
   __syncthreads();
-  // W and U0, a column a thread: beta_t times x_t - sum A_ts w_s, summed in 64 bits (2 us of 46; in 32 the error against 64
+  // W and U0, a column a thread: beta_t times x_t - sum A_ts w_s, summed in 64 bits (2 us of 52; in 32 the error against 64
   // bits is 5 % above that of token by token, not below).
   f32x4 *W = (f32x4*)item, *Q = W + 4 * DP, *K = Q + 4 * DP, *U0 = K + 4 * DP, *Bm = U0 + 4 * vp;
   if (channel) {

@@ -191,8 +191,8 @@ __global__ __launch_bounds__(kThreads) void time_mix_recurrence_kernel(
 // time_mix_scan_kernel walks a request's chunks.  Products of decays are taken of the decays themselves, never as quotients,
 // along a chunk in 64 bits, and so are B's sums; all else is float32.  A number that is not finite reaches no token ahead of its
 // own: B's zeros never meet it.
-// 1,944 tokens of six requests, the longest 801, 32 heads of 64 x 64: 188 us token by token, now 36 and 28; one request of 2,047
-// tokens 460, now 35 and 52; heads of 128 x 128, half as many, 280, now 37 and 48.  The first kernel is bound by its vector
+// 1,944 tokens of six requests, the longest 801, 32 heads of 64 x 64: 187 us token by token, now 36 and 29; one request of 2,047
+// tokens 458, now 36 and 54; heads of 128 x 128, half as many, 280, now 38 and 51.  The first kernel is bound by its vector
 // instructions, the second by a chain of 0.4 us a chunk.  Error against 64 bits (2-norm, 700 to 1,000 tokens): 9.1e-8, token
 // by token 9.5e-8; 128 x 128 9.2e-8 and 1.01e-7 (with B in float32 1.02e-7 and 1.05e-7, 8 us less).
 constexpr int kMaxChunkDim = 128;      // channels and value columns a head may have here

@@ -1573,3 +1573,67 @@ def test_the_clamped_epilogue_is_told_its_limit():
         k.linear(a, w, z, epilogue="clamped_glu")
     for epilogue, gate in (("clamped_glu", (0.0, 0.0, 0.0)), ("gelu_glu", None), ("swiglu", None)):
         assert torch.equal(k.linear(a, w, z.fill_(1.0), epilogue=epilogue, gate=gate), torch.zeros_like(z))
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(2, 64), (46, 192), (518, 704), (2046, 128), (2560, 2048), (4100, 1088), (30000, 64), (33000, 128)])
+def test_linear_whole_inner_size(M, N, K):
+    """17 to 64 rows: every cut of the rows and columns, both lengths of block, fewer blocks than waves, columns that end within a
+    group of four, rows that are gathered, and both sides of the norm hand-off."""
+    g = torch.Generator().manual_seed(M + N + K)
+    assert ops().linear_whole(M, N, K)
+    wide = torch.randn(M + 40, K + 8, generator=g).to(torch.bfloat16)      # rows with other numbers behind them
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
+    a, da, dw = wide[:M, :K], wide.to(DEV)[:M, :K], w.to(DEV)
+    res = torch.randn(M, N, generator=g)
+    nw = 1 + 0.1 * torch.randn(N, generator=g)
+    exact = a.double() @ w.double().T
+    # K products and their sums in any order, the factor and the last addition: at most K + 3 roundings of the absolute sum
+    bound = (K + 3) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + res.double().abs())
+    x, operand = res.clone().to(DEV), torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    sumsq = torch.full((M, ops().handoff_parts(M, N, K)), float("nan"), device=DEV)
+    if N % 8 == 0:
+        ops().linear_handoff(da, dw, x, x, emit=(nw.to(DEV), operand, sumsq))
+        assert torch.equal(operand.cpu(), (nw * x.cpu()).to(torch.bfloat16))
+        assert rel(sumsq.sum(dim=1), (x.double() ** 2).sum(dim=1)) < 1e-6
+    else:
+        ops().linear(da, dw, x, x)
+    assert ((x.cpu().double() - exact - res.double()).abs() <= bound).all()
+    # gathered rows, with the factors of a norm handed over in parts
+    rows = torch.randperm(M + 40, generator=g)[:M].to(torch.int32)
+    parts = torch.rand(M + 40, 70, generator=g) + 0.5
+    y = torch.empty(M, N, device=DEV)
+    ops().linear_handoff(wide.to(DEV)[:, :K], dw, y, rows=rows.to(DEV), prepared=(parts.to(DEV), 1e-5, K))
+    inv = 1.0 / torch.sqrt(parts[rows.long()].double().sum(dim=1, keepdim=True) / K + 1e-5)
+    gathered = wide[rows.long(), :K].double()
+    # the factor's own roundings beside them: a sum of 70 parts, a division, a root, a reciprocal and the product
+    assert ((y.cpu().double() - gathered @ w.double().T * inv).abs() <= (K + 80) * 2.0 ** -24 * (gathered.abs() @ w.double().abs().T) * inv).all()
+    # a row that is not finite is its own affair
+    da2 = da.clone()
+    da2[M // 2, K // 2] = float("inf")
+    z = torch.empty(M, N, device=DEV)
+    plain_z = torch.empty(M, N, device=DEV)
+    ops().linear(da2, dw, z)
+    ops().linear(da, dw, plain_z)
+    others = torch.arange(M) != M // 2
+    assert torch.equal(z.cpu()[others], plain_z.cpu()[others]) and not torch.isfinite(z[M // 2]).any()
+    for epilogue, gate in (("relu2", None), ("clamped_glu", (3.0, 1.702, 1.0)), ("gelu_glu", None)):
+        glu = epilogue != "relu2"
+        out = torch.full((M, N // 2 if glu else N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops().linear(da, dw, out, epilogue=epilogue, gate=gate)
+        assert torch.isfinite(out).all()
+        if not glu:
+            assert torch.equal(out, (plain_z.clamp(min=0) ** 2).to(torch.bfloat16))
+            continue
+        stored = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        want = torch.empty_like(out)
+        ops().linear(da, dw, stored)
+        stored = torch.cat([stored[:, 0::2], stored[:, 1::2]], dim=1)
+        ops().clamped_glu(stored, want, *gate) if gate else ops().gelu_glu(stored, want)
+        assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 14336, 4096), (64, 14336, 4096)])
+def test_long_inner_sizes_with_few_columns_are_split(M, K, N):
+    assert not ops().linear_whole(M, N, K) and ops().split_k(M, N, K) > 1
+    assert not ops().linear_whole(16, 2048, 2048) and not ops().linear_whole(65, 2048, 2048) and not ops().linear_whole(32, 2048, 2056)

@@ -13,7 +13,9 @@
 //    registers into two (v_mfma_f32_32x32x16_bf16; tile_mode says where); optionally over a share of the inner size (split k).
 //  * gemm_oneshot_bf16_kernel: the split product for few rows, operands streamed through a ring of
 //    LDS slabs filled straight from memory; splitk_reduce_kernel adds the parts and applies the epilogue.
-//  * gemm_skinny_bf16_kernel: at most 64 rows (decode steps), weights streamed once into registers.
+//  * gemm_skinny_bf16_kernel: at most 16 rows (decode steps), weights streamed once into registers; up to 64 for inner sizes that
+//    are no multiple of 64.
+//  * gemm_stripe_bf16_kernel: 17 to 64 rows, the inner size whole.
 #include <type_traits>
 
 #include "common.h"
@@ -1661,6 +1663,10 @@ __global__ __launch_bounds__(O_THREADS) void gemm_oneshot_bf16_kernel(const bf16
 // kernel).  The number of splits with the smallest estimated time: rounds of workgroups over the 256
 // compute units, each as long as a workgroup takes to fetch its share (about 35 GB/s), and the second
 // kernel's reading of the partial sums.
+static double oneshot_us(int M, int N, int K, int per) {
+  const int tiles = ((M + O_BM - 1) / O_BM) * ((N + O_BN - 1) / O_BN), splits = (K / O_SLAB_K + per - 1) / per;
+  return (tiles * splits + 255) / 256 * (2.0 + per * (O_SLAB_BYTES / 35e3)) + 1.5 + splits * (double)M * N * 4 / 3e6;
+}
 static int oneshot_plan(int M, int N, int K, int* slabs_per_split) {
   *slabs_per_split = 0;
   if (M <= 16 || K % O_SLAB_K || K < 4 * O_SLAB_K) return 1;
@@ -1681,8 +1687,7 @@ static int oneshot_plan(int M, int N, int K, int* slabs_per_split) {
     if (per < (nslabs >= 8 ? 4 : 2)) break;
     const int splits = (nslabs + per - 1) / per;
     if (splits < 2) continue;
-    const int rounds = (tiles * splits + 255) / 256;
-    const double t = rounds * (2.0 + per * (O_SLAB_BYTES / 35e3)) + 1.5 + splits * (double)M * N * 4 / 3e6;
+    const double t = oneshot_us(M, N, K, per);
     if (best == 1 || t < best_t) {
       best = splits;
       best_per = per;
@@ -2355,8 +2360,304 @@ static int launch_skinny(const SkinnyArgs& p, hipStream_t stream) {
   return TL_ERR_ARG;
 }
 
+// ============================================================ bfloat16, 17 to 64 rows
+// Bound by what a unit fetches: every workgroup needs its activation rows (64 of them are 256 KB at an inner size of 2,048, beside
+// 180 KB of weights), and a unit gets about 105 GB/s from its L2 in loads that take whole lines of 128 bytes (138 alone), but 37
+// in the matrix instructions' own order, 64 bytes of each of sixteen rows, in which gemm_skinny_bf16_kernel loads.  So a wave fetches
+// whole lines, turns them into operands through an area of LDS of its own (no barrier in the loop), and owns every eighth block of the
+// inner size, so that each row is fetched once by a workgroup; the waves' sums meet in LDS, in a fixed order.  The inner size stays whole: no second
+// kernel and no partial sums through memory, as splitting it over workgroups takes.  Blocks of 128 k where their LDS allows (64 otherwise),
+// one on its way: 64 rows of 2,048 by 11,264 pairs took 15.1 us so, 15.8 with two and 17.8 with three.  (Every workgroup beginning
+// with another block, so that they do not all ask for the same lines at once, took 14.7, but then a sum's order goes by its column.)
+// 64 rows, weights from memory, against the split product's two kernels: 2,560 x 2,048 10.9 -> 6.4 us, 2,048 x 2,048 10.0 ->
+// 5.5, 11,264 x 2,048 gated 18.1 -> 15.1, 2,048 x 5,632 14.4 -> 11.9.
+constexpr int T_MAX_INNER = 1 << 20;      // offsets within a workgroup's rows fit 31 bits
+
+template <int MT, int CT, int TK>
+struct Stripe {
+  static constexpr int kRows = MT * 16, kLd = CT * 16 + 4;                     // kLd: floats between rows of partial sums
+  static constexpr int kChunks = TK / 8, kRowsPerLoad = 64 / kChunks;          // 16-byte chunks of a row's share of a block
+  static constexpr int kA = kRows / kRowsPerLoad, kW = CT * 16 / kRowsPerLoad; // load instructions of a block
+  static constexpr int kWaveBytes = (kA + kW) * 1024;
+  static constexpr int kGroups = kRows * CT * 4;                               // groups of four columns of a row
+  static constexpr size_t kBody = (size_t)S_WAVES * (kWaveBytes > kRows * kLd * 4 ? kWaveBytes : kRows * kLd * 4);
+  static constexpr size_t kSmem = kBody + (size_t)(kRows + kGroups) * sizeof(float);
+};
+
+// p.cols_wg: a multiple of 4, at most 16 CT.  vec: the results' rows and addresses take groups of four columns.  GATHER: the input's
+// rows are p.rows' (through addresses of their own, as the input may be longer than a buffer's 31 bits).
+template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
+__global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const SkinnyArgs p, int groups_n, int vec) {
+  using S = Stripe<MT, CT, TK>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char stripe_smem[];
+  float* part = (float*)stripe_smem;                      // [S_WAVES][kRows][kLd], once the blocks are done with
+  float* scale_s = (float*)(stripe_smem + S::kBody);      // [kRows]
+  float* sq_s = scale_s + S::kRows;                       // [kRows][CT * 4]
+  const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TL_WAVE);
+  const int M = p.M, N = p.N, K = p.K, cw = p.cols_wg;
+  const int n0 = blockIdx.x * cw, m0 = blockIdx.y * S::kRows;
+  if (n0 >= N) return;
+
+  // A lane fetches chunk lc of row lr + kRowsPerLoad j.  Rows beyond the matrices and blocks beyond the inner size lie beyond the
+  // buffers: they read as zero and fetch nothing.
+  const int lr = lane / S::kChunks, lc = lane % S::kChunks, lda = (int)p.lda;
+  const auto buf_w = __builtin_amdgcn_make_buffer_rsrc((void*)(p.w + (int64_t)n0 * K), 0, min(cw, N - n0) * K * 2, 0x00020000);
+  const auto buf_a = __builtin_amdgcn_make_buffer_rsrc((void*)((const bf16_t*)p.a + (int64_t)m0 * lda), 0,
+                                                       ((min(S::kRows, M - m0) - 1) * lda + K) * 2, 0x00020000);
+  const int at_a = lr * lda * 2 + lc * 16, at_w = lr * K * 2 + lc * 16;
+  const int step_a = S::kRowsPerLoad * lda * 2, step_w = S::kRowsPerLoad * K * 2;
+  const int nblk = K / TK, mine = (nblk - wave + S_WAVES - 1) / S_WAVES;
+  const bf16_t* row_a[GATHER ? S::kA : 1];
+  if constexpr (GATHER)
+#pragma unroll
+    for (int j = 0; j < S::kA; ++j)
+      row_a[j] = (const bf16_t*)p.a + (int64_t)p.rows[min(m0 + j * S::kRowsPerLoad + lr, M - 1)] * p.lda + lc * 8;
+  struct Block {
+    bf16x8 a[S::kA], w[S::kW];
+  };
+  auto load = [&](Block& st, int i) {       // this wave's i-th block
+    const int k = i < mine ? (wave + i * S_WAVES) * TK * 2 : 0x70000000;
+#pragma unroll
+    for (int j = 0; j < S::kW; ++j)
+      st.w[j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(buf_w, at_w, k + j * step_w, 0));
+#pragma unroll
+    for (int j = 0; j < S::kA; ++j) {
+      if constexpr (GATHER) st.a[j] = i < mine ? *(const bf16x8*)(row_a[j] + k / 2) : bf16x8{};
+      else st.a[j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(buf_a, at_a, k + j * step_a, 0));
+    }
+  };
+  // chunk c of row r stands at place c ^ (r % kSwizzle) of its row, so that the operands of eight rows do not collide
+  constexpr int kSwizzle = S::kChunks < 16 ? S::kChunks : 16;
+  const int r16 = lane % 16, g = lane / 16;
+  unsigned char* own = stripe_smem + wave * S::kWaveBytes;
+  auto place = [&](int j) { return own + j * 1024 + lr * TK * 2 + (lc ^ ((j * S::kRowsPerLoad + lr) % kSwizzle)) * 16; };
+  f32x4 acc[MT][CT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) acc[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](Block& st, int next) {      // and requests the next block as soon as this one has left its registers
+#pragma unroll
+    for (int j = 0; j < S::kW; ++j) *(bf16x8*)place(S::kA + j) = st.w[j];
+#pragma unroll
+    for (int j = 0; j < S::kA; ++j) *(bf16x8*)place(j) = st.a[j];
+    load(st, next);
+#pragma unroll
+    for (int i = 0; i < TK / 32; ++i) {
+      const unsigned char* from = own + r16 * TK * 2 + ((i * 4 + g) ^ (r16 % kSwizzle)) * 16;
+      bf16x8 fa[MT], fw[CT];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) fw[ct] = *(const bf16x8*)(from + S::kA * 1024 + ct * 32 * TK);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) fa[mt] = *(const bf16x8*)(from + mt * 32 * TK);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          acc[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ct], fa[mt], acc[mt][ct], 0, 0, 0);
+    }
+  };
+  Block st;
+  load(st, 0);
+
+  // what the epilogue needs is requested behind the first block
+  constexpr int EPT = (S::kGroups + S_THREADS - 1) / S_THREADS;
+  f32x4 res_v[EPT], next_w[EPT];
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    res_v[j] = next_w[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (SWIGLU == 0 && sizeof(TO) == 4) {
+      const int e = tid + j * S_THREADS, c = e % (CT * 4) * 4, n = n0 + c;
+      const int m = min(m0 + e / (CT * 4), M - 1);
+      if (p.residual) {
+        const float* r = p.residual + (int64_t)m * p.ldo;
+        if (vec && n + 3 < N) res_v[j] = *(const f32x4*)(r + n);
+        else
+#pragma unroll
+          for (int q = 0; q < 4; ++q) res_v[j][q] = r[min(n + q, N - 1)];
+      }
+      if (p.emit_operand)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          next_w[j][q] = p.emit_w_is_f32 ? ((const float*)p.emit_w)[min(n + q, N - 1)] : (float)((const bf16_t*)p.emit_w)[min(n + q, N - 1)];
+    }
+  }
+  if (p.in_sumsq) {      // the rows' factors: one wave a row, in a fixed order
+    constexpr int RPW = S::kRows / S_WAVES;
+    float t[RPW];
+#pragma unroll
+    for (int ri = 0; ri < RPW; ++ri) {
+      const int m = min(m0 + wave * RPW + ri, M - 1);
+      const float* row = p.in_sumsq + (int64_t)(GATHER ? p.rows[m] : m) * p.in_parts;
+      t[ri] = lane < p.in_parts ? row[lane] : 0.f;
+      for (int q = lane + TL_WAVE; q < p.in_parts; q += TL_WAVE) t[ri] += row[q];
+    }
+#pragma unroll
+    for (int ri = 0; ri < RPW; ++ri) {
+      const float s = wave_sum(t[ri]);
+      if (lane == 0) scale_s[wave * RPW + ri] = 1.f / sqrtf(s / (float)p.in_width + p.in_eps);
+    }
+  }
+
+  for (int i = 0; i < mine; ++i) multiply(st, i + 1);
+
+  // a lane holds columns 4 g .. 4 g + 3 of row r16 of every tile
+  __syncthreads();
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) *(f32x4*)(part + (wave * S::kRows + mt * 16 + r16) * S::kLd + ct * 16 + g * 4) = acc[mt][ct];
+  __syncthreads();
+  TO* out = (TO*)p.out;
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    const int e = tid + j * S_THREADS;
+    if (e >= S::kGroups) break;
+    const int ml = e / (CT * 4), c = e % (CT * 4) * 4, m = m0 + ml, n = n0 + c;
+    const int left = m < M ? min(4, min(cw - c, N - n)) : 0;      // columns of this group that are results
+    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int wv = 0; wv < S_WAVES; ++wv) v += *(const f32x4*)(part + (wv * S::kRows + ml) * S::kLd + c);
+    float scale = 1.f;
+    if (p.row_scale) scale = p.row_scale[min(m, M - 1)];
+    if (p.in_sumsq) scale = scale_s[ml];
+    if constexpr (SWIGLU != 0) {      // two pairs (gate, up)
+      const TO y0 = from_f32<TO>(gated_pair<SWIGLU>(v[0] * scale, v[1] * scale, p.gate));
+      const TO y1 = from_f32<TO>(gated_pair<SWIGLU>(v[2] * scale, v[3] * scale, p.gate));
+      TO* to = out + (int64_t)m * p.ldo + n / 2;
+      if (left > 1) to[0] = y0;
+      if (left > 3) to[1] = y1;
+    } else {
+      float sq = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v[q] = v[q] * scale + res_v[j][q];
+        if constexpr (sizeof(TO) == 2) v[q] = act_value(v[q], p.act);
+        if (q < left) sq += v[q] * v[q];
+      }
+      TO* to = out + (int64_t)m * p.ldo + n;
+      if (vec && left == 4) {
+        if constexpr (sizeof(TO) == 4) *(f32x4*)to = v;
+        else *(bf16x4*)to = bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q < left) to[q] = from_f32<TO>(v[q]);
+      }
+      if constexpr (sizeof(TO) == 4) {
+        if (p.emit_operand) {
+          bf16_t* op = p.emit_operand + (int64_t)m * N + n;
+          const f32x4 x = next_w[j] * v;
+          if (vec && left == 4) *(bf16x4*)op = bf16x4{(bf16_t)x[0], (bf16_t)x[1], (bf16_t)x[2], (bf16_t)x[3]};
+          else
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              if (q < left) op[q] = (bf16_t)x[q];
+          sq_s[e] = sq;
+        }
+      }
+    }
+  }
+  if constexpr (SWIGLU == 0 && sizeof(TO) == 4) {
+    if (!p.emit_operand) return;      // uniform
+    __syncthreads();
+    if (tid < S::kRows && m0 + tid < M) {      // a part of a row's sum of squares per workgroup
+      float t = 0.f;
+#pragma unroll
+      for (int c = 0; c < CT * 4; ++c) t += sq_s[tid * CT * 4 + c];
+      p.emit_sumsq[(int64_t)(m0 + tid) * groups_n + blockIdx.x] = t;
+    }
+  }
+}
+
+template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
+static int launch_stripe_blocks(const SkinnyArgs& p, hipStream_t stream) {
+  const auto kernel = gemm_stripe_bf16_kernel<MT, CT, TK, TO, SWIGLU, GATHER>;
+  constexpr size_t smem = Stripe<MT, CT, TK>::kSmem;
+  static bool configured = false;
+  if (!configured) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return TL_ERR_LAUNCH;
+    configured = true;
+  }
+  const int vec = p.ldo % 4 == 0 && p.N % 4 == 0 && (uintptr_t)p.out % 16 == 0 && (uintptr_t)p.residual % 16 == 0 && (uintptr_t)p.emit_operand % 8 == 0;
+  const int groups_n = (p.N + p.cols_wg - 1) / p.cols_wg, groups_m = (p.M + MT * 16 - 1) / (MT * 16);
+  // several groups of rows: those of one group of columns fall on one die and find its weights in the L2 (48 rows of 5,120 x
+  // 5,120, three groups of 86: 32.3 us where they fell on different dies, 19.3 so)
+  dim3 g(groups_m > 1 ? (groups_n + kXcds - 1) / kXcds * kXcds : groups_n, groups_m), b(S_THREADS);
+  hipLaunchKernelGGL(kernel, g, b, smem, stream, p, groups_n, vec);
+  return TL_OK;
+}
+
+template <int MT, int CT, typename TO, int SWIGLU>
+static int launch_stripe_tile(const SkinnyArgs& p, hipStream_t stream) {
+  if constexpr (sizeof(TO) == 4) {      // the output head's
+    if (p.rows) {
+      if constexpr (MT + CT <= 4)
+        if (p.K % 128 == 0) return launch_stripe_blocks<MT, CT, 128, TO, SWIGLU, true>(p, stream);
+      return launch_stripe_blocks<MT, CT, 64, TO, SWIGLU, true>(p, stream);
+    }
+  }
+  if constexpr (MT + CT <= 4)
+    if (p.K % 128 == 0) return launch_stripe_blocks<MT, CT, 128, TO, SWIGLU, false>(p, stream);
+  return launch_stripe_blocks<MT, CT, 64, TO, SWIGLU, false>(p, stream);
+}
+
+// How this kernel takes a product of 17 to 64 rows, as tiles of sixteen rows and of sixteen columns a workgroup (false: not it).  A
+// workgroup's time goes by the rows that it fetches, of both operands, so the cheapest cut of the product has the smallest sum of
+// both, times the rounds of workgroups that it makes over the 256 units.  Timed for fifteen matrices of 1,024 x 704 to 27,648 x
+// 5,120 at 17, 32, 48 and 64 rows, every cut of each (1,270 in all): the one this picks is within 3 % of the fastest, 0.05 % on average.
+// The estimate (us) is compared with the split product's own (oneshot_plan; 4 us for its second launch), which is the faster way
+// for long inner sizes and few columns: 64 rows of 14,336 by 4,096 37.4 us here and 29.9 split; 5,120 x 5,120 19.0 and 19.7.
+struct StripePlan {
+  int mt, ct, cols;
+};
+static bool stripe_plan(int M, int N, int K, StripePlan* plan) {
+  if (M <= 16 || M > 64 || K % 64 || K > T_MAX_INNER) return false;
+  const int tiles = (M + 15) / 16;
+  int64_t least = 0;      // (of equal cuts the one with the fewest rows: 17 rows of 6,144 x 4,096 13.2 us in 1 x 3 tiles, 15.0 in 2 x 2)
+  for (int mt = 1; mt <= tiles; ++mt)
+    for (int ct = 1; ct <= 4; ++ct) {
+      const int64_t groups = (int64_t)((tiles + mt - 1) / mt) * ((N + 16 * ct - 1) / (16 * ct)), cost = (groups + 255) / 256 * (mt + ct);
+      if (least && cost >= least) continue;
+      least = cost;
+      // one round of three or four column tiles: as many columns as make 256 workgroups (64 rows of 5,120 x 5,120 20.6 -> 19.0 us)
+      const int even = (int)((N * (int64_t)((tiles + mt - 1) / mt) + 255) / 256 + 3) / 4 * 4;
+      *plan = {mt, ct, groups <= 256 && ct >= 3 && even > 16 * (ct - 1) && even < 16 * ct ? even : 16 * ct};
+    }
+  int slabs;
+  if (oneshot_plan(M, N, K, &slabs) < 2) return true;
+  return 2.4 + least * (K * 32 * 1.23e-5) + (double)N * K * 2 * 0.66 / 5.75e6 <= oneshot_us(M, N, K, slabs) + 4.0;
+}
+
+template <int MT, typename TO, int SWIGLU>
+static int launch_stripe_rows(const SkinnyArgs& p, int ct, hipStream_t stream) {
+  if (ct == 1) return launch_stripe_tile<MT, 1, TO, SWIGLU>(p, stream);
+  if (ct == 2) return launch_stripe_tile<MT, 2, TO, SWIGLU>(p, stream);
+  if (ct == 3) return launch_stripe_tile<MT, 3, TO, SWIGLU>(p, stream);
+  return launch_stripe_tile<MT, 4, TO, SWIGLU>(p, stream);
+}
+
+template <typename TO, int SWIGLU>
+static int launch_stripe(const SkinnyArgs& args, const StripePlan& plan, hipStream_t stream) {
+  SkinnyArgs p = args;
+  p.cols_wg = plan.cols;
+  if (plan.mt == 1) return launch_stripe_rows<1, TO, SWIGLU>(p, plan.ct, stream);
+  if (plan.mt == 2) return launch_stripe_rows<2, TO, SWIGLU>(p, plan.ct, stream);
+  if (plan.mt == 3) return launch_stripe_rows<3, TO, SWIGLU>(p, plan.ct, stream);
+  return launch_stripe_rows<4, TO, SWIGLU>(p, plan.ct, stream);
+}
+
 template <int PRO>
 static int launch_skinny_out(const SkinnyArgs& p, int out_dtype, bool swiglu, hipStream_t stream) {
+  if constexpr (PRO == PRO_NONE) {
+    StripePlan plan;
+    if (!(p.rows && out_dtype != 0) && p.lda <= T_MAX_INNER && stripe_plan(p.M, p.N, p.K, &plan)) {
+      if (out_dtype == 0 && !swiglu) return launch_stripe<float, 0>(p, plan, stream);
+      if (out_dtype == 1 && !swiglu) return launch_stripe<bf16_t, 0>(p, plan, stream);
+      if (out_dtype == 1 && p.gate.kind == kGateSilu) return launch_stripe<bf16_t, 1>(p, plan, stream);
+      if (out_dtype == 1) return launch_stripe<bf16_t, 2>(p, plan, stream);
+    }
+  }
   if (out_dtype == 0 && !swiglu) return launch_skinny<float, PRO, 0>(p, stream);
   if (out_dtype == 1 && !swiglu) return launch_skinny<bf16_t, PRO, 0>(p, stream);
   if (out_dtype == 1 && p.gate.kind == kGateSilu) return launch_skinny<bf16_t, PRO, 1>(p, stream);
@@ -2389,6 +2690,8 @@ static int f32_rows_col_tiles(int M, int N, int K, int cols, int* cols_wg = null
 }  // namespace
 
 extern "C" {
+
+int tl_linear_whole(int M, int N, int K);
 
 // Float32, at most 64 rows: out = rmsnorm(x; norm_w, eps) @ w.T, then the epilogue of tl_linear_tile
 // (0: + residual, 1: SiLU-gate), the norm inside the product's kernel.  Returns TL_ERR_ARG for sizes
@@ -2707,6 +3010,7 @@ int tl_linear_handoff(const void* a, const void* w, void* out, const float* resi
     p.emit_w_is_f32 = emit_w_dtype == 0 ? 1 : 0;
     p.emit_operand = (bf16_t*)emit_operand;
     p.emit_sumsq = emit_sumsq;
+    if (lda > T_MAX_INNER && tl_linear_whole(M, N, K)) return TL_ERR_ARG;      // its parts would not be tl_handoff_parts'
   }
   if (in_sumsq) {
     p.in_sumsq = in_sumsq;
@@ -2747,11 +3051,19 @@ int tl_linear_grouped(const void* a, const void* w, void* out, const int32_t* ti
   return tl_launch_status();
 }
 
+// Whether a bfloat16 product of these sizes keeps its inner size whole at 17 to 64 rows (see stripe_plan): it is not split then.
+int tl_linear_whole(int M, int N, int K) {
+  StripePlan plan;
+  return stripe_plan(M, N, K, &plan) ? 1 : 0;
+}
+
 // How many partial sums of squares per row tl_linear_handoff writes as a producer for these sizes
 // (few rows: one per workgroup, per 16 columns, or per 8 where workgroups own 8; beyond: one per 64
 // columns).
 int tl_handoff_parts(int M, int N, int K) {
   if (M > 64) return (N + 63) / 64;
+  StripePlan plan;
+  if (stripe_plan(M, N, K, &plan)) return (N + plan.cols - 1) / plan.cols;
   if (skinny_half(M, N, K)) return (N + 7) / 8;
   // one column tile a workgroup (see launch_skinny and launch_skinny_rows): a part per workgroup
   if (M <= 16 && N > 256 * S_COLS && N <= 4 * 256 * S_COLS) {       // two to four column tiles a workgroup

@@ -273,7 +273,9 @@ def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual: Option
             _fail("row scales are float32, one per row")
     if not (0 <= tile <= 4):
         _fail("tile is 0 (by size) or 1 to 4")
-    if dt == 1 and tile == 0 and M > 16:
+    whole = dt == 1 and linear_whole(M, N, K)
+    a = _near_rows(a, whole)
+    if dt == 1 and tile == 0 and M > 16 and not whole:
         splits = split_k(M, N, K)
         if splits > 1:
             return _linear_split(a, w, out, residual, code, row_scale, None, 0, 0.0, 0, None, splits, gate)
@@ -462,6 +464,24 @@ def split_k(rows: int, cols: int, inner: int) -> int:
 _SPLITS: dict = {}      # the plan is a pure function of the sizes
 
 
+def linear_whole(rows: int, cols: int, inner: int) -> bool:
+    """Whether the bfloat16 product [rows, inner] x [cols, inner]^T of 17 to 64 rows keeps its inner size whole, in one kernel: it
+    is then not split, whatever `split_k` says of its sizes."""
+    key = (rows, cols, inner)
+    n = _WHOLE.get(key)
+    if n is None:
+        n = _WHOLE[key] = 16 < rows <= FEW_ROWS and bool(_lib().tl_linear_whole(c_int(rows), c_int(cols), c_int(inner)))
+    return n
+
+
+_WHOLE: dict = {}
+WHOLE_MAX_STRIDE = 1 << 20      # elements between the input's rows: that kernel's offsets are 31 bits wide
+
+
+def _near_rows(a: torch.Tensor, whole: bool) -> torch.Tensor:
+    return a.contiguous() if whole and a.stride(0) > WHOLE_MAX_STRIDE else a
+
+
 def can_hand_off(rows: int, width: int, inner: int, dtype: torch.dtype) -> bool:
     """Whether `linear_handoff` can prepare a norm over `width` columns for `rows` rows, as the
     epilogue of the product with inner size `inner`: the few-row kernel, a product whose inner
@@ -475,7 +495,7 @@ def handoff_parts(rows: int, width: int, inner: int) -> int:
     """How many partial sums of squares per row the product [rows, inner] x [width, inner]^T writes
     when it prepares a norm: one per workgroup in the few-row kernel (16 or 8 columns), per 1024
     after a split inner size, per 64 in the tiled kernel."""
-    if split_k(rows, width, inner) > 1:
+    if split_k(rows, width, inner) > 1 and not linear_whole(rows, width, inner):
         return (width + 1023) // 1024
     if not (rows <= FEW_ROWS or width % 64 == 0):
         _fail(f"a norm is prepared for at most {FEW_ROWS} rows, with a split inner size or over a multiple of 64 columns")
@@ -523,7 +543,8 @@ def linear_handoff(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual
     M = a.shape[0] if rows is None else rows.numel()
     N = w.shape[0]
     swiglu = _epilogue(epilogue)
-    splits = split_k(M, N, K) if rows is None and M > 16 else 1
+    whole = linear_whole(M, N, K)
+    splits = split_k(M, N, K) if rows is None and M > 16 and not whole else 1
     if not (M > 0):
         _fail("no rows")
     if M > FEW_ROWS and splits == 1 and rows is not None:
@@ -567,6 +588,7 @@ def linear_handoff(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual
         if not (emit_sq.dtype == torch.float32 and emit_sq.is_contiguous()
                 and tuple(emit_sq.shape) == (M, handoff_parts(M, N, K))):
             _fail(f"sums of squares must be float32 [{M}, {handoff_parts(M, N, K)}]")
+    a = _near_rows(a, whole)
     if splits > 1:
         return _linear_split(a, w, out, residual, swiglu, None, sumsq_in, parts, eps, width, emit, splits)
     _check(_lib().tl_linear_handoff(

@@ -1637,3 +1637,49 @@ def test_linear_whole_inner_size(M, N, K):
 def test_long_inner_sizes_with_few_columns_are_split(M, K, N):
     assert not ops().linear_whole(M, N, K) and ops().split_k(M, N, K) > 1
     assert not ops().linear_whole(16, 2048, 2048) and not ops().linear_whole(65, 2048, 2048) and not ops().linear_whole(32, 2048, 2056)
+
+
+@pytest.mark.parametrize("T", [1, 6, 256, 257, 263])
+@pytest.mark.parametrize("K,experts,top,groups,keep,opts", [
+    (2048, 16, 4, 4, 2, {"score": "sigmoid", "group_top2": True}), (8, 1, 1, 1, 1, {}), (520, 5, 3, 1, 1, {"normalize": False}),
+    (2056, 17, 4, 1, 1, {}), (4104, 64, 9, 8, 4, {"score": "sigmoid"})])
+def test_router_in_one_kernel(T, K, experts, top, groups, keep, opts):
+    """Logits and choice in one kernel: one and four tokens a workgroup, more experts than waves, inner sizes that end within a
+    chunk.  The numbers are such that every order of addition gives the exact logits, so choice and weights are `moe_route`'s bits."""
+    g = torch.Generator().manual_seed(T + K + experts)
+    wide = torch.randint(-3, 4, (T, K + 8), generator=g).to(torch.bfloat16)
+    w = (torch.randint(-3, 4, (experts, K), generator=g) / 64).to(torch.bfloat16)
+    wide[T // 2, 3] = math.inf
+    z = (wide[:, :K].double() @ w.double().T).float()
+    bias, correction = (torch.randn(experts, generator=g) for _ in range(2))
+    for extra in ({}, {"bias": bias.to(DEV)}, {"correction": correction.to(DEV)}):
+        got = []
+        for call in (lambda *a, **o: ops().moe_route(z.to(DEV), *a, **o), lambda *a, **o: ops().moe_route_rows(wide.to(DEV)[:, :K], w.to(DEV), *a, **o)):
+            ids, wts = torch.full((T, top), -1, dtype=torch.int32, device=DEV), torch.full((T, top), -7.0, device=DEV)
+            call(ids, wts, groups, keep, 1.5, **extra, **opts)
+            got.append((ids.cpu(), wts.cpu()))
+        (want_ids, want_wts), (ids, wts) = got
+        assert ((ids >= 0) & (ids < experts)).all()
+        same = torch.arange(T) != T // 2      # the row with an infinity: NaN where it meets a zero, and then any expert may come
+        assert torch.equal(ids[same], want_ids[same]) and torch.equal(wts[same].view(torch.int32), want_wts[same].view(torch.int32))
+    with pytest.raises(Exception):
+        ops().moe_route_rows(wide.to(DEV)[:, :K], torch.zeros(65, K, dtype=torch.bfloat16, device=DEV), ids.to(DEV), wts.to(DEV))
+
+
+@pytest.mark.parametrize("T,cols", [(1, 3), (6, 1408), (257, 1025)])
+@pytest.mark.parametrize("experts", [16, 80])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_router_beside_an_activation(T, cols, experts, dtype):
+    """One kernel for both gives what the two give, by lanes and in the general form."""
+    g = torch.Generator().manual_seed(T + cols)
+    first = torch.randn(T, experts + cols, generator=g).to(DEV)
+    got = []
+    for one in (False, True):
+        ids, wts = torch.full((T, 4), -1, dtype=torch.int32, device=DEV), torch.full((T, 4), -7.0, device=DEV)
+        out = torch.full((T, cols), float("nan"), dtype=dtype, device=DEV)
+        beside = (first[:, experts:], out, "relu2")
+        ops().moe_route(first[:, :experts], ids, wts, 4, 2, 1.5, beside=beside if one else None)
+        if not one:
+            ops().activate_rows(*beside)
+        got.append((ids, wts, out))
+    assert all(torch.equal(x, y) for x, y in zip(*got)) and torch.isfinite(got[0][2]).all()

@@ -2570,6 +2570,10 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
   }
 }
 
+// Several groups of rows: those of one group of columns fall on one die and find its weights in the L2 (48 rows of 5,120 x 5,120,
+// three groups of 86 32.3 us where they fell on different dies, 19.3 so).
+static int stripe_grid_n(int groups_n, int groups_m) { return groups_m > 1 ? (groups_n + kXcds - 1) / kXcds * kXcds : groups_n; }
+
 template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
 static int launch_stripe_blocks(const SkinnyArgs& p, hipStream_t stream) {
   const auto kernel = gemm_stripe_bf16_kernel<MT, CT, TK, TO, SWIGLU, GATHER>;
@@ -2581,9 +2585,7 @@ static int launch_stripe_blocks(const SkinnyArgs& p, hipStream_t stream) {
   }
   const int vec = p.ldo % 4 == 0 && p.N % 4 == 0 && (uintptr_t)p.out % 16 == 0 && (uintptr_t)p.residual % 16 == 0 && (uintptr_t)p.emit_operand % 8 == 0;
   const int groups_n = (p.N + p.cols_wg - 1) / p.cols_wg, groups_m = (p.M + MT * 16 - 1) / (MT * 16);
-  // several groups of rows: those of one group of columns fall on one die and find its weights in the L2 (48 rows of 5,120 x
-  // 5,120, three groups of 86: 32.3 us where they fell on different dies, 19.3 so)
-  dim3 g(groups_m > 1 ? (groups_n + kXcds - 1) / kXcds * kXcds : groups_n, groups_m), b(S_THREADS);
+  dim3 g(stripe_grid_n(groups_n, groups_m), groups_m), b(S_THREADS);
   hipLaunchKernelGGL(kernel, g, b, smem, stream, p, groups_n, vec);
   return TL_OK;
 }
@@ -2617,11 +2619,12 @@ static bool stripe_plan(int M, int N, int K, StripePlan* plan) {
   int64_t least = 0;      // (of equal cuts the one with the fewest rows: 17 rows of 6,144 x 4,096 13.2 us in 1 x 3 tiles, 15.0 in 2 x 2)
   for (int mt = 1; mt <= tiles; ++mt)
     for (int ct = 1; ct <= 4; ++ct) {
-      const int64_t groups = (int64_t)((tiles + mt - 1) / mt) * ((N + 16 * ct - 1) / (16 * ct)), cost = (groups + 255) / 256 * (mt + ct);
+      const int groups_m = (tiles + mt - 1) / mt, groups_n = (N + 16 * ct - 1) / (16 * ct);
+      const int64_t groups = (int64_t)groups_m * stripe_grid_n(groups_n, groups_m), cost = (groups + 255) / 256 * (mt + ct);
       if (least && cost >= least) continue;
       least = cost;
       // one round of three or four column tiles: as many columns as make 256 workgroups (64 rows of 5,120 x 5,120 20.6 -> 19.0 us)
-      const int even = (int)((N * (int64_t)((tiles + mt - 1) / mt) + 255) / 256 + 3) / 4 * 4;
+      const int even = (int)((N * (int64_t)groups_m + 255) / 256 + 3) / 4 * 4;
       *plan = {mt, ct, groups <= 256 && ct >= 3 && even > 16 * (ct - 1) && even < 16 * ct ? even : 16 * ct};
     }
   int slabs;

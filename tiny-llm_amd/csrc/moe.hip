@@ -646,10 +646,17 @@ __device__ __forceinline__ Best wave_best(Best x) {
 __device__ __forceinline__ float lane_value(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
-__device__ __forceinline__ bool route_by_lanes(const float* zr, const float* bias, int32_t* ids, float* wts, int experts, int top,
-                                               int groups, int keep, float scale, int sigmoid, const float* correction,
-                                               int group_top2, int normalize) {
-  const int lane = threadIdx.x;
+struct RouteOptions {
+  const float* bias;
+  int experts, top, groups, keep;
+  float scale;
+  int sigmoid;
+  const float* correction;
+  int group_top2, normalize;
+};
+__device__ __forceinline__ bool route_by_lanes(const float* zr, const RouteOptions& o, int32_t* ids, float* wts, int lane) {
+  const float *bias = o.bias, *correction = o.correction;
+  const int experts = o.experts, top = o.top, groups = o.groups, keep = o.keep, sigmoid = o.sigmoid, group_top2 = o.group_top2;
   const bool in = lane < experts;
   float l = -INFINITY, extra = 0.f;
   if (in) {
@@ -696,7 +703,7 @@ __device__ __forceinline__ bool route_by_lanes(const float* zr, const float* bia
     const uint64_t at = __ballot(allowed && place == j);
     total += lane_value(score, __ffsll((unsigned long long)at) - 1);
   }
-  const float f = normalize ? scale / (total + 1e-20f) : scale;
+  const float f = o.normalize ? o.scale / (total + 1e-20f) : o.scale;
   if (allowed && place < top) {
     ids[place] = lane;
     wts[place] = score * f;
@@ -704,20 +711,18 @@ __device__ __forceinline__ bool route_by_lanes(const float* zr, const float* bia
   return true;
 }
 
-__global__ __launch_bounds__(TL_WAVE) void moe_route_kernel(const float* __restrict__ z, int64_t z_stride,
-                                                            const float* __restrict__ bias, int32_t* __restrict__ ids,
-                                                            float* __restrict__ wts, int experts, int top, int groups,
-                                                            int keep, float scale, int sigmoid,
-                                                            const float* __restrict__ correction, int group_top2,
-                                                            int normalize) {
-  __shared__ float s[kMaxRouted];         // choice scores; -inf once an expert is chosen or its run is out
-  __shared__ float gs[kMaxRouted];        // the runs' scores
-  __shared__ float plain[kMaxRouted];     // scores without the correction
-  const int t = blockIdx.x, lane = threadIdx.x;
-  const float* zr = z + (int64_t)t * z_stride;
-  if (experts <= TL_WAVE && route_by_lanes(zr, bias, ids + (int64_t)t * top, wts + (int64_t)t * top, experts, top, groups, keep,
-                                           scale, sigmoid, correction, group_top2, normalize))
-    return;
+// What the lanes of ONE wave have written to LDS is there for all of them (its LDS instructions run in order).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The general form, by one wave.  s: choice scores, -inf once an expert is chosen or its run is out; gs: the runs' scores;
+// plain: scores without the correction (all in LDS, o.experts long).
+__device__ void route_general(const float* zr, const RouteOptions& o, int32_t* ids, float* wts, int lane, float* s, float* gs, float* plain) {
+  const float *bias = o.bias, *correction = o.correction;
+  const int experts = o.experts, top = o.top, groups = o.groups, keep = o.keep, sigmoid = o.sigmoid, group_top2 = o.group_top2;
   float m = -INFINITY;
   for (int e = lane; e < experts; e += TL_WAVE) {     // the logits (a bias per expert added), kept in s for the next pass
     const float l = bias ? zr[e] + bias[e] : zr[e];
@@ -744,7 +749,7 @@ __global__ __launch_bounds__(TL_WAVE) void moe_route_kernel(const float* __restr
       s[e] += correction[e];
     }
   }
-  __syncthreads();
+  wave_sync();
   if (groups > 1 && keep < groups) {
     const int per = experts / groups;
     for (int g = lane; g < groups; g += TL_WAVE) {
@@ -755,18 +760,18 @@ __global__ __launch_bounds__(TL_WAVE) void moe_route_kernel(const float* __restr
       }
       gs[g] = group_top2 && per > 1 ? b + second : b;
     }
-    __syncthreads();
+    wave_sync();
     for (int k = 0; k < keep; ++k) {      // the best runs, one a pass; a kept run is marked with -inf
       Best b = {-INFINITY, 0x7fffffff};
       for (int g = lane; g < groups; g += TL_WAVE) b = better(b, Best{gs[g], g});
       b = wave_best(b);
-      __syncthreads();
+      wave_sync();
       if (lane == 0) gs[min(b.i, groups - 1)] = -INFINITY;      // (no index at all: every score is NaN)
-      __syncthreads();
+      wave_sync();
     }
     for (int e = lane; e < experts; e += TL_WAVE)
       if (gs[e / per] != -INFINITY) s[e] = -INFINITY;
-    __syncthreads();
+    wave_sync();
   }
   float total = 0.f;
   for (int j = 0; j < top; ++j) {         // the best of what is left, one a pass; gs now keeps the chosen scores
@@ -774,18 +779,115 @@ __global__ __launch_bounds__(TL_WAVE) void moe_route_kernel(const float* __restr
     for (int e = lane; e < experts; e += TL_WAVE) b = better(b, Best{s[e], e});
     b = wave_best(b);
     b.i = min(b.i, experts - 1);
-    __syncthreads();
+    wave_sync();
     const float score = correction ? plain[b.i] : b.v;
     if (lane == 0) {
       s[b.i] = -INFINITY;
       gs[j] = score;
-      ids[(int64_t)t * top + j] = b.i;
+      ids[j] = b.i;
     }
     total += score;
-    __syncthreads();
+    wave_sync();
   }
-  const float f = normalize ? scale / (total + 1e-20f) : scale;
-  for (int j = lane; j < top; j += TL_WAVE) wts[(int64_t)t * top + j] = gs[j] * f;
+  const float f = o.normalize ? o.scale / (total + 1e-20f) : o.scale;
+  for (int j = lane; j < top; j += TL_WAVE) wts[j] = gs[j] * f;
+}
+
+__global__ __launch_bounds__(TL_WAVE) void moe_route_kernel(const float* __restrict__ z, int64_t z_stride, RouteOptions o,
+                                                            int32_t* __restrict__ ids, float* __restrict__ wts) {
+  __shared__ float s[kMaxRouted], gs[kMaxRouted], plain[kMaxRouted];
+  const int t = blockIdx.x;
+  const float* zr = z + (int64_t)t * z_stride;
+  ids += (int64_t)t * o.top;
+  wts += (int64_t)t * o.top;
+  if (o.experts <= TL_WAVE && route_by_lanes(zr, o, ids, wts, threadIdx.x)) return;
+  route_general(zr, o, ids, wts, threadIdx.x, s, gs, plain);
+}
+
+// The same beside the activation of a shared expert's first product, whose columns lie behind the logits: blocks from n_tokens on
+// form out[t, c] = act(hidden[t, c]), 1,024 numbers each.  Neither waits for the other, and a decode step has a launch less (six
+// tokens, 16 experts, 1,408 columns: 5.0 -> 3.5 us).
+template <typename TO>
+__global__ __launch_bounds__(kThreads) void moe_route_beside_kernel(const float* __restrict__ z, int64_t z_stride, RouteOptions o,
+                                                                   int32_t* __restrict__ ids, float* __restrict__ wts, int n_tokens,
+                                                                   const float* __restrict__ hidden, TO* __restrict__ out, int cols,
+                                                                   int64_t total, int act) {
+  __shared__ float s[kMaxRouted], gs[kMaxRouted], plain[kMaxRouted];
+  const int t = blockIdx.x;
+  if (t < n_tokens) {
+    if (threadIdx.x >= TL_WAVE) return;
+    const float* zr = z + (int64_t)t * z_stride;
+    ids += (int64_t)t * o.top;
+    wts += (int64_t)t * o.top;
+    if (o.experts <= TL_WAVE && route_by_lanes(zr, o, ids, wts, threadIdx.x)) return;
+    route_general(zr, o, ids, wts, threadIdx.x, s, gs, plain);
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t i = ((int64_t)(t - n_tokens) * 4 + u) * kThreads + threadIdx.x;
+    if (i >= total) return;
+    const int64_t r = i / cols;
+    out[i] = from_f32<TO>(activate(hidden[r * z_stride + (i - r * cols)], act));
+  }
+}
+
+// A router whole, for at most 64 experts: its logits a [n_tokens, K] x w [experts, K] (bfloat16, float32 sums: a wave an expert at a
+// time, its lanes stride over the inner size, then a butterfly) and the choice, ROWS tokens a workgroup.  A product of 16 columns is no
+// work for the chip: six tokens, 16 experts, inner size 2,048 take 6.9 us as a product and a
+// choice and 4.6 so; 1,944 tokens, for which the tiled product spends a tile of 128 columns on 16, 13.8 and 10.4.  Four tokens a workgroup from 257 on: it fetches the weights (64 KB) once for them.
+constexpr int kRouteWaves = 16, kRouteFewRows = 256;
+template <int ROWS>
+__global__ __launch_bounds__(kRouteWaves * TL_WAVE) void moe_route_rows_kernel(const bf16_t* __restrict__ a, int64_t a_stride,
+                                                                              const bf16_t* __restrict__ w, int n_tokens, int K,
+                                                                              RouteOptions o, int32_t* __restrict__ ids,
+                                                                              float* __restrict__ wts) {
+  __shared__ float z[ROWS][TL_WAVE], s[ROWS][TL_WAVE], gs[ROWS][TL_WAVE], plain[ROWS][TL_WAVE];
+  const int lane = threadIdx.x % TL_WAVE, wave = threadIdx.x / TL_WAVE, t0 = blockIdx.x * ROWS;
+  constexpr int kAhead = ROWS == 1 ? 4 : 2, kStep = TL_WAVE * 8;      // chunks of 512 k on their way together
+  const bf16_t* row[ROWS];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) row[r] = a + (int64_t)min(t0 + r, n_tokens - 1) * a_stride;
+  for (int e = wave; e < o.experts; e += kRouteWaves) {
+    const bf16_t* we = w + (int64_t)e * K;
+    float acc[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) acc[r] = 0.f;
+    for (int k0 = lane * 8; k0 < K; k0 += kAhead * kStep) {
+      bf16x8 x[ROWS][kAhead], y[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int k = min(k0 + u * kStep, K - 8);
+        y[u] = *(const bf16x8*)(we + k);
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) x[r][u] = *(const bf16x8*)(row[r] + k);
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float v = fmaf((float)x[r][u][j], (float)y[u][j], acc[r]);
+            acc[r] = k0 + u * kStep < K ? v : acc[r];
+          }
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const float v = wave_sum(acc[r]);
+      if (lane == 0) z[r][e] = v;
+    }
+  }
+  __syncthreads();
+  if (wave >= ROWS || t0 + wave >= n_tokens) return;
+  ids += (int64_t)(t0 + wave) * o.top;
+  wts += (int64_t)(t0 + wave) * o.top;
+  if (!route_by_lanes(z[wave], o, ids, wts, lane)) route_general(z[wave], o, ids, wts, lane, s[wave], gs[wave], plain[wave]);
+}
+
+static bool route_ok(const RouteOptions& o) {
+  return o.experts > 0 && o.top > 0 && o.top <= o.experts && o.groups >= 0 &&
+         !(o.groups > 1 && (o.experts % o.groups || o.keep <= 0 || o.keep > o.groups || o.top > o.keep * (o.experts / o.groups)));
 }
 
 // out[i] = act(in[i]) over rows of `cols` elements (the input's rows may be wider).
@@ -994,11 +1096,48 @@ int tl_moe_route(const float* z, int64_t z_stride, const float* bias, int32_t* i
                  int top, int groups, int keep, float scale, int sigmoid, const float* correction, int group_top2,
                  int normalize, hipStream_t stream) {
   if (n_tokens <= 0) return TL_OK;
-  if (experts <= 0 || experts > kMaxRouted || top <= 0 || top > experts || z_stride < experts || !z || !ids || !wts ||
-      groups < 0 || (groups > 1 && (experts % groups || keep <= 0 || keep > groups || top > keep * (experts / groups))))
+  const RouteOptions o{bias, experts, top, groups, keep, scale, sigmoid, correction, group_top2, normalize};
+  if (experts > kMaxRouted || !route_ok(o) || z_stride < experts || !z || !ids || !wts) return TL_ERR_ARG;
+  hipLaunchKernelGGL(moe_route_kernel, dim3(n_tokens), dim3(TL_WAVE), 0, stream, z, z_stride, o, ids, wts);
+  return tl_launch_status();
+}
+
+// The same, and out [n_tokens, cols] (contiguous, float32 0 or bfloat16 1) = act(hidden), hidden's rows as far apart as the logits'.
+int tl_moe_route_beside(const float* z, int64_t z_stride, const float* bias, int32_t* ids, float* wts, int n_tokens, int experts,
+                        int top, int groups, int keep, float scale, int sigmoid, const float* correction, int group_top2,
+                        int normalize, const float* hidden, void* out, int cols, int act, int dtype_out, hipStream_t stream) {
+  if (n_tokens <= 0) return TL_OK;
+  const RouteOptions o{bias, experts, top, groups, keep, scale, sigmoid, correction, group_top2, normalize};
+  if (experts > kMaxRouted || !route_ok(o) || z_stride < experts || !z || !ids || !wts || cols <= 0 || z_stride < cols || !hidden || !out ||
+      (act != kActNone && act != kActRelu2) || (dtype_out != 0 && dtype_out != 1))
     return TL_ERR_ARG;
-  hipLaunchKernelGGL(moe_route_kernel, dim3(n_tokens), dim3(TL_WAVE), 0, stream, z, z_stride, bias, ids, wts, experts, top,
-                     groups, keep, scale, sigmoid, correction, group_top2, normalize);
+  const int64_t total = (int64_t)n_tokens * cols, blocks = n_tokens + ceil_div64(total, 4 * kThreads);
+  if (blocks > 0x7fffffff) return TL_ERR_ARG;
+  if (dtype_out == 0)
+    hipLaunchKernelGGL(moe_route_beside_kernel<float>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, z, z_stride, o, ids, wts,
+                       n_tokens, hidden, (float*)out, cols, total, act);
+  else
+    hipLaunchKernelGGL(moe_route_beside_kernel<bf16_t>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, z, z_stride, o, ids, wts,
+                       n_tokens, hidden, (bf16_t*)out, cols, total, act);
+  return tl_launch_status();
+}
+
+// The same of the logits a [n_tokens, K] (bfloat16, rows a_stride apart) x w [experts, K]^T, for at most 64 experts; rows and
+// weights at multiples of 16 bytes.
+int tl_moe_route_rows(const void* a, int64_t a_stride, const void* w, const float* bias, int32_t* ids, float* wts, int n_tokens,
+                      int K, int experts, int top, int groups, int keep, float scale, int sigmoid, const float* correction,
+                      int group_top2, int normalize, hipStream_t stream) {
+  if (n_tokens <= 0) return TL_OK;
+  const RouteOptions o{bias, experts, top, groups, keep, scale, sigmoid, correction, group_top2, normalize};
+  if (experts > TL_WAVE || !route_ok(o) || K <= 0 || K % 8 || a_stride % 8 || a_stride < K || !a || !w || !ids || !wts ||
+      (((uintptr_t)a | (uintptr_t)w) & 15))
+    return TL_ERR_ARG;
+  if (n_tokens <= kRouteFewRows)
+    hipLaunchKernelGGL(moe_route_rows_kernel<1>, dim3(n_tokens), dim3(kRouteWaves * TL_WAVE), 0, stream, (const bf16_t*)a, a_stride,
+                       (const bf16_t*)w, n_tokens, K, o, ids, wts);
+  else
+    hipLaunchKernelGGL(moe_route_rows_kernel<4>, dim3((n_tokens + 3) / 4), dim3(kRouteWaves * TL_WAVE), 0, stream, (const bf16_t*)a,
+                       a_stride, (const bf16_t*)w, n_tokens, K, o, ids, wts);
   return tl_launch_status();
 }
 

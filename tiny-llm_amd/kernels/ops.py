@@ -2503,7 +2503,7 @@ MOE_SCORES = ("softmax", "sigmoid")
 
 def moe_route(z: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, groups: int = 1, keep: int = 1,
               scale: float = 1.0, bias: Optional[torch.Tensor] = None, score: str = "softmax",
-              correction: Optional[torch.Tensor] = None, group_top2: bool = False, normalize: bool = True) -> None:
+              correction: Optional[torch.Tensor] = None, group_top2: bool = False, normalize: bool = True, beside=None) -> None:
     """A router over the logits z (float32 [T, E], rows may be wider apart; `bias`, float32 [E], is added to every
     row if given): scores s = softmax(z) over all experts;
     the experts lie in `groups` equal runs of neighbours, a run's score is its largest, and only experts of the
@@ -2512,7 +2512,8 @@ def moe_route(z: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, groups:
     their scores / (their sum + 1e-20) * scale.
     Options: `score` "sigmoid" (s = sigmoid(z)); `correction` (float32 [E]) is added to the scores wherever experts or
     runs are chosen, never to the weights; `group_top2`: a run is ranked by its two best experts together; `normalize` False:
-    the weights are the scores * scale."""
+    the weights are the scores * scale.  `beside`: (x, out, act) as `activate_rows` takes them, x float32 of z's row stride, done
+    by the same kernel."""
     _dev(z, ids, weights, correction)
     _f32_vec(correction, z.shape[1], "moe_route correction")
     _need(score in MOE_SCORES, f"moe_route: scores {score!r} are not built")
@@ -2530,10 +2531,58 @@ def moe_route(z: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, groups:
     if groups > 1:
         _need(E % groups == 0 and 0 < keep <= groups and top <= keep * (E // groups),
               "moe_route: equal groups, 1 to `groups` of them kept, holding at least `top` experts")
-    _check(_lib().tl_moe_route(_ptr(z), c_int64(z.stride(0)), _ptr(bias), _ptr(ids), _ptr(weights), c_int(T), c_int(E), c_int(top),
-                               c_int(groups), c_int(keep), c_float(scale), c_int(MOE_SCORES.index(score)),
-                               _ptr(correction), c_int(1 if group_top2 else 0), c_int(1 if normalize else 0), _stream()),
-           "moe_route")
+    args = (_ptr(z), c_int64(z.stride(0)), _ptr(bias), _ptr(ids), _ptr(weights), c_int(T), c_int(E), c_int(top), c_int(groups),
+            c_int(keep), c_float(scale), c_int(MOE_SCORES.index(score)), _ptr(correction), c_int(1 if group_top2 else 0),
+            c_int(1 if normalize else 0))
+    if beside is None:
+        _check(_lib().tl_moe_route(*args, _stream()), "moe_route")
+        return
+    x, out, act = beside
+    _dev(x, out)
+    _rows_2d(x, "moe_route: the rows beside")
+    _need(act in MOE_ACTIVATIONS, f"moe_route: activation {act!r} is not built")
+    _need(x.dtype == torch.float32 and x.stride(0) == z.stride(0) and x.shape[0] == T and out.is_contiguous() and out.shape == x.shape,
+          "moe_route: the rows beside are float32, as far apart as the logits', their results contiguous")
+    _check(_lib().tl_moe_route_beside(*args, _ptr(x), _ptr(out), c_int(x.shape[1]), c_int(MOE_ACTIVATIONS[act]), c_int(_dt(out)),
+                                      _stream()), "moe_route_beside")
+
+
+def moe_route_rows_ok(dtype: torch.dtype, experts: int, inner: int) -> bool:
+    """Whether `moe_route_rows` takes a router of these sizes."""
+    return dtype == torch.bfloat16 and 0 < experts <= 64 and inner % 8 == 0
+
+
+def moe_route_rows_pay(rows: int, experts: int, inner: int) -> bool:
+    """Where one kernel is faster than the product and `moe_route`: every workgroup of it fetches the weights, so up to 64 K of them,
+    and not for the longest prompts (16 experts of 2,048: 6 rows 6.9 -> 4.6 us, 256 10.4 -> 4.9, 1,944 13.8 -> 10.4, 4,096 17.7 and
+    18.0; 64 experts of 4,096: 6 rows 10.8 and 15.1)."""
+    return experts * inner <= 1 << 16 and rows <= 2048
+
+
+def moe_route_rows(h: torch.Tensor, w: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, groups: int = 1, keep: int = 1,
+                   scale: float = 1.0, bias: Optional[torch.Tensor] = None, score: str = "softmax",
+                   correction: Optional[torch.Tensor] = None, group_top2: bool = False, normalize: bool = True) -> None:
+    """`moe_route` of the logits h @ w.T (h [T, K], w [E, K], bfloat16, up to 64 experts; float32 sums), in one kernel with them."""
+    _dev(h, w, ids, weights, correction, bias)
+    _rows_2d(h, "moe_route_rows input")
+    T, K = h.shape
+    _need(w.dim() == 2 and w.is_contiguous() and w.shape[1] == K, f"moe_route_rows: weights are contiguous [E, {K}]")
+    E, top = w.shape[0], ids.shape[1] if ids.dim() == 2 else 0
+    _need(h.dtype == w.dtype and moe_route_rows_ok(h.dtype, E, K) and h.stride(0) % 8 == 0,
+          "moe_route_rows: bfloat16, up to 64 experts, rows of a multiple of 8")
+    _need(score in MOE_SCORES, f"moe_route_rows: scores {score!r} are not built")
+    _need(ids.dtype == torch.int32 and ids.is_contiguous() and tuple(ids.shape) == (T, top) and 0 < top <= E,
+          "moe_route_rows: ids are contiguous int32 [T, top], top within the experts")
+    _f32_vec(weights, T * top, "moe_route_rows weights")
+    _f32_vec(bias, E, "moe_route_rows bias")
+    _f32_vec(correction, E, "moe_route_rows correction")
+    if groups > 1:
+        _need(E % groups == 0 and 0 < keep <= groups and top <= keep * (E // groups),
+              "moe_route_rows: equal groups, 1 to `groups` of them kept, holding at least `top` experts")
+    _check(_lib().tl_moe_route_rows(_ptr(h, 16), c_int64(h.stride(0)), _ptr(w, 16), _ptr(bias), _ptr(ids), _ptr(weights), c_int(T),
+                                    c_int(K), c_int(E), c_int(top), c_int(groups), c_int(keep), c_float(scale),
+                                    c_int(MOE_SCORES.index(score)), _ptr(correction), c_int(1 if group_top2 else 0),
+                                    c_int(1 if normalize else 0), _stream()), "moe_route_rows")
 
 
 def activate_rows(x: torch.Tensor, out: torch.Tensor, act: Optional[str]) -> torch.Tensor:

@@ -178,6 +178,7 @@ class RoutedMoE(FeedForward):
                                  intermediate_size=int(shared["intermediate_size"]),
                                  activation=shared.get("activation", activation))
         self.w_up = self.w_down = self.w_router = None
+        self.route_whole = ops.moe_route_rows_ok(dtype, self.num_experts, self.hidden_size)      # logits and choice in one kernel
 
     def weights(self) -> List[WeightSpec]:
         p, W, F = self.prefix, self.hidden_size, self.intermediate_size
@@ -231,14 +232,17 @@ class RoutedMoE(FeedForward):
             Fs = self.shared.intermediate_size
             first = ops.scratch("moe_first", (T, self.shared_off + Fs), torch.float32, dev)
             ops.linear(h, self.w_first, first)
-            ops.moe_route(first[:, :E], ids, wts, self.groups, self.keep, self.scale, self.b_router,
-                          correction=self.correction_w, **self.route_options)
-            zs = ops.activate_rows(first[:, self.shared_off:], ops.scratch("ffn_gated", (T, Fs), self.dtype, dev),
-                                   self.shared.activation)
+            zs = ops.scratch("ffn_gated", (T, Fs), self.dtype, dev)
+            ops.moe_route(first[:, :E], ids, wts, self.groups, self.keep, self.scale, self.b_router, correction=self.correction_w,
+                          beside=(first[:, self.shared_off:], zs, self.shared.activation), **self.route_options)
             if residual is None:
                 base = ops.linear(zs, self.shared.w_down, ops.scratch("sublayer_out", (T, self.hidden_size), torch.float32, dev))
             else:
                 base = ops.linear(zs, self.shared.w_down, residual, residual)
+        elif self.route_whole and ops.moe_route_rows_pay(T, E, self.hidden_size):
+            ops.moe_route_rows(h, self.w_router, ids, wts, self.groups, self.keep, self.scale, self.b_router,
+                               correction=self.correction_w, **self.route_options)
+            base = residual
         else:
             logits = ops.scratch("moe_router", (T, E), torch.float32, dev)
             ops.linear(h, self.w_router, logits)

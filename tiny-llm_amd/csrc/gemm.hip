@@ -13,9 +13,9 @@
 //    registers into two (v_mfma_f32_32x32x16_bf16; tile_mode says where); optionally over a share of the inner size (split k).
 //  * gemm_oneshot_bf16_kernel: the split product for few rows, operands streamed through a ring of
 //    LDS slabs filled straight from memory; splitk_reduce_kernel adds the parts and applies the epilogue.
-//  * gemm_skinny_bf16_kernel: at most 16 rows (decode steps), weights streamed once into registers; up to 64 for inner sizes that
+//  * gemm_skinny_bf16_kernel: the fewest rows (decode steps), weights streamed once into registers; up to 64 for inner sizes that
 //    are no multiple of 64.
-//  * gemm_stripe_bf16_kernel: 17 to 64 rows, the inner size whole.
+//  * gemm_stripe_bf16_kernel: 6 to 64 rows (stripe_plan says which), the inner size whole.
 #include <type_traits>
 
 #include "common.h"
@@ -2360,7 +2360,7 @@ static int launch_skinny(const SkinnyArgs& p, hipStream_t stream) {
   return TL_ERR_ARG;
 }
 
-// ============================================================ bfloat16, 17 to 64 rows
+// ============================================================ bfloat16, 6 to 64 rows
 // Bound by what a unit fetches: every workgroup needs its activation rows (64 of them are 256 KB at an inner size of 2,048, beside
 // 180 KB of weights), and a unit gets about 105 GB/s from its L2 in loads that take whole lines of 128 bytes (138 alone), but 37
 // in the matrix instructions' own order, 64 bytes of each of sixteen rows, in which gemm_skinny_bf16_kernel loads.  So a wave fetches
@@ -2457,6 +2457,24 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
           acc[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ct], fa[mt], acc[mt][ct], 0, 0, 0);
     }
   };
+  // The parts of the rows' sums of squares are requested ahead of everything else, up to 256 of a row together, and added up once the
+  // first block has been requested (behind it, and one request after the other: a decode step of 8 rows 3.4 % slower).
+  constexpr int RPW = S::kRows / S_WAVES, PRE = 4;      // rows a wave, requests a row
+  float pre[RPW][PRE];
+  const float* row_sq[RPW];
+  if (p.in_sumsq) {
+#pragma unroll
+    for (int ri = 0; ri < RPW; ++ri) {
+      const int m = min(m0 + wave * RPW + ri, M - 1);
+      row_sq[ri] = p.in_sumsq + (int64_t)(GATHER ? p.rows[m] : m) * p.in_parts;
+#pragma unroll
+      for (int h = 0; h < PRE; ++h) {
+        pre[ri][h] = 0.f;
+        if (h * TL_WAVE >= p.in_parts) continue;      // uniform
+        if (lane + h * TL_WAVE < p.in_parts) pre[ri][h] = row_sq[ri][lane + h * TL_WAVE];
+      }
+    }
+  }
   Block st;
   load(st, 0);
 
@@ -2483,19 +2501,12 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
     }
   }
   if (p.in_sumsq) {      // the rows' factors: one wave a row, in a fixed order
-    constexpr int RPW = S::kRows / S_WAVES;
-    float t[RPW];
 #pragma unroll
     for (int ri = 0; ri < RPW; ++ri) {
-      const int m = min(m0 + wave * RPW + ri, M - 1);
-      const float* row = p.in_sumsq + (int64_t)(GATHER ? p.rows[m] : m) * p.in_parts;
-      t[ri] = lane < p.in_parts ? row[lane] : 0.f;
-      for (int q = lane + TL_WAVE; q < p.in_parts; q += TL_WAVE) t[ri] += row[q];
-    }
-#pragma unroll
-    for (int ri = 0; ri < RPW; ++ri) {
-      const float s = wave_sum(t[ri]);
-      if (lane == 0) scale_s[wave * RPW + ri] = 1.f / sqrtf(s / (float)p.in_width + p.in_eps);
+      float t = (pre[ri][0] + pre[ri][1]) + (pre[ri][2] + pre[ri][3]);
+      for (int q = lane + PRE * TL_WAVE; q < p.in_parts; q += TL_WAVE) t += row_sq[ri][q];
+      t = wave_sum(t);
+      if (lane == 0) scale_s[wave * RPW + ri] = 1.f / sqrtf(t / (float)p.in_width + p.in_eps);
     }
   }
 
@@ -2592,41 +2603,54 @@ static int launch_stripe_blocks(const SkinnyArgs& p, hipStream_t stream) {
 
 template <int MT, int CT, typename TO, int SWIGLU>
 static int launch_stripe_tile(const SkinnyArgs& p, hipStream_t stream) {
+  // (four tiles of a short inner size go by shorter blocks: 64 rows of 2,560 x 2,048 in 2 x 2 tiles 7.8 us and 7.3, 16 of 11,264 x
+  // 2,048 in 1 x 3 12.4 and 11.6, but 17 of 6,144 x 4,096 in 1 x 3 13.2 and 14.1)
+  const bool long_blocks = p.K % 128 == 0 && (MT + CT <= 3 || p.K > 2048);
   if constexpr (sizeof(TO) == 4) {      // the output head's
     if (p.rows) {
       if constexpr (MT + CT <= 4)
-        if (p.K % 128 == 0) return launch_stripe_blocks<MT, CT, 128, TO, SWIGLU, true>(p, stream);
+        if (long_blocks) return launch_stripe_blocks<MT, CT, 128, TO, SWIGLU, true>(p, stream);
       return launch_stripe_blocks<MT, CT, 64, TO, SWIGLU, true>(p, stream);
     }
   }
   if constexpr (MT + CT <= 4)
-    if (p.K % 128 == 0) return launch_stripe_blocks<MT, CT, 128, TO, SWIGLU, false>(p, stream);
+    if (long_blocks) return launch_stripe_blocks<MT, CT, 128, TO, SWIGLU, false>(p, stream);
   return launch_stripe_blocks<MT, CT, 64, TO, SWIGLU, false>(p, stream);
 }
 
-// How this kernel takes a product of 17 to 64 rows, as tiles of sixteen rows and of sixteen columns a workgroup (false: not it).  A
-// workgroup's time goes by the rows that it fetches, of both operands, so the cheapest cut of the product has the smallest sum of
-// both, times the rounds of workgroups that it makes over the 256 units.  Timed for fifteen matrices of 1,024 x 704 to 27,648 x
-// 5,120 at 17, 32, 48 and 64 rows, every cut of each (1,270 in all): the one this picks is within 3 % of the fastest, 0.05 % on average.
-// The estimate (us) is compared with the split product's own (oneshot_plan; 4 us for its second launch), which is the faster way
-// for long inner sizes and few columns: 64 rows of 14,336 by 4,096 37.4 us here and 29.9 split; 5,120 x 5,120 19.0 and 19.7.
+// How this kernel takes a product of 6 to 64 rows, as tiles of sixteen rows and of sixteen columns a workgroup and the columns that
+// it owns of them (false: not it).  A workgroup's time goes by the rows that it fetches, of both operands, so the cheapest cut of the product has
+// the smallest sum of both, times the rounds of workgroups that it makes over the 256 units.  Timed for fifteen matrices of 1,024 x 704 to
+// 27,648 x 5,120 at 17, 32, 48 and 64 rows, every cut of each (1,270 in all): the one this picks is within 3 % of the fastest, 0.05 % on average.
+//  * Beyond 16 rows the estimate (us) is compared with the split product's own (oneshot_us; 4 us for its second launch), which is the
+//    faster way for long inner sizes and few columns: 64 rows of 14,336 by 4,096 37.4 us here and 29.9 split; 5,120 x 5,120 19.0 and 19.7.
+//  * 9 to 16 rows: faster than the few-row kernel at each of eleven matrices (16 rows: 2,560 x 2,048 5.9 -> 5.0 us, 2,048 x 2,048 5.7 ->
+//    4.6, 2,048 x 5,632 11.8 -> 9.0, 11,264 x 2,048 gated 12.8 -> 11.6, 4,096 x 14,336 34.7 -> 26.2).
+//  * 6 to 8 rows: in one round, where the few-row kernel has no form of eight columns and a workgroup's columns are not just one
+//    tile of a short inner size (8 rows: 2,560 x 2,048 5.2 -> 4.7, 11,264 x 2,048 12.1 -> 11.6, 6,144 x 4,096 13.1 -> 11.7, 4,096 x
+//    14,336 28.9 -> 25.2, but 4,096 x 4,096 9.7 and 10.0, 2,048 x 2,048 4.6 both).  At 1 row the few-row kernel is the faster one.
 struct StripePlan {
   int mt, ct, cols;
 };
 static bool stripe_plan(int M, int N, int K, StripePlan* plan) {
-  if (M <= 16 || M > 64 || K % 64 || K > T_MAX_INNER) return false;
+  if (M < 6 || M > 64 || K % 64 || K > T_MAX_INNER) return false;
   const int tiles = (M + 15) / 16;
-  int64_t least = 0;      // (of equal cuts the one with the fewest rows: 17 rows of 6,144 x 4,096 13.2 us in 1 x 3 tiles, 15.0 in 2 x 2)
+  int64_t least = 0, fewest = 0;      // (of equal cuts the one with the fewest rows: 17 rows of 6,144 x 4,096 13.2 us in 1 x 3 tiles, 15.0 in 2 x 2)
   for (int mt = 1; mt <= tiles; ++mt)
     for (int ct = 1; ct <= 4; ++ct) {
       const int groups_m = (tiles + mt - 1) / mt, groups_n = (N + 16 * ct - 1) / (16 * ct);
       const int64_t groups = (int64_t)groups_m * stripe_grid_n(groups_n, groups_m), cost = (groups + 255) / 256 * (mt + ct);
       if (least && cost >= least) continue;
       least = cost;
-      // one round of three or four column tiles: as many columns as make 256 workgroups (64 rows of 5,120 x 5,120 20.6 -> 19.0 us)
-      const int even = (int)((N * (int64_t)groups_m + 255) / 256 + 3) / 4 * 4;
-      *plan = {mt, ct, groups <= 256 && ct >= 3 && even > 16 * (ct - 1) && even < 16 * ct ? even : 16 * ct};
+      fewest = groups;
+      // one round of three or four column tiles, or of up to 16 rows: as many columns as make 256 workgroups, at least 8 (64 rows of
+      // 5,120 x 5,120 20.6 -> 19.0 us, 16 rows of 2,048 x 5,632 10.3 -> 9.0)
+      int even = (int)((N * (int64_t)groups_m + 255) / 256 + 3) / 4 * 4;
+      if (tiles == 1 && even < 8) even = 8;
+      *plan = {mt, ct, groups <= 256 && (ct >= 3 || tiles == 1) && even > 16 * (ct - 1) && even < 16 * ct ? even : 16 * ct};
     }
+  if (M <= 8) return fewest <= 256 && N > 2048 && (plan->cols != 16 || K > 4096);
+  if (M <= 16) return true;
   int slabs;
   if (oneshot_plan(M, N, K, &slabs) < 2) return true;
   return 2.4 + least * (K * 32 * 1.23e-5) + (double)N * K * 2 * 0.66 / 5.75e6 <= oneshot_us(M, N, K, slabs) + 4.0;
@@ -3054,7 +3078,7 @@ int tl_linear_grouped(const void* a, const void* w, void* out, const int32_t* ti
   return tl_launch_status();
 }
 
-// Whether a bfloat16 product of these sizes keeps its inner size whole at 17 to 64 rows (see stripe_plan): it is not split then.
+// Whether a bfloat16 product of these sizes is gemm_stripe_bf16_kernel's (see stripe_plan): it is not split then.
 int tl_linear_whole(int M, int N, int K) {
   StripePlan plan;
   return stripe_plan(M, N, K, &plan) ? 1 : 0;

@@ -545,13 +545,13 @@ static int launch_f32_ring_any(const float* a, const float* w, float* out, const
   return TL_ERR_ARG;
 }
 
-// The same product for few rows (decode steps): the weights stream once, straight from memory
-// into the matrix instruction's operand registers.  A workgroup owns 16 output columns (8 where
+// The same product for 17 to 64 rows (and up to 256 where the tiled kernel has too few tiles), and with a norm in front: the weights stream
+// once, straight from memory into the matrix instruction's operand registers.  A workgroup owns 16 output columns (8 with a norm where
 // 16 would leave compute units without work: the matrix tile's other 8 rows then repeat them and
 // are dropped); its eight waves deal the k blocks of 256 out among themselves, a wave requests a
-// whole block (16 KB) at once and the next one before it multiplies; the block sums meet in LDS and
+// whole block (16 KB) at once; the block sums meet in LDS and
 // are added in ascending order: the order of gemm_f32_kernel, to the bit.  Rows come in tiles of
-// 16 (up to four).
+// 16.  (Up to 16 rows: gemm_f32_lines_kernel.)
 constexpr int FR_WAVES = 8, FR_THREADS = FR_WAVES * TL_WAVE, FR_MAX_MT = 4;
 
 //
@@ -561,20 +561,6 @@ constexpr int FR_WAVES = 8, FR_THREADS = FR_WAVES * TL_WAVE, FR_MAX_MT = 4;
 // blocks in ascending order, so a row's factor depends on nothing but the row), and the factor is
 // applied to the block sums' total.  That saves the norm's kernel in front of the product.
 //
-// CT (one row tile only): a workgroup owns CT column tiles side by side.  The activations of a k block,
-// which weigh as much as one tile's weights, are fetched once for all of them, and a wide product
-// (gate and up, the output head) becomes one or two rounds of workgroups instead of three to eight.
-// The weights come as a chain of pieces, the block's tiles and then the wave's next block, each
-// requested while the piece before it is multiplied.  A tile's block sums are what they are with one
-// tile a workgroup, bit for bit.
-//
-// PAIR (8 columns, at most 8 rows, no norm): the matrix tile of 16 x 16 then holds two k blocks at
-// once.  Operand rows 0 to 7 are the 8 columns (and the 8 activation rows) at the k of one block, rows
-// 8 to 15 the same columns and rows at the k of the next; the two diagonal 8 x 8 blocks of the result
-// are the two block sums, each accumulated from zero in the order it has everywhere else, and the
-// rest of the tile is dropped.  Without it the second half of the tile repeats the first: every load
-// instruction then fetches half of what it could, and 8 columns are what bounds these products,
-// since a workgroup is as fast as its loads.  A wave takes pairs of blocks instead of blocks.
 // The norm's arguments come first and as a structure, so that no argument is preloaded into registers (kernels are compiled to
 // find the leading plain ones there).  Preloaded, eighteen such products took 0.7 % more on average: 16 rows of 2,048 x 2,048
 // 10.9 -> 11.1 us, 65 of 2,048 x 5,632 49.4 -> 50.5, 100 of 2,560 x 2,048 35.2 -> 35.8, though the main loop's registers are
@@ -583,41 +569,30 @@ struct F32RowsNorm {
   const float* w;
   float eps;
 };
-template <bool SWIGLU, int COLS, bool NORM = false, bool WIDE = false, int CT = 1, bool PAIR = false>
+template <bool SWIGLU, int COLS, bool NORM, bool WIDE>
 __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const F32RowsNorm norm, const float* __restrict__ a,
                                                                    const float* __restrict__ w,
                                                                    float* __restrict__ out,
                                                                    const float* __restrict__ residual, int M,
                                                                    int N, int K, int64_t lda, int64_t ldo,
                                                                    const float* __restrict__ row_scale = nullptr,
-                                                                   int tiles_wg = FR_MAX_MT, int cols_wg = 0) {
+                                                                   int tiles_wg = FR_MAX_MT) {
   const float* __restrict__ norm_w = norm.w;
   const float eps = norm.eps;
-  // cols_wg (even, with CT column tiles of which the last is partly used): the columns a workgroup owns
-  // where whole tiles would not make whole rounds of 256 workgroups; the tile's other columns repeat
-  // the last one and are dropped.
   // WIDE (more than 16 rows): blockIdx.y picks a group of `tiles_wg` row tiles, so that a product with
   // few column tiles still gives every compute unit a workgroup with whole matrix tiles (16 columns)
   // instead of half-used ones (8 columns); the activations of the next row tile are requested before
   // this one is multiplied, and the registers that takes are those of the next block's weights, which
   // are requested behind the block's last row tile instead.
-  static_assert(!(NORM && WIDE), "the norm rides in the product of one row tile");
-  static_assert(CT >= 1 && CT <= 3 && !(WIDE && CT > 1) && !(NORM && CT > 1), "several column tiles go with one row tile and no norm");
-  static_assert(!PAIR || (COLS == 8 && !NORM && !WIDE && CT == 1), "pairs of k blocks: 8 columns, one row tile of at most 8 rows");
-  extern __shared__ float rows_smem[];      // [m tiles][CT][k blocks][16 rows][COLS columns], NORM: + [m tiles][k blocks][16]
+  static_assert(NORM != WIDE, "the norm rides in the product of few row tiles");
+  extern __shared__ float rows_smem[];      // [m tiles][k blocks][16 rows][COLS columns], NORM: + [m tiles][k blocks][16]
   const int nkb = (K + F_KBLOCK - 1) / F_KBLOCK;
   const int mt0 = WIDE ? blockIdx.y * tiles_wg : 0;                       // first row tile of this workgroup
   const int mts = WIDE ? min(tiles_wg, (M + 15) / 16 - mt0) : (M + 15) / 16;   // and how many it owns
   const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = tid / TL_WAVE;
   const int l16 = lane % 16, kk = lane / 16;
-  // a wave's unit of work: a k block, or a pair of them, of which this lane feeds the first or the second
-  constexpr int UNIT = PAIR ? 2 : 1;
-  const int second = PAIR ? l16 / 8 : 0;
-  const int units = (nkb + UNIT - 1) / UNIT;
-  const int cw = cols_wg > 0 ? cols_wg : COLS * CT;
-  const int n0 = blockIdx.x * cw;
-  auto wrow_of = [&](int ct) { return w + (int64_t)min(n0 + min(ct * COLS + l16 % COLS, cw - 1), N - 1) * K; };
-  const float* wrow = wrow_of(0);
+  const int n0 = blockIdx.x * COLS;
+  const float* wrow = w + (int64_t)min(n0 + l16 % COLS, N - 1) * K;
   // A k block that lies wholly inside K is loaded without a predicate per load (each would be a
   // branch of its own, and the waits around branches are placed for the worst case); only the last,
   // partial block of an inner size that is no multiple of 256 takes the predicated loads.  The loop
@@ -629,26 +604,22 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const F32Rows
       else dst[g] = load_k4<true>(row, k0 + g * 16 + kk * 4, K);
     }
   };
-  auto a_row = [&](int mt) { return a + (int64_t)min((mt0 + mt) * 16 + (PAIR ? l16 % 8 : l16), M - 1) * lda; };
-  f32x4 wv[16], wnext[WIDE ? 1 : 16];
-  if (wave < units) {
-    if ((wave + 1) * UNIT * F_KBLOCK <= K) load16(std::true_type{}, wv, wrow, (wave * UNIT + second) * F_KBLOCK);
-    else load16(std::false_type{}, wv, wrow, (wave * UNIT + second) * F_KBLOCK);
+  auto a_row = [&](int mt) { return a + (int64_t)min((mt0 + mt) * 16 + l16, M - 1) * lda; };
+  f32x4 wv[16];
+  if (wave < nkb) {
+    if ((wave + 1) * F_KBLOCK <= K) load16(std::true_type{}, wv, wrow, wave * F_KBLOCK);
+    else load16(std::false_type{}, wv, wrow, wave * F_KBLOCK);
   }
-  float* ss_smem = rows_smem + mts * CT * nkb * 16 * COLS;
-  // one row tile and column tile of one k block: the block sum of 16 rows x COLS columns goes to LDS
-  auto multiply = [&](f32x4 (&av)[16], int mt, int b, int ct = 0) {
+  float* ss_smem = rows_smem + mts * nkb * 16 * COLS;
+  // one row tile of one k block: the block sum of 16 rows x COLS columns goes to LDS
+  auto multiply = [&](f32x4 (&av)[16], int mt, int b) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int g = 0; g < 16; ++g)
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[g][e], av[g][e], acc, 0, 0, 0);
     // lane (l16, kk): row m = l16, columns 4 kk + r
-    if constexpr (PAIR) {     // rows 0..7 x columns 0..7: this lane's block is the first; 8..15 x 8..15: the second
-      if ((l16 < 8) == (kk < 2) && b < nkb) *(f32x4*)(&rows_smem[(b * 16 + l16 % 8) * COLS + (kk % 2) * 4]) = acc;
-    } else {
-      if (kk * 4 < COLS) *(f32x4*)(&rows_smem[(((mt * CT + ct) * nkb + b) * 16 + l16) * COLS + kk * 4]) = acc;
-    }
+    if (kk * 4 < COLS) *(f32x4*)(&rows_smem[((mt * nkb + b) * 16 + l16) * COLS + kk * 4]) = acc;
   };
   // NORM: the rows times the norm's weights, their squares added up on the way (one row tile of one k block)
   auto scale_rows = [&](auto whole, f32x4 (&av)[16], int mt, int b) {
@@ -667,17 +638,10 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const F32Rows
     ss += __shfl_xor(ss, 32, TL_WAVE);
     if (kk == 0) ss_smem[(mt * nkb + b) * 16 + l16] = ss;
   };
-  constexpr int AHEAD = FR_WAVES * UNIT * F_KBLOCK;        // from a wave's unit to its next
-  auto block = [&](auto whole, auto next_whole, int u) {
-    const int b = u * UNIT + second;          // this lane's k block
+  constexpr int AHEAD = FR_WAVES * F_KBLOCK;        // from a wave's block to its next
+  auto block = [&](auto whole, auto next_whole, int b) {
     const int kb = b * F_KBLOCK;
-    // (NORM keeps the norm's weights in registers beside the rows instead of the next block's
-    // weights; those are requested once this block is done.  The norm's products have the hidden
-    // size as their inner size: one block a wave up to 2048, two at 4096.)
-    // The first row tile's activations are requested BEFORE the next block's weights: loads come
-    // back in the order they were asked for, and the matrix instructions below wait for the
-    // activations; asked for behind the weights they would wait for those as well, and the block
-    // ahead would hide nothing.
+    // The next block's weights are requested once this block is done: the norm's weights, or the next row tile, have the registers.
     f32x4 av[16];
     load16(whole, av, a_row(0), kb);
     if constexpr (WIDE) {
@@ -690,63 +654,217 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const F32Rows
           multiply(av2, mt + 1, b);
         }
       }
-      if (u + FR_WAVES < units) load16(next_whole, wv, wrow, kb + AHEAD);
-    } else if constexpr (CT > 1) {
-      // one row tile, no norm
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        const bool more = ct + 1 < CT || u + FR_WAVES < units;
-        if (ct + 1 < CT) load16(whole, wnext, wrow_of(ct + 1), kb);
-        else if (u + FR_WAVES < units) load16(next_whole, wnext, wrow, kb + AHEAD);
-        multiply(av, 0, b, ct);
-        if (more) {
-#pragma unroll
-          for (int g = 0; g < 16; ++g) wv[g] = wnext[g];
-        }
-      }
+      if (b + FR_WAVES < nkb) load16(next_whole, wv, wrow, kb + AHEAD);
     } else {
-      if (!NORM && u + FR_WAVES < units) load16(next_whole, wnext, wrow, kb + AHEAD);
       for (int mt = 0; mt < mts; ++mt) {
         if (mt > 0) load16(whole, av, a_row(mt), kb);
-        if constexpr (NORM) scale_rows(whole, av, mt, b);
+        scale_rows(whole, av, mt, b);
         multiply(av, mt, b);
       }
-      if constexpr (NORM) {
-        if (u + FR_WAVES < units) load16(next_whole, wv, wrow, kb + AHEAD);
-      } else {
-#pragma unroll
-        for (int g = 0; g < 16; ++g) wv[g] = wnext[g];
-      }
+      if (b + FR_WAVES < nkb) load16(next_whole, wv, wrow, kb + AHEAD);
     }
   };
-  for (int u = wave; u < units; u += FR_WAVES) {
-    const bool whole = (u + 1) * UNIT * F_KBLOCK <= K, next_whole = (u + FR_WAVES + 1) * UNIT * F_KBLOCK <= K;
-    if (whole && next_whole) block(std::true_type{}, std::true_type{}, u);
-    else if (whole) block(std::true_type{}, std::false_type{}, u);
-    else block(std::false_type{}, std::false_type{}, u);
+  for (int b = wave; b < nkb; b += FR_WAVES) {
+    const bool whole = (b + 1) * F_KBLOCK <= K, next_whole = (b + FR_WAVES + 1) * F_KBLOCK <= K;
+    if (whole && next_whole) block(std::true_type{}, std::true_type{}, b);
+    else if (whole) block(std::true_type{}, std::false_type{}, b);
+    else block(std::false_type{}, std::false_type{}, b);
   }
   __syncthreads();
-  for (int e = tid; e < mts * CT * 16 * COLS; e += FR_THREADS) {
-    const int tile = e / (16 * COLS), mt = tile / CT, ct = tile % CT, r = (e % (16 * COLS)) / COLS, c = e % COLS;
+  for (int e = tid; e < mts * 16 * COLS; e += FR_THREADS) {
+    const int mt = e / (16 * COLS), r = (e % (16 * COLS)) / COLS, c = e % COLS;
     float t = 0.f;
-    for (int b = 0; b < nkb; ++b) t += rows_smem[((tile * nkb + b) * 16 + r) * COLS + c];
+    for (int b = 0; b < nkb; ++b) t += rows_smem[((mt * nkb + b) * 16 + r) * COLS + c];
     if constexpr (NORM) {
       float q = 0.f;
       for (int b = 0; b < nkb; ++b) q += ss_smem[(mt * nkb + b) * 16 + r];
       t *= f32_norm_factor(q, K, eps);
     }
-    const int m = (mt0 + mt) * 16 + r, n = n0 + ct * COLS + c;
+    const int m = (mt0 + mt) * 16 + r, n = n0 + c;
     if constexpr (!NORM) {
       if (row_scale && m < M) t *= row_scale[m];    // the factor of a norm in front (norm_prescale_f32_kernel)
     }
     if constexpr (SWIGLU) {   // columns (2j, 2j+1) = (gate_j, up_j); N and n0 are even
       const float u = __shfl_down(t, 1, TL_WAVE);
-      if (m < M && n < N && ct * COLS + c < cw && (c & 1) == 0) out[(int64_t)m * ldo + n / 2] = swiglu_pair(t, u);
+      if (m < M && n < N && (c & 1) == 0) out[(int64_t)m * ldo + n / 2] = swiglu_pair(t, u);
     } else {
-      if (m < M && n < N && ct * COLS + c < cw) {
+      if (m < M && n < N) {
         const int64_t at = (int64_t)m * ldo + n;
         out[at] = residual ? t + residual[at] : t;
       }
+    }
+  }
+}
+
+// The same product for one tile of rows (decode steps of up to 16), by whole lines.  gemm_f32_rows_kernel loads in the matrix instruction's order, 64
+// bytes of each of sixteen rows an instruction, at 37 GB/s a unit; a unit gets 105 from its L2 in whole lines.  Here a wave fetches runs
+// of 512 bytes, half a k block of sixteen rows at a time, of activations and of each column tile, and turns them into
+// operands through 8 KB of LDS of its own; the next half block is on its way meanwhile.  Same blocks, same groups, same order: the bits of gemm_f32_kernel.
+// 8 rows, weights from memory: 2,560 x 2,048 10.7 -> 8.5 us, 2,048 x 2,048 8.1 -> 6.6, 11,264 x 2,048 gated 23.0 -> 21.4, 2,048 x 5,632 16.4 ->
+// 13.0, 32,000 x 2,048 63.7 -> 58.2, 6,144 x 4,096 28.3 -> 22.6; 16 rows of 2,048 x 5,632 25.4 -> 16.5.
+// NORM: the product is that of `a`'s RMSNorm, as described there.
+//
+// CT (one row tile only): a workgroup owns CT column tiles side by side.  The activations of a k block,
+// which weigh as much as one tile's weights, are fetched once for all of them, and a wide product
+// (gate and up, the output head) becomes one or two rounds of workgroups instead of three to eight.
+// The weights come as a chain of pieces, the block's tiles and then the wave's next block, each
+// requested while the piece before it is multiplied.  A tile's block sums are what they are with one
+// tile a workgroup, bit for bit.
+//
+// PAIR (8 columns, at most 8 rows, no norm): the matrix tile of 16 x 16 then holds two k blocks at
+// once.  Operand rows 0 to 7 are the 8 columns (and the 8 activation rows) at the k of one block, rows
+// 8 to 15 the same columns and rows at the k of the next; the two diagonal 8 x 8 blocks of the result
+// are the two block sums, each accumulated from zero in the order it has everywhere else, and the
+// rest of the tile is dropped.  Without it the second half of the tile repeats the first: every load
+// instruction then fetches half of what it could, and 8 columns are what bounds these products,
+// since a workgroup is as fast as its loads.  A wave takes pairs of blocks instead of blocks.
+constexpr int FL_HALF = F_KBLOCK / 2, FL_AREA = 16 * FL_HALF;      // k of a step; floats of a wave's area
+constexpr int64_t FL_MAX_STRIDE = 1 << 24;                         // floats between rows: offsets within sixteen rows fit 31 bits
+constexpr size_t FL_STAGE_BYTES = (size_t)FR_WAVES * FL_AREA * sizeof(float), FL_SUM_BYTES = 96 * 1024;      // together a unit's LDS
+template <bool SWIGLU, int CT, bool PAIR, bool NORM>
+__global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32RowsNorm norm, const float* __restrict__ a, const float* __restrict__ w,
+                                                                    float* __restrict__ out, const float* __restrict__ residual,
+                                                                    int M, int N, int K, int64_t lda, int64_t ldo,
+                                                                    const float* __restrict__ row_scale, int cw) {
+  static_assert(CT == 1 || (!PAIR && !NORM), "pairs of k blocks and the norm: one column tile");
+  constexpr int COLS = PAIR ? 8 : 16, UNIT = PAIR ? 2 : 1;
+  extern __shared__ __attribute__((aligned(16))) float lines_smem[];
+  constexpr int ROWS = PAIR ? 8 : 16;
+  const int nkb = (K + F_KBLOCK - 1) / F_KBLOCK, units = (nkb + UNIT - 1) / UNIT;
+  float* sums = lines_smem + FR_WAVES * FL_AREA;            // [CT][k blocks][ROWS][COLS], NORM: + [k blocks][ROWS]
+  float* squares = sums + CT * nkb * ROWS * COLS;
+  const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TL_WAVE);
+  const int l16 = lane % 16, kk = lane / 16, lr = lane / 32, lc = lane % 32;
+  const int n0 = blockIdx.x * cw, stride_a = (int)lda;
+  // Both operands as buffers: rows beyond the matrices, and steps beyond this wave's, read as zeros and fetch nothing
+  auto rows_of = [&](const float* base, int stride, int rows) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, rows > 0 ? ((rows - 1) * stride + K) * 4 : 0, 0x00020000);
+  };
+  const auto buf_w = rows_of(w + (int64_t)n0 * K, K, min(cw, N - n0)), buf_a = rows_of(a, stride_a, M);
+  const int at_w = (lr * K + lc * 4) * 4, at_a = (lr * stride_a + lc * 4) * 4;
+  const int mine = wave < units ? 2 * ((units - wave + FR_WAVES - 1) / FR_WAVES) : 0;      // half blocks (PAIR: of two blocks)
+  // load i of a step: 16 bytes of row 2 i + lane / 32 (PAIR: from row 8 on the rows 0 .. of the next k block), k 4 (lane % 32) ..
+  struct Step {
+    f32x4 a[8], w[CT][8];
+  };
+  auto first_k = [&](int s) { return ((wave + s / 2 * FR_WAVES) * UNIT * F_KBLOCK) + s % 2 * FL_HALF; };
+  auto load_tile = [&](f32x4 (&v)[8], auto buf, int at, int stride, int row0, int s) {
+    const int k0 = first_k(s);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const bool up = PAIR && i >= 4;
+      const int row = row0 + 2 * i - (up ? 8 : 0), k = k0 + (up ? F_KBLOCK : 0);
+      v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, at, s < mine ? (row * stride + k) * 4 : 0x70000000, 0));
+    }
+  };
+  float* own = lines_smem + wave * FL_AREA;
+  auto sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // chunk c of row r stands at place c ^ r of its 32; what lies beyond K is zero
+  auto put = [&](f32x4 (&v)[8], int k0) {
+    if (k0 + (PAIR ? F_KBLOCK : 0) + FL_HALF > K)      // uniform
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const bool in = k0 + (PAIR && i >= 4 ? F_KBLOCK : 0) + lc * 4 < K;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] = in ? v[i][e] : 0.f;
+      }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *(f32x4*)(own + (2 * i + lr) * FL_HALF + (lc ^ (2 * i + lr)) * 4) = v[i];
+    sync();
+  };
+  auto get = [&](f32x4 (&v)[8]) {
+#pragma unroll
+    for (int g = 0; g < 8; ++g) v[g] = *(const f32x4*)(own + l16 * FL_HALF + ((g * 4 + kk) ^ l16) * 4);
+    sync();
+  };
+  Step st;
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) load_tile(st.w[ct], buf_w, at_w, K, ct * 16, 0);
+  load_tile(st.a, buf_a, at_a, stride_a, 0, 0);
+  // NORM: the norm's weights of a step, as operands (4 K bytes, from the caches), requested a step ahead
+  f32x4 nw[NORM ? 8 : 1];
+  auto load_norm = [&](int s) {
+    if constexpr (NORM)
+#pragma unroll
+      for (int g = 0; g < 8; ++g)
+        nw[g] = load_k4<true>(norm.w, first_k(min(s, mine - 1)) + (PAIR && l16 >= 8 ? F_KBLOCK : 0) + g * 16 + kk * 4, K);
+  };
+  if (mine > 0) load_norm(0);
+  f32x4 acc[CT];
+  float ss = 0.f;
+  for (int s = 0; s < mine; ++s) {
+    const int k0 = first_k(s);
+    if (s % 2 == 0) {
+      ss = 0.f;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    f32x4 av[8];
+    put(st.a, k0);
+    load_tile(st.a, buf_a, at_a, stride_a, 0, s + 1);
+    get(av);
+    if constexpr (NORM) {      // the rows times the norm's weights, their squares added up on the way
+#pragma unroll
+      for (int g = 0; g < 8; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          ss = __builtin_fmaf(av[g][e], av[g][e], ss);
+          av[g][e] *= nw[g][e];
+        }
+      load_norm(s + 1);
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      f32x4 wv[8];
+      put(st.w[ct], k0);
+      load_tile(st.w[ct], buf_w, at_w, K, ct * 16, s + 1);
+      get(wv);
+#pragma unroll
+      for (int g = 0; g < 8; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[g][e], av[g][e], acc[ct], 0, 0, 0);
+    }
+    if (s % 2 == 1) {      // the block's sums: lane (l16, kk) has row l16, columns 4 kk + r
+      const int b = (wave + s / 2 * FR_WAVES) * UNIT + (PAIR ? l16 / 8 : 0);
+      if constexpr (NORM) {      // the four lanes of a row, one per k quarter: (s0 + s1) + (s2 + s3)
+        ss += __shfl_xor(ss, 16, TL_WAVE);
+        ss += __shfl_xor(ss, 32, TL_WAVE);
+        if (kk == 0 && b < nkb) squares[b * ROWS + l16 % ROWS] = ss;
+      }
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        if constexpr (PAIR) {     // rows 0..7 x columns 0..7: the first block; 8..15 x 8..15: the second
+          if ((l16 < 8) == (kk < 2) && b < nkb) *(f32x4*)(&sums[(b * ROWS + l16 % 8) * COLS + (kk % 2) * 4]) = acc[ct];
+        } else {
+          *(f32x4*)(&sums[((ct * nkb + b) * ROWS + l16) * COLS + kk * 4]) = acc[ct];
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < CT * ROWS * COLS; e += FR_THREADS) {
+    const int ct = e / (ROWS * COLS), r = e % (ROWS * COLS) / COLS, c = e % COLS;
+    float t = 0.f;
+    for (int b = 0; b < nkb; ++b) t += sums[((ct * nkb + b) * ROWS + r) * COLS + c];
+    const int n = n0 + ct * COLS + c;
+    if constexpr (NORM) {
+      float q = 0.f;
+      for (int b = 0; b < nkb; ++b) q += squares[b * ROWS + r];
+      t *= f32_norm_factor(q, K, norm.eps);
+    } else if (row_scale && r < M) {
+      t *= row_scale[r];      // the factor of a norm in front (norm_prescale_f32_kernel)
+    }
+    const bool there = r < M && n < N && ct * COLS + c < cw;
+    if constexpr (SWIGLU) {   // columns (2j, 2j+1) = (gate_j, up_j); N and n0 are even
+      const float u = __shfl_down(t, 1, TL_WAVE);
+      if (there && (c & 1) == 0) out[(int64_t)r * ldo + n / 2] = swiglu_pair(t, u);
+    } else if (there) {
+      const int64_t at = (int64_t)r * ldo + n;
+      out[at] = residual ? t + residual[at] : t;
     }
   }
 }
@@ -2714,6 +2832,55 @@ static int f32_rows_col_tiles(int M, int N, int K, int cols, int* cols_wg = null
   return 1;
 }
 
+template <bool SWIGLU, int CT, bool PAIR, bool NORM>
+static int launch_f32_lines_form(const F32RowsNorm& norm, const float* a, const float* w, float* out, const float* residual, int M, int N, int K,
+                                 int64_t lda, int64_t ldo, const float* row_scale, int cw, size_t sums, hipStream_t stream) {
+  const auto kernel = gemm_f32_lines_kernel<SWIGLU, CT, PAIR, NORM>;
+  static bool configured = false;
+  if (!configured) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(FL_STAGE_BYTES + FL_SUM_BYTES)) != hipSuccess)
+      return TL_ERR_LAUNCH;
+    configured = true;
+  }
+  hipLaunchKernelGGL(kernel, dim3((N + cw - 1) / cw), dim3(FR_THREADS), FL_STAGE_BYTES + sums, stream, norm, a, w, out, residual, M, N, K, lda, ldo,
+                     row_scale, cw);
+  return TL_OK;
+}
+
+// Whether and how the float32 product of at most 16 rows goes by whole lines: 8 columns a workgroup where that still is one round of
+// workgroups over the 256 compute units (pairs of k blocks up to 8 rows), else as many (even) as make 256 workgroups up to 16, else one to three column
+// tiles (f32_rows_col_tiles).  With a norm one column tile at most.
+struct F32Lines {
+  int ct, cw;
+  bool pair;
+  size_t sums;      // bytes of block sums
+};
+static bool f32_lines_plan(int M, int N, int K, int64_t lda, bool norm, F32Lines* p) {
+  if (M > 16 || lda > FL_MAX_STRIDE || K > FL_MAX_STRIDE) return false;
+  const int nkb = (K + F_KBLOCK - 1) / F_KBLOCK;
+  const bool eight = (N + 7) / 8 <= 256;
+  p->pair = eight && M <= 8;
+  p->cw = 0;
+  p->ct = eight || norm ? 1 : f32_rows_col_tiles(M, N, K, 16, &p->cw);
+  if (p->cw == 0) {
+    const int even = ((N + 255) / 256 + 1) / 2 * 2;
+    p->cw = eight ? 8 : p->ct == 1 && even < 16 ? even : 16 * p->ct;
+  }
+  p->sums = (size_t)nkb * (p->pair ? 8 * 8 : 16 * 16 * p->ct) * sizeof(float) + (norm ? (size_t)nkb * 16 * sizeof(float) : 0);
+  return p->sums <= FL_SUM_BYTES;
+}
+
+template <bool SWIGLU, bool NORM>
+static int launch_f32_lines(const F32Lines& p, const F32RowsNorm& norm, const float* a, const float* w, float* out, const float* residual, int M, int N,
+                            int K, int64_t lda, int64_t ldo, const float* row_scale, hipStream_t stream) {
+#define TL_LINES(CT, PAIR, NRM) launch_f32_lines_form<SWIGLU, CT, PAIR, NRM>(norm, a, w, out, residual, M, N, K, lda, ldo, row_scale, p.cw, p.sums, stream)
+  if (p.pair) return TL_LINES(1, true, NORM);
+  if (p.ct == 2) return TL_LINES(2, false, false);
+  if (p.ct == 3) return TL_LINES(3, false, false);
+  return TL_LINES(1, false, NORM);
+#undef TL_LINES
+}
+
 }  // namespace
 
 extern "C" {
@@ -2749,17 +2916,24 @@ int tl_linear_norm_f32(const float* x, const float* norm_w, float eps, const flo
   const int nkb = (K + F_KBLOCK - 1) / F_KBLOCK, mts = (M + 15) / 16;
   const int cols = (N + 7) / 8 <= 256 ? 8 : 16;
   const size_t smem = (size_t)mts * nkb * 16 * (cols + 1) * sizeof(float);
+  F32Lines lines;
+  if (f32_lines_plan(M, N, K, lda, true, &lines)) {
+    const F32RowsNorm norm{norm_w, eps};
+    const int rc = swiglu ? launch_f32_lines<true, true>(lines, norm, x, w, out, residual, M, N, K, lda, ldo, nullptr, stream)
+                          : launch_f32_lines<false, true>(lines, norm, x, w, out, residual, M, N, K, lda, ldo, nullptr, stream);
+    return rc == TL_OK ? tl_launch_status() : rc;
+  }
   static bool configured = false;
   if (!configured) {
-    const void* kernels[4] = {(const void*)gemm_f32_rows_kernel<true, 16, true>, (const void*)gemm_f32_rows_kernel<false, 16, true>,
-                              (const void*)gemm_f32_rows_kernel<true, 8, true>, (const void*)gemm_f32_rows_kernel<false, 8, true>};
+    const void* kernels[4] = {(const void*)gemm_f32_rows_kernel<true, 16, true, false>, (const void*)gemm_f32_rows_kernel<false, 16, true, false>,
+                              (const void*)gemm_f32_rows_kernel<true, 8, true, false>, (const void*)gemm_f32_rows_kernel<false, 8, true, false>};
     for (const void* k : kernels)
       if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) return TL_ERR_LAUNCH;
     configured = true;
   }
   dim3 gr((N + cols - 1) / cols);
 #define TL_F32_ROWS_NORM(SW, CO)                                                                                 \
-  hipLaunchKernelGGL((gemm_f32_rows_kernel<SW, CO, true>), gr, dim3(FR_THREADS), smem, stream, F32RowsNorm{norm_w, eps}, x, w, out, \
+  hipLaunchKernelGGL((gemm_f32_rows_kernel<SW, CO, true, false>), gr, dim3(FR_THREADS), smem, stream, F32RowsNorm{norm_w, eps}, x, w, out, \
                      residual, M, N, K, lda, ldo)
   if (swiglu && cols == 16) TL_F32_ROWS_NORM(true, 16);
   else if (swiglu) TL_F32_ROWS_NORM(true, 8);
@@ -2814,24 +2988,25 @@ int tl_linear_tile(const void* a, const void* w, void* out, const float* residua
     const bool vec = K % 4 == 0 && lda % 4 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
     const int nkb = (K + F_KBLOCK - 1) / F_KBLOCK;
     const int mts = (M + 15) / 16;
-    // One row tile: 8 columns a workgroup where that still is one round of workgroups over the 256
-    // compute units (a workgroup fills a compute unit: more than 256 of them would run in two rounds).
-    // More row tiles (17 to 64 rows, up to 256 by the estimate below): whole matrix tiles of 16 columns, and the row tiles shared out
-    // over as many groups of workgroups (1, 2 or 4) as it takes to give every compute unit a
-    // workgroup and to fit the block sums into LDS.
-    int cols = (N + 7) / 8 <= 256 ? 8 : 16, groups = 1;
-    if (mts > 1) {
-      cols = 16;
-      const int col_tiles = (N + 15) / 16;
-      // (more groups only while they stay within one round of 256 workgroups: a second, partly filled
-      // round costs as much as a full one)
-      while (groups < mts && (col_tiles * groups * 2 <= 256 || (size_t)((mts + groups - 1) / groups) * nkb * 16 * cols * sizeof(float) > 96 * 1024))
-        groups *= 2;
+    F32Lines lines;
+    if (vec && f32_lines_plan(M, N, K, lda, false, &lines)) {
+      const F32RowsNorm none{};
+      const int rc = swiglu ? launch_f32_lines<true, false>(lines, none, (const float*)a, (const float*)w, (float*)out, residual, M, N, K, lda,
+                                                            ldo, row_scale, stream)
+                            : launch_f32_lines<false, false>(lines, none, (const float*)a, (const float*)w, (float*)out, residual, M, N, K, lda,
+                                                             ldo, row_scale, stream);
+      return rc == TL_OK ? tl_launch_status() : rc;
     }
+    // 17 to 64 rows, up to 256 by the estimate below (and what the kernel above does not take): matrix tiles of 16 columns, and the row
+    // tiles shared out over as many groups of workgroups (1, 2 or 4) as it takes to give every compute unit a
+    // workgroup and to fit the block sums into LDS (more groups only while they stay within one round of 256 workgroups: a second, partly
+    // filled round costs as much as a full one).
+    int groups = 1;
+    const int col_tiles = (N + 15) / 16;
+    while (groups < mts && (col_tiles * groups * 2 <= 256 || (size_t)((mts + groups - 1) / groups) * nkb * 16 * 16 * sizeof(float) > 96 * 1024))
+      groups *= 2;
     const int tiles_wg = (mts + groups - 1) / groups;
-    int cols_wg = 0;
-    const int ct = f32_rows_col_tiles(M, N, K, cols, &cols_wg);
-    const size_t rows_smem = (size_t)tiles_wg * nkb * 16 * cols * ct * sizeof(float);
+    const size_t rows_smem = (size_t)tiles_wg * nkb * 16 * 16 * sizeof(float);
     // Up to 64 rows the few-row kernel; up to 256 where it is estimated faster than the tiled kernel, whose few
     // tiles each walk the whole inner size (f32_ring_us; where rows are no whole vectors, measured at inner size 2048: 87 us a
     // round of up to 352 tiles of 64 x 64, 204 us a round of 128 x 128; the few-row kernel 0.66 us per row tile and million
@@ -2853,45 +3028,19 @@ int tl_linear_tile(const void* a, const void* w, void* out, const float* residua
     if (few_rows && vec && rows_smem <= 96 * 1024) {
       static bool configured = false;
       if (!configured) {
-        const void* kernels[12] = {(const void*)gemm_f32_rows_kernel<true, 8, false, false, 1, true>,
-                                   (const void*)gemm_f32_rows_kernel<false, 8, false, false, 1, true>,
-                                   (const void*)gemm_f32_rows_kernel<true, 16>, (const void*)gemm_f32_rows_kernel<false, 16>,
-                                   (const void*)gemm_f32_rows_kernel<true, 8>, (const void*)gemm_f32_rows_kernel<false, 8>,
-                                   (const void*)gemm_f32_rows_kernel<true, 16, false, true>,
-                                   (const void*)gemm_f32_rows_kernel<false, 16, false, true>,
-                                   (const void*)gemm_f32_rows_kernel<true, 16, false, false, 2>,
-                                   (const void*)gemm_f32_rows_kernel<false, 16, false, false, 2>,
-                                   (const void*)gemm_f32_rows_kernel<true, 16, false, false, 3>,
-                                   (const void*)gemm_f32_rows_kernel<false, 16, false, false, 3>};
+        const void* kernels[2] = {(const void*)gemm_f32_rows_kernel<true, 16, false, true>, (const void*)gemm_f32_rows_kernel<false, 16, false, true>};
         for (const void* k : kernels)
           if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess)
             return TL_ERR_LAUNCH;
         configured = true;
       }
-      const int cw = cols_wg > 0 ? cols_wg : cols * ct;
-      dim3 gr((N + cw - 1) / cw, (mts + tiles_wg - 1) / tiles_wg);
-#define TL_F32_ROWS_K(...)                                                                                          \
-  hipLaunchKernelGGL((gemm_f32_rows_kernel<__VA_ARGS__>), gr, dim3(FR_THREADS), rows_smem, stream, F32RowsNorm{}, (const float*)a, \
-                     (const float*)w, (float*)out, residual, M, N, K, lda, ldo, row_scale, \
-                     tiles_wg, cols_wg)
-#define TL_F32_ROWS(SW, CO, WI, CTI) TL_F32_ROWS_K(SW, CO, false, WI, CTI)
-#define TL_F32_ROWS_CT(SW)                                                                                           \
-  do {                                                                                                               \
-    if (ct == 3) TL_F32_ROWS(SW, 16, false, 3);                                                                      \
-    else if (ct == 2) TL_F32_ROWS(SW, 16, false, 2);                                                                 \
-    else TL_F32_ROWS(SW, 16, false, 1);                                                                              \
-  } while (0)
-      if (mts > 1 && swiglu) TL_F32_ROWS(true, 16, true, 1);
-      else if (mts > 1) TL_F32_ROWS(false, 16, true, 1);
-      else if (swiglu && cols == 16) TL_F32_ROWS_CT(true);
-      else if (swiglu && M <= 8) TL_F32_ROWS_K(true, 8, false, false, 1, true);      // cols == 8: pairs of k blocks
-      else if (swiglu) TL_F32_ROWS(true, 8, false, 1);
-      else if (cols == 16) TL_F32_ROWS_CT(false);
-      else if (M <= 8) TL_F32_ROWS_K(false, 8, false, false, 1, true);
-      else TL_F32_ROWS(false, 8, false, 1);
-#undef TL_F32_ROWS_CT
+      dim3 gr((N + 15) / 16, (mts + tiles_wg - 1) / tiles_wg);
+#define TL_F32_ROWS(SW)                                                                                              \
+  hipLaunchKernelGGL((gemm_f32_rows_kernel<SW, 16, false, true>), gr, dim3(FR_THREADS), rows_smem, stream, F32RowsNorm{}, (const float*)a, \
+                     (const float*)w, (float*)out, residual, M, N, K, lda, ldo, row_scale, tiles_wg)
+      if (swiglu) TL_F32_ROWS(true);
+      else TL_F32_ROWS(false);
 #undef TL_F32_ROWS
-#undef TL_F32_ROWS_K
       return tl_launch_status();
     }
     if (f32_ring_ok(vec, K, lda)) {

@@ -1684,3 +1684,26 @@ def test_router_beside_an_activation(T, cols, experts, dtype):
             ops().activate_rows(*beside)
         got.append((ids, wts, out))
     assert all(torch.equal(x, y) for x, y in zip(*got)) and torch.isfinite(got[0][2]).all()
+
+
+@pytest.mark.parametrize("shapes", [[(3,)], [(1,), (4096,), (2, 4099), (16, 1024), (1, 5)], [(7,)] * 200])
+def test_rows_of_many_tensors(shapes):
+    """Rows cleared and copied in as few launches as they fit, whole vectors and single numbers, both 4-byte types; the other rows stay."""
+    g = torch.Generator().manual_seed(len(shapes))
+    tensors = [torch.randn(70, *s, generator=g) if i % 3 else torch.randint(-9, 9, (70, *s), generator=g, dtype=torch.int32) for i, s in enumerate(shapes)]
+    dev = [t.to(DEV) for t in tensors]
+    for slots in ([69], [5, 0, 33], list(range(64))):
+        for t, copy in zip(tensors, ops().tensor_rows(dev, slots, save=True)):
+            assert copy.dtype == t.dtype and torch.equal(copy.cpu(), t[slots])
+    dev[0][5] = float("nan") if dev[0].is_floating_point() else 3
+    for slots in ([5, 0, 33], [69]):
+        ops().tensor_rows(dev, slots)
+        for t, d in zip(tensors, dev):
+            t[slots] = 0
+            assert torch.equal(d.cpu(), t)
+    ops().tensor_rows(dev, list(range(70)))
+    assert not any(d.any() for d in dev)
+    with pytest.raises(Exception):
+        ops().tensor_rows(dev, [70])
+    with pytest.raises(Exception):
+        ops().tensor_rows([d.to(torch.bfloat16) for d in dev], [0])

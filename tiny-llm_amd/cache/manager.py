@@ -175,15 +175,29 @@ class CacheManager:
     def free_slots(self) -> int:
         return len(self._free_slots)
 
-    def add_request(self, req_id) -> int:
+    def _rows(self, slots: Sequence[int], save: bool = False):
+        """The state rows of `slots` in every tensor: cleared, or copied ({owner: [slots, ...]}); on the device one launch for all."""
+        states = list(self.states.values())
+        if states[0].is_cuda and len(slots) <= 64 and all(t.element_size() == 4 and t.is_contiguous() for t in states):
+            from ..kernels import ops
+            copies = ops.tensor_rows(states, slots, save)
+            return dict(zip(self.states, copies)) if save else None
+        idx = torch.tensor(slots, dtype=torch.long, device=states[0].device)
+        if save:
+            return {owner: st.index_select(0, idx) for owner, st in self.states.items()}
+        for st in states:
+            st.index_fill_(0, idx, 0)
+
+    def add_request(self, req_id, clear: bool = True) -> int:
+        """`clear`: the request's state begins as zeros (False: the caller sees to it)."""
         if req_id in self.requests:
             raise CacheError(f"request {req_id!r} is already live")
         if not self._free_slots:
             raise NoFreeSlot(f"all {self.max_seqs} request slots are taken")
         slot = self._free_slots.pop()
         self.requests[req_id] = RequestCache(slot, 0, [[] for _ in self.groups])
-        for st in self.states.values():
-            st[slot].zero_()
+        if clear and self.states:
+            self._rows([slot])
         return slot
 
     def num_tokens(self, req_id) -> int:
@@ -267,11 +281,11 @@ class CacheManager:
         if self.states:
             slots = [self.requests[rid].slot for rid, _ in entries if rid in self.requests]
             if slots:
-                idx = torch.tensor(slots, dtype=torch.long, device=next(iter(self.states.values())).device)
-                saved = (idx, {owner: st.index_select(0, idx) for owner, st in self.states.items()})
+                saved = (slots, self._rows(slots, save=True))
         self._reservation = (list(new), lengths, [rid for rid, _ in growing], saved)
-        for rid in new:
-            self.add_request(rid)
+        admitted = [self.add_request(rid, clear=False) for rid in new]
+        if admitted and self.states:
+            self._rows(admitted)
         for rid, new_len in growing:
             self.grow(rid, new_len)
         return before
@@ -286,7 +300,8 @@ class CacheManager:
         new, lengths, order, saved = self._reservation
         self._reservation = None
         if saved is not None:
-            idx, by_owner = saved
+            slots, by_owner = saved
+            idx = torch.tensor(slots, dtype=torch.long, device=next(iter(self.states.values())).device)
             for owner, values in by_owner.items():
                 self.states[owner].index_copy_(0, idx, values)
         if order:

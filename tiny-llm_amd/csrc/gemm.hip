@@ -2848,8 +2848,8 @@ static int launch_f32_lines_form(const F32RowsNorm& norm, const float* a, const 
 }
 
 // Whether and how the float32 product of at most 16 rows goes by whole lines: 8 columns a workgroup where that still is one round of
-// workgroups over the 256 compute units (pairs of k blocks up to 8 rows), else as many (even) as make 256 workgroups up to 16, else one to three column
-// tiles (f32_rows_col_tiles).  With a norm one column tile at most.
+// workgroups over the 256 compute units (pairs of k blocks up to 8 rows), else one to three column tiles (f32_rows_col_tiles), one of as many
+// (even) as make whole rounds of 256 workgroups.  With a norm one column tile.
 struct F32Lines {
   int ct, cw;
   bool pair;
@@ -2863,8 +2863,8 @@ static bool f32_lines_plan(int M, int N, int K, int64_t lda, bool norm, F32Lines
   p->cw = 0;
   p->ct = eight || norm ? 1 : f32_rows_col_tiles(M, N, K, 16, &p->cw);
   if (p->cw == 0) {
-    const int even = ((N + 255) / 256 + 1) / 2 * 2;
-    p->cw = eight ? 8 : p->ct == 1 && even < 16 ? even : 16 * p->ct;
+    const int rounds = (N + 256 * 16 - 1) / (256 * 16), even = ((N + 256 * rounds - 1) / (256 * rounds) + 1) / 2 * 2;
+    p->cw = eight ? 8 : p->ct == 1 ? even : 16 * p->ct;
   }
   p->sums = (size_t)nkb * (p->pair ? 8 * 8 : 16 * 16 * p->ct) * sizeof(float) + (norm ? (size_t)nkb * 16 * sizeof(float) : 0);
   return p->sums <= FL_SUM_BYTES;

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 
@@ -1207,6 +1207,37 @@ def cast_rows(x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
         _fail("cast_rows takes contiguous operands of one shape, the input in float32")
     _check(_lib().tl_cast_rows(_ptr(x), _ptr(out), c_int64(x.numel()), c_int(_dt(out)), _stream()), "cast_rows")
     return out
+
+
+ROW_TENSORS, ROW_SLOTS = 96, 64      # most tensors and rows one launch of `tensor_rows` takes
+
+
+def tensor_rows(tensors: Sequence[torch.Tensor], slots: Sequence[int], save: bool = False):
+    """Rows `slots` of every tensor (contiguous, 4-byte numbers) in one launch for up to 96 tensors and 64 rows: cleared, or (`save`)
+    copied; returns a list of [len(slots), ...] copies then."""
+    n_slots = len(slots)
+    for t in tensors:
+        _need(t.is_contiguous() and t.element_size() == 4 and t.dim() >= 1, "tensor_rows: contiguous tensors of 4-byte numbers")
+        _need(all(0 <= s < t.shape[0] for s in slots), "tensor_rows: a row outside a tensor")
+    _dev(*tensors)
+    words = [t.numel() // max(1, t.shape[0]) for t in tensors]
+    first = [sum(-(-w // 4) * 4 for w in words[:i]) for i in range(len(words) + 1)]
+    buf = torch.empty(first[-1] * n_slots, dtype=torch.int32, device=tensors[0].device) if save and tensors else None
+    for i in range(0, len(tensors), ROW_TENSORS):
+        part = slice(i, min(i + ROW_TENSORS, len(tensors)))
+        k = part.stop - part.start
+        longs = lambda v: (ctypes.c_int64 * k)(*v[part])  # noqa: E731
+        for j in range(0, n_slots, ROW_SLOTS):
+            some = slots[j:j + ROW_SLOTS]
+            if save and n_slots > ROW_SLOTS:
+                _fail(f"tensor_rows copies at most {ROW_SLOTS} rows")
+            _check(_lib().tl_tensor_rows((ctypes.c_void_p * k)(*[t.data_ptr() for t in tensors[part]]), longs(words), longs(words),
+                                         longs(first), c_int(k), (ctypes.c_int32 * len(some))(*some), c_int(len(some)), _ptr(buf),
+                                         _stream()), "tensor_rows")
+    if not save:
+        return None
+    return [buf[first[i] * n_slots:first[i] * n_slots + words[i] * n_slots].view(t.dtype).view(n_slots, *t.shape[1:])
+            for i, t in enumerate(tensors)]
 
 
 def gelu_table_rows(gate: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor, off: int, dim: int,

@@ -1707,3 +1707,19 @@ def test_rows_of_many_tensors(shapes):
         ops().tensor_rows(dev, [70])
     with pytest.raises(Exception):
         ops().tensor_rows([d.to(torch.bfloat16) for d in dev], [0])
+
+
+@pytest.mark.parametrize("M,K,n", [(1, 64, 3), (6, 2048, 64), (16, 704, 250)])
+def test_linear_set_leaves_tanh(M, K, n):
+    """A product of a set whose results leave as tanh in bfloat16: the bits of the product in float32 and `tanh_rows`, beside a plain one."""
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    a, w = (torch.randn(*s, device=DEV, generator=g).bfloat16() for s in ((M, K), (n, K)))
+    w = (w.float() / math.sqrt(K)).bfloat16()
+    plain_out, beside = torch.empty(M, n, device=DEV), torch.full((M, n + 3), 7.0, device=DEV)
+    low = torch.full((M, n + 3), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops().linear_set([(a, w, plain_out)])
+    ops().linear_set([(a, w, beside[:, :n]), (a, w, low[:, :n])])
+    assert torch.equal(beside[:, :n], plain_out) and (beside[:, n:] == 7.0).all() and (low[:, n:] == 7.0).all()
+    assert torch.equal(low[:, :n], ops().tanh_rows(plain_out, torch.empty(M, n, dtype=torch.bfloat16, device=DEV)))
+    with pytest.raises(Exception):      # inner sizes that are no multiple of 64 have no such form
+        ops().linear_set([(a[:, :K - 8], w[:, :K - 8].contiguous(), low[:, :n])])

@@ -37,7 +37,7 @@ constexpr int F_LD = F_BK + 4;    // LDS row stride in floats (80 bytes: 16-byte
 
 // What a bfloat16 product may apply to its float32 sums before they are rounded (a run-time choice, the same for the whole
 // launch; epilogue 2 of the entry points): the square of max(v, 0).
-constexpr int kActNone = 0, kActRelu2 = 2;
+constexpr int kActNone = 0, kActRelu2 = 2, kActTanh = 5;      // tanh: products of a set only, rounded to bfloat16 as they are stored
 __device__ __forceinline__ float act_value(float v, int act) {
   if (act == kActRelu2) {
     v = fmaxf(v, 0.f);
@@ -2345,6 +2345,7 @@ __global__ __launch_bounds__(S_THREADS) void gemm_skinny_bf16_kernel(const Skinn
 constexpr int S_SET = 6;
 struct SkinnySet {
   SkinnyArgs p[S_SET];
+  int vec;                  // every result's rows and address take groups of four columns
 };
 __global__ __launch_bounds__(S_THREADS) void gemm_skinny_set_kernel(const SkinnySet set) {
   const SkinnyArgs& p = set.p[blockIdx.y];
@@ -2504,8 +2505,9 @@ struct Stripe {
 
 // p.cols_wg: a multiple of 4, at most 16 CT.  vec: the results' rows and addresses take groups of four columns.  GATHER: the input's
 // rows are p.rows' (through addresses of their own, as the input may be longer than a buffer's 31 bits).
-template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
-__global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const SkinnyArgs p, int groups_n, int vec) {
+// SET: one of several products in a launch, whose results may leave as the tanh of the sums.
+template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER, bool SET>
+__device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n, int vec, int block_n, int block_m) {
   using S = Stripe<MT, CT, TK>;
   extern __shared__ __attribute__((aligned(16))) unsigned char stripe_smem[];
   float* part = (float*)stripe_smem;                      // [S_WAVES][kRows][kLd], once the blocks are done with
@@ -2513,7 +2515,7 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
   float* sq_s = scale_s + S::kRows;                       // [kRows][CT * 4]
   const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TL_WAVE);
   const int M = p.M, N = p.N, K = p.K, cw = p.cols_wg;
-  const int n0 = blockIdx.x * cw, m0 = blockIdx.y * S::kRows;
+  const int n0 = block_n * cw, m0 = block_m * S::kRows;
   if (n0 >= N) return;
 
   // A lane fetches chunk lc of row lr + kRowsPerLoad j.  Rows beyond the matrices and blocks beyond the inner size lie beyond the
@@ -2664,6 +2666,15 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
         if constexpr (sizeof(TO) == 2) v[q] = act_value(v[q], p.act);
         if (q < left) sq += v[q] * v[q];
       }
+      if constexpr (SET) {
+        if (p.act == kActTanh) {      // uniform
+          bf16_t* low = (bf16_t*)p.out + (int64_t)m * p.ldo + n;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (q < left) low[q] = (bf16_t)tanhf(v[q]);
+          continue;
+        }
+      }
       TO* to = out + (int64_t)m * p.ldo + n;
       if (vec && left == 4) {
         if constexpr (sizeof(TO) == 4) *(f32x4*)to = v;
@@ -2694,9 +2705,44 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
       float t = 0.f;
 #pragma unroll
       for (int c = 0; c < CT * 4; ++c) t += sq_s[tid * CT * 4 + c];
-      p.emit_sumsq[(int64_t)(m0 + tid) * groups_n + blockIdx.x] = t;
+      p.emit_sumsq[(int64_t)(m0 + tid) * groups_n + block_n] = t;
     }
   }
+}
+
+template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
+__global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const SkinnyArgs p, int groups_n, int vec) {
+  stripe_product<MT, CT, TK, TO, SWIGLU, GATHER, false>(p, groups_n, vec, blockIdx.x, blockIdx.y);
+}
+
+// Several products of up to 16 rows that do not wait for each other as ONE launch (SkinnySet): blockIdx.y names the product, a
+// workgroup owns up to 16 CT of its columns.  Five products of a decode step's six rows (four of 2,048 columns and one of 64, inner size 2,048)
+// take 21.8 us as launches of their own, 11.9 in gemm_skinny_set_kernel (16 columns, two rounds of workgroups) and 9.6 so (36 columns, one round).
+template <int CT, int TK>
+__global__ __launch_bounds__(S_THREADS) void gemm_stripe_set_kernel(const SkinnySet set) {
+  stripe_product<1, CT, TK, float, 0, false, true>(set.p[blockIdx.y], 0, set.vec, blockIdx.x, 0);
+}
+template <int CT, int TK>
+static int launch_stripe_set(SkinnySet& set, int count, int most, int cols, hipStream_t stream) {
+  constexpr size_t smem = Stripe<1, CT, TK>::kSmem;
+  static bool configured = false;
+  if (!configured) {
+    if (hipFuncSetAttribute((const void*)gemm_stripe_set_kernel<CT, TK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+      return TL_ERR_LAUNCH;
+    configured = true;
+  }
+  for (int i = 0; i < count; ++i) set.p[i].cols_wg = cols;
+  hipLaunchKernelGGL((gemm_stripe_set_kernel<CT, TK>), dim3((most + cols - 1) / cols, count), dim3(S_THREADS), smem, stream, set);
+  return TL_OK;
+}
+// As few columns a workgroup (8 to 48, a multiple of 4) as make one round of the 256 units, else 16.
+static int stripe_set_cols(const SkinnySet& set, int count) {
+  for (int cols = 8; cols <= 48; cols += 4) {
+    int64_t groups = 0;
+    for (int i = 0; i < count; ++i) groups += (set.p[i].N + cols - 1) / cols;
+    if (groups <= 256) return cols;
+  }
+  return S_COLS;
 }
 
 // Several groups of rows: those of one group of columns fall on one die and find its weights in the L2 (48 rows of 5,120 x 5,120,
@@ -3110,20 +3156,38 @@ int tl_linear(const void* a, const void* w, void* out, const float* residual, co
   return tl_linear_tile(a, w, out, residual, row_scale, M, N, K, lda, ldo, dtype, out_dtype, epilogue, 0, 0.f, 0.f, 0.f, stream);
 }
 
+// Whether tl_linear_set may be told to leave a product's results as tanh in bfloat16 (inner sizes of whole 64).
+int tl_linear_set_tanh(int K) { return K > 0 && K % 64 == 0 && K <= T_MAX_INNER; }
+
 // `count` products of at most 16 rows, one inner size: out[i] (float32 [M, n[i]], rows ldo[i] apart) = a[i] @ w[i]^T,
-// a[i] bfloat16 [M, K] with rows lda[i] apart, w[i] bfloat16 [n[i], K].  The arrays are read here, before the launch.
-// Five products of a decode step's six rows (four of 2,048 columns and one of 64, inner size 2,048) take 21.8 us as
-// launches of their own and 11.5 us so (12.4 with 32 columns a workgroup).
+// a[i] bfloat16 [M, K] with rows lda[i] apart, w[i] bfloat16 [n[i], K]; tanh[i] (where tl_linear_set_tanh says so): out[i] is bfloat16, the tanh of
+// the sums.  The arrays are read here, before the launch.
 int tl_linear_set(const void* const* a, const void* const* w, void* const* out, const int32_t* n, const int64_t* lda,
-                  const int64_t* ldo, int count, int M, int K, hipStream_t stream) {
+                  const int64_t* ldo, const int32_t* tanh, int count, int M, int K, hipStream_t stream) {
   if (count <= 0 || M <= 0) return TL_OK;
   if (count > S_SET || M > 16 || K <= 0 || K % 8) return TL_ERR_ARG;
   SkinnySet set{};
   int most = 0;
+  bool whole = tl_linear_set_tanh(K), any_tanh = false;
+  set.vec = 1;
   for (int i = 0; i < count; ++i) {
     if (n[i] <= 0 || lda[i] % 8 || lda[i] < K || ldo[i] < n[i] || !a[i] || !w[i] || !out[i]) return TL_ERR_ARG;
     set.p[i] = SkinnyArgs{a[i], (const bf16_t*)w[i], out[i], nullptr, nullptr, nullptr, nullptr, 0.f, 0, M, n[i], K, lda[i], ldo[i]};
+    set.p[i].act = tanh[i] ? kActTanh : kActNone;
+    any_tanh = any_tanh || tanh[i];
+    whole = whole && lda[i] <= T_MAX_INNER;
+    if (!tanh[i] && (ldo[i] % 4 || n[i] % 4 || (uintptr_t)out[i] % 16)) set.vec = 0;
     most = n[i] > most ? n[i] : most;
+  }
+  if (any_tanh && !whole) return TL_ERR_ARG;
+  if (whole) {
+    const int cols = stripe_set_cols(set, count);
+    const int rc = cols > 32 ? launch_stripe_set<3, 64>(set, count, most, cols, stream)
+                   : cols > 16 ? (K % 128 == 0 ? launch_stripe_set<2, 128>(set, count, most, cols, stream)
+                                               : launch_stripe_set<2, 64>(set, count, most, cols, stream))
+                   : K % 128 == 0 ? launch_stripe_set<1, 128>(set, count, most, cols, stream)
+                                  : launch_stripe_set<1, 64>(set, count, most, cols, stream);
+    return rc == TL_OK ? tl_launch_status() : rc;
   }
   const size_t smem = (size_t)S_WAVES * 16 * 17 * sizeof(float) + (size_t)(S_WAVES + 1) * 16 * sizeof(float);
   hipLaunchKernelGGL(gemm_skinny_set_kernel, dim3((most + S_COLS - 1) / S_COLS, count), dim3(S_THREADS), smem, stream, set);

@@ -426,7 +426,8 @@ LINEAR_SET_MOST = 6     # most products of a set
 
 def linear_set(products) -> None:
     """out = a @ w.T for every (a, w, out) of `products` (2 to 6 of them, of one inner size and at most 16 rows,
-    bfloat16 in, float32 out) in one launch: products that do not wait for each other."""
+    bfloat16 in, float32 out) in one launch: products that do not wait for each other.  An out in bfloat16 gets tanh of the
+    float32 sums (`linear_set_tanh` says where)."""
     a0 = products[0][0]
     M, K = a0.shape
     _need(0 < len(products) <= LINEAR_SET_MOST and M <= LINEAR_SET_ROWS and K % 8 == 0, "linear_set: up to 6 products of up to 16 rows")
@@ -434,7 +435,8 @@ def linear_set(products) -> None:
         _dev(a, w, out)
         _rows_2d(a, "linear_set input")
         _rows_2d(out, "linear_set output")
-        _need(a.dtype == w.dtype == torch.bfloat16 and out.dtype == torch.float32, "linear_set: bfloat16 in, float32 out")
+        _need(a.dtype == w.dtype == torch.bfloat16 and (out.dtype == torch.float32 or linear_set_tanh(K) and out.dtype == torch.bfloat16
+                                                        and a.stride(0) <= WHOLE_MAX_STRIDE), "linear_set: bfloat16 in, float32 out")
         _need(tuple(a.shape) == (M, K) and a.stride(0) % 8 == 0 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
               and tuple(out.shape) == (M, w.shape[0]), "linear_set: a [M, K], w [N, K], out [M, N]")
     n = len(products)
@@ -442,7 +444,13 @@ def linear_set(products) -> None:
     a, w, out = zip(*products)
     _check(_lib().tl_linear_set(ptrs(a, 16), ptrs(w, 16), ptrs(out, 4), (ctypes.c_int32 * n)(*[t.shape[0] for t in w]),
                                 (ctypes.c_int64 * n)(*[t.stride(0) for t in a]), (ctypes.c_int64 * n)(*[t.stride(0) for t in out]),
-                                c_int(n), c_int(M), c_int(K), _stream()), "linear_set")
+                                (ctypes.c_int32 * n)(*[int(t.dtype == torch.bfloat16) for t in out]), c_int(n), c_int(M), c_int(K),
+                                _stream()), "linear_set")
+
+
+def linear_set_tanh(inner: int) -> bool:
+    """Whether a product of a `linear_set` of this inner size may leave its results as tanh in bfloat16."""
+    return bool(_lib().tl_linear_set_tanh(c_int(inner)))
 
 
 FEW_ROWS = 64   # most rows the few-row product takes

@@ -96,15 +96,19 @@ class TimeMix(Mixer):
             ops.shift_save(h, state, self.s_floats, ctx.cu_seqlens_q, ctx.state_slots)
         x = ops.scratch("time_mix_in", (T, 4 * seg), torch.float32, dev)
         gate = ops.scratch("time_mix_gate", (T, S), torch.float32, dev)
-        low = ops.scratch("time_mix_low", (T, self.rank), torch.float32, dev)
+        few = self.dtype == torch.bfloat16 and T <= ops.LINEAR_SET_ROWS
+        act = ops.scratch("time_mix_low_act", (T, self.rank), self.dtype, dev)
+        in_set = few and ops.linear_set_tanh(self.hidden_size)        # the small product's tanh rides in the launch
+        low = act if in_set else ops.scratch("time_mix_low", (T, self.rank), torch.float32, dev)
         products = [(mixes[0], self.w_r, x[:, 0:S]), (mixes[1], self.w_k, x[:, seg:seg + S]),
                     (mixes[2], self.w_v, x[:, 2 * seg:2 * seg + S]), (mixes[3], self.w_g, gate), (mixes[4], self.w1, low)]
-        if self.dtype == torch.bfloat16 and T <= ops.LINEAR_SET_ROWS:
+        if few:
             ops.linear_set(products)
         else:
             for a, w, out in products:
                 ops.linear(a, w, out)
-        act = ops.tanh_rows(low, ops.scratch("time_mix_low_act", (T, self.rank), self.dtype, dev))
+        if not in_set:
+            ops.tanh_rows(low, act)
         ops.linear(act, self.w2, x[:, 3 * seg:3 * seg + S])
         o = ops.scratch("time_mix_o", (T * S,), torch.float32, dev)
         if not single and self.form(ctx.sizes):

@@ -2506,7 +2506,7 @@ struct Stripe {
 // p.cols_wg: a multiple of 4, at most 16 CT.  vec: the results' rows and addresses take groups of four columns.  GATHER: the input's
 // rows are p.rows' (through addresses of their own, as the input may be longer than a buffer's 31 bits).
 // SET: one of several products in a launch, whose results may leave as the tanh of the sums.
-template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER, bool SET>
+template <int MT, int CT, int TK, int SUMS, typename TO, int SWIGLU, bool GATHER, bool SET>
 __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n, int vec, int block_n, int block_m) {
   using S = Stripe<MT, CT, TK>;
   extern __shared__ __attribute__((aligned(16))) unsigned char stripe_smem[];
@@ -2551,11 +2551,15 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
   const int r16 = lane % 16, g = lane / 16;
   unsigned char* own = stripe_smem + wave * S::kWaveBytes;
   auto place = [&](int j) { return own + j * 1024 + lr * TK * 2 + (lc ^ ((j * S::kRowsPerLoad + lr) % kSwizzle)) * 16; };
-  f32x4 acc[MT][CT];
+  // SUMS 2: sums of their own for every other step of 32 k, added at the end, half the roundings in a row (2,048 x 5,632 against
+  // 64 bits: 1.61e-7 of the result with one, 1.20e-7 with two; split over workgroups, as such products were, 1.30e-7).
+  f32x4 acc[SUMS][MT][CT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int h = 0; h < SUMS; ++h)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) acc[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) acc[h][mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto multiply = [&](Block& st, int next) {      // and requests the next block as soon as this one has left its registers
 #pragma unroll
     for (int j = 0; j < S::kW; ++j) *(bf16x8*)place(S::kA + j) = st.w[j];
@@ -2574,7 +2578,7 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
-          acc[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ct], fa[mt], acc[mt][ct], 0, 0, 0);
+          acc[i % SUMS][mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ct], fa[mt], acc[i % SUMS][mt][ct], 0, 0, 0);
     }
   };
   // The parts of the rows' sums of squares are requested ahead of everything else, up to 256 of a row together, and added up once the
@@ -2637,7 +2641,11 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) *(f32x4*)(part + (wave * S::kRows + mt * 16 + r16) * S::kLd + ct * 16 + g * 4) = acc[mt][ct];
+    for (int ct = 0; ct < CT; ++ct) {
+      f32x4 v = acc[0][mt][ct];
+      if constexpr (SUMS == 2) v += acc[1][mt][ct];
+      *(f32x4*)(part + (wave * S::kRows + mt * 16 + r16) * S::kLd + ct * 16 + g * 4) = v;
+    }
   __syncthreads();
   TO* out = (TO*)p.out;
 #pragma unroll
@@ -2710,9 +2718,9 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
   }
 }
 
-template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
+template <int MT, int CT, int TK, int SUMS, typename TO, int SWIGLU, bool GATHER>
 __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const SkinnyArgs p, int groups_n, int vec) {
-  stripe_product<MT, CT, TK, TO, SWIGLU, GATHER, false>(p, groups_n, vec, blockIdx.x, blockIdx.y);
+  stripe_product<MT, CT, TK, SUMS, TO, SWIGLU, GATHER, false>(p, groups_n, vec, blockIdx.x, blockIdx.y);
 }
 
 // Several products of up to 16 rows that do not wait for each other as ONE launch (SkinnySet): blockIdx.y names the product, a
@@ -2720,7 +2728,7 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
 // take 21.8 us as launches of their own, 11.9 in gemm_skinny_set_kernel (16 columns, two rounds of workgroups) and 9.6 so (36 columns, one round).
 template <int CT, int TK>
 __global__ __launch_bounds__(S_THREADS) void gemm_stripe_set_kernel(const SkinnySet set) {
-  stripe_product<1, CT, TK, float, 0, false, true>(set.p[blockIdx.y], 0, set.vec, blockIdx.x, 0);
+  stripe_product<1, CT, TK, 1, float, 0, false, true>(set.p[blockIdx.y], 0, set.vec, blockIdx.x, 0);
 }
 template <int CT, int TK>
 static int launch_stripe_set(SkinnySet& set, int count, int most, int cols, hipStream_t stream) {
@@ -2749,9 +2757,9 @@ static int stripe_set_cols(const SkinnySet& set, int count) {
 // three groups of 86 32.3 us where they fell on different dies, 19.3 so).
 static int stripe_grid_n(int groups_n, int groups_m) { return groups_m > 1 ? (groups_n + kXcds - 1) / kXcds * kXcds : groups_n; }
 
-template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
-static int launch_stripe_blocks(const SkinnyArgs& p, hipStream_t stream) {
-  const auto kernel = gemm_stripe_bf16_kernel<MT, CT, TK, TO, SWIGLU, GATHER>;
+template <int MT, int CT, int TK, int SUMS, typename TO, int SWIGLU, bool GATHER>
+static int launch_stripe_sums(const SkinnyArgs& p, hipStream_t stream) {
+  const auto kernel = gemm_stripe_bf16_kernel<MT, CT, TK, SUMS, TO, SWIGLU, GATHER>;
   constexpr size_t smem = Stripe<MT, CT, TK>::kSmem;
   static bool configured = false;
   if (!configured) {
@@ -2763,6 +2771,14 @@ static int launch_stripe_blocks(const SkinnyArgs& p, hipStream_t stream) {
   dim3 g(stripe_grid_n(groups_n, groups_m), groups_m), b(S_THREADS);
   hipLaunchKernelGGL(kernel, g, b, smem, stream, p, groups_n, vec);
   return TL_OK;
+}
+
+// Two sums beyond 2,048 k (up to there one is as close to 64 bits as what took such products before), where the registers allow.
+template <int MT, int CT, int TK, typename TO, int SWIGLU, bool GATHER>
+static int launch_stripe_blocks(const SkinnyArgs& p, hipStream_t stream) {
+  if constexpr (MT * CT <= 4)
+    if (p.K > 2048) return launch_stripe_sums<MT, CT, TK, 2, TO, SWIGLU, GATHER>(p, stream);
+  return launch_stripe_sums<MT, CT, TK, 1, TO, SWIGLU, GATHER>(p, stream);
 }
 
 template <int MT, int CT, typename TO, int SWIGLU>
@@ -2811,7 +2827,8 @@ static bool stripe_plan(int M, int N, int K, StripePlan* plan) {
       // 5,120 x 5,120 20.6 -> 19.0 us, 16 rows of 2,048 x 5,632 10.3 -> 9.0)
       int even = (int)((N * (int64_t)groups_m + 255) / 256 + 3) / 4 * 4;
       if (tiles == 1 && even < 8) even = 8;
-      *plan = {mt, ct, groups <= 256 && (ct >= 3 || tiles == 1) && even > 16 * (ct - 1) && even < 16 * ct ? even : 16 * ct};
+      const bool one_round = (int64_t)groups_m * stripe_grid_n((N + even - 1) / even, groups_m) <= 256;      // also as the grid is filled up
+      *plan = {mt, ct, one_round && (ct >= 3 || tiles == 1) && even > 16 * (ct - 1) && even < 16 * ct ? even : 16 * ct};
     }
   if (M <= 8) return fewest <= 256 && N > 2048 && (plan->cols != 16 || K > 4096);
   if (M <= 16) return true;

@@ -1723,3 +1723,41 @@ def test_linear_set_leaves_tanh(M, K, n):
     assert torch.equal(low[:, :n], ops().tanh_rows(plain_out, torch.empty(M, n, dtype=torch.bfloat16, device=DEV)))
     with pytest.raises(Exception):      # inner sizes that are no multiple of 64 have no such form
         ops().linear_set([(a[:, :K - 8], w[:, :K - 8].contiguous(), low[:, :n])])
+
+
+@pytest.mark.parametrize("M", [1, 6, 9, 17, 33, 64, 65])
+@pytest.mark.parametrize("N,K", [(518, 704), (2046, 128), (2560, 2048), (4102, 1088), (4096, 64), (300, 72)])
+def test_linear_residual_of_bfloat16_results(M, N, K):
+    """A float32 residual of results that leave in bfloat16: by every kernel that takes such a product, rows of their own stride
+    and side by side, columns that end within a group of four; beside it the hand-off and the norm in front."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
+    exact, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    da, dw = a.to(DEV), w.to(DEV)
+    inv = torch.rand(M, generator=g) + 0.5
+    x = torch.randn(M, K, generator=g)
+    nw = 1 + 0.1 * torch.randn(K, generator=g)
+    for pad in (0, 8, 6):
+        wide = torch.randn(M, N + pad, generator=g)
+        res = wide[:, :N].double()
+        dr = wide.to(DEV)[:, :N]
+
+        def check(call, exact, size):
+            full = torch.full((M, N + pad), 7.0, dtype=torch.bfloat16, device=DEV)
+            out = full[:, :N]
+            call(out)
+            # the result's own rounding to 8 bits beside at most K + 3 roundings of the float32 sum, its factor and the addition
+            bound = 2.0 ** -8 * (exact + res).abs() + 1.01 * (K + 3) * 2.0 ** -24 * (size + res.abs())
+            assert ((out.cpu().double() - exact - res).abs() <= bound).all()
+            assert (full[:, N:] == 7.0).all()
+
+        check(lambda out: ops().linear(da, dw, out, dr), exact, size)
+        f = inv.double()[:, None]
+        check(lambda out: ops().linear(da, dw, out, dr, row_scale=inv.to(DEV)), exact * f, size * f)
+        check(lambda out: ops().linear_handoff(da, dw, out, dr), exact, size)
+        # the norm's operand is rounded to bfloat16 ahead of the product: that is the product's input
+        h = (nw * x).to(torch.bfloat16).double()
+        f = 1.0 / torch.sqrt((x.double() ** 2).mean(dim=1, keepdim=True) + 1e-5)
+        # (the factor, a root of a sum of K squares and a reciprocal, is no further off than the sums: twice their bound)
+        check(lambda out: ops().linear_norm(x.to(DEV), nw.to(DEV), 1e-5, dw, out, dr), (h @ w.double().T) * f, 2 * (h.abs() @ w.double().abs().T) * f)

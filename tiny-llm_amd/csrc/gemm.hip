@@ -2608,7 +2608,7 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
     res_v[j] = next_w[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (SWIGLU == 0 && sizeof(TO) == 4) {
+    if constexpr (SWIGLU == 0) {      // the residual is float32 whatever the results are
       const int e = tid + j * S_THREADS, c = e % (CT * 4) * 4, n = n0 + c;
       const int m = min(m0 + e / (CT * 4), M - 1);
       if (p.residual) {
@@ -2618,10 +2618,11 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
 #pragma unroll
           for (int q = 0; q < 4; ++q) res_v[j][q] = r[min(n + q, N - 1)];
       }
-      if (p.emit_operand)
+      if constexpr (sizeof(TO) == 4)
+        if (p.emit_operand)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          next_w[j][q] = p.emit_w_is_f32 ? ((const float*)p.emit_w)[min(n + q, N - 1)] : (float)((const bf16_t*)p.emit_w)[min(n + q, N - 1)];
+          for (int q = 0; q < 4; ++q)
+            next_w[j][q] = p.emit_w_is_f32 ? ((const float*)p.emit_w)[min(n + q, N - 1)] : (float)((const bf16_t*)p.emit_w)[min(n + q, N - 1)];
     }
   }
   if (p.in_sumsq) {      // the rows' factors: one wave a row, in a fixed order

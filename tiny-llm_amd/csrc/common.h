@@ -93,6 +93,14 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// What the lanes of ONE wave have written to LDS is there for all of them behind it, and what they have read is read: its LDS
+// instructions run in order, so this only holds the compiler to the order (no instruction).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Maximum and minimum over a row of 16 lanes (integers); every lane of the row gets the result.
 __device__ __forceinline__ int row_max_i32(int v) {
   v = max(v, dpp_i32<TL_DPP_ROR8>(v));

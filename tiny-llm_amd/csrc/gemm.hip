@@ -758,11 +758,6 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
     }
   };
   float* own = lines_smem + wave * FL_AREA;
-  auto sync = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
   // chunk c of row r stands at place c ^ r of its 32; what lies beyond K is zero
   auto put = [&](f32x4 (&v)[8], int k0) {
     if (k0 + (PAIR ? F_KBLOCK : 0) + FL_HALF > K)      // uniform
@@ -774,12 +769,12 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
       }
 #pragma unroll
     for (int i = 0; i < 8; ++i) *(f32x4*)(own + (2 * i + lr) * FL_HALF + (lc ^ (2 * i + lr)) * 4) = v[i];
-    sync();
+    wave_sync();
   };
   auto get = [&](f32x4 (&v)[8]) {
 #pragma unroll
     for (int g = 0; g < 8; ++g) v[g] = *(const f32x4*)(own + l16 * FL_HALF + ((g * 4 + kk) ^ l16) * 4);
-    sync();
+    wave_sync();
   };
   Step st;
 #pragma unroll
@@ -1380,9 +1375,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
               f32x4{c[q * 4 + 0], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
     auto leave = [&](auto form) {
       constexpr int FORM = decltype(form)::value;
       constexpr bool AHEAD = FORM != kNoResidual && sizeof(TO) == 4 && !NEXT;
@@ -1511,9 +1504,7 @@ __global__ __launch_bounds__(WM * WN * TL_WAVE) void gemm_bf16_kernel(const bf16
     else if (!SWIGLU && residual && vec_ok) leave(std::integral_constant<int, kResidual>{});
     else leave(std::integral_constant<int, kNoResidual>{});
     // the area is written again for the next 32 rows
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
   }
 }
 
@@ -2566,6 +2557,7 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
 #pragma unroll
     for (int j = 0; j < S::kA; ++j) *(bf16x8*)place(j) = st.a[j];
     load(st, next);
+    wave_sync();      // other lanes read them
 #pragma unroll
     for (int i = 0; i < TK / 32; ++i) {
       const unsigned char* from = own + r16 * TK * 2 + ((i * 4 + g) ^ (r16 % kSwizzle)) * 16;
@@ -2580,6 +2572,7 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
         for (int mt = 0; mt < MT; ++mt)
           acc[i % SUMS][mt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ct], fa[mt], acc[i % SUMS][mt][ct], 0, 0, 0);
     }
+    wave_sync();      // the area is written again for the next block
   };
   // The parts of the rows' sums of squares are requested ahead of everything else, up to 256 of a row together, and added up once the
   // first block has been requested (behind it, and one request after the other: a decode step of 8 rows 3.4 % slower).

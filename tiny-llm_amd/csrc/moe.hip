@@ -711,13 +711,6 @@ __device__ __forceinline__ bool route_by_lanes(const float* zr, const RouteOptio
   return true;
 }
 
-// What the lanes of ONE wave have written to LDS is there for all of them (its LDS instructions run in order).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The general form, by one wave.  s: choice scores, -inf once an expert is chosen or its run is out; gs: the runs' scores;
 // plain: scores without the correction (all in LDS, o.experts long).
 __device__ void route_general(const float* zr, const RouteOptions& o, int32_t* ids, float* wts, int lane, float* s, float* gs, float* plain) {

@@ -68,3 +68,21 @@ def test_a_wave_reads_a_block_once_it_is_written_whole(kernels):
         assert exchanges(main_loop(lines), (mt + ct) * tk // 32), name
         seen += 1
     assert seen
+
+
+def scalar_offsets(lines):
+    """The scalar offsets of a listing's buffer loads."""
+    return [re.split(r",\s*(?![^\[]*\])", line)[3].split()[0] for line in lines if line.startswith("buffer_load_")]
+
+
+def test_rows_beyond_a_matrix_are_beyond_a_lane_s_own_offset(kernels):
+    """The kernels that fetch whole lines ask for rows beyond the matrices and for blocks beyond the inner size, and rely on the
+    buffers' ends: of an offset only a lane's own part is sure to be compared with them."""
+    assert scalar_offsets(["buffer_load_dwordx4 v[8:11], v94, s[4:7], s14 offen", "buffer_load_dword v8, v94, s[4:7], 0 offen"]) == ["s14", "0"]
+    seen = 0
+    for name, lines in kernels.items():
+        if "gemm_stripe_" in name or "gemm_f32_lines_" in name:
+            offsets = scalar_offsets(lines)
+            seen += len(offsets)
+            assert set(offsets) <= {"0"}, name
+    assert seen

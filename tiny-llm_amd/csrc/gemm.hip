@@ -719,7 +719,7 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const F32Rows
 // instruction then fetches half of what it could, and 8 columns are what bounds these products,
 // since a workgroup is as fast as its loads.  A wave takes pairs of blocks instead of blocks.
 constexpr int FL_HALF = F_KBLOCK / 2, FL_AREA = 16 * FL_HALF;      // k of a step; floats of a wave's area
-constexpr int64_t FL_MAX_STRIDE = 1 << 24;                         // floats between rows: offsets within sixteen rows fit 31 bits
+constexpr int64_t FL_MAX_STRIDE = 1 << 24;                         // floats between rows: sixteen rows end below 2^30 bytes, and offsets below twice that
 constexpr size_t FL_STAGE_BYTES = (size_t)FR_WAVES * FL_AREA * sizeof(float), FL_SUM_BYTES = 96 * 1024;      // together a unit's LDS
 template <bool SWIGLU, int CT, bool PAIR, bool NORM>
 __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32RowsNorm norm, const float* __restrict__ a, const float* __restrict__ w,
@@ -736,26 +736,35 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
   const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TL_WAVE);
   const int l16 = lane % 16, kk = lane / 16, lr = lane / 32, lc = lane % 32;
   const int n0 = blockIdx.x * cw, stride_a = (int)lda;
-  // Both operands as buffers: rows beyond the matrices, and steps beyond this wave's, read as zeros and fetch nothing
+  // Both operands as buffers: rows beyond the matrices, and steps beyond this wave's, read as zeros and fetch nothing.  All of an
+  // offset is a lane's own (scalar offset 0): that is what the check of a buffer's end is documented for.
   auto rows_of = [&](const float* base, int stride, int rows) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, rows > 0 ? ((rows - 1) * stride + K) * 4 : 0, 0x00020000);
   };
   const auto buf_w = rows_of(w + (int64_t)n0 * K, K, min(cw, N - n0)), buf_a = rows_of(a, stride_a, M);
-  const int at_w = (lr * K + lc * 4) * 4, at_a = (lr * stride_a + lc * 4) * 4;
   const int mine = wave < units ? 2 * ((units - wave + FR_WAVES - 1) / FR_WAVES) : 0;      // half blocks (PAIR: of two blocks)
+  auto first_k = [&](int s) { return ((wave + s / 2 * FR_WAVES) * UNIT * F_KBLOCK) + s % 2 * FL_HALF; };
   // load i of a step: 16 bytes of row 2 i + lane / 32 (PAIR: from row 8 on the rows 0 .. of the next k block), k 4 (lane % 32) ..
+  constexpr int PLACES = PAIR ? 4 : 8, BEYOND = 0x40000000;      // bytes: beyond every buffer here
+  int at_w[PLACES], at_a[PLACES];
+#pragma unroll
+  for (int i = 0; i < PLACES; ++i) {
+    const int from = mine > 0 ? first_k(0) * 4 : BEYOND;
+    at_w[i] = ((2 * i + lr) * K + lc * 4) * 4 + from;
+    at_a[i] = ((2 * i + lr) * stride_a + lc * 4) * 4 + from;
+  }
+  auto advance = [&](int (&at)[PLACES], int s) {      // from step s to the next
+    const int by = s + 1 >= mine ? BEYOND : (s % 2 == 0 ? FL_HALF : FR_WAVES * UNIT * F_KBLOCK - FL_HALF) * 4;
+#pragma unroll
+    for (int i = 0; i < PLACES; ++i) at[i] += by;
+  };
   struct Step {
     f32x4 a[8], w[CT][8];
   };
-  auto first_k = [&](int s) { return ((wave + s / 2 * FR_WAVES) * UNIT * F_KBLOCK) + s % 2 * FL_HALF; };
-  auto load_tile = [&](f32x4 (&v)[8], auto buf, int at, int stride, int row0, int s) {
-    const int k0 = first_k(s);
+  auto load_tile = [&](f32x4 (&v)[8], auto buf, const int (&at)[PLACES], int tile) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const bool up = PAIR && i >= 4;
-      const int row = row0 + 2 * i - (up ? 8 : 0), k = k0 + (up ? F_KBLOCK : 0);
-      v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, at, s < mine ? (row * stride + k) * 4 : 0x70000000, 0));
-    }
+    for (int i = 0; i < 8; ++i)
+      v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, at[i % PLACES] + tile + i / PLACES * F_KBLOCK * 4, 0, 0));
   };
   float* own = lines_smem + wave * FL_AREA;
   // chunk c of row r stands at place c ^ r of its 32; what lies beyond K is zero
@@ -777,9 +786,10 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
     wave_sync();
   };
   Step st;
+  load_tile(st.a, buf_a, at_a, 0);      // in the order in which they are needed
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) load_tile(st.w[ct], buf_w, at_w, K, ct * 16, 0);
-  load_tile(st.a, buf_a, at_a, stride_a, 0, 0);
+  for (int ct = 0; ct < CT; ++ct) load_tile(st.w[ct], buf_w, at_w, ct * 16 * K * 4);
   // NORM: the norm's weights of a step, as operands (4 K bytes, from the caches), requested a step ahead
   f32x4 nw[NORM ? 8 : 1];
   auto load_norm = [&](int s) {
@@ -800,7 +810,8 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
     }
     f32x4 av[8];
     put(st.a, k0);
-    load_tile(st.a, buf_a, at_a, stride_a, 0, s + 1);
+    advance(at_a, s);
+    load_tile(st.a, buf_a, at_a, 0);
     get(av);
     if constexpr (NORM) {      // the rows times the norm's weights, their squares added up on the way
 #pragma unroll
@@ -816,7 +827,8 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
     for (int ct = 0; ct < CT; ++ct) {
       f32x4 wv[8];
       put(st.w[ct], k0);
-      load_tile(st.w[ct], buf_w, at_w, K, ct * 16, s + 1);
+      if (ct == 0) advance(at_w, s);
+      load_tile(st.w[ct], buf_w, at_w, ct * 16 * K * 4);
       get(wv);
 #pragma unroll
       for (int g = 0; g < 8; ++g)
@@ -2510,7 +2522,8 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
   if (n0 >= N) return;
 
   // A lane fetches chunk lc of row lr + kRowsPerLoad j.  Rows beyond the matrices and blocks beyond the inner size lie beyond the
-  // buffers: they read as zero and fetch nothing.
+  // buffers: they read as zero and fetch nothing.  All of an offset is a lane's own (scalar offset 0): that is what the check of a
+  // buffer's end is documented for.
   const int lr = lane / S::kChunks, lc = lane % S::kChunks, lda = (int)p.lda;
   const auto buf_w = __builtin_amdgcn_make_buffer_rsrc((void*)(p.w + (int64_t)n0 * K), 0, min(cw, N - n0) * K * 2, 0x00020000);
   const auto buf_a = __builtin_amdgcn_make_buffer_rsrc((void*)((const bf16_t*)p.a + (int64_t)m0 * lda), 0,
@@ -2530,11 +2543,11 @@ __device__ __forceinline__ void stripe_product(const SkinnyArgs& p, int groups_n
     const int k = i < mine ? (wave + i * S_WAVES) * TK * 2 : 0x70000000;
 #pragma unroll
     for (int j = 0; j < S::kW; ++j)
-      st.w[j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(buf_w, at_w, k + j * step_w, 0));
+      st.w[j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(buf_w, at_w + k + j * step_w, 0, 0));
 #pragma unroll
     for (int j = 0; j < S::kA; ++j) {
       if constexpr (GATHER) st.a[j] = i < mine ? *(const bf16x8*)(row_a[j] + k / 2) : bf16x8{};
-      else st.a[j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(buf_a, at_a, k + j * step_a, 0));
+      else st.a[j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(buf_a, at_a + k + j * step_a, 0, 0));
     }
   };
   // chunk c of row r stands at place c ^ (r % kSwizzle) of its row, so that the operands of eight rows do not collide

@@ -1761,3 +1761,31 @@ def test_linear_residual_of_bfloat16_results(M, N, K):
         f = 1.0 / torch.sqrt((x.double() ** 2).mean(dim=1, keepdim=True) + 1e-5)
         # (the factor, a root of a sum of K squares and a reciprocal, is no further off than the sums: twice their bound)
         check(lambda out: ops().linear_norm(x.to(DEV), nw.to(DEV), 1e-5, dw, out, dr), (h @ w.double().T) * f, 2 * (h.abs() @ w.double().abs().T) * f)
+
+
+@pytest.mark.parametrize("M,N,K", [(12, 512, 32768), (9, 100, 24580), (16, 2048, 24832), (16, 10, 49152), (8, 512, 49152)])
+def test_few_float32_rows_of_long_inner_sizes(M, N, K):
+    """9 to 16 rows, eight columns a workgroup, inner sizes of 24,577 to 49,152: still the kernel of few rows, and the bits of the tiled one."""
+    assert ops().linear_f32_lines(M, N, K, K) and (M <= 8 or not ops().linear_f32_lines(M, N, 49156, 49156))
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    a, w, scale = rnd(300, K), rnd(N, K) / math.sqrt(K), torch.rand(300, device=DEV, generator=g) + 0.5
+    x = rnd(300, N)
+    many, few = x.clone(), x[:M].clone()
+    ops().linear(a, w, many, many, row_scale=scale)
+    ops().linear(a[:M], w, few, few, row_scale=scale[:M])
+    assert torch.equal(few, many[:M])
+    exact = (a[:M].double() @ w.double().T) * scale[:M].double()[:, None] + x[:M].double()
+    size = (a[:M].double().abs() @ w.double().abs().T) * scale[:M].double()[:, None] + x[:M].double().abs()
+    assert ((few.double() - exact).abs() <= (K + 3) * 2.0 ** -24 * size).all()
+    many, few = torch.empty(300, N // 2, device=DEV), torch.empty(M, N // 2, device=DEV)
+    ops().linear(a, w, many, epilogue="swiglu")
+    ops().linear(a[:M], w, few, epilogue="swiglu")
+    assert torch.equal(few, many[:M])
+    if ops().linear_norm_f32_ok(M, N, K, K):
+        nw = rnd(K)
+        inside, apart = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+        ops().linear_norm_f32(a[:M], nw, 1e-5, w, inside)
+        h, inv = ops().norm_prescale_f32(a[:M], nw, 1e-5)
+        ops().linear(h, w, apart, row_scale=inv)
+        assert torch.equal(inside, apart)

@@ -727,12 +727,13 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
                                                                     int M, int N, int K, int64_t lda, int64_t ldo,
                                                                     const float* __restrict__ row_scale, int cw) {
   static_assert(CT == 1 || (!PAIR && !NORM), "pairs of k blocks and the norm: one column tile");
-  constexpr int COLS = PAIR ? 8 : 16, UNIT = PAIR ? 2 : 1;
+  constexpr int UNIT = PAIR ? 2 : 1;
   extern __shared__ __attribute__((aligned(16))) float lines_smem[];
   constexpr int ROWS = PAIR ? 8 : 16;
   const int nkb = (K + F_KBLOCK - 1) / F_KBLOCK, units = (nkb + UNIT - 1) / UNIT;
-  float* sums = lines_smem + FR_WAVES * FL_AREA;            // [CT][k blocks][ROWS][COLS], NORM: + [k blocks][ROWS]
-  float* squares = sums + CT * nkb * ROWS * COLS;
+  const int col_bits = PAIR || (CT == 1 && cw <= 8) ? 3 : 4, cols = 1 << col_bits;      // columns of a tile that have sums
+  float* sums = lines_smem + FR_WAVES * FL_AREA;            // [CT][k blocks][ROWS][cols], NORM: + [k blocks][ROWS]
+  float* squares = sums + CT * nkb * ROWS * cols;
   const int tid = threadIdx.x, lane = tid % TL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TL_WAVE);
   const int l16 = lane % 16, kk = lane / 16, lr = lane / 32, lc = lane % 32;
   const int n0 = blockIdx.x * cw, stride_a = (int)lda;
@@ -845,19 +846,19 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
         if constexpr (PAIR) {     // rows 0..7 x columns 0..7: the first block; 8..15 x 8..15: the second
-          if ((l16 < 8) == (kk < 2) && b < nkb) *(f32x4*)(&sums[(b * ROWS + l16 % 8) * COLS + (kk % 2) * 4]) = acc[ct];
+          if ((l16 < 8) == (kk < 2) && b < nkb) *(f32x4*)(&sums[(b * ROWS + l16 % 8) * 8 + (kk % 2) * 4]) = acc[ct];
         } else {
-          *(f32x4*)(&sums[((ct * nkb + b) * ROWS + l16) * COLS + kk * 4]) = acc[ct];
+          if (kk * 4 < cols) *(f32x4*)(&sums[(((ct * nkb + b) * ROWS + l16) << col_bits) + kk * 4]) = acc[ct];
         }
       }
     }
   }
   __syncthreads();
-  for (int e = tid; e < CT * ROWS * COLS; e += FR_THREADS) {
-    const int ct = e / (ROWS * COLS), r = e % (ROWS * COLS) / COLS, c = e % COLS;
+  for (int e = tid; e < CT * ROWS * cols; e += FR_THREADS) {
+    const int ct = e / ROWS >> col_bits, r = (e >> col_bits) % ROWS, c = e % cols;
     float t = 0.f;
-    for (int b = 0; b < nkb; ++b) t += sums[((ct * nkb + b) * ROWS + r) * COLS + c];
-    const int n = n0 + ct * COLS + c;
+    for (int b = 0; b < nkb; ++b) t += sums[(((ct * nkb + b) * ROWS + r) << col_bits) + c];
+    const int n = n0 + ct * 16 + c;
     if constexpr (NORM) {
       float q = 0.f;
       for (int b = 0; b < nkb; ++b) q += squares[b * ROWS + r];
@@ -865,7 +866,7 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_lines_kernel(const F32Row
     } else if (row_scale && r < M) {
       t *= row_scale[r];      // the factor of a norm in front (norm_prescale_f32_kernel)
     }
-    const bool there = r < M && n < N && ct * COLS + c < cw;
+    const bool there = r < M && n < N && ct * 16 + c < cw;
     if constexpr (SWIGLU) {   // columns (2j, 2j+1) = (gate_j, up_j); N and n0 are even
       const float u = __shfl_down(t, 1, TL_WAVE);
       if (there && (c & 1) == 0) out[(int64_t)r * ldo + n / 2] = swiglu_pair(t, u);
@@ -2936,7 +2937,8 @@ static bool f32_lines_plan(int M, int N, int K, int64_t lda, bool norm, F32Lines
     const int rounds = (N + 256 * 16 - 1) / (256 * 16), even = ((N + 256 * rounds - 1) / (256 * rounds) + 1) / 2 * 2;
     p->cw = eight ? 8 : p->ct == 1 ? even : 16 * p->ct;
   }
-  p->sums = (size_t)nkb * (p->pair ? 8 * 8 : 16 * 16 * p->ct) * sizeof(float) + (norm ? (size_t)nkb * 16 * sizeof(float) : 0);
+  // (eight columns have sums for eight: 9 to 16 rows of up to 2,048 columns and inner sizes of 24,577 to 49,152 fit so)
+  p->sums = (size_t)nkb * (p->pair ? 8 * 8 : 16 * (p->cw <= 8 ? 8 : 16 * p->ct)) * sizeof(float) + (norm ? (size_t)nkb * 16 * sizeof(float) : 0);
   return p->sums <= FL_SUM_BYTES;
 }
 
@@ -2973,6 +2975,12 @@ int tl_linear_norm_f32_ok(int M, int N, int K, int64_t lda) {
 // workgroup's activation rows once per column tile; the bits are the same either way.
 int tl_linear_f32_col_tiles(int M, int N, int K) {
   return f32_rows_col_tiles(M, N, K, (N + 7) / 8 <= 256 ? 8 : 16);
+}
+
+// Whether the float32 product of these sizes, rows in whole vectors, is gemm_f32_lines_kernel's (norm: with the norm inside).
+int tl_linear_f32_lines(int M, int N, int K, int64_t lda, int norm) {
+  F32Lines lines;
+  return M > 0 && N > 0 && K > 0 && K % 4 == 0 && lda % 4 == 0 && f32_lines_plan(M, N, K, lda, norm != 0, &lines) ? 1 : 0;
 }
 
 int tl_linear_norm_f32(const float* x, const float* norm_w, float eps, const float* w, float* out,

@@ -363,6 +363,11 @@ def linear_f32_col_tiles(rows: int, cols: int, inner: int) -> int:
     return int(_lib().tl_linear_f32_col_tiles(c_int(rows), c_int(cols), c_int(inner)))
 
 
+def linear_f32_lines(rows: int, cols: int, inner: int, row_stride: int, norm: bool = False) -> bool:
+    """Whether the float32 product of these sizes (up to 16 rows, in whole vectors) fetches whole lines, with the norm inside or without."""
+    return bool(_lib().tl_linear_f32_lines(c_int(rows), c_int(cols), c_int(inner), c_int64(row_stride), c_int(1 if norm else 0)))
+
+
 def linear_norm_f32(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w: torch.Tensor, out: torch.Tensor,
                     residual: Optional[torch.Tensor] = None, epilogue: Optional[str] = None) -> torch.Tensor:
     """out = rmsnorm(x; norm_weight, eps) @ w.T, then the epilogue of `linear`, all float32 and for few

@@ -1789,3 +1789,28 @@ def test_few_float32_rows_of_long_inner_sizes(M, N, K):
         h, inv = ops().norm_prescale_f32(a[:M], nw, 1e-5)
         ops().linear(h, w, apart, row_scale=inv)
         assert torch.equal(inside, apart)
+
+
+@pytest.mark.parametrize("M", [9, 17, 33, 64])
+@pytest.mark.parametrize("K", [704, 832, 1088, 1984])
+def test_sums_of_uneven_blocks_meet_in_pairs(M, K):
+    """Inner sizes that are an odd multiple of 64: the eight waves' sums are added in pairs.  2^24 and twice 1 in three waves' shares
+    give 2^24 + 2 in pairs, and 2^24 one after the other; and random products are no further from 64 bits than they were in blocks of 128."""
+    a, w = torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(520, K, dtype=torch.bfloat16)
+    for k, v in ((0, 4096.0), (2 * 64 + 5, 1.0), (3 * 64 + 63, 1.0)):
+        a[:, k], w[:, k] = v, v
+    out = torch.empty(M, 520, device=DEV)
+    ops().linear(a.to(DEV), w.to(DEV), out)
+    assert (out == 2.0 ** 24 + 2).all()
+    if M <= 16:
+        ops().linear_set([(a.to(DEV), w.to(DEV), out.zero_())])
+        assert (out == 2.0 ** 24 + 2).all()
+    g = torch.Generator().manual_seed(K)
+    a, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(1024, K, generator=g) / math.sqrt(K)).bfloat16()
+    out = torch.empty(M, 1024, device=DEV)
+    ops().linear(a.to(DEV), w.to(DEV), out)
+    exact = a.double() @ w.double().T
+    # what blocks of 128 k left at these sizes and 9 to 17 rows (sums over 9,216 and more results, so that two draws agree to 1 %;
+    # in pairs it is 5 to 8 % less)
+    former = {704: 7.65e-8, 832: 8.0e-8, 1088: 8.5e-8, 1984: 1.015e-7}[K]
+    assert float((out.cpu().double() - exact).norm() / exact.norm()) <= former

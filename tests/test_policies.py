@@ -181,3 +181,11 @@ def test_the_delta_rule_runs_in_chunks_where_its_longest_portion_pays_for_them()
         assert pays(lens), lens
     assert not pays([1] * 239 + [62], 32, 48, 64) and not pays([1] * 94 + [43], 64, 33, 33)
     assert not pays([2047], dim=32) and not pays([2047], dim=129) and not pays([2047], vdim=129) and not pays([2047], taps=5)
+
+
+def test_no_plan_is_kept_for_rows_that_have_none():
+    """A product of more rows than the kernel of whole lines takes leaves nothing behind: prompts have any length."""
+    kept = len(ops._WHOLE)
+    assert not any(ops.linear_whole(rows, 2048, 2048) for rows in range(65, 600))
+    assert len(ops._WHOLE) == kept
+    assert ops.linear_whole(64, 2048, 2048) and ops.linear_whole(9, 2048, 2048) and not ops.linear_whole(5, 2560, 2048)

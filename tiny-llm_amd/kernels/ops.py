@@ -480,10 +480,12 @@ _SPLITS: dict = {}      # the plan is a pure function of the sizes
 def linear_whole(rows: int, cols: int, inner: int) -> bool:
     """Whether the bfloat16 product [rows, inner] x [cols, inner]^T of 6 to 64 rows goes, its inner size whole, to the kernel that
     fetches whole lines: it is then not split, whatever `split_k` says of its sizes."""
+    if rows > FEW_ROWS:
+        return False        # nothing is kept: a server's prompts have any length
     key = (rows, cols, inner)
     n = _WHOLE.get(key)
     if n is None:
-        n = _WHOLE[key] = rows <= FEW_ROWS and bool(_lib().tl_linear_whole(c_int(rows), c_int(cols), c_int(inner)))
+        n = _WHOLE[key] = bool(_lib().tl_linear_whole(c_int(rows), c_int(cols), c_int(inner)))
     return n
 
 

@@ -189,3 +189,17 @@ def test_no_plan_is_kept_for_rows_that_have_none():
     assert not any(ops.linear_whole(rows, 2048, 2048) for rows in range(65, 600))
     assert len(ops._WHOLE) == kept
     assert ops.linear_whole(64, 2048, 2048) and ops.linear_whole(9, 2048, 2048) and not ops.linear_whole(5, 2560, 2048)
+
+
+def test_few_rows_of_short_inner_sizes_keep_their_kernel():
+    """Where the kernel of whole lines was timed slower than the few-row one (inner sizes of up to 2,048): products of one and of several
+    rounds of workgroups; odd multiples of 64 and longer inner sizes, whose sums are closer to 64 bits so, stay with whole lines."""
+    whole = ops.linear_whole
+    for rows, cols, inner in ((9, 32000, 2048), (16, 32000, 2048), (12, 128256, 2048), (9, 8192, 2048), (10, 6144, 1024), (8, 8192, 2048),
+                              (6, 4704, 640), (8, 2560, 512), (16, 560, 256), (12, 2048, 640), (17, 3072, 256), (24, 4096, 512), (32, 2560, 256),
+                              (9, 18432, 2048), (16, 40960, 1024)):
+        assert not whole(rows, cols, inner), (rows, cols, inner)
+    for rows, cols, inner in ((9, 32000, 2112), (9, 28672, 4096), (16, 28672, 1536), (11, 8192, 2048), (8, 8192, 2560), (8, 2560, 2048), (16, 560, 320),
+                              (16, 1024, 512), (16, 2560, 704), (17, 2048, 256), (25, 4096, 512), (33, 3072, 256), (16, 11264, 2048),
+                              (8, 11264, 2048), (64, 2560, 128)):
+        assert whole(rows, cols, inner), (rows, cols, inner)

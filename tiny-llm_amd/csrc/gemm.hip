@@ -2822,14 +2822,38 @@ static int launch_stripe_tile(const SkinnyArgs& p, hipStream_t stream) {
 // 27,648 x 5,120 at 17, 32, 48 and 64 rows, every cut of each (1,270 in all): the one this picks is within 3 % of the fastest, 0.05 % on average.
 //  * Beyond 16 rows the estimate (us) is compared with the split product's own (oneshot_us; 4 us for its second launch), which is the
 //    faster way for long inner sizes and few columns: 64 rows of 14,336 by 4,096 37.4 us here and 29.9 split; 5,120 x 5,120 19.0 and 19.7.
-//  * 9 to 16 rows: faster than the few-row kernel at each of eleven matrices (16 rows: 2,560 x 2,048 5.9 -> 5.0 us, 2,048 x 2,048 5.7 ->
-//    4.6, 2,048 x 5,632 11.8 -> 9.0, 11,264 x 2,048 gated 12.8 -> 11.6, 4,096 x 14,336 34.7 -> 26.2).
 //  * 6 to 8 rows: in one round, where the few-row kernel has no form of eight columns and a workgroup's columns are not just one
 //    tile of a short inner size (8 rows: 2,560 x 2,048 5.2 -> 4.7, 11,264 x 2,048 12.1 -> 11.6, 6,144 x 4,096 13.1 -> 11.7, 4,096 x
 //    14,336 28.9 -> 25.2, but 4,096 x 4,096 9.7 and 10.0, 2,048 x 2,048 4.6 both).  At 1 row the few-row kernel is the faster one.
+//  * Up to 32 rows and 2,048 k: not where the few-row kernel is the faster one, see below.
 struct StripePlan {
   int mt, ct, cols;
 };
+
+// Whether the few-row kernel is the faster one for up to 32 rows of a short inner size.  Both timed at 3,700 products of 6 to 64 rows, 128 to
+// 151,936 columns and 64 to 16,384 k, weights from memory (us, whole lines and few-row kernel):
+//  * 6 to 8 rows: one column tile a workgroup below 1,536 k (8 rows of 2,560: 512 k 1.09 times as long, 1,024 k 1.01, 1,536 k 0.96),
+//    two up to 2,048 (4,097 to 8,192 columns: 1.15 at 128 k, 8,192 x 2,048 10.2 and 9.3, 0.96 at 2,560 k).
+//  * 9 to 16 rows in one round of up to 8,192 columns: 256 and 384 k 1.02 to 1.12 times, and beyond 1,024 columns up to 640 k 0.98 to 1.10;
+//    at 9 and 10 rows up to 768 k (1.02 to 1.08), beyond 4,096 columns up to 2,048 k (9 rows of 8,192 x 2,048 10.3 and 9.4).
+//  * 9 to 16 rows in several rounds: two or four column tiles a workgroup (9 rows of 32,000 x 2,048 31.8 and 27.1, 16 rows 31.7 and 29.4; 40,960
+//    columns, two tiles, 1.1 to 1.34 times), three up to 12 rows beyond 1,024 k (18,432 x 2,048 1.08 to 1.15 times); from 11 rows on only
+//    where its stages of 1,024 k are full (16 rows of 28,672 x 1,536 22.0 and 23.2).
+//  * 17 to 32 rows of 2,049 to 4,096 columns: up to 512 k (17 rows 1.03 to 1.16 times), beyond 24 rows 256 k (1.0 to 1.07).
+// An odd multiple of 64 stays: the few-row kernel pads it, and its sums of such inner sizes are further from 64 bits.  So do longer inner sizes, some
+// of which cost up to a tenth more so (9 rows of 28,672 x 4,096 50.3 and 44.0; 48 rows of 5,120 x 5,120 20.0 and 18.2 split): their sums
+// are closer to 64 bits by a quarter and more (1.15e-7 and 1.74e-7 of the result for the latter).
+static bool stripe_few_rows_pay(int M, int N, int K, const StripePlan& plan, bool several_rounds) {
+  if (K > 2048 || (K % 128 && K != 64)) return false;
+  if (M <= 8) return plan.ct == 1 ? K < 1536 : plan.ct == 2;
+  if (K < 256) return false;
+  if (M <= 16) {
+    if (several_rounds) return (M <= 10 ? K >= 512 : K == 512 || K % 1024 == 0) && (plan.ct != 3 || (M <= 12 && K > 1024));
+    if (N > 8192) return false;
+    return K < 512 || (N > 1024 && (K <= 640 || (M <= 10 && K <= (N <= 4096 ? 768 : 2048))));
+  }
+  return M <= 32 && N > 2048 && N <= 4096 && K <= (M <= 24 ? 512 : 256);
+}
 static bool stripe_plan(int M, int N, int K, StripePlan* plan) {
   if (M < 6 || M > 64 || K % 64 || K > T_MAX_INNER) return false;
   const int tiles = (M + 15) / 16;
@@ -2848,6 +2872,7 @@ static bool stripe_plan(int M, int N, int K, StripePlan* plan) {
       const bool one_round = (int64_t)groups_m * stripe_grid_n((N + even - 1) / even, groups_m) <= 256;      // also as the grid is filled up
       *plan = {mt, ct, one_round && (ct >= 3 || tiles == 1) && even > 16 * (ct - 1) && even < 16 * ct ? even : 16 * ct};
     }
+  if (stripe_few_rows_pay(M, N, K, *plan, fewest > 256)) return false;
   if (M <= 8) return fewest <= 256 && N > 2048 && (plan->cols != 16 || K > 4096);
   if (M <= 16) return true;
   int slabs;

@@ -203,3 +203,13 @@ def test_few_rows_of_short_inner_sizes_keep_their_kernel():
                               (16, 1024, 512), (16, 2560, 704), (17, 2048, 256), (25, 4096, 512), (33, 3072, 256), (16, 11264, 2048),
                               (8, 11264, 2048), (64, 2560, 128)):
         assert whole(rows, cols, inner), (rows, cols, inner)
+
+
+def test_norms_of_short_float32_rows_ride_where_a_block_is_one_request():
+    """The float32 product with a norm inside: by whole lines only where a wave has more than the one or two blocks that the other
+    kernel asks for at once."""
+    lines = lambda rows, cols, inner: ops.linear_f32_lines(rows, cols, inner, inner, norm=True)
+    assert not any(lines(rows, cols, inner) for rows in (1, 8, 12) for cols in (64, 2048, 6144) for inner in (64, 256, 512, 640, 768))
+    assert not lines(16, 512, 512) and lines(16, 512, 768) and lines(1, 512, 896) and lines(8, 2048, 2048) and lines(16, 6144, 4096)
+    assert not lines(1, 4096, 1152) and lines(8, 4096, 1152) and lines(1, 4096, 2048) and lines(1, 2048, 1152)
+    assert all(ops.linear_f32_lines(rows, 512, inner, inner) for rows in (1, 16) for inner in (64, 512, 2048))      # without a norm

@@ -2955,7 +2955,11 @@ static int launch_f32_lines_form(const F32RowsNorm& norm, const float* a, const 
 
 // Whether and how the float32 product of at most 16 rows goes by whole lines: 8 columns a workgroup where that still is one round of
 // workgroups over the 256 compute units (pairs of k blocks up to 8 rows), else one to three column tiles (f32_rows_col_tiles), one of as many
-// (even) as make whole rounds of 256 workgroups.  With a norm one column tile.
+// (even) as make whole rounds of 256 workgroups.  With a norm one column tile, and not for the shortest inner sizes, where a wave has one block and
+// gemm_f32_rows_kernel asks for all of it at once (us, that kernel and this one, which takes two steps: 1 row of 256 x 256 4.3 and 6.2, 512 x 512 5.0
+// and 6.0, 768 x 768 6.2 and 6.5, 16 rows 6.6 and 6.4; beyond 2,048 columns, which have no pairs of blocks, 1 row of 4,096 x 1,152 1.08 times as long, 1,536
+// 1.03, 2,048 1.01).  951 such products are 4 % faster on average for it; inner sizes that end just behind a block of 256, as 772 and 1,028, still are up to 1.11
+// times as long as in that kernel.
 struct F32Lines {
   int ct, cw;
   bool pair;
@@ -2963,6 +2967,7 @@ struct F32Lines {
 };
 static bool f32_lines_plan(int M, int N, int K, int64_t lda, bool norm, F32Lines* p) {
   if (M > 16 || lda > FL_MAX_STRIDE || K > FL_MAX_STRIDE) return false;
+  if (norm && (K <= 640 || (K <= 768 && M <= 12) || (M < 8 && N > 2048 && K > 1024 && K <= 1536))) return false;
   const int nkb = (K + F_KBLOCK - 1) / F_KBLOCK;
   const bool eight = (N + 7) / 8 <= 256;
   p->pair = eight && M <= 8;

@@ -1814,3 +1814,20 @@ def test_sums_of_uneven_blocks_meet_in_pairs(M, K):
     # in pairs it is 5 to 8 % less)
     former = {704: 7.65e-8, 832: 8.0e-8, 1088: 8.5e-8, 1984: 1.015e-7}[K]
     assert float((out.cpu().double() - exact).norm() / exact.norm()) <= former
+
+
+@pytest.mark.parametrize("T", [1, 7, 256, 257, 258])
+@pytest.mark.parametrize("K,experts", [(520, 16), (1032, 24), (8, 25), (2056, 32), (520, 33), (1024, 40), (1032, 41), (512, 64)])
+def test_router_of_several_experts_a_wave(T, K, experts):
+    """One, two and four experts of a wave together, the last of them absent, one and four tokens a workgroup: numbers of which every order of
+    addition gives the exact logits, so choice and weights are `moe_route`'s bits."""
+    g = torch.Generator().manual_seed(T + K + experts)
+    a = torch.randint(-3, 4, (T, K), generator=g).to(torch.bfloat16)
+    w = (torch.randint(-3, 4, (experts, K), generator=g) / 64).to(torch.bfloat16)
+    z = (a.double() @ w.double().T).float().to(DEV)
+    got = []
+    for call in (lambda *x: ops().moe_route(z, *x), lambda *x: ops().moe_route_rows(a.to(DEV), w.to(DEV), *x)):
+        ids, wts = torch.full((T, 5), -1, dtype=torch.int32, device=DEV), torch.full((T, 5), -7.0, device=DEV)
+        call(ids, wts)
+        got.append((ids, wts))
+    assert all(torch.equal(x, y) for x, y in zip(*got))

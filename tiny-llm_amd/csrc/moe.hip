@@ -829,47 +829,59 @@ __global__ __launch_bounds__(kThreads) void moe_route_beside_kernel(const float*
 // time, its lanes stride over the inner size, then a butterfly) and the choice, ROWS tokens a workgroup.  A product of 16 columns is no
 // work for the chip: six tokens, 16 experts, inner size 2,048 take 6.9 us as a product and a
 // choice and 4.6 so; 1,944 tokens, for which the tiled product spends a tile of 128 columns on 16, 13.8 and 10.4.  Four tokens a workgroup from 257 on: it fetches the weights (64 KB) once for them.
+// PER experts of a wave go together (the same sums): one after the other, a wave's four experts of 64 are four chains of loads.  Four tokens a
+// workgroup then ask for one chunk at a time, so that a unit holds two workgroups (64 registers).  64 experts of 1,024: 6 tokens 9.1 -> 7.7 us,
+// 1,024 14.7 -> 10.5, 2,048 19.9 -> 14.7; 32 of 2,048: 2,048 tokens 16.7 -> 11.9.
 constexpr int kRouteWaves = 16, kRouteFewRows = 256;
-template <int ROWS>
+template <int ROWS, int PER>
 __global__ __launch_bounds__(kRouteWaves * TL_WAVE) void moe_route_rows_kernel(const bf16_t* __restrict__ a, int64_t a_stride,
                                                                               const bf16_t* __restrict__ w, int n_tokens, int K,
                                                                               RouteOptions o, int32_t* __restrict__ ids,
                                                                               float* __restrict__ wts) {
   __shared__ float z[ROWS][TL_WAVE], s[ROWS][TL_WAVE], gs[ROWS][TL_WAVE], plain[ROWS][TL_WAVE];
   const int lane = threadIdx.x % TL_WAVE, wave = threadIdx.x / TL_WAVE, t0 = blockIdx.x * ROWS;
-  constexpr int kAhead = ROWS == 1 ? 4 : 2, kStep = TL_WAVE * 8;      // chunks of 512 k on their way together
+  constexpr int kAhead = ROWS == 1 ? 4 : PER == 1 ? 2 : 1, kStep = TL_WAVE * 8;      // chunks of 512 k on their way together
   const bf16_t* row[ROWS];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) row[r] = a + (int64_t)min(t0 + r, n_tokens - 1) * a_stride;
-  for (int e = wave; e < o.experts; e += kRouteWaves) {
-    const bf16_t* we = w + (int64_t)e * K;
-    float acc[ROWS];
+  for (int e0 = wave; e0 < o.experts; e0 += kRouteWaves * PER) {
+    const bf16_t* we[PER];
+    float acc[PER][ROWS];
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) acc[r] = 0.f;
+    for (int p = 0; p < PER; ++p) {
+      we[p] = w + (int64_t)min(e0 + p * kRouteWaves, o.experts - 1) * K;
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) acc[p][r] = 0.f;
+    }
     for (int k0 = lane * 8; k0 < K; k0 += kAhead * kStep) {
-      bf16x8 x[ROWS][kAhead], y[kAhead];
+      bf16x8 x[ROWS][kAhead], y[PER][kAhead];
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
         const int k = min(k0 + u * kStep, K - 8);
-        y[u] = *(const bf16x8*)(we + k);
+#pragma unroll
+        for (int p = 0; p < PER; ++p) y[p][u] = *(const bf16x8*)(we[p] + k);
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) x[r][u] = *(const bf16x8*)(row[r] + k);
       }
 #pragma unroll
       for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r)
+        for (int p = 0; p < PER; ++p)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float v = fmaf((float)x[r][u][j], (float)y[u][j], acc[r]);
-            acc[r] = k0 + u * kStep < K ? v : acc[r];
-          }
+          for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float v = fmaf((float)x[r][u][j], (float)y[p][u][j], acc[p][r]);
+              acc[p][r] = k0 + u * kStep < K ? v : acc[p][r];
+            }
     }
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-      const float v = wave_sum(acc[r]);
-      if (lane == 0) z[r][e] = v;
-    }
+    for (int p = 0; p < PER; ++p)
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const float v = wave_sum(acc[p][r]);
+        if (lane == 0 && e0 + p * kRouteWaves < o.experts) z[r][e0 + p * kRouteWaves] = v;
+      }
   }
   __syncthreads();
   if (wave >= ROWS || t0 + wave >= n_tokens) return;
@@ -1125,12 +1137,19 @@ int tl_moe_route_rows(const void* a, int64_t a_stride, const void* w, const floa
   if (experts > TL_WAVE || !route_ok(o) || K <= 0 || K % 8 || a_stride % 8 || a_stride < K || !a || !w || !ids || !wts ||
       (((uintptr_t)a | (uintptr_t)w) & 15))
     return TL_ERR_ARG;
-  if (n_tokens <= kRouteFewRows)
-    hipLaunchKernelGGL(moe_route_rows_kernel<1>, dim3(n_tokens), dim3(kRouteWaves * TL_WAVE), 0, stream, (const bf16_t*)a, a_stride,
-                       (const bf16_t*)w, n_tokens, K, o, ids, wts);
-  else
-    hipLaunchKernelGGL(moe_route_rows_kernel<4>, dim3((n_tokens + 3) / 4), dim3(kRouteWaves * TL_WAVE), 0, stream, (const bf16_t*)a,
-                       a_stride, (const bf16_t*)w, n_tokens, K, o, ids, wts);
+#define TL_ROUTE(ROWS, PER)                                                                                                        \
+  hipLaunchKernelGGL((moe_route_rows_kernel<ROWS, PER>), dim3((n_tokens + ROWS - 1) / ROWS), dim3(kRouteWaves * TL_WAVE), 0, stream, \
+                     (const bf16_t*)a, a_stride, (const bf16_t*)w, n_tokens, K, o, ids, wts)
+  if (n_tokens <= kRouteFewRows) {      // (between 33 and 40 experts, and up to 24, the share that most waves would not have costs more)
+    if (experts > 40) TL_ROUTE(1, 4);
+    else if (experts > 24 && experts <= 32) TL_ROUTE(1, 2);
+    else TL_ROUTE(1, 1);
+  } else {
+    if (experts > 32) TL_ROUTE(4, 4);
+    else if (experts > 16) TL_ROUTE(4, 2);
+    else TL_ROUTE(4, 1);
+  }
+#undef TL_ROUTE
   return tl_launch_status();
 }
 

@@ -2599,9 +2599,12 @@ def moe_route_rows_ok(dtype: torch.dtype, experts: int, inner: int) -> bool:
 
 
 def moe_route_rows_pay(rows: int, experts: int, inner: int) -> bool:
-    """Where one kernel is faster than the product and `moe_route`: every workgroup of it fetches the weights, so up to 64 K of them,
-    and not for the longest prompts (16 experts of 2,048: 6 rows 6.9 -> 4.6 us, 256 10.4 -> 4.9, 1,944 13.8 -> 10.4, 4,096 17.7 and
-    18.0; 64 experts of 4,096: 6 rows 10.8 and 15.1)."""
+    """Where one kernel is used instead of the product and `moe_route`: every workgroup of it fetches the weights, so up to 64 K of them,
+    and not for the longest prompts (4,096 rows of 16 experts and 2,048 inner elements 17.7 us and 18.0).  Both timed at 58 sizes of 4 to 64 experts
+    and 256 to 8,192 inner elements and 13 numbers of rows (us, both and one): 6 rows of 16 x 2,048 6.4 and 4.0, of 64 x 1,024 7.9 and
+    7.8; 1,024 rows of 64 x 1,024 13.7 and 9.7; 2,048 of 16 x 2,048 13.1 and 9.6, of 32 x 2,048 13.7 and 11.9, of 64 x 1,024 14.9 and 14.8.  It is the
+    slower one for 40 experts and more of 256 inner elements (1.05 to 1.13 times) and beyond 256 rows of 8,192 (1.1 to 1.5 times): its weights
+    are closer to 64 bits (0.95e-7, by both 1.05e-7 to 1.3e-7), so it stays there too."""
     return experts * inner <= 1 << 16 and rows <= 2048
 
 

@@ -617,3 +617,20 @@ def test_runs_of_decode_steps_in_a_window_group():
     # after the commit only the window's blocks are held: positions 23.. -> logical blocks 5 and 6
     assert [b != RELEASED for b in cm.block_table("a", 1)] == [False] * 5 + [True] * 2
     assert cm.free_blocks() == [20 - 7, 6 - 2]
+
+
+def test_state_rows_go_in_one_launch_on_their_own_device_only(monkeypatch):
+    """The kernel for many tensors' rows runs on the current device: states of another one are cleared and copied by torch, which
+    goes by each tensor's own."""
+    from types import SimpleNamespace
+
+    import torch
+
+    def states(index, size=4, dense=True):
+        return [SimpleNamespace(is_cuda=True, device=torch.device("cuda", index), element_size=lambda: size, is_contiguous=lambda: dense)] * 3
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    assert CacheManager._one_launch(states(0), 64)
+    assert not CacheManager._one_launch(states(1), 1) and not CacheManager._one_launch(states(0) + states(1), 1)
+    assert not CacheManager._one_launch(states(0), 65) and not CacheManager._one_launch(states(0, size=2), 1)
+    assert not CacheManager._one_launch(states(0, dense=False), 1) and not CacheManager._one_launch([torch.zeros(2, 3)], 1)

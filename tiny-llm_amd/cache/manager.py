@@ -175,10 +175,16 @@ class CacheManager:
     def free_slots(self) -> int:
         return len(self._free_slots)
 
+    @staticmethod
+    def _one_launch(states: Sequence[torch.Tensor], rows: int) -> bool:
+        """Whether the kernel takes these tensors: it runs on the current device, so only theirs will do."""
+        return (states[0].is_cuda and rows <= 64 and all(t.element_size() == 4 and t.is_contiguous() for t in states)
+                and all(t.device.index == torch.cuda.current_device() for t in states))
+
     def _rows(self, slots: Sequence[int], save: bool = False):
         """The state rows of `slots` in every tensor: cleared, or copied ({owner: [slots, ...]}); on the device one launch for all."""
         states = list(self.states.values())
-        if states[0].is_cuda and len(slots) <= 64 and all(t.element_size() == 4 and t.is_contiguous() for t in states):
+        if self._one_launch(states, len(slots)):
             from ..kernels import ops
             copies = ops.tensor_rows(states, slots, save)
             return dict(zip(self.states, copies)) if save else None

@@ -419,7 +419,8 @@ def test_linear_f32_tiles_cut_to_fit(M, N, K):
 @pytest.mark.parametrize("K,N", [(5632, 2048), (2048, 4100), (1096, 518), (2048, 2046), (256, 2560), (4096, 6144)])
 def test_linear_split_k(M, K, N):
     """Products with few output tiles split their inner size over workgroups and add the parts up
-    in a second kernel, which also applies every epilogue and both sides of the norm hand-off."""
+    in a second kernel, which also applies every epilogue and both sides of the norm hand-off.  (Up to 64 rows `split_k` says the
+    same of these sizes, but `linear` keeps their inner size whole; `test_linear_split_k_of_up_to_64_rows` has sizes that are split.)"""
     g = torch.Generator().manual_seed(M + K + N)
     a = torch.randn(M, K, generator=g).to(torch.bfloat16)
     w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
@@ -434,7 +435,7 @@ def test_linear_split_k(M, K, N):
     else:
         must_split = K >= 512 and few_tiles
     if must_split:
-        assert splits > 1                     # these sizes are here because they are split
+        assert splits > 1                     # these sizes are here because they are split (beyond 64 rows)
     out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
     ops().linear(a.to(DEV), w.to(DEV), out)
     assert rel(out, ref) < 6e-3
@@ -1579,7 +1580,7 @@ def test_the_clamped_epilogue_is_told_its_limit():
 @pytest.mark.parametrize("N,K", [(2, 64), (46, 192), (518, 704), (2046, 128), (2560, 2048), (4100, 1088), (30000, 64), (33000, 128)])
 def test_linear_whole_inner_size(M, N, K):
     """6 to 64 rows: every cut of the rows and columns, both lengths of block, fewer blocks than waves, columns that end within a
-    group of four, rows that are gathered, and both sides of the norm hand-off."""
+    group of four, rows that are gathered, and both sides of the norm hand-off.  (One sum a tile at these inner sizes; the next test has two.)"""
     g = torch.Generator().manual_seed(M + N + K)
     assert ops().linear_whole(M, N, K) or M < 9
     wide = torch.randn(M + 40, K + 8, generator=g).to(torch.bfloat16)      # rows with other numbers behind them
@@ -1831,3 +1832,107 @@ def test_router_of_several_experts_a_wave(T, K, experts):
         call(ids, wts)
         got.append((ids, wts))
     assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 16384, 2112), (16, 1030, 2112), (9, 2560, 4096), (17, 4100, 2176), (32, 518, 2304), (33, 2046, 2112), (33, 4096, 4096),
+                                   (48, 5120, 2240), (64, 4608, 2304), (17, 16384, 2112)])
+def test_linear_whole_inner_size_in_two_sums(M, N, K):
+    """Inner sizes beyond 2,048: two sums a tile (one to four tiles a workgroup, four column tiles of few rows among them), by both lengths
+    of block, and one where the registers do not allow two."""
+    assert ops().linear_whole(M, N, K)
+    test_linear_whole_inner_size(M, N, K)
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 14336, 4096), (50, 13824, 5120), (64, 14336, 4096), (48, 12096, 1776)])
+def test_linear_split_k_of_up_to_64_rows(M, K, N):
+    """Long inner sizes with few columns: up to 64 rows they are split too, a single slab of rows in the ring kernel."""
+    assert ops().split_k(M, N, K) > 1 and not ops().linear_whole(M, N, K)
+    test_linear_split_k(M, K, N)
+
+
+@pytest.mark.parametrize("M,K,cols", [(6, 2048, (2048, 2048, 2048, 2048, 64)), (16, 704, (1200, 1200, 1200, 1200, 1198)), (13, 256, (2050, 2050, 2050, 70)),
+                                      (1, 192, (2500, 2500, 2500, 2500, 33)), (9, 128, (4096, 4096, 4096, 4096, 4096, 10)), (16, 2112, (1030, 66))])
+def test_linear_set_by_whole_lines(M, K, cols):
+    """Sets of one, two and three column tiles a workgroup (8 to 48 columns), by both lengths of block, and sets too wide for one round; the last,
+    often far narrower than the others, leaves tanh: the bits of the product in float32 and `tanh_rows`; nothing beyond is written."""
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    sets, whole, plain_sets = [], [], []
+    for i, n in enumerate(cols):
+        a, w = rnd(M, K + 8).bfloat16()[:, :K], (rnd(n, K) / math.sqrt(K)).bfloat16()
+        full = torch.full((M, n + 3), 7.0, device=DEV, dtype=torch.bfloat16 if i + 1 == len(cols) else torch.float32)
+        whole.append(full)
+        sets.append((a, w, full[:, :n]))
+        plain_sets.append((a, w, torch.empty(M, n, device=DEV)))
+    ops().linear_set(sets)
+    ops().linear_set(plain_sets)
+    for (a, w, out), full, (_, _, sums) in zip(sets, whole, plain_sets):
+        n = out.shape[1]
+        want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+        assert ((sums.double() - want).abs() <= K * 2.0 ** -24 * size).all()
+        if out.dtype == torch.float32:
+            assert torch.equal(out, sums)
+        else:
+            assert torch.equal(out, ops().tanh_rows(sums, torch.empty(M, n, dtype=torch.bfloat16, device=DEV)))
+        assert (full[:, n:] == 7.0).all()
+
+
+def test_input_rows_far_apart():
+    """Input rows more than 2^20 elements apart, beyond the offsets of the kernel of whole lines: the bits of rows side by side."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    far = torch.empty(17, (1 << 20) + 8, dtype=torch.bfloat16, device=DEV)[:, :704]
+    near = torch.randn(17, 704, device=DEV, generator=g).bfloat16()
+    far.copy_(near)
+    w, res = (torch.randn(2048, 704, device=DEV, generator=g) / 27).bfloat16(), torch.randn(17, 2048, device=DEV, generator=g)
+    nw, rows = torch.rand(2048, device=DEV, generator=g), torch.arange(16, 4, -1, dtype=torch.int32, device=DEV)
+    got = []
+    for a in (near, far):
+        x, y, z = res.clone(), torch.empty(12, 2048, device=DEV), torch.empty(9, 2048, dtype=torch.bfloat16, device=DEV)
+        operand, sumsq = torch.empty(17, 2048, dtype=torch.bfloat16, device=DEV), torch.empty(17, ops().handoff_parts(17, 2048, 704), device=DEV)
+        ops().linear_handoff(a, w, x, x, emit=(nw, operand, sumsq))
+        ops().linear_handoff(a, w, y, rows=rows)
+        ops().linear(a[:9], w, z)
+        got.append((x, operand, sumsq, y, z))
+    assert all(torch.equal(p, q) for p, q in zip(*got))
+    exact = near.double() @ w.double().T
+    assert rel(got[1][0], exact + res.double()) < 1e-5 and rel(got[1][3], exact[rows.long()]) < 1e-5
+    out = [torch.empty(17, 300, device=DEV)[:6] for _ in range(2)]
+    for a, o in zip((near, far), out):
+        ops().linear_set([(a[:6], w[:300], o)])
+        assert rel(o, exact[:6, :300]) < 1e-5
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("K,N", [(700, 100), (900, 3000), (2052, 5000), (1028, 2304)])
+def test_few_float32_rows_ignore_what_lies_behind_them(M, K, N):
+    """The float32 kernel of whole lines reads on behind a row's end where an inner size ends within a block: numbers there that are not finite,
+    and those at the start of the next weight row, stay out of a row's results; a row and a column of such numbers keep to themselves."""
+    g = torch.Generator(device=DEV).manual_seed(M + K + N)
+    wide = torch.full((M, K + 260), float("nan"), device=DEV)
+    wide[:, K + 8:] = float("inf")
+    wide[:, :K] = torch.randn(M, K, device=DEV, generator=g)
+    a, w = wide[:, :K], torch.randn(N, K, device=DEV, generator=g) / math.sqrt(K)
+    nw = torch.rand(K, device=DEV, generator=g) + 0.5
+    calls = [lambda x, w, o: ops().linear(x, w, o)]
+    if ops().linear_norm_f32_ok(M, N, K, a.stride(0)):
+        calls.append(lambda x, w, o: ops().linear_norm_f32(x, nw, 1e-5, w, o))
+    assert ops().linear_f32_lines(M, N, K, a.stride(0))
+    bad_w = w.clone()
+    bad_w[N // 2, :4] = float("inf")       # the first numbers of a weight row: behind the end of the row ahead of it
+    bad_a = wide.clone()[:, :K]
+    bad_a[M // 2, :4] = float("nan")
+    columns, rows = torch.arange(N, device=DEV) != N // 2, torch.arange(M, device=DEV) != M // 2
+    for call in calls:
+        out, bad = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+        call(a, w, out)
+        assert torch.isfinite(out).all()
+        call(a.contiguous(), w, bad)
+        assert torch.equal(out, bad)
+        call(a, bad_w, bad)
+        assert torch.equal(bad[:, columns], out[:, columns]) and not torch.isfinite(bad[:, N // 2]).any()
+        call(bad_a, w, bad)
+        assert torch.equal(bad[rows], out[rows]) and not torch.isfinite(bad[M // 2]).any()
+    want = a.double() @ w.double().T
+    out = torch.empty(M, N, device=DEV)
+    ops().linear(a, w, out)
+    assert ((out.double() - want).abs() <= (K + 3) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all()

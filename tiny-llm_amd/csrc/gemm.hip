@@ -707,11 +707,10 @@ __global__ __launch_bounds__(FR_THREADS) void gemm_f32_rows_kernel(const F32Rows
 // CT (one row tile only): a workgroup owns CT column tiles side by side.  The activations of a k block,
 // which weigh as much as one tile's weights, are fetched once for all of them, and a wide product
 // (gate and up, the output head) becomes one or two rounds of workgroups instead of three to eight.
-// The weights come as a chain of pieces, the block's tiles and then the wave's next block, each
-// requested while the piece before it is multiplied.  A tile's block sums are what they are with one
-// tile a workgroup, bit for bit.
+// Each tile's next half block is requested as soon as this one has left its registers for LDS.  A tile's block sums are what they are
+// with one tile a workgroup, bit for bit.
 //
-// PAIR (8 columns, at most 8 rows, no norm): the matrix tile of 16 x 16 then holds two k blocks at
+// PAIR (8 columns, at most 8 rows): the matrix tile of 16 x 16 then holds two k blocks at
 // once.  Operand rows 0 to 7 are the 8 columns (and the 8 activation rows) at the k of one block, rows
 // 8 to 15 the same columns and rows at the k of the next; the two diagonal 8 x 8 blocks of the result
 // are the two block sums, each accumulated from zero in the order it has everywhere else, and the
@@ -1781,7 +1780,8 @@ __global__ __launch_bounds__(O_THREADS) void gemm_oneshot_bf16_kernel(const bf16
   }
 }
 
-// Whether and how this kernel takes a product of 17 to 64 rows: slabs of 64 k per split (0: not this
+// Whether and how this kernel takes a product of 17 to 64 rows that is split at all (stripe_plan, which compares its time
+// with this estimate, keeps most of them whole): slabs of 64 k per split (0: not this
 // kernel).  The number of splits with the smallest estimated time: rounds of workgroups over the 256
 // compute units, each as long as a workgroup takes to fetch its share (about 35 GB/s), and the second
 // kernel's reading of the partial sums.
@@ -2744,6 +2744,8 @@ __global__ __launch_bounds__(S_THREADS) void gemm_stripe_bf16_kernel(const Skinn
 // Several products of up to 16 rows that do not wait for each other as ONE launch (SkinnySet): blockIdx.y names the product, a
 // workgroup owns up to 16 CT of its columns.  Five products of a decode step's six rows (four of 2,048 columns and one of 64, inner size 2,048)
 // take 21.8 us as launches of their own, 11.9 in gemm_skinny_set_kernel (16 columns, two rounds of workgroups) and 9.6 so (36 columns, one round).
+// Of 40 sets at 1 to 16 rows (inner sizes of 256 to 4,096) it takes 0.52 to 1.0 times as long for all but a few: inner size 256, 1.0 to 1.05
+// times 2.7 us, up to 6 rows of 1,024 + 256 + 256 columns 1.04 to 1.08 times 4.3, of five times 4,096 by 2,048 1.05 to 1.09 times 20.
 template <int CT, int TK>
 __global__ __launch_bounds__(S_THREADS) void gemm_stripe_set_kernel(const SkinnySet set) {
   stripe_product<1, CT, TK, 1, float, 0, false, true>(set.p[blockIdx.y], 0, set.vec, blockIdx.x, 0);
@@ -2821,7 +2823,7 @@ static int launch_stripe_tile(const SkinnyArgs& p, hipStream_t stream) {
 // the smallest sum of both, times the rounds of workgroups that it makes over the 256 units.  Timed for fifteen matrices of 1,024 x 704 to
 // 27,648 x 5,120 at 17, 32, 48 and 64 rows, every cut of each (1,270 in all): the one this picks is within 3 % of the fastest, 0.05 % on average.
 //  * Beyond 16 rows the estimate (us) is compared with the split product's own (oneshot_us; 4 us for its second launch), which is the
-//    faster way for long inner sizes and few columns: 64 rows of 14,336 by 4,096 37.4 us here and 29.9 split; 5,120 x 5,120 19.0 and 19.7.
+//    faster way for long inner sizes and few columns: 64 rows of 14,336 by 4,096 37.4 us here and 29.9 split; 5,120 x 5,120 20.4 and 19.9.
 //  * 6 to 8 rows: in one round, where the few-row kernel has no form of eight columns and a workgroup's columns are not just one
 //    tile of a short inner size (8 rows: 2,560 x 2,048 5.2 -> 4.7, 11,264 x 2,048 12.1 -> 11.6, 6,144 x 4,096 13.1 -> 11.7, 4,096 x
 //    14,336 28.9 -> 25.2, but 4,096 x 4,096 9.7 and 10.0, 2,048 x 2,048 4.6 both).  At 1 row the few-row kernel is the faster one.
@@ -3369,9 +3371,9 @@ int tl_linear_whole(int M, int N, int K) {
   return stripe_plan(M, N, K, &plan) ? 1 : 0;
 }
 
-// How many partial sums of squares per row tl_linear_handoff writes as a producer for these sizes
-// (few rows: one per workgroup, per 16 columns, or per 8 where workgroups own 8; beyond: one per 64
-// columns).
+// How many partial sums of squares per row tl_linear_handoff writes as a producer for these sizes: by whole lines one per workgroup,
+// whose columns are stripe_plan's (any multiple of 4 from 8 to 64); other products of up to 64 rows one per workgroup and column
+// tile (8 or 16 columns, or as many as make whole rounds); beyond 64 rows one per 64 columns.
 int tl_handoff_parts(int M, int N, int K) {
   if (M > 64) return (N + 63) / 64;
   StripePlan plan;

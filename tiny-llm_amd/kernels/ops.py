@@ -464,7 +464,7 @@ FEW_ROWS = 64   # most rows the few-row product takes
 def split_k(rows: int, cols: int, inner: int) -> int:
     """Into how many parts the bfloat16 product [rows, inner] x [cols, inner]^T has its inner size
     split over workgroups (1: not at all): products with few output tiles and more rows than the
-    few-row kernel likes."""
+    few-row kernel likes.  (Up to 64 rows `linear_whole` comes first.)"""
     if inner % 8:
         return 1
     key = (rows, cols, inner)
@@ -499,7 +499,7 @@ def _near_rows(a: torch.Tensor, whole: bool) -> torch.Tensor:
 
 def can_hand_off(rows: int, width: int, inner: int, dtype: torch.dtype) -> bool:
     """Whether `linear_handoff` can prepare a norm over `width` columns for `rows` rows, as the
-    epilogue of the product with inner size `inner`: the few-row kernel, a product whose inner
+    epilogue of the product with inner size `inner`: the kernels for up to 64 rows, a product whose inner
     size is split, or the tiled kernel where the width is a multiple of 64."""
     if dtype != torch.bfloat16 or rows <= 0 or width % 8 or inner % 8:
         return False
@@ -508,7 +508,8 @@ def can_hand_off(rows: int, width: int, inner: int, dtype: torch.dtype) -> bool:
 
 def handoff_parts(rows: int, width: int, inner: int) -> int:
     """How many partial sums of squares per row the product [rows, inner] x [width, inner]^T writes
-    when it prepares a norm: one per workgroup in the few-row kernel (16 or 8 columns), per 1024
+    when it prepares a norm: up to 64 rows one per workgroup (by whole lines, `linear_whole`, any multiple of 4 columns from 8
+    to 64; in the few-row kernel 8 or 16, or as many as make whole rounds), one per 1024 columns
     after a split inner size, per 64 in the tiled kernel."""
     if split_k(rows, width, inner) > 1 and not linear_whole(rows, width, inner):
         return (width + 1023) // 1024
@@ -549,8 +550,9 @@ def linear_handoff(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, residual
     and the sums of out^2 over groups of columns.  prepared = (sumsq [R, P], eps, width): `a` is
     such an operand ([R, K]; `rows` picks rows of both) and the product is multiplied by
     1 / sqrt(sum(sumsq[row]) / width + eps): together the two are rmsnorm(out) @ w.T.
-    At most 64 rows go to the few-row kernel, a product whose inner size is split (`split_k`) to
-    its two kernels, any other to the tiled kernel (no `rows` then; emitting needs N % 64 == 0)."""
+    6 to 64 rows go by whole lines where `linear_whole` says so, a product whose inner size is split (`split_k`, beyond 16 rows and
+    not `rows`) to its two kernels, others of up to 64 rows to the few-row kernel, and any other to the tiled kernel (no `rows` then;
+    emitting needs N % 64 == 0)."""
     _dev(a, w, out, residual, rows)
     _rows_2d(a, "linear input")
     _rows_2d(out, "linear output")

@@ -627,7 +627,7 @@ def test_state_rows_go_in_one_launch_on_their_own_device_only(monkeypatch):
     import torch
 
     def states(index, size=4, dense=True):
-        return [SimpleNamespace(is_cuda=True, device=torch.device("cuda", index), element_size=lambda: size, is_contiguous=lambda: dense)] * 3
+        return [SimpleNamespace(is_cuda=True, get_device=lambda: index, element_size=lambda: size, is_contiguous=lambda: dense)] * 3
 
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     assert CacheManager._one_launch(states(0), 64)

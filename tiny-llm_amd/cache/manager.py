@@ -178,8 +178,10 @@ class CacheManager:
     @staticmethod
     def _one_launch(states: Sequence[torch.Tensor], rows: int) -> bool:
         """Whether the kernel takes these tensors: it runs on the current device, so only theirs will do."""
-        return (states[0].is_cuda and rows <= 64 and all(t.element_size() == 4 and t.is_contiguous() for t in states)
-                and all(t.device.index == torch.cuda.current_device() for t in states))
+        if not states[0].is_cuda or rows > 64:
+            return False
+        here = torch.cuda.current_device()
+        return all(t.element_size() == 4 and t.is_contiguous() and t.get_device() == here for t in states)
 
     def _rows(self, slots: Sequence[int], save: bool = False):
         """The state rows of `slots` in every tensor: cleared, or copied ({owner: [slots, ...]}); on the device one launch for all."""
